@@ -14,9 +14,11 @@
 // Parameters, flat, row-major [out][in]: W1, b1, W2, b2, W3, b3.
 // Loss: L = 1/(2B) * sum_b sum_o (y_bo - t_bo)^2.
 //
-// Sizes are tiny (din <= 256, h <= 128, dout <= 8); one block per sample for
-// the per-sample passes, one thread per parameter for the batch reductions
-// (deterministic sums, no float atomics).
+// Sizes are tiny (din <= 256, h <= 128, dout <= 8), so latency bounds every
+// kernel: one block per sample for the per-sample passes, one block per
+// output neuron for the batch reductions (deterministic sums, no float
+// atomics).  A gradient of 256 samples is two launches and 27 us with its
+// synchronisation (four launches and 100 us before).
 
 #include <hip/hip_runtime.h>
 
@@ -46,110 +48,188 @@ struct MlpDims {
   __host__ __device__ size_t total() const { return b3() + dout; }
 };
 
-// Forward pass, one block (kMaxHidden threads) per sample.  Keeps the
-// activations for the backward pass when a1/a2 are given.
-__global__ void __launch_bounds__(kMaxHidden) k_mlp_fwd(MlpDims d, int B, const float* __restrict__ X,
-                                                        const float* __restrict__ P, float* __restrict__ A1,
-                                                        float* __restrict__ A2, float* __restrict__ Y) {
-  __shared__ float x[kMaxIn], a1[kMaxHidden], a2[kMaxHidden];
-  const int b = blockIdx.x, j = threadIdx.x;
-  if (b >= B) return;
-  for (int i = j; i < d.din; i += blockDim.x) x[i] = X[(size_t)b * d.din + i];
-  __syncthreads();
-  if (j < d.h) {
-    const float* w = P + d.w1() + (size_t)j * d.din;
-    float z = P[d.b1() + j];
-    for (int i = 0; i < d.din; i++) z = fmaf(w[i], x[i], z);
-    a1[j] = tanhf(z);
-    if (A1) A1[(size_t)b * d.h + j] = a1[j];
-  }
-  __syncthreads();
-  if (j < d.h) {
-    const float* w = P + d.w2() + (size_t)j * d.h;
-    float z = P[d.b2() + j];
-    for (int i = 0; i < d.h; i++) z = fmaf(w[i], a1[i], z);
-    a2[j] = tanhf(z);
-    if (A2) A2[(size_t)b * d.h + j] = a2[j];
-  }
-  __syncthreads();
-  if (j < d.dout) {
-    const float* w = P + d.w3() + (size_t)j * d.h;
-    float z = P[d.b3() + j];
-    for (int i = 0; i < d.h; i++) z = fmaf(w[i], a2[i], z);
-    Y[(size_t)b * d.dout + j] = z;
+// A sample is one block of kMlpThreads threads.  Four threads share each dot
+// product (lane groups of four read consecutive weights of a row; partial
+// sums added by two shuffles): a row is 72 or 64 weights, so a thread's
+// chain is 18 fused multiply-adds with their loads in flight together, where
+// a thread per row waited on 72.
+constexpr int kMlpThreads = 256;
+constexpr int kDotLanes = 4;
+
+// z[j] = bias[j] + sum_i W[j][i] in[i] for every j < nout, then f(j, z).
+template <class F>
+__device__ inline void dense_rows(const float* __restrict__ W, const float* __restrict__ bias, const float* in, int nin,
+                                  int nout, F&& f) {
+  const int q = threadIdx.x % kDotLanes;
+  for (int j = threadIdx.x / kDotLanes; j < nout; j += kMlpThreads / kDotLanes) {
+    const float* w = W + (size_t)j * nin;
+    float z = 0.f;
+#pragma unroll 6
+    for (int i = q; i < nin; i += kDotLanes) z = fmaf(w[i], in[i], z);
+    z += __shfl_xor(z, 1);
+    z += __shfl_xor(z, 2);
+    if (q == 0) f(j, z + bias[j]);
   }
 }
 
-// Per-sample deltas: D3 = dL/dz3 = (y - t)/B, D2 = (W3^T D3) * (1 - a2^2),
-// D1 = (W2^T D2) * (1 - a1^2); per-sample loss terms.
-__global__ void __launch_bounds__(kMaxHidden) k_mlp_delta(MlpDims d, int B, const float* __restrict__ T,
-                                                          const float* __restrict__ P,
-                                                          const float* __restrict__ A1,
-                                                          const float* __restrict__ A2,
-                                                          const float* __restrict__ Y, float* __restrict__ D1,
-                                                          float* __restrict__ D2, float* __restrict__ D3,
-                                                          float* __restrict__ lossb) {
-  __shared__ float d3[kMaxOut], d2[kMaxHidden];
-  const int b = blockIdx.x, j = threadIdx.x;
+// Activations and output of one sample, in LDS (x already there).
+__device__ inline void forward_sample(const MlpDims& d, const float* __restrict__ P, const float* x, float* a1,
+                                      float* a2, float* y) {
+  dense_rows(P + d.w1(), P + d.b1(), x, d.din, d.h, [&](int j, float z) { a1[j] = tanhf(z); });
+  __syncthreads();
+  dense_rows(P + d.w2(), P + d.b2(), a1, d.h, d.h, [&](int j, float z) { a2[j] = tanhf(z); });
+  __syncthreads();
+  dense_rows(P + d.w3(), P + d.b3(), a2, d.h, d.dout, [&](int j, float z) { y[j] = z; });
+  __syncthreads();
+}
+
+// Forward pass, one block per sample.
+__global__ void __launch_bounds__(kMlpThreads) k_mlp_fwd(MlpDims d, int B, const float* __restrict__ X,
+                                                         const float* __restrict__ P, float* __restrict__ Y) {
+  __shared__ float x[kMaxIn], a1[kMaxHidden], a2[kMaxHidden], y[kMaxOut];
+  const int b = blockIdx.x;
   if (b >= B) return;
-  if (j == 0) {
-    float l = 0.f;
-    for (int o = 0; o < d.dout; o++) {
-      float e = Y[(size_t)b * d.dout + o] - T[(size_t)b * d.dout + o];
-      d3[o] = e / (float)B;
-      D3[(size_t)b * d.dout + o] = d3[o];
-      l = fmaf(e, e, l);
-    }
-    lossb[b] = 0.5f * l / (float)B;
+  for (int i = threadIdx.x; i < d.din; i += kMlpThreads) x[i] = X[(size_t)b * d.din + i];
+  __syncthreads();
+  forward_sample(d, P, x, a1, a2, y);
+  if ((int)threadIdx.x < d.dout) Y[(size_t)b * d.dout + threadIdx.x] = y[threadIdx.x];
+}
+
+// Forward and backward of one sample: activations A1, A2, deltas D3 =
+// dL/dz3 = (y - t)/B, D2 = (W3^T D3) * (1 - a2^2), D1 = (W2^T D2) *
+// (1 - a1^2), and the sample's loss term.  One launch instead of a forward
+// and a delta kernel (6.6 + 5.2 us at 256 samples, and the gap between):
+// the deltas need nothing but this sample's activations, which stay in LDS.
+__global__ void __launch_bounds__(kMlpThreads) k_mlp_sample(MlpDims d, int B, const float* __restrict__ X,
+                                                            const float* __restrict__ T, const float* __restrict__ P,
+                                                            float* __restrict__ A1, float* __restrict__ A2,
+                                                            float* __restrict__ D1, float* __restrict__ D2,
+                                                            float* __restrict__ D3, float* __restrict__ lossb) {
+  constexpr int kWaves = kMlpThreads / 64;
+  __shared__ float x[kMaxIn], a1[kMaxHidden], a2[kMaxHidden], y[kMaxOut], d3[kMaxOut], d2[kMaxHidden];
+  __shared__ float part[kWaves][64];
+  const int b = blockIdx.x, tid = threadIdx.x;
+  if (b >= B) return;
+  for (int i = tid; i < d.din; i += kMlpThreads) x[i] = X[(size_t)b * d.din + i];
+  __syncthreads();
+  forward_sample(d, P, x, a1, a2, y);
+  for (int j = tid; j < d.h; j += kMlpThreads) {
+    A1[(size_t)b * d.h + j] = a1[j];
+    A2[(size_t)b * d.h + j] = a2[j];
+  }
+  if (tid < d.dout) {
+    const float e = y[tid] - T[(size_t)b * d.dout + tid];
+    y[tid] = e;
+    d3[tid] = e / (float)B;
+    D3[(size_t)b * d.dout + tid] = d3[tid];
   }
   __syncthreads();
-  if (j < d.h) {
+  if (tid == 0) {
+    float l = 0.f;
+    for (int o = 0; o < d.dout; o++) l = fmaf(y[o], y[o], l);
+    lossb[b] = 0.5f * l / (float)B;
+  }
+  for (int j = tid; j < d.h; j += kMlpThreads) {
     float s = 0.f;
     for (int o = 0; o < d.dout; o++) s = fmaf(P[d.w3() + (size_t)o * d.h + j], d3[o], s);
-    float a = A2[(size_t)b * d.h + j];
-    d2[j] = s * (1.f - a * a);
+    d2[j] = s * (1.f - a2[j] * a2[j]);
     D2[(size_t)b * d.h + j] = d2[j];
   }
   __syncthreads();
-  if (j < d.h) {
+  // a column of W2 per lane, its rows split over the waves
+  const int lane = tid & 63, w = tid >> 6;
+  for (int j0 = 0; j0 < d.h; j0 += 64) {
+    const int j = j0 + lane;
     float s = 0.f;
-    for (int o = 0; o < d.h; o++) s = fmaf(P[d.w2() + (size_t)o * d.h + j], d2[o], s);
-    float a = A1[(size_t)b * d.h + j];
-    D1[(size_t)b * d.h + j] = s * (1.f - a * a);
-  }
-}
-
-// Gradient of every parameter, summed over the batch in sample order:
-// dW[o][i] = sum_b D[b][o] * in[b][i], db[o] = sum_b D[b][o].
-__global__ void k_mlp_grad(MlpDims d, int B, const float* __restrict__ X, const float* __restrict__ A1,
-                           const float* __restrict__ A2, const float* __restrict__ D1,
-                           const float* __restrict__ D2, const float* __restrict__ D3, float* __restrict__ G) {
-  const size_t n = d.total();
-  for (size_t p = (size_t)blockIdx.x * blockDim.x + threadIdx.x; p < n; p += (size_t)gridDim.x * blockDim.x) {
-    const float *Dv, *In;
-    int nout, nin, o, i;
-    bool bias;
-    if (p < d.b1()) { Dv = D1; In = X; nout = d.h; nin = d.din; o = (int)(p / d.din); i = (int)(p % d.din); bias = false; }
-    else if (p < d.w2()) { Dv = D1; In = nullptr; nout = d.h; nin = 0; o = (int)(p - d.b1()); i = 0; bias = true; }
-    else if (p < d.b2()) { size_t q = p - d.w2(); Dv = D2; In = A1; nout = d.h; nin = d.h; o = (int)(q / d.h); i = (int)(q % d.h); bias = false; }
-    else if (p < d.w3()) { Dv = D2; In = nullptr; nout = d.h; nin = 0; o = (int)(p - d.b2()); i = 0; bias = true; }
-    else if (p < d.b3()) { size_t q = p - d.w3(); Dv = D3; In = A2; nout = d.dout; nin = d.h; o = (int)(q / d.h); i = (int)(q % d.h); bias = false; }
-    else { Dv = D3; In = nullptr; nout = d.dout; nin = 0; o = (int)(p - d.b3()); i = 0; bias = true; }
-    float s = 0.f;
-    for (int b = 0; b < B; b++) {
-      float dv = Dv[(size_t)b * nout + o];
-      s = bias ? s + dv : fmaf(dv, In[(size_t)b * nin + i], s);
+    if (j < d.h) {
+#pragma unroll 8
+      for (int o = w; o < d.h; o += kWaves) s = fmaf(P[d.w2() + (size_t)o * d.h + j], d2[o], s);
     }
-    G[p] = s;
+    part[w][lane] = s;
+    __syncthreads();
+    if (w == 0 && j < d.h) {
+      for (int v = 1; v < kWaves; v++) s += part[v][lane];
+      D1[(size_t)b * d.h + j] = s * (1.f - a1[j] * a1[j]);
+    }
+    __syncthreads();
   }
 }
 
-__global__ void k_loss_sum(int B, const float* __restrict__ lossb, float* __restrict__ out) {
-  if (blockIdx.x == 0 && threadIdx.x == 0) {
+// Gradient of every parameter, summed over the batch: dW[o][i] = sum_b
+// D[b][o] * in[b][i], db[o] = sum_b D[b][o].  One block per output neuron:
+// lanes take consecutive inputs (whole lines of In), the block's 16 waves
+// take every 16th sample, and the waves' sums are added in a fixed order in
+// LDS (the same bits from call to call).  A thread per parameter walked the
+// whole batch alone: 36 blocks and a chain of 256 loads, 66 us at 256
+// samples.  The last block adds up the loss terms (a serial chain of its own
+// launch before, 11 us).
+constexpr int kGradThreads = 1024, kGradWaves = kGradThreads / 64;
+constexpr int kGradCols = (kMaxIn > kMaxHidden ? kMaxIn : kMaxHidden) / 64;
+__global__ void __launch_bounds__(kGradThreads) k_mlp_grad(MlpDims d, int B, const float* __restrict__ X,
+                                                           const float* __restrict__ A1, const float* __restrict__ A2,
+                                                           const float* __restrict__ D1, const float* __restrict__ D2,
+                                                           const float* __restrict__ D3,
+                                                           const float* __restrict__ lossb, float* __restrict__ G,
+                                                           float* __restrict__ loss) {
+  __shared__ float part[kGradWaves][64];
+  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+  // the waves' sums of a column, added in wave order
+  auto across = [&](float s) {
+    part[w][lane] = s;
+    __syncthreads();
+    float z = 0.f;
+    if (w == 0)
+      for (int v = 0; v < kGradWaves; v++) z += part[v][lane];
+    __syncthreads();
+    return z;
+  };
+  int o = blockIdx.x;
+  if (o == 2 * d.h + d.dout) {
     float s = 0.f;
-    for (int b = 0; b < B; b++) s += lossb[b];
-    *out = s;
+    for (int b = threadIdx.x; b < B; b += kGradThreads) s += lossb[b];
+    s = across(s);
+    if (w == 0) {
+#pragma unroll
+      for (int m = 32; m > 0; m >>= 1) s += __shfl_xor(s, m);
+      if (lane == 0 && loss) *loss = s;
+    }
+    return;
   }
+  const float *Dv, *In;
+  float *gw, *gb;
+  int nout, nin;
+  if (o < d.h) {
+    Dv = D1; In = X; nout = d.h; nin = d.din; gw = G + d.w1(); gb = G + d.b1();
+  } else if (o < 2 * d.h) {
+    o -= d.h;
+    Dv = D2; In = A1; nout = d.h; nin = d.h; gw = G + d.w2(); gb = G + d.b2();
+  } else {
+    o -= 2 * d.h;
+    Dv = D3; In = A2; nout = d.dout; nin = d.h; gw = G + d.w3(); gb = G + d.b3();
+  }
+  float s[kGradCols], sb = 0.f;
+#pragma unroll
+  for (int c = 0; c < kGradCols; c++) s[c] = 0.f;
+#pragma unroll 4
+  for (int b = w; b < B; b += kGradWaves) {
+    const float dv = Dv[(size_t)b * nout + o];
+    sb += dv;
+#pragma unroll
+    for (int c = 0; c < kGradCols; c++)
+      if (64 * c < nin) {
+        const int i = 64 * c + lane;
+        s[c] = fmaf(dv, i < nin ? In[(size_t)b * nin + i] : 0.f, s[c]);
+      }
+  }
+#pragma unroll
+  for (int c = 0; c < kGradCols; c++)
+    if (64 * c < nin) {
+      const float z = across(s[c]);
+      const int i = 64 * c + lane;
+      if (w == 0 && i < nin) gw[(size_t)o * nin + i] = z;
+    }
+  const float z = across(sb);  // every lane of a wave holds its bias sum
+  if (threadIdx.x == 0) gb[o] = z;
 }
 
 // Adam (Kingma & Ba 2015) with bias correction; step t starts at 1.
@@ -219,29 +299,22 @@ void ensure_batch(gx_mlp* m, int B) {
 }
 
 // Device arrays of one gradient pass: inputs X [B][din], T [B][dout];
-// scratch A1, A2, D1, D2 [B][h], Y, D3 [B][dout], lossb [B] (every element
+// scratch A1, A2, D1, D2 [B][h], D3 [B][dout], lossb [B] (every element
 // written before it is read); outputs G [params] and, when given, loss.
 struct GradBufs {
   const float *X, *T;
-  float *A1, *A2, *Y, *D1, *D2, *D3, *lossb, *G, *loss;
+  float *A1, *A2, *D1, *D2, *D3, *lossb, *G, *loss;
 };
 
-// forward + deltas + gradient + loss sum, enqueued on st
+// forward + deltas, then gradient + loss sum, enqueued on st
 void mlp_gradient_on(const gx_mlp* m, const GradBufs& g, int B, hipStream_t st) {
   const MlpDims& d = m->d;
-  hipLaunchKernelGGL(k_mlp_fwd, dim3(B), dim3(kMaxHidden), 0, st, d, B, g.X, m->P.as<float>(), g.A1, g.A2, g.Y);
-  GX_HIP(hipGetLastError());
-  hipLaunchKernelGGL(k_mlp_delta, dim3(B), dim3(kMaxHidden), 0, st, d, B, g.T, m->P.as<float>(), g.A1, g.A2, g.Y,
+  hipLaunchKernelGGL(k_mlp_sample, dim3(B), dim3(kMlpThreads), 0, st, d, B, g.X, g.T, m->P.as<float>(), g.A1, g.A2,
                      g.D1, g.D2, g.D3, g.lossb);
   GX_HIP(hipGetLastError());
-  size_t n = d.total();
-  hipLaunchKernelGGL(k_mlp_grad, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, st, d, B, g.X, g.A1, g.A2, g.D1,
-                     g.D2, g.D3, g.G);
+  hipLaunchKernelGGL(k_mlp_grad, dim3(2 * d.h + d.dout + 1), dim3(kGradThreads), 0, st, d, B, g.X, g.A1, g.A2, g.D1,
+                     g.D2, g.D3, g.lossb, g.G, g.loss);
   GX_HIP(hipGetLastError());
-  if (g.loss) {
-    hipLaunchKernelGGL(k_loss_sum, dim3(1), dim3(64), 0, st, B, g.lossb, g.loss);
-    GX_HIP(hipGetLastError());
-  }
 }
 
 // forward + deltas + gradient into m->G; returns the loss
@@ -250,7 +323,7 @@ float mlp_gradient(gx_mlp* m, const float* x, const float* t, int B) {
   ensure_batch(m, B);
   GX_HIP(hipMemcpyAsync(m->X.p, x, (size_t)B * d.din * 4, hipMemcpyHostToDevice, m->st));
   GX_HIP(hipMemcpyAsync(m->T.p, t, (size_t)B * d.dout * 4, hipMemcpyHostToDevice, m->st));
-  const GradBufs g{m->X.as<float>(), m->T.as<float>(), m->A1.as<float>(), m->A2.as<float>(), m->Y.as<float>(),
+  const GradBufs g{m->X.as<float>(), m->T.as<float>(), m->A1.as<float>(), m->A2.as<float>(),
                    m->D1.as<float>(), m->D2.as<float>(), m->D3.as<float>(), m->lossb.as<float>(), m->G.as<float>(),
                    m->loss.as<float>()};
   mlp_gradient_on(m, g, B, m->st);
@@ -261,13 +334,13 @@ float mlp_gradient(gx_mlp* m, const float* x, const float* t, int B) {
 }
 
 // Scratch of the allocation-free gradient (gx_mlp_gradient_noalloc): one
-// array per device, holding A1, A2, D1, D2, Y, D3 and the per-sample loss of
+// array per device, holding A1, A2, D1, D2, D3 and the per-sample loss of
 // a batch of at most kNoAllocBatch samples at the largest network
-// dimensions (8.3 MiB).  In host code `scratch` only names the symbol; its
+// dimensions (8.1 MiB).  In host code `scratch` only names the symbol; its
 // device address comes from hipGetSymbolAddress, once per device.
 constexpr int kNoAllocBatch = 4096;
 constexpr size_t kNoAllocFloats =
-    (size_t)kNoAllocBatch * (4 * kMaxHidden + 2 * kMaxOut + 1);
+    (size_t)kNoAllocBatch * (4 * kMaxHidden + kMaxOut + 1);
 static __device__ __align__(256) float scratch[kNoAllocFloats];
 
 constexpr int kMaxDevices = 64;
@@ -294,8 +367,7 @@ float* scratch_on(int device) {
 int gx_mlp_forward_device(gx_mlp* m, const float* dX, int B, float* dY, hipStream_t st) {
   return mlp_guard(m, [&] {
     GX_HIP(hipSetDevice(m->device));
-    hipLaunchKernelGGL(k_mlp_fwd, dim3(B), dim3(kMaxHidden), 0, st, m->d, B, dX, m->P.as<float>(), nullptr, nullptr,
-                       dY);
+    hipLaunchKernelGGL(k_mlp_fwd, dim3(B), dim3(kMlpThreads), 0, st, m->d, B, dX, m->P.as<float>(), dY);
     GX_HIP(hipGetLastError());
   });
 }
@@ -373,8 +445,8 @@ int gx_mlp_forward(gx_mlp* m, const float* x, int batch, float* y) {
     ensure_batch(m, batch);
     const MlpDims& d = m->d;
     GX_HIP(hipMemcpyAsync(m->X.p, x, (size_t)batch * d.din * 4, hipMemcpyHostToDevice, m->st));
-    hipLaunchKernelGGL(k_mlp_fwd, dim3(batch), dim3(kMaxHidden), 0, m->st, d, batch, m->X.as<float>(),
-                       m->P.as<float>(), nullptr, nullptr, m->Y.as<float>());
+    hipLaunchKernelGGL(k_mlp_fwd, dim3(batch), dim3(kMlpThreads), 0, m->st, d, batch, m->X.as<float>(),
+                       m->P.as<float>(), m->Y.as<float>());
     GX_HIP(hipGetLastError());
     GX_HIP(hipMemcpyAsync(y, m->Y.p, (size_t)batch * d.dout * 4, hipMemcpyDeviceToHost, m->st));
     GX_HIP(hipStreamSynchronize(m->st));
@@ -405,7 +477,7 @@ int gx_mlp_gradient_noalloc(gx_mlp* m, const float* x, const float* t, int batch
     float* sp = scratch_on(m->device);
     const MlpDims& d = m->d;
     const size_t bh = (size_t)batch * d.h, bo = (size_t)batch * d.dout;
-    GradBufs g{x, t, sp, sp + bh, sp + 4 * bh, sp + 2 * bh, sp + 3 * bh, sp + 4 * bh + bo, sp + 4 * bh + 2 * bo,
+    GradBufs g{x, t, sp, sp + bh, sp + 2 * bh, sp + 3 * bh, sp + 4 * bh, sp + 4 * bh + bo,
                grad ? grad : m->G.as<float>(), loss};
     hipStream_t st = stream ? static_cast<hipStream_t>(stream) : m->st;
     mlp_gradient_on(m, g, batch, st);

@@ -51,7 +51,7 @@ int gx_mlp_gradient(gx_mlp* m, const float* x, const float* t, int batch, float*
  * grad (params floats) and loss (one float) are device outputs, either may
  * be NULL (the gradient then stays in the network's own buffer).  The
  * activations and deltas live in a fixed device array of the library (one
- * per GPU, 8.3 MiB, kept until the process ends), so batch must not exceed
+ * per GPU, 8.1 MiB, kept until the process ends), so batch must not exceed
  * 4096 samples (GX_EINVAL otherwise) and the call makes no device
  * allocation.  stream: a hipStream_t to enqueue on (the call then returns
  * without waiting), or NULL for the network's own stream, synchronized

@@ -67,6 +67,29 @@ def test_mlp_gradient_matches_oracle(sizer, B):
     assert np.max(np.abs(g - gref)) < 1e-4 * scale
 
 
+@pytest.mark.parametrize("din,h,dout", [(1, 1, 1), (65, 63, 3), (256, 128, 8)])
+@pytest.mark.parametrize("B", [1, 17, 1025])
+def test_mlp_gradient_at_the_dimension_limits(sizer, din, h, dout, B):
+    """Rows that are not a multiple of the lanes sharing a dot product,
+    networks narrower and wider than a wave, batches below and above one
+    sample per wave of the gradient's blocks."""
+    rng = np.random.default_rng(din + B)
+    n = din * h + h + h * h + h + dout * h + dout
+    p = (rng.standard_normal(n) * 0.1).astype(np.float32)
+    X = rng.uniform(0, 1, (B, din)).astype(np.float32)
+    T = rng.normal(0, 1, (B, dout)).astype(np.float32)
+    m = sizer.Mlp(din, h, dout, params=p)
+    g, loss = m.gradient(X, T)
+    ref = sr.loss(p, X, T, din, h, dout)
+    gref = sr.gradient(p, X, T, din, h, dout)
+    # chains of at most B / 16 + 16 batch sums of terms with about 3 * 64 roundings each
+    tol = (B / 16 + 208) * 2.0 ** -24
+    assert abs(loss - ref) <= 4 * tol * max(1.0, abs(ref))
+    assert np.max(np.abs(g - gref)) <= 4 * tol * max(np.max(np.abs(gref)), 1e-3)
+    y, _ = sr.forward(p, X, din, h, dout)
+    assert np.allclose(m.forward(X), y, rtol=1e-5, atol=1e-5)
+
+
 def test_adam_step_matches_oracle(sizer):
     p = sizer.init_params(seed=9)
     m = sizer.Mlp(params=p)

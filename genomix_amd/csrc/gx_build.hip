@@ -2394,7 +2394,7 @@ __device__ inline int back_side(uint32_t t) { return (t == ET_FF || t == ET_RF) 
 // Initial walk records of a node end (ranking by walks, below): not yet
 // walked, or the end of a node that merges with nothing.
 constexpr uint64_t kEndUnvisited = ~0ull, kEndSingle = ~0ull - 1;
-constexpr uint32_t kWalkCap = 4096;
+constexpr uint32_t kWalkCap = 1024;  // claims of one walk; a longer path is ranked by walks between splitters
 
 // Neighbour y of k-mer v (reverse complement rv) for mask bit 4t + x:
 // FF w[1:]+x, FR rc(w[1:]+x) = comp(x)+rc(w)[:-1], RF rc(x+w[:-1]) =
@@ -2583,8 +2583,9 @@ __device__ inline bool mergeable(uint64_t i, int d, const uint32_t* lnk, const u
 // Chains are short in read graphs (errors end them every few letters: the
 // 5 Mbp workload's longest has ~130 nodes), so one dependent read per node
 // replaces several full passes over all ends.  A walker longer than the
-// cap, cycles (no endpoint) and even k (a palindromic k-mer links both its
-// sides to one neighbour) take the pointer-jumping ranking instead.
+// cap and graphs of long paths are ranked by walks between splitters
+// (below); cycles (no endpoint) and even k (a palindromic k-mer links both
+// its sides to one neighbour) take the pointer-jumping ranking instead.
 
 // One 16-byte entry per node end: .x = the next end on its path (kEnd at
 // the path's end), .z/.w = a 64-bit record; node i's record is the one of
@@ -2661,13 +2662,100 @@ __global__ void k_walk_join(uint32_t nwalk, const uint64_t* __restrict__ claim, 
   }
 }
 
+// Ranking by walks between splitters (odd k, long paths).  A walk from each
+// endpoint is a chain of dependent reads as long as half its path, so a
+// graph of long paths (a cleaned one: 5 M nodes in 16 K unitigs of up to
+// 10^5) waits on its longest few walks.  Here every path is cut at
+// splitters -- its endpoints, and one in kSplitEvery of its other nodes by
+// a hash of the node number -- and each splitter walks to the next one in
+// both directions: about 2 nn / kSplitEvery walks of kSplitEvery nodes on
+// average (the longest of 10^5 walks ~12 times that).  The splitters' own
+// chains are ranked by pointer jumping over 2 records each, and every
+// node's position follows from its walk's.  Both walks of a segment write a
+// record to each of its nodes (either gives the node the same rank), so no
+// claim is needed.  A cleaned 5 Mbp graph: 12 ms (walks that gave up at
+// their cap, then 18 rounds over 10 M node ends) -> 0.8 ms (the walks 0.4,
+// bound by their random lines; 19 rounds over 0.7 M records 0.2).
+constexpr uint32_t kSplitEvery = 16;
+// Mean path length from which the splitters pay: below it the walks from
+// the endpoints alone are short (18 nodes per path in an uncleaned read
+// graph: 3.5 ms for 55 M nodes, where splitters would read each node twice
+// and rank 2 M of them).
+constexpr uint64_t kSplitMean = 64;
+
+// Nodes that end a path or split one (endpoint: from k_links / k_link_ends).
+__global__ void k_split_flags(uint64_t nn, const uint32_t* __restrict__ lnk, const uint32_t* __restrict__ endpoint,
+                              uint32_t* __restrict__ flag) {
+  for (uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; i < nn; i += (uint64_t)gridDim.x * blockDim.x) {
+    const uint2 l = reinterpret_cast<const uint2*>(lnk)[i];
+    const bool inner = l.x != kEnd && l.y != kEnd;
+    flag[i] = endpoint[i] || (inner && ((uint32_t)i * 2654435761u >> 16) % kSplitEvery == 0) ? 1u : 0u;
+  }
+}
+
+// The splitters in node order; both entries of a splitter carry its number
+// + 1 in .y (0 for the other nodes), so a walk reads one entry per node.
+__global__ void k_split_list(uint64_t nn, const uint32_t* __restrict__ flag, const uint64_t* __restrict__ at,
+                             uint32_t* __restrict__ list, uint4* __restrict__ E) {
+  for (uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; i < nn; i += (uint64_t)gridDim.x * blockDim.x)
+    if (flag[i]) {
+      const uint32_t a = (uint32_t)at[i];
+      list[a] = (uint32_t)i;
+      E[2 * i].y = a + 1;
+      E[2 * i + 1].y = a + 1;
+    }
+}
+
+// Element 2a + d leaves splitter a through side d and walks to the next
+// splitter: R[element] = (the element it continues as, nodes to it, the
+// smallest 2 * node + side left of the nodes before it, itself), the form
+// k_pj_round ranks; a path's end has no successor.  Every node crossed gets
+// the record (element, side left, nodes from the splitter).
+__global__ void __launch_bounds__(kBlock) k_split_walk(uint32_t nel, uint64_t nn, const uint32_t* __restrict__ list,
+                                                       uint4* __restrict__ E, uint4* __restrict__ R) {
+  for (uint32_t w = blockIdx.x * blockDim.x + threadIdx.x; w < nel; w += gridDim.x * blockDim.x) {
+    uint32_t e = 2 * list[w >> 1] + (w & 1), mn = e, n = 0, to = kEnd;
+    uint32_t x = E[e].x;
+    reinterpret_cast<uint64_t*>(E + (e & ~1u))[1] = ((uint64_t)w << 32) | ((uint64_t)(e & 1) << 31);
+    while (x != kEnd && n < nn) {  // n < nn: a path visits no node twice
+      e = x;
+      n++;
+      const uint2 q = *reinterpret_cast<const uint2*>(E + e);  // next end, splitter
+      if (q.y) {
+        to = 2 * (q.y - 1) + (e & 1);
+        break;
+      }
+      mn = min(mn, e);
+      reinterpret_cast<uint64_t*>(E + (e & ~1u))[1] = ((uint64_t)w << 32) | ((uint64_t)(e & 1) << 31) | n;
+      x = q.x;
+    }
+    R[w] = make_uint4(to, to == kEnd ? 0u : n, mn, w);
+  }
+}
+
+// Per element, from the ranks of both elements of its splitter: the path's
+// summary (as k_walk_join) and the nodes before the splitter.  An element
+// still following its chain lies on a cycle and gets no summary.
+__global__ void k_split_join(uint32_t nel, const uint4* __restrict__ R, uint64_t* __restrict__ sum,
+                             uint32_t* __restrict__ before) {
+  for (uint32_t w = blockIdx.x * blockDim.x + threadIdx.x; w < nel; w += gridDim.x * blockDim.x) {
+    const uint4 f = R[w], o = R[w ^ 1];  // the nodes ahead, and those behind
+    const uint64_t len = (uint64_t)f.y + o.y + 1;
+    const bool ahead = (f.z >> 1) <= (o.z >> 1);  // the smallest node; walks the other way leave it by the other side
+    const uint32_t mn = ahead ? f.z >> 1 : o.z >> 1, rev = ahead ? f.z & 1 : 1 - (o.z & 1);
+    const bool cyc = f.x != kEnd || o.x != kEnd;
+    sum[w] = cyc ? ~0ull : (len << 32) | ((uint64_t)rev << 31) | mn;
+    before[w] = o.y;
+  }
+}
+
 // Per node from its record: representative, orientation, position; a node
 // without a record lies on a cycle or beyond the cap.  The claiming walker
 // reads the unitig backwards when it leaves the smallest node by its R side
 // (bit 31 of its sum); the node reads backwards when that differs from the
 // side it leaves the node by.
 __global__ void k_walk_final(uint64_t nn, const uint4* __restrict__ E, uint64_t nwalk, const uint64_t* __restrict__ sum,
-                             uint32_t* __restrict__ urep, uint32_t* __restrict__ upos, uint32_t* __restrict__ isrep,
+                             const uint32_t* __restrict__ before, uint32_t* __restrict__ urep, uint32_t* __restrict__ upos, uint32_t* __restrict__ isrep,
                              uint64_t* __restrict__ ulen_of_rep, uint32_t* __restrict__ unranked) {
   for (uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; i < nn; i += (uint64_t)gridDim.x * blockDim.x) {
     const uint64_t r = end_record(E[2 * i]);
@@ -2687,7 +2775,10 @@ __global__ void k_walk_final(uint64_t nn, const uint4* __restrict__ E, uint64_t 
       *unranked = 1u;
       continue;
     }
-    const uint32_t len = (uint32_t)(s >> 32), mn = (uint32_t)s & 0x7fffffffu, a = (uint32_t)r & 0x7fffffffu;
+    const uint32_t len = (uint32_t)(s >> 32), mn = (uint32_t)s & 0x7fffffffu;
+    // position from the path's start as this walker crosses it (a walk
+    // between splitters starts `before` nodes into its path)
+    const uint32_t a = ((uint32_t)r & 0x7fffffffu) + (before ? before[r >> 32] : 0u);
     const bool against = ((s >> 31) & 1) != 0;  // the unitig reads against this walker
     const bool side = ((r >> 31) & 1) != 0;      // the walker leaves this node by its R side
     urep[i] = mn | (against != side ? 0x80000000u : 0u);
@@ -2719,7 +2810,8 @@ __global__ void k_pj_init(uint64_t nn, const uint32_t* __restrict__ lnk, const u
 
 __global__ void __launch_bounds__(kBlock) k_pj_round(uint64_t ne, const uint4* __restrict__ Rc,
                                                      uint4* __restrict__ Rn, uint8_t* __restrict__ bflag,
-                                                     unsigned long long* __restrict__ nread) {
+                                                     uint64_t* __restrict__ breads) {
+  __shared__ uint32_t wreads[kBlock / 64];
   int any = 0;
   uint32_t reads = 0;  // successor records read (ends still following their chain)
   typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
@@ -2737,9 +2829,24 @@ __global__ void __launch_bounds__(kBlock) k_pj_round(uint64_t ne, const uint4* _
     __builtin_nontemporal_store(r, Rnv + e);
   }
   for (int o = 32; o > 0; o >>= 1) reads += __shfl_xor(reads, o);
-  if ((threadIdx.x & 63) == 0 && reads) atomicAdd(nread, (unsigned long long)reads);
+  if ((threadIdx.x & 63) == 0) wreads[threadIdx.x >> 6] = reads;
   any = __syncthreads_or(any);
-  if (threadIdx.x == 0) bflag[blockIdx.x] = any ? 1 : 0;
+  if (threadIdx.x == 0) {
+    bflag[blockIdx.x] = any ? 1 : 0;
+    // the block's own counter, summed once after the last round: an atomic
+    // per wave on one address took 40 us of a 50 us round over 0.3 M records
+    uint64_t s = 0;
+    for (int w = 0; w < kBlock / 64; w++) s += wreads[w];
+    breads[blockIdx.x] += s;
+  }
+}
+
+__global__ void __launch_bounds__(kBlock) k_sum_reads(const uint64_t* __restrict__ breads, uint32_t n,
+                                                      uint64_t* __restrict__ out) {
+  uint64_t s = 0, tot;
+  for (uint32_t j = threadIdx.x; j < n; j += kBlock) s += breads[j];
+  (void)block_exclusive_scan<uint64_t>(s, &tot);
+  if (threadIdx.x == 0) *out = tot;
 }
 
 __global__ void __launch_bounds__(kBlock) k_flag_or(const uint8_t* __restrict__ bflag, uint32_t n, uint32_t* out) {
@@ -4507,50 +4614,96 @@ static void run_unitigs(gx_build* b) {
   uint32_t* isrep = buf<uint32_t>(b->u_isrep, nn + 1);
   uint64_t* ulen_of_rep = buf<uint64_t>(b->u_lenrep, nn + 1);
   // ranking by walks (odd k), pointer jumping when a walk cannot rank every node
+  const unsigned jgrid = 8192;
+  uint64_t* breads = buf<uint64_t>(b->u_flag, jgrid + jgrid / 8);  // per-block counters of the jumping rounds, flags
+  uint8_t* bflag = reinterpret_cast<uint8_t*>(breads + jgrid);
+  GX_HIP(hipMemsetAsync(breads, 0, jgrid * 8, st));
+  int rounds = 0;
   bool walked = false;
   b->u_walkers = 0;
   if (walk) {
     ph_begin(b, PH_KWALK);
     uint64_t* at = buf<uint64_t>(b->u_uid, nn + 1);
     uint32_t* ws = buf<uint32_t>(b->u_any, 4);  // [0] capped, [1] unranked nodes
-    GX_HIP(hipMemsetAsync(ws, 0, 16, st));
     const unsigned gn = grid_for(nn, kBlock, G * 4);
     exclusive_scan<uint32_t, uint64_t>(endp, at, nn, scratch_for(b, scan_scratch_bytes<uint64_t>(nn)), st);
     const uint64_t nw = read1(st, at + nn);
-    uint32_t* walkers = buf<uint32_t>(b->u_walk2, nw + 1);
-    uint64_t* sum = buf<uint64_t>(b->u_ptr[1], 3 * (nw + 1));  // path sums, walker claims, meeting records
-    uint64_t* claim = sum + (nw + 1);
-    uint64_t* met = claim + (nw + 1);
-    GX_HIP(hipMemsetAsync(sum, 0xff, (nw + 1) * 8, st));  // a sum no join writes sends the pass to pointer jumping
-    if (nw) {
-      hipLaunchKernelGGL(k_walk_list, dim3(gn), dim3(kBlock), 0, st, nn, endp, at, E, walkers);
+    // nodes from the walkers' records; true when every node has its rank
+    auto finish_walks = [&](uint64_t nwalk, const uint64_t* sum, const uint32_t* before, uint32_t* wr) {
+      hipLaunchKernelGGL(k_walk_final, dim3(gn), dim3(kBlock), 0, st, nn, E, nwalk, sum, before, urep, upos, isrep,
+                         ulen_of_rep, ws + 1);
       GX_HIP(hipGetLastError());
-      // one resident wave set, each lane walking ~a dozen paths in turn: a
-      // wave then waits for the longest of its lanes' sums, not of single paths
-      hipLaunchKernelGGL(k_walk, dim3(grid_for(nw, kBlock, G)), dim3(kBlock), 0, st, (uint32_t)nw, walkers, E, claim,
-                         met, ws);
+      GX_HIP(hipMemcpyAsync(wr, ws, 16, hipMemcpyDeviceToHost, st));
+      GX_HIP(hipStreamSynchronize(st));
+      b->u_walkers = nwalk;
+      return wr[0] == 0 && wr[1] == 0;
+    };
+    auto walk_splits = [&] {
+      uint32_t* flag = upos;  // until k_walk_final
+      hipLaunchKernelGGL(k_split_flags, dim3(gn), dim3(kBlock), 0, st, nn, lnk, endp, flag);
       GX_HIP(hipGetLastError());
-      hipLaunchKernelGGL(k_walk_join, dim3(grid_for(nw, kBlock, G)), dim3(kBlock), 0, st, (uint32_t)nw, claim, met,
-                         sum);
+      exclusive_scan<uint32_t, uint64_t>(flag, at, nn, scratch_for(b, scan_scratch_bytes<uint64_t>(nn)), st);
+      GX_HIP(hipMemsetAsync(ws, 0, 16, st));
+      const uint64_t na = read1(st, at + nn), nel = 2 * na;
+      uint32_t* list = buf<uint32_t>(b->u_walk2, na + 1);
+      uint4* S[2];
+      S[0] = buf<uint4>(b->u_ptr[1], 2 * nel + (3 * nel + 3) / 4 + 1);  // two ranking buffers, sums, nodes before
+      S[1] = S[0] + nel;
+      uint64_t* sum = reinterpret_cast<uint64_t*>(S[1] + nel);
+      uint32_t* before = reinterpret_cast<uint32_t*>(sum + nel);
+      hipLaunchKernelGGL(k_split_list, dim3(gn), dim3(kBlock), 0, st, nn, flag, at, list, E);
       GX_HIP(hipGetLastError());
+      hipLaunchKernelGGL(k_split_walk, dim3(grid_for(nel, kBlock, jgrid)), dim3(kBlock), 0, st, (uint32_t)nel, nn, list,
+                         E, S[0]);
+      GX_HIP(hipGetLastError());
+      int cur = 0;
+      for (uint64_t reach = 1; reach < na; reach <<= 1) {  // after r rounds an element has followed 2^r segments
+        pj_begin(b);
+        hipLaunchKernelGGL(k_pj_round, dim3(grid_for(nel, kBlock, jgrid)), dim3(kBlock), 0, st, nel, S[cur],
+                           S[cur ^ 1], bflag, breads);
+        GX_HIP(hipGetLastError());
+        pj_end(b);
+        cur ^= 1;
+        rounds++;
+      }
+      hipLaunchKernelGGL(k_split_join, dim3(grid_for(nel, kBlock, G)), dim3(kBlock), 0, st, (uint32_t)nel, S[cur], sum,
+                         before);
+      GX_HIP(hipGetLastError());
+      uint32_t wr[4];
+      return finish_walks(nel, sum, before, wr);
+    };
+    if (nw && nn > kSplitMean * (nw / 2)) {
+      walked = walk_splits();
+    } else {
+      uint32_t* walkers = buf<uint32_t>(b->u_walk2, nw + 1);
+      uint64_t* sum = buf<uint64_t>(b->u_ptr[1], 3 * (nw + 1));  // path sums, walker claims, meeting records
+      uint64_t* claim = sum + (nw + 1);
+      uint64_t* met = claim + (nw + 1);
+      GX_HIP(hipMemsetAsync(ws, 0, 16, st));
+      GX_HIP(hipMemsetAsync(sum, 0xff, (nw + 1) * 8, st));  // a sum no join writes leaves its nodes unranked
+      if (nw) {
+        hipLaunchKernelGGL(k_walk_list, dim3(gn), dim3(kBlock), 0, st, nn, endp, at, E, walkers);
+        GX_HIP(hipGetLastError());
+        // one resident wave set, each lane walking ~a dozen paths in turn: a
+        // wave then waits for the longest of its lanes' sums, not of single paths
+        hipLaunchKernelGGL(k_walk, dim3(grid_for(nw, kBlock, G)), dim3(kBlock), 0, st, (uint32_t)nw, walkers, E, claim,
+                           met, ws);
+        GX_HIP(hipGetLastError());
+        hipLaunchKernelGGL(k_walk_join, dim3(grid_for(nw, kBlock, G)), dim3(kBlock), 0, st, (uint32_t)nw, claim, met,
+                           sum);
+        GX_HIP(hipGetLastError());
+      }
+      uint32_t wr[4];
+      walked = finish_walks(nw, sum, nullptr, wr);
+      if (wr[0]) walked = walk_splits();  // a walk met its cap: this graph has long paths after all
     }
-    hipLaunchKernelGGL(k_walk_final, dim3(gn), dim3(kBlock), 0, st, nn, E, nw, sum, urep, upos, isrep, ulen_of_rep,
-                       ws + 1);
-    GX_HIP(hipGetLastError());
     ph_end(b, PH_KWALK);
-    uint32_t wr[4];
-    GX_HIP(hipMemcpyAsync(wr, ws, sizeof(wr), hipMemcpyDeviceToHost, st));
-    GX_HIP(hipStreamSynchronize(st));
-    walked = wr[0] == 0 && wr[1] == 0;
-    b->u_walkers = nw;
   }
   uint4* R[2] = {nullptr, nullptr};
-  const unsigned jgrid = 8192;
-  uint8_t* bflag = buf<uint8_t>(b->u_flag, jgrid);
   uint32_t* anyflag = buf<uint32_t>(b->u_any, 4);
   int rmax = 2;
   while ((1ull << rmax) < ne + 1) rmax++;
-  int cur = 0, rounds = 0;
+  int cur = 0;
   if (!walked) {
   R[0] = buf<uint4>(b->u_ptr[0], ne + 1);
   R[1] = buf<uint4>(b->u_ptr[1], ne + 1);
@@ -4565,7 +4718,7 @@ static void run_unitigs(gx_build* b) {
     for (int r = 0; r <= rmax && act; r++) {
       unsigned g = grid_for(ne, kBlock, jgrid);
       pj_begin(b);
-      hipLaunchKernelGGL(k_pj_round, dim3(g), dim3(kBlock), 0, st, ne, R[cur], R[cur ^ 1], bflag, errw + 2);
+      hipLaunchKernelGGL(k_pj_round, dim3(g), dim3(kBlock), 0, st, ne, R[cur], R[cur ^ 1], bflag, breads);
       GX_HIP(hipGetLastError());
       pj_end(b);
       hipLaunchKernelGGL(k_flag_or, dim3(1), dim3(kBlock), 0, st, bflag, g, anyflag);
@@ -4585,9 +4738,15 @@ static void run_unitigs(gx_build* b) {
     GX_HIP(hipGetLastError());
   }
   }  // pointer jumping
-  unsigned long long e = read1(st, errw);
-  if (e != ~0ull) throw GxError(GX_EDEVICE, "internal error: neighbour k-mer missing from the table");
-  b->u_succ_reads = read1(st, errw + 2);
+  if (rounds) {
+    hipLaunchKernelGGL(k_sum_reads, dim3(1), dim3(kBlock), 0, st, breads, jgrid, reinterpret_cast<uint64_t*>(errw + 2));
+    GX_HIP(hipGetLastError());
+  }
+  unsigned long long ew[3];  // [0] first node without its neighbour, [2] successor reads of the jumping rounds
+  GX_HIP(hipMemcpyAsync(ew, errw, sizeof(ew), hipMemcpyDeviceToHost, st));
+  GX_HIP(hipStreamSynchronize(st));
+  if (ew[0] != ~0ull) throw GxError(GX_EDEVICE, "internal error: neighbour k-mer missing from the table");
+  b->u_succ_reads = ew[2];
 
   uint64_t* uid_of_rep = buf<uint64_t>(b->u_uid, nn + 1);
   exclusive_scan<uint32_t, uint64_t>(isrep, uid_of_rep, nn, scratch_for(b, scan_scratch_bytes<uint64_t>(nn)), st);

@@ -129,10 +129,12 @@ int gx_unitig_emit(gx_build* b, uint8_t* dst, size_t cap, size_t* written);
 
 /* How the unitig pass ranks the nodes of its merge paths:
  * GX_RANK_AUTO (default) walks each path from both its endpoints toward
- * each other when k is odd and falls back to pointer jumping for even k
- * (palindromic k-mers), cycles and walks of more than 4096 nodes (every
- * path of more than 8192); GX_RANK_POINTER_JUMPING always uses pointer
- * jumping.  The records are the same either way. */
+ * each other when k is odd; graphs of long paths (more than 64 nodes on
+ * average, or a walk of more than 1024) are walked between splitter nodes,
+ * whose chains are ranked by pointer jumping.  It falls back to pointer
+ * jumping over every node for even k (palindromic k-mers) and cycles;
+ * GX_RANK_POINTER_JUMPING always uses that.  The records are the same
+ * either way. */
 #define GX_RANK_AUTO 0
 #define GX_RANK_POINTER_JUMPING 1
 int gx_unitig_set_ranking(gx_build* b, int mode);
@@ -152,11 +154,11 @@ int gx_unitig_limits(uint64_t* max_nodes, uint64_t* max_head_offset);
  * count predicted by an attached sizing network (0 if none, genomix_sizer.h),
  * [8] table rebuilds after overflow, [9] records sorted by the global
  * fallback for oversized key buckets (sorted aggregation), [10] pointer-
- * jumping rounds of the last unitig run, [11] key-range passes of the build
+ * jumping rounds of the last unitig run (over nodes or splitters), [11] key-range passes of the build
  * (genomix_stream.h), [12] successor records read by those pointer-jumping
  * rounds (node ends still following their chain, summed over the rounds),
- * [13] path endpoints that walked their paths in the last unitig run (0 when
- * it ranked by pointer jumping only), [14] device allocations the last
+ * [13] walks that ranked the last unitig run: one per path endpoint, or two
+ * per splitter (0 when it ranked by pointer jumping only), [14] device allocations the last
  * finish made (0 when a repeated build reuses every buffer of the handle),
  * [15] buffers of earlier builds or phases it freed to make room. */
 int gx_build_stats(gx_build* b, uint64_t* out, int n);

@@ -115,6 +115,35 @@ def test_walk_falls_back_on_cycles_and_long_paths(gx):
     assert got == oracle.unitigs(oracle.build_graph(lin, k)[0], k)
 
 
+@pytest.mark.parametrize("k", [21, 33])
+@pytest.mark.parametrize("lengths,circular", [((90, 95, 88, 4000), 0), ((2300, 2500), 0), ((40,) * 60 + (5200,), 0),
+                                              ((3000, 150, 151), 1), ((30000,), 0)])
+def test_splitter_walks_equal_pointer_jumping(gx, k, lengths, circular):
+    """Graphs of long paths are ranked by walks between splitters: paths of
+    about one and of many splitters, paths that first meet the plain walks'
+    cap (a low mean length with one long path), and a circular genome beside
+    them, against pointer jumping and the oracle."""
+    rng = random.Random(sum(lengths) + k)
+    lines = []
+    for c, G in enumerate(lengths):
+        g = "".join(rng.choice("ACGT") for _ in range(G + k))
+        if c < circular:
+            g += g[:200]
+        for p in range(0, max(1, len(g) - 119), 30):
+            s = g[p:p + 120 + (len(g) - 120) % 30] if p + 150 > len(g) else g[p:p + 120]
+            lines.append(s if rng.random() < 0.5 else rc(s))
+    text = "".join(f"{4 * i + 2}\t{s}\n" for i, s in enumerate(lines)).encode()
+    outs = []
+    for mode in ("auto", "pointer_jumping"):
+        with gx.GraphBuilder(k) as b:
+            b.set_ranking(mode)
+            b.add_reads(text)
+            b.finish()
+            outs.append(b.unitigs())
+    assert outs[0] == outs[1]
+    assert outs[0] == oracle.unitigs(oracle.build_graph(text, k)[0], k)
+
+
 def test_cycles_and_tandems(gx):
     rng = random.Random(3)
     lines = []

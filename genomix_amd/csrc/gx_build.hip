@@ -3033,22 +3033,62 @@ __global__ void k_unitig_heads(uint64_t nn, const uint64_t* __restrict__ hstart,
   }
 }
 
-__global__ void k_uhead_unique(uint64_t nh, const Key128* __restrict__ key, uint32_t* __restrict__ uflag,
-                               uint32_t* __restrict__ hu, uint32_t* __restrict__ hf) {
-  for (uint64_t j = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; j < nh; j += (uint64_t)gridDim.x * blockDim.x) {
-    bool first = j == 0 || key[j].lo != key[j - 1].lo || key[j].hi != key[j - 1].hi;
-    uflag[j] = first ? 1 : 0;
-    if (first) atomicAdd(((key[j].lo >> 53) & 1) ? &hf[key[j].hi] : &hu[key[j].hi], 1u);
+// Bytes of a read head in a record: mate flag, uuid, the read and its mate
+// as VKmers.
+__device__ inline uint32_t uhead_bytes(const uint32_t* __restrict__ mlen, uint32_t m) {
+  const uint32_t L = mlen[m], Lm = mlen[m ^ 1];
+  return 1 + 8 + 4 + (L + 3) / 4 + (Lm > 0 ? 4 + (Lm + 3) / 4 : 0);
+}
+
+// Unique heads (TreeSet keeps the first of equal keys): their flags and
+// record bytes, and the counts per unitig of unflipped / flipped ones.  The
+// heads are sorted, so the lanes of a wave that share a unitig and flag are
+// neighbours and add their count with one atomic: a cleaned graph's unitigs
+// carry 10^4 heads each, and an atomic per head waited on those few
+// addresses (2.4 ms for 1.7 M heads; 56 us now).
+__global__ void __launch_bounds__(kBlock) k_uhead_unique(uint64_t nh, const Key128* __restrict__ key,
+                                                         const uint32_t* __restrict__ val,
+                                                         const uint32_t* __restrict__ mlen,
+                                                         uint32_t* __restrict__ uflag, uint32_t* __restrict__ usz,
+                                                         uint32_t* __restrict__ hu, uint32_t* __restrict__ hf) {
+  const int lane = threadIdx.x & 63;
+  for (uint64_t j0 = (uint64_t)blockIdx.x * kBlock; j0 < nh; j0 += (uint64_t)gridDim.x * kBlock) {
+    const uint64_t j = j0 + threadIdx.x;
+    Key128 x{0, 0}, before{0, 0};
+    if (j < nh) x = key[j];
+    if (j > 0 && j < nh) before = key[j - 1];
+    const bool first = j < nh && (j == 0 || x.lo != before.lo || x.hi != before.hi);
+    const uint32_t flip = (uint32_t)(x.lo >> 53) & 1;
+    const bool head = j < nh && (lane == 0 || x.hi != before.hi || flip != ((uint32_t)(before.lo >> 53) & 1));
+    if (j < nh) {
+      uflag[j] = first ? 1 : 0;
+      usz[j] = first ? uhead_bytes(mlen, val[j] & 0x7fffffffu) : 0;
+    }
+    const uint64_t uniq = __ballot(first), heads = __ballot(head);
+    if (head) {
+      const uint64_t later = lane == 63 ? 0ull : heads >> (lane + 1) << (lane + 1);  // the next group's first lane
+      const uint64_t upto = later ? (later & (0 - later)) - 1 : ~0ull;
+      const uint32_t n = (uint32_t)__popcll(uniq & upto & (~0ull << lane));
+      if (n) atomicAdd(flip ? &hf[x.hi] : &hu[x.hi], n);
+    }
   }
 }
 
+// The unique heads in order, each with its unitig and the record bytes of
+// the unique heads before it (nhead + 1 entries).
 __global__ void k_uhead_compact(uint64_t nh, const uint32_t* __restrict__ uflag, const uint64_t* __restrict__ upos_,
-                                const Key128* __restrict__ key, const uint32_t* __restrict__ val,
-                                uint64_t* __restrict__ ukey_lo, uint32_t* __restrict__ uval_out) {
+                                const uint64_t* __restrict__ ubytes, const Key128* __restrict__ key,
+                                const uint32_t* __restrict__ val, uint64_t* __restrict__ ukey_lo,
+                                uint32_t* __restrict__ uval_out, uint32_t* __restrict__ uunit,
+                                uint64_t* __restrict__ hbytes) {
   for (uint64_t j = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; j < nh; j += (uint64_t)gridDim.x * blockDim.x) {
+    if (j == nh - 1) hbytes[upos_[nh]] = ubytes[nh];
     if (!uflag[j]) continue;
-    ukey_lo[upos_[j]] = key[j].lo;
-    uval_out[upos_[j]] = val[j];
+    const uint64_t q = upos_[j];
+    ukey_lo[q] = key[j].lo;
+    uval_out[q] = val[j];
+    uunit[q] = (uint32_t)key[j].hi;
+    hbytes[q] = ubytes[j];
   }
 }
 
@@ -3066,7 +3106,7 @@ struct USerCtx {
   const uint32_t *hu, *hf;
   const uint64_t* hkey;    // offset etc.
   const uint32_t* hval;    // mate index | flipped << 31
-  const uint64_t* hbytes;  // head-rich unitigs: bytes of the unflipped / flipped heads
+  const uint64_t* hbytes;  // record bytes of the heads before each head
   const uint32_t* mlen;
   const uint64_t* wbase;
   const uint64_t* words;
@@ -3098,15 +3138,8 @@ __device__ inline uint32_t next_letter(const USerCtx& c, uint32_t o) {
 __device__ inline uint64_t useq_len(const USerCtx& c, uint64_t u) { return c.ulen[u] + c.k - 1; }
 
 // Unitigs with more than kHeadsLong read heads have their heads written by
-// k_uheads_long (a wave per unitig, lanes over heads); k_useq_write leaves
-// the bytes to it.
+// k_uheads_long (a thread per head); k_useq_write leaves the bytes to it.
 constexpr uint32_t kHeadsLong = 32;
-
-__device__ inline uint64_t uhead_bytes(const USerCtx& c, uint64_t j) {
-  const uint32_t m = c.hval[j] & 0x7fffffffu;
-  const uint32_t L = c.mlen[m], Lm = c.mlen[m ^ 1];
-  return 1 + 8 + 4 + (L + 3) / 4 + (Lm > 0 ? 4 + (Lm + 3) / 4 : 0);
-}
 
 // One read head of unitig records: mate flag, uuid (offset in the unitig,
 // mate, readId), the read and its mate as VKmers.
@@ -3133,36 +3166,11 @@ __device__ inline uint64_t unitig_record_size(const USerCtx& c, uint64_t u) {
   for (int f = 0; f < 2; f++) {
     uint32_t n = f ? nf : nu_;
     if (!n) continue;
-    val += 1 + 4;
-    if (nu_ + nf > kHeadsLong) {  // summed by k_uhead_bytes_long
-      val += c.hbytes[2 * u + f];
-      continue;
-    }
-    uint64_t a = h0 + (f ? nu_ : 0);
-    for (uint64_t j = a; j < a + n; j++) val += uhead_bytes(c, j);
+    const uint64_t a = h0 + (f ? nu_ : 0);
+    val += 1 + 4 + c.hbytes[a + n] - c.hbytes[a];
   }
   if (c.ulen[u] > 1) val += 4 + (useq_len(c, u) + 3) / 4;
   return 8 + 4 + c.nb + val;
-}
-
-// Bytes of the heads of head-rich unitigs (more than kHeadsLong), a wave
-// per unitig.
-__global__ void __launch_bounds__(kBlock) k_uhead_bytes_long(USerCtx c, uint64_t* __restrict__ hbytes) {
-  const int lane = threadIdx.x & 63;
-  const uint64_t nw = (uint64_t)gridDim.x * (kBlock / 64);
-  for (uint64_t u = (uint64_t)blockIdx.x * (kBlock / 64) + (threadIdx.x >> 6); u < c.nu; u += nw) {
-    const uint32_t nu_ = c.hu[u], nf = c.hf[u];
-    if (nu_ + nf <= kHeadsLong) continue;
-    for (int f = 0; f < 2; f++) {
-      const uint32_t n = f ? nf : nu_;
-      const uint64_t a = c.hstart[u] + (f ? nu_ : 0);
-      uint64_t sum = 0;
-      for (uint32_t q = lane; q < n; q += 64) sum += uhead_bytes(c, a + q);
-#pragma unroll
-      for (int o = 32; o > 0; o >>= 1) sum += __shfl_xor(sum, o, 64);
-      if (lane == 0) hbytes[2 * u + f] = sum;
-    }
-  }
 }
 
 __global__ void k_useq_size(USerCtx c, uint64_t* __restrict__ rsize) {
@@ -3259,7 +3267,7 @@ __device__ inline void write_unitig_record(const USerCtx& c, uint64_t u, uint8_t
       uint64_t a = h0 + (f ? nu_ : 0);
       if (nu_ + nf > kHeadsLong) {  // k_uheads_long writes these heads
         head_at[2 * u + f] = rec_at + (uint64_t)(p - rs);
-        p += c.hbytes[2 * u + f];
+        p += c.hbytes[a + n] - c.hbytes[a];
       } else {
         for (uint64_t j = a; j < a + n; j++) write_uhead(c, j, p);
       }
@@ -3342,52 +3350,69 @@ __global__ void __launch_bounds__(kBlock) k_useq_write(USerCtx c, const uint64_t
     __builtin_nontemporal_store(src[x], dst + x);  // written once, read by the caller later
 }
 
-// Heads of unitigs with many of them: a wave per unitig; each pass places
-// 64 heads by a wave prefix sum of their sizes.
-__global__ void __launch_bounds__(kBlock) k_uheads_long(USerCtx c, const uint64_t* __restrict__ head_at,
+// Heads of unitigs with many of them: a thread per head, placed by the
+// prefix sum of the heads' bytes.  (A wave per unitig, 64 heads at a time,
+// left the longest unitigs of a cleaned graph to a few waves: 6.2 ms for
+// 1.7 M heads; 0.56 ms now, 0.3 TB/s, bound by its 8-byte stores at
+// a stride of a head.)
+__global__ void __launch_bounds__(kBlock) k_uheads_long(USerCtx c, const uint64_t* __restrict__ nhead,
+                                                       const uint32_t* __restrict__ uunit,
+                                                       const uint64_t* __restrict__ head_at,
                                                        uint8_t* __restrict__ out) {
-  const int lane = threadIdx.x & 63;
-  const uint64_t nw = (uint64_t)gridDim.x * (kBlock / 64);
-  for (uint64_t u = (uint64_t)blockIdx.x * (kBlock / 64) + (threadIdx.x >> 6); u < c.nu; u += nw) {
+  const uint64_t n = *nhead;
+  for (uint64_t j = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; j < n; j += (uint64_t)gridDim.x * blockDim.x) {
+    const uint32_t u = uunit[j];
     const uint32_t nu_ = c.hu[u], nf = c.hf[u];
     if (nu_ + nf <= kHeadsLong) continue;
-    for (int f = 0; f < 2; f++) {
-      const uint32_t n = f ? nf : nu_;
-      if (!n) continue;
-      const uint64_t a = c.hstart[u] + (f ? nu_ : 0);
-      uint64_t at = head_at[2 * u + f];
-      for (uint32_t q0 = 0; q0 < n; q0 += 64) {
-        const uint32_t q = q0 + lane;
-        const uint32_t sz = q < n ? (uint32_t)uhead_bytes(c, a + q) : 0u;  // < 2^16 per head
-        uint32_t inc = sz;
-#pragma unroll
-        for (int o = 1; o < 64; o <<= 1) {
-          const uint32_t y = __shfl_up(inc, o, 64);
-          if (lane >= o) inc += y;
-        }
-        if (q < n) {
-          uint8_t* p = out + at + (inc - sz);
-          write_uhead(c, a + q, p);
-        }
-        at += (uint32_t)__shfl(inc, 63, 64);
-      }
-    }
+    const uint32_t f = c.hval[j] >> 31;
+    uint8_t* p = out + head_at[2 * (uint64_t)u + f] + (c.hbytes[j] - c.hbytes[c.hstart[u] + (f ? nu_ : 0)]);
+    write_uhead(c, j, p);
   }
 }
 
-template <int W>
-__global__ void __launch_bounds__(kBlock) k_useq_long(USerCtx c, const uint64_t* __restrict__ seq_at,
-                                                     uint8_t* __restrict__ out) {
+// Long sequences in chunks of kSeqChunk bytes, so that one unitig's letters
+// are gathered by many waves: (unitig, chunk) entries, in any order.  A
+// unitig of m nodes longer than kUseqLong letters has at most m / 64 chunks.
+constexpr uint32_t kSeqChunk = 64;
+static_assert(kUseqLong >= 256 && kSeqChunk == 64, "the chunk table holds nn / 64 + 1 entries");
+__global__ void __launch_bounds__(kBlock) k_useq_chunks(USerCtx c, uint2* __restrict__ chunk,
+                                                       unsigned long long* __restrict__ nchunk) {
   const int lane = threadIdx.x & 63;
-  const uint64_t nw = (uint64_t)gridDim.x * (kBlock / 64);
-  for (uint64_t u = (uint64_t)blockIdx.x * (kBlock / 64) + (threadIdx.x >> 6); u < c.nu; u += nw) {
-    if (c.ulen[u] <= 1) continue;
-    const uint64_t len = useq_len(c, u);
-    if (len <= kUseqLong) continue;
-    const uint64_t nbl = (len + 3) / 4;
-    const uint32_t* ord = c.order + c.ubase[u];
-    uint8_t* p = out + seq_at[u];
-    for (uint64_t bq = lane; bq < nbl; bq += 64) p[bq] = useq_byte<W>(c, ord, len, nbl - 1 - bq);
+  for (uint64_t u0 = (uint64_t)blockIdx.x * kBlock; u0 < c.nu; u0 += (uint64_t)gridDim.x * kBlock) {
+    const uint64_t u = u0 + threadIdx.x;
+    uint32_t n = 0;
+    if (u < c.nu && c.ulen[u] > 1) {
+      const uint64_t len = useq_len(c, u);
+      if (len > kUseqLong) n = (uint32_t)(((len + 3) / 4 + kSeqChunk - 1) / kSeqChunk);
+    }
+    if (!__ballot(n > 0)) continue;
+    uint32_t incl = n;
+#pragma unroll
+    for (int o = 1; o < 64; o <<= 1) {
+      const uint32_t y = __shfl_up(incl, o);
+      if (lane >= o) incl += y;
+    }
+    unsigned long long at = 0;
+    if (lane == 63) at = atomicAdd(nchunk, (unsigned long long)incl);
+    at = __shfl(at, 63) + incl - n;
+    for (uint32_t q = 0; q < n; q++) chunk[at + q] = make_uint2((uint32_t)u, q);
+  }
+}
+
+// A wave per chunk, a byte (four letters) per lane.  (A wave per unitig
+// before: 2.1 ms for the 5 M letters of a cleaned graph, whose longest
+// unitigs have 10^5; 40 us now.)
+template <int W>
+__global__ void __launch_bounds__(kBlock) k_useq_long(USerCtx c, const uint2* __restrict__ chunk,
+                                                     const unsigned long long* __restrict__ nchunk,
+                                                     const uint64_t* __restrict__ seq_at, uint8_t* __restrict__ out) {
+  const int lane = threadIdx.x & 63;
+  const uint64_t n = *nchunk, nw = (uint64_t)gridDim.x * (kBlock / 64);
+  for (uint64_t q = (uint64_t)blockIdx.x * (kBlock / 64) + (threadIdx.x >> 6); q < n; q += nw) {
+    const uint2 x = chunk[q];
+    const uint64_t u = x.x, len = useq_len(c, u), nbl = (len + 3) / 4;
+    const uint64_t bq = (uint64_t)x.y * kSeqChunk + lane;
+    if (bq < nbl) out[seq_at[u] + bq] = useq_byte<W>(c, c.order + c.ubase[u], len, nbl - 1 - bq);
   }
 }
 
@@ -3447,7 +3472,8 @@ struct gx_build {
   DevBuf nix_dir, nix_slots;  // key -> node index
   DevBuf rcode;               // replay codes, one byte per record in node order
   DevBuf u_seqat;             // unitig pass: byte position of long sequences
-  DevBuf u_hbytes;            // unitig pass: head bytes of head-rich unitigs
+  DevBuf u_hbytes;            // unitig pass: record bytes of the heads before each head
+  DevBuf u_chunk;             // unitig pass: chunks of long sequences
   DevBuf u_headat;            // unitig pass: byte position of the heads of head-rich unitigs
   DevBuf u_ends;              // unitig pass: each node's outer letters, one byte per node
   DevBuf s_acc, s_k1, s_k2, s_v1, s_v2, s_flag, s_pos, s_bval, s_bst, s_out;  // statistics, FASTA
@@ -3705,7 +3731,7 @@ static void for_each_buf(gx_build* b, F&& f) {
         &b->u_base, &b->u_order, &b->u_cov, &b->u_edge, &b->u_ecnt, &b->u_hk, &b->u_hk2, &b->u_hv, &b->u_hv2,
         &b->u_uflag, &b->u_uposh, &b->u_hu, &b->u_hf, &b->u_htot, &b->u_hstart, &b->u_hklo, &b->u_hvc, &b->u_rsize,
         &b->u_roff, &b->u_out, &b->ppid, &b->pidx, &b->ppid2, &b->pidx2, &b->pbound, &b->sva, &b->svb,
-        &b->nix_dir, &b->nix_slots, &b->rcode, &b->u_seqat, &b->u_hbytes, &b->tophist, &b->outacc, &b->blist, &b->hist2,
+        &b->nix_dir, &b->nix_slots, &b->rcode, &b->u_seqat, &b->u_hbytes, &b->u_chunk, &b->tophist, &b->outacc, &b->blist, &b->hist2,
         &b->hregs, &b->sfeat, &b->spred, &b->c_keep, &b->c_pos, &b->c_klo, &b->c_khi, &b->c_cnt, &b->c_msk,
         &b->c_hcu, &b->c_hcf, &b->c_htot, &b->c_hstart, &b->c_uval, &b->hoff, &b->c_hoff, &b->bb_min, &b->bb_maj,
         &b->bb_typ, &b->bb_np, &b->bb_pbase, &b->bb_pairs, &b->bb_ed, &b->bb_into, &b->bb_hn, &b->bb_hb,
@@ -4807,7 +4833,9 @@ static void run_unitigs(gx_build* b) {
   bool fl = radix_sort<Key128>(hk, hv, hk2, hv2, nh, 0, 12, scratch_for(b, radix_scratch_bytes<Key128>(nh)), st);
   if (fl) { std::swap(hk, hk2); std::swap(hv, hv2); }
   uint32_t* uflag = buf<uint32_t>(b->u_uflag, nh + 1);
-  uint64_t* uposh = buf<uint64_t>(b->u_uposh, nh + 1);
+  uint64_t* uposh = buf<uint64_t>(b->u_uposh, 2 * nh + 2);  // unique heads before each head, and their bytes
+  uint64_t* ubytes = uposh + nh + 1;
+  uint32_t* usz = hv2;  // the sort's spare buffer
   uint32_t* hu = buf<uint32_t>(b->u_hu, nu + 1);
   uint32_t* hf = buf<uint32_t>(b->u_hf, nu + 1);
   uint64_t* htot = buf<uint64_t>(b->u_htot, nu + 1);
@@ -4815,15 +4843,19 @@ static void run_unitigs(gx_build* b) {
   GX_HIP(hipMemsetAsync(hu, 0, (nu + 1) * 4, st));
   GX_HIP(hipMemsetAsync(hf, 0, (nu + 1) * 4, st));
   if (nh) {
-    hipLaunchKernelGGL(k_uhead_unique, dim3(grid_for(nh, kBlock, G)), dim3(kBlock), 0, st, nh, hk, uflag, hu, hf);
+    hipLaunchKernelGGL(k_uhead_unique, dim3(grid_for(nh, kBlock, G)), dim3(kBlock), 0, st, nh, hk, hv,
+                       b->mlen.as<uint32_t>(), uflag, usz, hu, hf);
     GX_HIP(hipGetLastError());
   }
   exclusive_scan<uint32_t, uint64_t>(uflag, uposh, nh, scratch_for(b, scan_scratch_bytes<uint64_t>(nh)), st);
+  exclusive_scan<uint32_t, uint64_t>(usz, ubytes, nh, scratch_for(b, scan_scratch_bytes<uint64_t>(nh)), st);
   uint64_t* hkey_lo = buf<uint64_t>(b->u_hklo, nh + 1);
-  uint32_t* hval_c = buf<uint32_t>(b->u_hvc, nh + 1);
+  uint32_t* hval_c = buf<uint32_t>(b->u_hvc, 2 * (nh + 1));  // values, and unitigs
+  uint32_t* hunit = hval_c + nh + 1;
+  uint64_t* hbytes = buf<uint64_t>(b->u_hbytes, nh + 1);
   if (nh) {
-    hipLaunchKernelGGL(k_uhead_compact, dim3(grid_for(nh, kBlock, G)), dim3(kBlock), 0, st, nh, uflag, uposh, hk, hv,
-                       hkey_lo, hval_c);
+    hipLaunchKernelGGL(k_uhead_compact, dim3(grid_for(nh, kBlock, G)), dim3(kBlock), 0, st, nh, uflag, uposh, ubytes,
+                       hk, hv, hkey_lo, hval_c, hunit, hbytes);
     GX_HIP(hipGetLastError());
   }
   if (nu) {
@@ -4844,14 +4876,10 @@ static void run_unitigs(gx_build* b) {
     GX_HIP(hipGetLastError());
   }
   c.ends = ends;
-  uint64_t* hbytes = buf<uint64_t>(b->u_hbytes, 2 * nu + 2);
   c.hbytes = hbytes;
   uint64_t* rsize = buf<uint64_t>(b->u_rsize, nu + 1);
   uint64_t* roff = buf<uint64_t>(b->u_roff, nu + 1);
   if (nu) {
-    hipLaunchKernelGGL(k_uhead_bytes_long, dim3(grid_for(nu, kBlock / 64, 1u << 16)), dim3(kBlock), 0, st, c,
-                       hbytes);
-    GX_HIP(hipGetLastError());
     hipLaunchKernelGGL(k_useq_size, dim3(grid_for(nu, kBlock, G)), dim3(kBlock), 0, st, c, rsize);
     GX_HIP(hipGetLastError());
   }
@@ -4865,10 +4893,19 @@ static void run_unitigs(gx_build* b) {
     hipLaunchKernelGGL(k_useq_write<W>, dim3(grid_for(nu, kBlock, 0xffffffffu)), dim3(kBlock), 0, st, c, roff, out,
                        seq_at, head_at);
     GX_HIP(hipGetLastError());
-    hipLaunchKernelGGL(k_uheads_long, dim3(grid_for(nu, kBlock / 64, 1u << 16)), dim3(kBlock), 0, st, c, head_at,
-                       out);
+    if (nh) {
+      hipLaunchKernelGGL(k_uheads_long, dim3(grid_for(nh, kBlock, 1u << 16)), dim3(kBlock), 0, st, c, uposh + nh, hunit,
+                         head_at, out);
+      GX_HIP(hipGetLastError());
+    }
+    unsigned long long* nchunk = buf<unsigned long long>(b->u_chunk, nn / 64 + 2);  // the count, then the chunks
+    uint2* chunk = reinterpret_cast<uint2*>(nchunk + 1);
+    hipLaunchKernelGGL(k_set_u64, dim3(1), dim3(1), 0, st, reinterpret_cast<uint64_t*>(nchunk), 0ull);
     GX_HIP(hipGetLastError());
-    hipLaunchKernelGGL(k_useq_long<W>, dim3(grid_for(nu, kBlock / 64, 1u << 16)), dim3(kBlock), 0, st, c, seq_at, out);
+    hipLaunchKernelGGL(k_useq_chunks, dim3(grid_for(nu, kBlock, G)), dim3(kBlock), 0, st, c, chunk, nchunk);
+    GX_HIP(hipGetLastError());
+    hipLaunchKernelGGL(k_useq_long<W>, dim3(grid_for(nn / 64 + 1, kBlock / 64, 4096)), dim3(kBlock), 0, st, c, chunk,
+                       nchunk, seq_at, out);
     GX_HIP(hipGetLastError());
   }
   ph_end(b, PH_UNITIG);

@@ -39,6 +39,28 @@ def test_stats_and_fasta_match_oracle(gx, k, paired):
         assert b.fasta("unitigs") == oracle.dump_fasta(cleaned, k)
 
 
+@pytest.mark.parametrize("copies", [1, 1023, 1500])
+def test_stats_of_wide_ranges(gx, copies):
+    """Coverages, head counts and seed scores inside and beyond a block's
+    counting window, and (a long unitig that carries many heads) beyond the
+    widest histogram, where the values are sorted."""
+    import random
+    rng = random.Random(copies)
+    k = 21
+    one = "".join(rng.choice("ACGT") for _ in range(60))
+    genome = "".join(rng.choice("ACGT") for _ in range(6000))
+    reads = [one] * copies + [genome[p:p + 100] for p in range(0, 5901, 2)]
+    text = "".join(f"{4 * i + 2}\t{s}\n" for i, s in enumerate(reads)).encode()
+    with gx.GraphBuilder(k) as b:
+        b.add_reads(text)
+        b.finish()
+        assert b.graph_stats("nodes") == oracle.graph_stats(b.part_bytes(0), k)
+        u = b.unitigs()
+        got = b.graph_stats("unitigs")
+        assert got == oracle.graph_stats(u, k)
+        assert got["maximum"]["scaffoldSeedScore"] > 1 << 22
+
+
 def test_stats_errors(gx):
     with gx.GraphBuilder(21) as b:
         b.add_reads(_text(3, G=5000, paired=False))

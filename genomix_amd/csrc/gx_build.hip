@@ -836,7 +836,7 @@ __device__ inline uint32_t sort_bucket(const SK& sk, int nb, int bkb) {
 
 // Key -> node index, built from the sorted nodes without global atomics:
 // the nodes of each key bucket (the top bkb bytes of the sort key: 2, or 3
-// above 2^26 nodes) are contiguous (dir[b] = first node), and each bucket
+// above 2 * 10^8 nodes) are contiguous (dir[b] = first node), and each bucket
 // owns a private open-addressing region of two slots per node, filled in
 // LDS by one block.  A lookup is the bucket's two dir entries plus one or
 // two slot probes.
@@ -894,59 +894,105 @@ __global__ void k_fill_u32(uint32_t* __restrict__ p, uint64_t from, uint64_t to,
     p[i] = v;
 }
 
-constexpr int kNixLds = 4096;  // slots of one bucket region built in LDS (two-byte buckets)
-constexpr int kNixLdsSmall = 1024;  // three-byte buckets: smaller regions, more blocks per CU
-template <int W, int LCAP>
-__global__ void __launch_bounds__(kBlock) k_nix_build(const uint64_t* __restrict__ klo, const uint64_t* __restrict__ khi,
-                                                      const uint32_t* __restrict__ msk, const uint32_t* __restrict__ dir,
-                                                      void* slots, uint32_t b0, uint32_t b1) {
-  using S = typename std::conditional<W == 1, Slot1, Slot2>::type;
-  __shared__ S lt[LCAP];
-  for (uint32_t bk = b0 + blockIdx.x; bk < b1; bk += gridDim.x) {
-    const uint32_t lo = dir[bk], hi = dir[bk + 1];
-    if (lo >= hi) continue;
-    const uint64_t R = 2ull * (hi - lo), base = 2ull * lo;
-    const bool local = R <= LCAP;
-    S* T = local ? lt : (S*)slots + base;
-    for (uint64_t i = threadIdx.x; i < R; i += kBlock) {
-      S e{};
-      if (W == 1) ((Slot1*)&e)->key = kEmpty;
-      else ((Slot2*)&e)->hi = kEmpty;
-      T[i] = e;
-    }
-    __syncthreads();
-    for (uint64_t n = lo + threadIdx.x; n < hi; n += kBlock) {
-      KV key = node_key<W>(klo, khi, n);
-      uint64_t s = slot_home(khash<W>(key), R);
-      for (uint64_t probe = 0; probe < R; probe++) {
-        if (W == 1) {
-          Slot1* e = (Slot1*)&T[s];
-          if (atomicCAS((unsigned long long*)&e->key, (unsigned long long)kEmpty, (unsigned long long)key.lo) ==
-              kEmpty) {
-            e->count = (uint32_t)n;
-            e->mask = msk[n] & 0xFFFFu;
-            break;
-          }
-        } else {  // distinct keys: a taken slot always holds another key
-          Slot2* e = (Slot2*)&T[s];
-          if (atomicCAS((unsigned long long*)&e->hi, (unsigned long long)kEmpty, (unsigned long long)key.hi) ==
-              kEmpty) {
-            e->lo = key.lo;
-            e->count = (uint32_t)n;
-            e->mask = msk[n] & 0xFFFFu;
-            break;
-          }
-        }
-        s = s + 1 == R ? 0 : s + 1;
-      }
-    }
-    __syncthreads();
-    if (local)
-      for (uint64_t i = threadIdx.x; i < R; i += kBlock) ((S*)slots)[base + i] = lt[i];
-    __syncthreads();  // lt is reused by the next bucket
+// Regions of the index, `span` consecutive buckets at a time: their slots
+// are claimed in LDS, where a slot is the node's number in the span (4 bytes
+// whatever the key's width), then written out whole, each slot gathering its
+// node's key and mask from the span's few lines.  Claims on whole slots took
+// 16 or 32 bytes of LDS each: 4 waves per CU with two-word keys, and a block
+// per bucket of six nodes above 2^26 nodes.  54.7 M nodes 1.25 -> 0.79 ms (2.8
+// TB/s of keys, masks and slots), 107 M 10.3 -> 1.4 ms, 250 K (most buckets
+// hold a few) 152 -> 7.5 us, four ranges of two-word nodes 7.9 -> 2.8 ms.  A
+// span that exceeds LDS is taken bucket by bucket, a bucket that does in HBM.
+template <int W>
+__device__ inline void nix_slot(void* slots, uint64_t at, KV key, uint32_t node, uint32_t mask) {
+  if (W == 1) {
+    Slot1 e;
+    e.key = key.lo;
+    e.count = node;
+    e.mask = mask;
+    ((Slot1*)slots)[at] = e;
+  } else {
+    Slot2 e;
+    e.hi = key.hi;
+    e.lo = key.lo;
+    e.count = node;
+    e.mask = mask;
+    e.pad = 0;
+    ((Slot2*)slots)[at] = e;
   }
 }
 
+template <int W, int LCAP, int NT>
+__global__ void __launch_bounds__(NT) k_nix_build(const uint64_t* __restrict__ klo, const uint64_t* __restrict__ khi,
+                                                  const uint32_t* __restrict__ msk, const uint32_t* __restrict__ dir,
+                                                  void* __restrict__ slots, int nb, int bkb, uint32_t b0, uint32_t b1,
+                                                  uint32_t span) {
+  __shared__ uint32_t lt[LCAP];
+  // buckets [ba, bb), whose slots fit LDS
+  auto build = [&](uint32_t ba, uint32_t bb) {
+    const uint32_t first = dir[ba], n = dir[bb] - first, R = 2 * n;
+    for (uint32_t i = threadIdx.x; i < R; i += NT) lt[i] = kEnd;
+    __syncthreads();
+    for (uint32_t q = threadIdx.x; q < n; q += NT) {
+      const KV key = node_key<W>(klo, khi, (uint64_t)first + q);
+      const uint32_t bk = bb - ba > 1 ? node_bucket<W>(key, nb, bkb) : ba;
+      const uint32_t lo = dir[bk] - first, Rb = 2 * (dir[bk + 1] - first - lo);
+      uint32_t* T = lt + 2 * lo;
+      uint32_t s = (uint32_t)slot_home(khash<W>(key), Rb);
+      for (uint32_t probe = 0; probe < Rb; probe++) {  // distinct keys: a taken slot always holds another key
+        if (atomicCAS(&T[s], kEnd, q) == kEnd) break;
+        s = s + 1 == Rb ? 0 : s + 1;
+      }
+    }
+    __syncthreads();
+    for (uint32_t i = threadIdx.x; i < R; i += NT) {
+      const uint32_t q = lt[i];
+      KV key{kEmpty, kEmpty};
+      uint32_t node = 0, mask = 0;
+      if (q != kEnd) {
+        node = first + q;
+        key = node_key<W>(klo, khi, node);
+        mask = msk[node] & 0xFFFFu;
+      }
+      nix_slot<W>(slots, 2ull * first + i, key, node, mask);
+    }
+    __syncthreads();  // lt is reused
+  };
+  for (uint64_t ga = b0 + (uint64_t)blockIdx.x * span; ga < b1; ga += (uint64_t)gridDim.x * span) {
+    const uint32_t gb = (uint32_t)min((uint64_t)b1, ga + span);
+    if (dir[gb] - dir[ga] <= LCAP / 2) {
+      if (dir[gb] > dir[ga]) build((uint32_t)ga, gb);
+      continue;
+    }
+    for (uint32_t bk = (uint32_t)ga; bk < gb; bk++) {
+      const uint32_t lo = dir[bk], hi = dir[bk + 1];
+      if (lo >= hi) continue;
+      if (hi - lo <= LCAP / 2) {
+        build(bk, bk + 1);
+        continue;
+      }
+      const uint64_t R = 2ull * (hi - lo), base = 2ull * lo;
+      for (uint64_t i = threadIdx.x; i < R; i += NT) nix_slot<W>(slots, base + i, KV{kEmpty, kEmpty}, 0, 0);
+      __syncthreads();
+      for (uint64_t n = lo + threadIdx.x; n < hi; n += NT) {
+        const KV key = node_key<W>(klo, khi, n);
+        uint64_t s = slot_home(khash<W>(key), R);
+        for (uint64_t probe = 0; probe < R; probe++) {
+          unsigned long long* word = W == 1 ? (unsigned long long*)&((Slot1*)slots)[base + s].key
+                                            : (unsigned long long*)&((Slot2*)slots)[base + s].hi;
+          if (atomicCAS(word, (unsigned long long)kEmpty, (unsigned long long)(W == 1 ? key.lo : key.hi)) == kEmpty) {
+            nix_slot<W>(slots, base + s, key, (uint32_t)n, msk[n] & 0xFFFFu);
+            break;
+          }
+          s = s + 1 == R ? 0 : s + 1;
+        }
+      }
+      __syncthreads();
+    }
+  }
+}
+
+constexpr int kNixSmall = 8192, kNixLarge = 16384;  // LDS slots of k_nix_build: 32 KB (512 threads), 64 KB (1024)
 constexpr int kBucketCap = 8192;  // records sorted per bucket in one block (72 KB / 144 KB of LDS)
 // HBM of a key-range pass, per occurrence (sizes the ranges): the records
 // (two key and two neighbour-code arrays, the sorted codes) and, per node (dfrac
@@ -3685,7 +3731,11 @@ static NodeIndex build_node_index(gx_build* b, hipStream_t st, uint64_t nn, cons
   const int nb = b->nb;
   const unsigned G = b->grid;
   const size_t slotsz = W == 1 ? sizeof(Slot1) : sizeof(Slot2);
-  const int xbkb = nb < 2 ? 1 : (nb >= 4 && nn > (1ull << 26)) ? 3 : 2;
+  // two-byte buckets while the larger LDS table holds 2.5 times the mean
+  // bucket (the canonical choice skews the top byte between 0.1 and 2 times
+  // the mean); beyond that three-byte ones
+  const uint64_t slots2 = 5 * nn / 65536;  // slots of a two-byte bucket of 2.5 times the mean size
+  const int xbkb = nb < 2 ? 1 : (nb >= 4 && slots2 > kNixLarge) ? 3 : 2;
   const uint32_t nbk = 1u << (8 * xbkb);
   const uint32_t xb0 = tlo << (8 * (xbkb - 1)), xb1 = thi << (8 * (xbkb - 1));
   b->nix_bkb = xbkb;
@@ -3703,12 +3753,19 @@ static NodeIndex build_node_index(gx_build* b, hipStream_t st, uint64_t nn, cons
   hipLaunchKernelGGL(k_nix_dir<W>, dim3(grid_for(nn + 1, kBlock, G)), dim3(kBlock), 0, st, nn, klo, khi, nb, xbkb, xb0,
                      xb1, ndir);
   GX_HIP(hipGetLastError());
-  if (xbkb == 3)
-    hipLaunchKernelGGL((k_nix_build<W, kNixLdsSmall>), dim3(std::min(xb1 - xb0, 65536u)), dim3(kBlock), 0, st, klo,
-                       khi, msk, ndir, nslots, xb0, xb1);
+  // buckets per block: as many as fill the small table, but at least 512
+  // blocks; the large table (two blocks per CU) where one mean bucket would
+  // not leave the small one room for the skew
+  const uint64_t per = std::max<uint64_t>(1, 5 * nn / nbk);
+  uint32_t span = 1;
+  while ((uint64_t)span * 2 * per <= kNixSmall && (xb1 - xb0) / (span * 2) >= 512) span *= 2;
+  const unsigned blocks = std::min((xb1 - xb0 + span - 1) / span, 65536u);
+  if (per <= kNixSmall)
+    hipLaunchKernelGGL((k_nix_build<W, kNixSmall, 512>), dim3(blocks), dim3(512), 0, st, klo, khi, msk, ndir, nslots,
+                       nb, xbkb, xb0, xb1, span);
   else
-    hipLaunchKernelGGL((k_nix_build<W, kNixLds>), dim3(std::min(xb1 - xb0, 65536u)), dim3(kBlock), 0, st, klo, khi,
-                       msk, ndir, nslots, xb0, xb1);
+    hipLaunchKernelGGL((k_nix_build<W, kNixLarge, 1024>), dim3(blocks), dim3(1024), 0, st, klo, khi, msk, ndir, nslots,
+                       nb, xbkb, xb0, xb1, span);
   GX_HIP(hipGetLastError());
   return NodeIndex{ndir, nslots, nb, nbk, xbkb};
 }

@@ -222,3 +222,19 @@ def test_head_beyond_offset_field_is_refused(gx):
         assert "23 bits" in str(e.value)
     with pytest.raises(oracle.OracleError):
         oracle.make_uuid(0, 0, 2, lim + 1)
+
+
+@pytest.mark.parametrize("k", [21, 33])
+@pytest.mark.parametrize("n", [1500, 6000, 30000])
+def test_node_index_of_uneven_buckets(gx, k, n):
+    """K-mers that share their first eight letters fill one bucket of the node
+    index beside many small ones: within a span of buckets, one bucket alone
+    in LDS, and one that only fits in HBM."""
+    rng = random.Random(n + k)
+    lines = []
+    for i in range(n):
+        s = "ACGTACGT" + "".join(rng.choice("ACGT") for _ in range(k - 6))
+        lines.append(s if rng.random() < 0.5 else rc(s))
+    g = "".join(rng.choice("ACGT") for _ in range(3000))
+    lines += [g[p:p + 100] for p in range(0, 2900, 20)]
+    check(gx, "".join(f"{4 * i + 2}\t{s}\n" for i, s in enumerate(lines)).encode(), k)

@@ -1704,26 +1704,52 @@ __device__ inline void type_sizes(uint32_t mask, int n[4]) {
   for (int t = 0; t < 4; t++) n[t] = __popc((mask >> (4 * t)) & 0xF);
 }
 
-// Nodes whose lists need the replay: some list holds >= 2 k-mers.  Marks
-// the slot (kNeedsBit), counts the records to replay and emits the replay
-// list key (count, clamped) for length-balanced scheduling.
+// Nodes whose lists need the replay: some list holds >= 2 k-mers.  needs =
+// the number of such lists; with a table (hash method) also marks the slot
+// (kNeedsBit) and stores the node's records in selcnt.  tot: [0] records and
+// [1] nodes to replay, [2] their lists; a set of atomics per block, on one of
+// kTotLines cache lines that the host adds up (atomics on one line follow
+// each other at 13 ns: 84 us of this kernel for the 5 M nodes of a 500 kbp
+// genome).
+constexpr int kTotLines = 32, kTotLine = 16;  // lines, words per line
 template <int W>
-__global__ void k_node_info(uint64_t nn, const uint32_t* __restrict__ msk, const uint32_t* __restrict__ cnt,
-                            const uint32_t* __restrict__ nslot, void* table, int jdk7,
-                            uint32_t* __restrict__ needs, uint64_t* __restrict__ selcnt,
-                            unsigned long long* maxcnt) {
+__global__ void __launch_bounds__(kBlock) k_node_info(uint64_t nn, const uint32_t* __restrict__ msk,
+                                                      const uint32_t* __restrict__ cnt,
+                                                      const uint32_t* __restrict__ nslot, void* table, int jdk7,
+                                                      uint32_t* __restrict__ needs, uint64_t* __restrict__ selcnt,
+                                                      unsigned long long* __restrict__ tot,
+                                                      unsigned long long* maxcnt) {
+  tot += kTotLine * (blockIdx.x % kTotLines);
+  uint64_t rec = 0, nodes = 0, entries = 0;
+  uint32_t most = 0;
   for (uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; i < nn; i += (uint64_t)gridDim.x * blockDim.x) {
-    if (cnt[i] > 255) atomicMax(maxcnt, (unsigned long long)cnt[i]);
+    const uint32_t c = cnt[i];
+    most = max(most, c);
     int n[4];
     type_sizes(msk[i], n);
-    bool need = jdk7 && (n[0] > 1 || n[1] > 1 || n[2] > 1 || n[3] > 1);
-    needs[i] = need ? 1 : 0;
-    selcnt[i] = need ? cnt[i] : 0;
-    if (need && table) {
+    const uint32_t lists = jdk7 ? (n[0] > 1) + (n[1] > 1) + (n[2] > 1) + (n[3] > 1) : 0;
+    needs[i] = lists;
+    entries += lists;
+    if (lists) {
+      rec += c;
+      nodes++;
+    }
+    if (selcnt) selcnt[i] = lists ? c : 0;
+    if (lists && table) {
       uint32_t s = nslot[i];
       uint32_t* m = W == 1 ? &((Slot1*)table)[s].mask : &((Slot2*)table)[s].mask;
       *m |= kNeedsBit;
     }
+  }
+  for (int o = 32; o > 0; o >>= 1) most = max(most, (uint32_t)__shfl_xor((int)most, o));
+  if ((threadIdx.x & 63) == 0 && most > 255) atomicMax(maxcnt, (unsigned long long)most);
+  uint64_t all;
+  (void)block_exclusive_scan<uint64_t>(rec, &all);
+  if (threadIdx.x == 0 && all) atomicAdd(&tot[0], (unsigned long long)all);
+  (void)block_exclusive_scan<uint64_t>((nodes << 32) | entries, &all);  // at most 4 * 2^30 / blocks entries each
+  if (threadIdx.x == 0 && all) {
+    atomicAdd(&tot[1], (unsigned long long)(all >> 32));
+    atomicAdd(&tot[2], (unsigned long long)(all & 0xffffffffull));
   }
 }
 
@@ -1772,17 +1798,50 @@ __global__ void k_sel_write(uint64_t nocc, const uint32_t* __restrict__ occ_slot
   }
 }
 
-// Replay list: nodes needing the replay, keyed by descending record count
-// so that one wave gets nodes of similar length.
-__global__ void k_replay_list(uint64_t nn, const uint32_t* __restrict__ needs, const uint64_t* __restrict__ rpos,
-                              const uint32_t* __restrict__ cnt, uint32_t* __restrict__ rkey,
-                              uint32_t* __restrict__ rval) {
-  for (uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; i < nn; i += (uint64_t)gridDim.x * blockDim.x) {
-    if (needs[i]) {
-      uint64_t p = rpos[i];
-      uint32_t c = cnt[i] > 0xffffu ? 0xffffu : cnt[i];
-      rkey[p] = 0xffffu - c;
-      rval[p] = (uint32_t)i;
+// Replay list: an entry per list of two or more k-mers, keyed by descending
+// record count (so that one wave gets runs of similar length) with the edge
+// type above the sorted 16 bits.  Each block takes a contiguous share of the
+// nodes and reserves its entries with one atomic; their order among equal
+// counts does not matter.
+constexpr int kRTypeShift = 16;
+__global__ void __launch_bounds__(kBlock) k_replay_list(uint64_t nn, const uint32_t* __restrict__ needs,
+                                                        const uint32_t* __restrict__ msk,
+                                                        const uint32_t* __restrict__ cnt,
+                                                        unsigned long long* __restrict__ next,
+                                                        uint32_t* __restrict__ rkey, uint32_t* __restrict__ rval) {
+  __shared__ unsigned long long base;
+  constexpr int kPer = 4;  // nodes per thread and scan
+  const uint64_t per = (nn + gridDim.x - 1) / gridDim.x;
+  const uint64_t a = blockIdx.x * per, e = min(nn, a + per);
+  uint64_t mine = 0, all;
+  for (uint64_t i = a + threadIdx.x; i < e; i += kBlock) mine += needs[i];
+  (void)block_exclusive_scan<uint64_t>(mine, &all);
+  if (threadIdx.x == 0) base = all ? atomicAdd(next, (unsigned long long)all) : 0;
+  __syncthreads();
+  if (!all) return;
+  uint64_t at = base;
+  for (uint64_t i0 = a; i0 < e; i0 += kPer * kBlock) {
+    uint32_t n[kPer], sum = 0, tile;
+#pragma unroll
+    for (int r = 0; r < kPer; r++) {
+      const uint64_t i = i0 + r * kBlock + threadIdx.x;
+      n[r] = i < e ? needs[i] : 0;
+      sum += n[r];
+    }
+    uint64_t p = at + block_exclusive_scan<uint32_t>(sum, &tile);
+    at += tile;
+#pragma unroll
+    for (int r = 0; r < kPer; r++) {
+      if (!n[r]) continue;
+      const uint64_t i = i0 + r * kBlock + threadIdx.x;
+      const uint32_t c = min(cnt[i], 0xffffu);
+      int sz[4];
+      type_sizes(msk[i], sz);
+      for (uint32_t t = 0; t < 4; t++)
+        if (sz[t] > 1) {
+          rkey[p] = (0xffffu - c) | (t << kRTypeShift);
+          rval[p++] = (uint32_t)i;
+        }
     }
   }
 }
@@ -1845,185 +1904,103 @@ __device__ inline LList j7_union(LList L, int sym, uint32_t hb) {
   return o;
 }
 
-// Long runs (a repeat k-mer carries thousands of records) are replayed by
-// four lanes per node, one per edge type: the four lists are independent
-// state machines over the same records, so the serial chain per lane is a
-// quarter of the work.  Lanes 4q..4q+3 hold node q; the four 16-bit results
-// are merged with lane shuffles.  Each lane caches its last eight
-// transitions (n, order, symbol class) -> (n', order'): a list of fixed
-// letters moves between a handful of orders under the two reorderings (a
-// union with no letter, with a letter present), so after a few records every
-// lane hits its cache and the wave no longer runs the full union whenever
-// one of its 64 lanes misses.
-constexpr uint32_t kLongReplay = 64;
-
-__device__ inline int code_sym(uint32_t code, int t) {
-  uint32_t sn = code & 0xF, pn = (code >> 4) & 0xF;
-  if (t == ET_FF || t == ET_FR) return ((sn & 8) && (((sn & 4) != 0) == (t == ET_FR))) ? (int)(sn & 3) : -1;
-  return ((pn & 8) && (((pn & 4) != 0) == (t == ET_RF))) ? (int)(pn & 3) : -1;
+// The order a list is in takes one of 65 states (no letter, then the orders
+// of 1 to 4 of the 4 letters), numbered by size, then letter by letter among
+// those not used yet.
+constexpr int kReplayStates = 65;
+__device__ inline uint32_t replay_state(const LList& l) {
+  uint32_t idx = 0, left = 0xFu;
+  for (int j = 0; j < l.n; j++) {
+    const uint32_t x = ll_get(l, j);
+    idx = idx * (4 - j) + __popc(left & ((1u << x) - 1));
+    left &= ~(1u << x);
+  }
+  return idx + (l.n == 0 ? 0 : l.n == 1 ? 1 : l.n == 2 ? 5 : l.n == 3 ? 17 : 41);
+}
+__device__ inline LList replay_order(uint32_t s) {
+  LList l{0, s == 0 ? 0 : s < 5 ? 1 : s < 17 ? 2 : s < 41 ? 3 : 4};
+  if (l.n == 0) return l;
+  uint32_t idx = s - (l.n == 1 ? 1 : l.n == 2 ? 5 : l.n == 3 ? 17 : 41);
+  uint32_t digit[4] = {0, 0, 0, 0};
+  for (int j = l.n - 1; j >= 0; j--) {
+    digit[j] = idx % (4 - j);
+    idx /= 4 - j;
+  }
+  uint32_t left = 0xFu;
+  for (int j = 0; j < l.n; j++) {
+    uint32_t m = left;
+    for (uint32_t q = 0; q < digit[j]; q++) m &= m - 1;
+    const uint32_t x = (uint32_t)__builtin_ctz(m);
+    l.bits |= x << (2 * j);
+    left &= ~(1u << x);
+  }
+  return l;
 }
 
-template <int W>
-__global__ void k_replay_long(uint64_t nlong, const uint32_t* __restrict__ rlist, const uint64_t* __restrict__ seg,
-                              const uint8_t* __restrict__ codes, const uint64_t* __restrict__ klo,
-                              const uint64_t* __restrict__ khi, const uint32_t* __restrict__ msk, int k, int nb,
-                              uint64_t* __restrict__ lists) {
-  for (uint64_t gid = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; gid < 4 * nlong;
-       gid += (uint64_t)gridDim.x * blockDim.x) {
-    const uint64_t q = gid >> 2;
-    const int t = (int)(gid & 3);
-    const uint32_t i = rlist[q];
-    const uint32_t mask = msk[i];
-    const bool active = __popc((mask >> (4 * t)) & 0xF) > 1;
-    uint64_t part = 0;
-    if (active) {
-      KV v = node_key<W>(klo, khi, i);
-      uint32_t hb = 0;
-      for (uint32_t x = 0; x < 4; x++)
-        hb |= ((uint32_t)jdk7_spread(java_hash_vkmer<W>(neighbour<W>(v, k, (uint32_t)t, x), k, nb)) & 7u) << (3 * x);
-      LList l{0, 0};
-      uint32_t memo[8];  // key << 11 | (n' << 8 | order'); all ones = empty (keys have 14 bits)
-#pragma unroll
-      for (int m = 0; m < 8; m++) memo[m] = 0xffffffffu;
-      uint32_t rr = 0;  // slot the next miss fills
-      const uint64_t a = seg[i], e = seg[i + 1];
-      uint64_t g = a & ~15ull;
-      uint4 cur = *reinterpret_cast<const uint4*>(codes + g);
-      while (g < e) {
-        const uint64_t gn = g + 16;
-        const uint4 nxt = gn < e ? *reinterpret_cast<const uint4*>(codes + gn) : make_uint4(0, 0, 0, 0);
-        const uint64_t lo64 = (uint64_t)cur.x | ((uint64_t)cur.y << 32), hi64 = (uint64_t)cur.z | ((uint64_t)cur.w << 32);
-        const int j0 = g < a ? (int)(a - g) : 0, j1 = e - g < 16 ? (int)(e - g) : 16;
-        for (int j = j0; j < j1; j++) {
-          uint32_t code = (uint32_t)((j < 8 ? lo64 >> (8 * j) : hi64 >> (8 * (j - 8))) & 0xff);
-          int sy = code_sym(code, t);
-          if (l.n <= 1 && (sy < 0 || (l.n == 1 && (int)ll_get(l, 0) == sy))) continue;
-          if (l.n == 0) { l.bits = (uint32_t)sy; l.n = 1; continue; }
-          uint32_t cls = 5;
-          if (sy >= 0) {
-            cls = (uint32_t)sy;
-            for (int jj = 0; jj < l.n; jj++)
-              if ((int)ll_get(l, jj) == sy) cls = 4;
-          }
-          uint32_t key = ((uint32_t)l.n << 11) | (l.bits << 3) | cls;
-          uint32_t hit = 0xffffffffu;
-#pragma unroll
-          for (int m = 0; m < 8; m++) hit = (memo[m] >> 11) == key ? memo[m] : hit;
-          if (hit != 0xffffffffu) { l.n = (hit >> 8) & 7; l.bits = hit & 0xff; continue; }
-          LList o = j7_union(l, sy, hb);
-          const uint32_t nv = (key << 11) | ((uint32_t)o.n << 8) | o.bits;
-#pragma unroll
-          for (int m = 0; m < 8; m++) memo[m] = m == (int)rr ? nv : memo[m];
-          rr = (rr + 1) & 7;
-          l = o;
-        }
-        cur = nxt;
-        g = gn;
-      }
-      LList f = j7_union(l, -1, hb);  // cross aggregator init
-      part = ((uint64_t)f.n | ((uint64_t)f.bits << 3)) << (16 * t);
-    }
-    uint32_t plo = (uint32_t)part, phi = (uint32_t)(part >> 32);
-    plo |= __shfl_xor(plo, 1);
-    phi |= __shfl_xor(phi, 1);
-    plo |= __shfl_xor(plo, 2);
-    phi |= __shfl_xor(phi, 2);
-    if (t == 0) lists[i] = ((uint64_t)phi << 32) | plo;
+// Letter a record adds to list t (0..3), or 4: the record has no such edge.
+__device__ inline uint32_t code_letter(uint32_t code, uint32_t t) {
+  const uint32_t nib = t < 2 ? code & 0xF : code >> 4;
+  const uint32_t want = 8u | ((t == ET_FR || t == ET_RF) ? 4u : 0u);
+  return (nib & 0xC) == want ? nib & 3 : 4u;
+}
+
+// A union's result depends only on the list's state, the record's letter and
+// the 12 hash bits of the four neighbours (hb): one table for every k-mer,
+// made once per handle, a row per hb.  A row starts on a cache line and its
+// first line holds the states of up to two letters.
+constexpr int kReplayRow = 384, kReplayRows = 4096;
+static_assert(kReplayStates * 5 <= kReplayRow, "row of a state's five successors");
+__global__ void k_replay_table(uint8_t* __restrict__ tab) {
+  for (uint32_t q = blockIdx.x * blockDim.x + threadIdx.x; q < (uint32_t)kReplayRows * kReplayRow;
+       q += gridDim.x * blockDim.x) {
+    const uint32_t hb = q / kReplayRow, at = q % kReplayRow, s = at / 5, letter = at % 5;
+    if (s < kReplayStates) tab[q] = (uint8_t)replay_state(j7_union(replay_order(s), letter < 4 ? (int)letter : -1, hb));
   }
 }
 
-__global__ void k_count_long(uint64_t n, const uint32_t* __restrict__ rkey, uint32_t lim,
-                             unsigned long long* __restrict__ cnt) {
-  uint64_t c = 0;
-  for (uint64_t q = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; q < n; q += (uint64_t)gridDim.x * blockDim.x)
-    c += rkey[q] <= lim;
-  for (int o = 32; o > 0; o >>= 1) c += __shfl_xor(c, o, 64);
-  if ((threadIdx.x & 63) == 0 && c) atomicAdd(cnt, (unsigned long long)c);  // one add per wave
-}
-
-// One thread per node of the replay list.  Only lists that end with >= 2
-// k-mers are simulated; a list with <= 1 k-mer has one order.  Fast paths:
-// unions that cannot reorder (empty or one-element list, no new element)
-// are skipped, and a union's result depends only on (list size, order,
-// symbol class) -- a new letter, a letter already present, or none -- so
-// the last two transitions of each list are cached.
+// One lane per list: a record costs one read of the table's row, which the
+// caches hold after a list's first few records; the chain of those reads
+// bounds a long run (3000 records of a repeat k-mer).  Before, a thread took
+// all four lists of a node and remembered two transitions of each, computing
+// the others' unions, and runs of 64 records or more went four lanes per node
+// on a second stream: 206 us for a 5 kbp genome, 1.0 + 1.8 ms (side by side)
+// for the 5 Mbp workload; now 12 us and 0.54 ms.
+constexpr uint64_t kReplayResident = 256 * 2048;  // lanes that run at once
 template <int W>
-__global__ void k_replay(uint64_t nrep, const uint32_t* __restrict__ rlist, const uint64_t* __restrict__ seg,
-                         const uint8_t* __restrict__ codes, const uint64_t* __restrict__ klo,
-                         const uint64_t* __restrict__ khi, const uint32_t* __restrict__ msk, int k, int nb,
-                         uint64_t* __restrict__ lists) {
-  for (uint64_t q = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; q < nrep; q += (uint64_t)gridDim.x * blockDim.x) {
-    uint32_t i = rlist[q];
-    KV v = node_key<W>(klo, khi, i);
-    uint32_t mask = msk[i];
-    uint32_t rel = 0;
-    int nfin[4];
-    for (int t = 0; t < 4; t++) {
-      nfin[t] = __popc((mask >> (4 * t)) & 0xF);
-      if (nfin[t] > 1) rel |= 1u << t;
-    }
+__global__ void __launch_bounds__(64) k_replay(uint64_t n, const uint32_t* __restrict__ rkey,
+                                               const uint32_t* __restrict__ rval, const uint64_t* __restrict__ seg,
+                                               const uint8_t* __restrict__ codes, const uint64_t* __restrict__ klo,
+                                               const uint64_t* __restrict__ khi, const uint8_t* __restrict__ tab, int k,
+                                               int nb, uint64_t* __restrict__ lists) {
+  for (uint64_t q = (uint64_t)blockIdx.x * 64 + threadIdx.x; q < n; q += (uint64_t)gridDim.x * 64) {
+    const uint32_t i = rval[q], t = rkey[q] >> kRTypeShift;
+    const uint64_t a = seg[i], e = seg[i + 1];
+    const KV v = node_key<W>(klo, khi, i);
     // low 3 bits of the JDK-7-spread VKmer.hashCode of each stored neighbour
-    uint32_t hb[4] = {0, 0, 0, 0};
-    for (uint32_t t = 0; t < 4; t++)
-      if ((rel >> t) & 1)
-        for (uint32_t x = 0; x < 4; x++)
-          hb[t] |= ((uint32_t)jdk7_spread(java_hash_vkmer<W>(neighbour<W>(v, k, t, x), k, nb)) & 7u) << (3 * x);
-    LList L[4] = {{0, 0}, {0, 0}, {0, 0}, {0, 0}};
-    // two-entry transition cache per list: (n, order, symbol class) ->
-    // (n', order'); an all-ones word is empty (no valid key has n = 7)
-    uint32_t cache[4][2];
-    for (int t = 0; t < 4; t++) cache[t][0] = cache[t][1] = 0xffffffffu;
-    uint64_t a = seg[i], e = seg[i + 1];
+    uint32_t hb = 0;
+    for (uint32_t x = 0; x < 4; x++)
+      hb |= ((uint32_t)jdk7_spread(java_hash_vkmer<W>(neighbour<W>(v, k, t, x), k, nb)) & 7u) << (3 * x);
+    const uint8_t* row = tab + (size_t)hb * kReplayRow;
+    uint32_t s = 0;
     // Codes are bytes, read 16 at a time with aligned 16-byte loads; the
-    // next group is loaded before the current one is replayed, so a long
-    // list (a repeat k-mer has thousands of records) waits on memory only
-    // once per group.  The code array is padded to a multiple of 16 bytes.
+    // next group is loaded before the current one is replayed.  The code
+    // array is padded to a multiple of 16 bytes.
     uint64_t g = a & ~15ull;
     uint4 cur = a < e ? *reinterpret_cast<const uint4*>(codes + g) : make_uint4(0, 0, 0, 0);
     while (g < e) {
       const uint64_t gn = g + 16;
       const uint4 nxt = gn < e ? *reinterpret_cast<const uint4*>(codes + gn) : make_uint4(0, 0, 0, 0);
-      const uint64_t lo64 = (uint64_t)cur.x | ((uint64_t)cur.y << 32), hi64 = (uint64_t)cur.z | ((uint64_t)cur.w << 32);
-      const int j0 = g < a ? (int)(a - g) : 0, j1 = e - g < 16 ? (int)(e - g) : 16;
-      for (int j = j0; j < j1; j++) {
-        uint32_t code = (uint32_t)((j < 8 ? lo64 >> (8 * j) : hi64 >> (8 * (j - 8))) & 0xff);
-        int sym[4] = {-1, -1, -1, -1};
-        uint32_t sn = code & 0xF, pn = (code >> 4) & 0xF;
-        if (sn & 8) sym[(sn & 4) ? ET_FR : ET_FF] = (int)(sn & 3);
-        if (pn & 8) sym[(pn & 4) ? ET_RF : ET_RR] = (int)(pn & 3);
-        for (int t = 0; t < 4; t++) {
-          if (!((rel >> t) & 1)) continue;
-          int sy = sym[t];
-          LList& l = L[t];
-          if (l.n <= 1 && (sy < 0 || (l.n == 1 && (int)ll_get(l, 0) == sy))) continue;
-          if (l.n == 0) { l.bits = (uint32_t)sy; l.n = 1; continue; }
-          // symbol class: the new letter, 4 = a letter already present, 5 = none
-          uint32_t cls = 5;
-          if (sy >= 0) {
-            cls = (uint32_t)sy;
-            for (int j = 0; j < l.n; j++)
-              if ((int)ll_get(l, j) == sy) cls = 4;
-          }
-          uint32_t key = ((uint32_t)l.n << 11) | (l.bits << 3) | cls;  // 14 bits
-          uint32_t c0 = cache[t][0], c1 = cache[t][1];
-          if ((c0 >> 11) == key) { l.n = (c0 >> 8) & 7; l.bits = c0 & 0xff; continue; }
-          if ((c1 >> 11) == key) { l.n = (c1 >> 8) & 7; l.bits = c1 & 0xff; continue; }
-          LList o = j7_union(l, sy, hb[t]);
-          cache[t][1] = c0;
-          cache[t][0] = (key << 11) | ((uint32_t)o.n << 8) | o.bits;
-          l = o;
-        }
-      }
+      const uint32_t j0 = g < a ? (uint32_t)(a - g) : 0, jn = (e - g < 16 ? (uint32_t)(e - g) : 16) - j0;
+      const uint32_t w[4] = {cur.x, cur.y, cur.z, cur.w};
+#pragma unroll
+      for (uint32_t j = 0; j < 16; j++)
+        if (j - j0 < jn) s = row[s * 5 + code_letter((w[j / 4] >> (8 * (j % 4))) & 0xff, t)];
       cur = nxt;
       g = gn;
     }
-    uint64_t out = 0;
-    for (int t = 0; t < 4; t++) {
-      if (!((rel >> t) & 1)) continue;
-      LList f = j7_union(L[t], -1, hb[t]);  // cross aggregator init
-      out |= ((uint64_t)f.n | ((uint64_t)f.bits << 3)) << (16 * t);
-    }
-    lists[i] = out;
+    s = row[s * 5 + 4];  // cross aggregator init
+    const LList f = replay_order(s);
+    reinterpret_cast<uint16_t*>(lists + i)[t] = (uint16_t)((uint32_t)f.n | (f.bits << 3));
   }
 }
 
@@ -3476,10 +3453,9 @@ struct gx_build {
   gx_build_cfg cfg{};
   int W = 1, nb = 0;
   hipStream_t st = nullptr;
-  // a second stream for work that overlaps the main stream's (the replay
-  // of the longest record runs beside the heads, the unitigs' outer edges
-  // beside their coverage and heads): ordered by events, created on first
-  // use
+  // a second stream for work that overlaps the main stream's (the unitigs'
+  // outer edges beside their coverage and heads): ordered by events, created
+  // on first use
   hipStream_t st2 = nullptr;
   hipEvent_t ev_fork = nullptr, ev_join = nullptr;
   std::string err;
@@ -3494,7 +3470,7 @@ struct gx_build {
   DevBuf text, scratch, blk, blk2, term, rid, mstart, mlen, wcnt, wbase, words, valid, nocc, occbase, hmask, hidx;
   DevBuf table, occ_slot, occ_code, claimed;
   DevBuf ckey, cval, ckey2, cval2, nslot, klo, khi, cnt, msk, needs, selcnt, seg;
-  DevBuf selflag, selpos, selk, selv, selk2, selv2, lists, rpos, rkey, rval, rkey2, rval2;
+  DevBuf selflag, selpos, selk, selv, selk2, selv2, lists, rtot, rkey, rval, rkey2, rval2;
   DevBuf hkey, hval, hkey2, hval2, uflag, upos, uval, hcu, hcf, htot, hstart, rsize, roff, out;
   DevBuf errw;
   uint64_t stats[16] = {};
@@ -3516,6 +3492,7 @@ struct gx_build {
   DevBuf ppid, pidx, ppid2, pidx2, pbound;
   DevBuf sva, svb;  // sorted aggregation: record neighbour codes
   DevBuf nix_dir, nix_slots;  // key -> node index
+  DevBuf rtab;                // replay transitions by hash bits (k_replay_table), the same for every build
   DevBuf rcode;               // replay codes, one byte per record in node order
   DevBuf u_seqat;             // unitig pass: byte position of long sequences
   DevBuf u_hbytes;            // unitig pass: record bytes of the heads before each head
@@ -3781,7 +3758,7 @@ static void for_each_buf(gx_build* b, F&& f) {
         &b->term, &b->rid, &b->mstart, &b->mlen, &b->wcnt, &b->wbase, &b->words, &b->valid, &b->nocc, &b->occbase,
         &b->hmask, &b->hidx, &b->table, &b->occ_slot, &b->occ_code, &b->claimed, &b->ckey, &b->cval, &b->ckey2,
         &b->cval2, &b->nslot, &b->klo, &b->khi, &b->cnt, &b->msk, &b->needs, &b->selcnt, &b->seg, &b->selflag,
-        &b->selpos, &b->selk, &b->selv, &b->selk2, &b->selv2, &b->lists, &b->rpos, &b->rkey, &b->rval, &b->rkey2,
+        &b->selpos, &b->selk, &b->selv, &b->selk2, &b->selv2, &b->lists, &b->rtot, &b->rkey, &b->rval, &b->rkey2,
         &b->rval2, &b->hkey, &b->hval, &b->hkey2, &b->hval2, &b->uflag, &b->upos, &b->uval, &b->hcu, &b->hcf,
         &b->htot, &b->hstart, &b->rsize, &b->roff, &b->out, &b->errw, &b->u_lnk, &b->u_tand, &b->u_cut, &b->u_flag,
         &b->u_any, &b->u_rep, &b->u_pos, &b->u_isrep, &b->u_lenrep, &b->u_uid, &b->u_repnode, &b->u_len,
@@ -4314,26 +4291,35 @@ static void run_build(gx_build* b) {
   const NodeIndex nix = build_node_index<W>(b, st, nn, klo, khi, msk, tlo, thi);
   if (sorted) cap = 2 * nn;
   ph_end(b, PH_NIX);
-  bool side_open = false;  // k_replay_long runs on the side stream, not joined yet
 
   // 6. replay
   ph_begin(b, PH_REPLAY);
   const int jdk7 = b->cfg.edge_order == GX_EDGE_ORDER_JDK7;
   uint32_t* needs = buf<uint32_t>(b->needs, nn + 1);
-  uint64_t* selcnt = buf<uint64_t>(b->selcnt, nn + 1);
-  uint64_t* seg = buf<uint64_t>(b->seg, nn + 1);
+  // records, nodes and lists to replay, per line; then the entries placed
+  unsigned long long* rtot = buf<unsigned long long>(b->rtot, kTotLine * kTotLines + 1);
+  GX_HIP(hipMemsetAsync(rtot, 0, (kTotLine * kTotLines + 1) * 8, st));
+  uint64_t* selcnt = sorted ? nullptr : buf<uint64_t>(b->selcnt, nn + 1);
   if (nn) {
     hipLaunchKernelGGL(k_node_info<W>, dim3(grid_for(nn, kBlock, G)), dim3(kBlock), 0, st, nn, msk, cnt, nslot,
-                       sorted ? nullptr : table, jdk7, needs, selcnt, errw + 3);
+                       sorted ? nullptr : table, jdk7, needs, selcnt, rtot, errw + 3);
     GX_HIP(hipGetLastError());
   }
-  exclusive_scan<uint64_t, uint64_t>(selcnt, seg, nn, scratch_for(b, scan_scratch_bytes<uint64_t>(nn)), st);
-  uint64_t nsel = read1(st, seg + nn);
+  unsigned long long rt[kTotLine * kTotLines];
+  GX_HIP(hipMemcpyAsync(rt, rtot, sizeof(rt), hipMemcpyDeviceToHost, st));
+  GX_HIP(hipStreamSynchronize(st));
+  uint64_t nsel = 0, nrep = 0, nent = 0;
+  for (int l = 0; l < kTotLines; l++) {
+    nsel += rt[kTotLine * l];
+    nrep += rt[kTotLine * l + 1];
+    nent += rt[kTotLine * l + 2];
+  }
   uint64_t* lists = buf<uint64_t>(b->lists, nn + 1);
-  uint64_t nrep = 0;
   if (nsel) {
     const uint32_t* codes = nullptr;
     if (!sorted) {
+    uint64_t* seg = buf<uint64_t>(b->seg, nn + 1);
+    exclusive_scan<uint64_t, uint64_t>(selcnt, seg, nn, scratch_for(b, scan_scratch_bytes<uint64_t>(nn)), st);
     uint32_t* flag = buf<uint32_t>(b->selflag, N + 1);
     uint64_t* pos = buf<uint64_t>(b->selpos, N + 1);
     hipLaunchKernelGGL(k_sel_flags<W>, dim3(grid_for(N, kBlock, G)), dim3(kBlock), 0, st, N, occ_slot, table, flag);
@@ -4361,49 +4347,35 @@ static void run_build(gx_build* b) {
                                                    &b->selv, &b->selk2, &b->selv2, &b->table});
     table = nullptr;
     }
-    // replay list ordered by descending record count
-    uint64_t* rpos = buf<uint64_t>(b->rpos, nn + 1);
-    exclusive_scan<uint32_t, uint64_t>(needs, rpos, nn, scratch_for(b, scan_scratch_bytes<uint64_t>(nn)), st);
-    nrep = read1(st, rpos + nn);
-    uint32_t* rk = buf<uint32_t>(b->rkey, nrep + 1);
-    uint32_t* rv = buf<uint32_t>(b->rval, nrep + 1);
-    uint32_t* rk2 = buf<uint32_t>(b->rkey2, nrep + 1);
-    uint32_t* rv2 = buf<uint32_t>(b->rval2, nrep + 1);
-    hipLaunchKernelGGL(k_replay_list, dim3(grid_for(nn, kBlock, G)), dim3(kBlock), 0, st, nn, needs, rpos, cnt, rk, rv);
+    uint32_t* rk = buf<uint32_t>(b->rkey, nent + 1);
+    uint32_t* rv = buf<uint32_t>(b->rval, nent + 1);
+    hipLaunchKernelGGL(k_replay_list, dim3(grid_for(nn, 8 * kBlock, G)), dim3(kBlock), 0, st, nn, needs, msk, cnt,
+                       rtot + kTotLine * kTotLines, rk, rv);
     GX_HIP(hipGetLastError());
-    bool f4 = radix_sort<uint32_t>(rk, rv, rk2, rv2, nrep, 0, 2, scratch_for(b, radix_scratch_bytes<uint32_t>(nrep)),
-                                   st);
-    uint32_t* rlist = f4 ? rv2 : rv;
-    const uint32_t* rkeys = f4 ? rk2 : rk;
-    // the longest runs (a prefix of the list) go to the four-lane kernel
-    GX_HIP(hipMemsetAsync(errw + 2, 0, 8, st));
-    hipLaunchKernelGGL(k_count_long, dim3(grid_for(nrep, kBlock, G)), dim3(kBlock), 0, st, nrep, rkeys,
-                       0xffffu - kLongReplay, errw + 2);
-    GX_HIP(hipGetLastError());
-    const uint64_t nlong = read1(st, errw + 2);
+    // by descending record count once the lists exceed the resident lanes;
+    // fewer all run at once, as long as their longest in any order
+    if (nent > kReplayResident) {
+      uint32_t* rk2 = buf<uint32_t>(b->rkey2, nent + 1);
+      uint32_t* rv2 = buf<uint32_t>(b->rval2, nent + 1);
+      if (radix_sort<uint32_t>(rk, rv, rk2, rv2, nent, 0, 2, scratch_for(b, radix_scratch_bytes<uint32_t>(nent)), st)) {
+        rk = rk2;
+        rv = rv2;
+      }
+    }
+    if (!b->rtab.p) {
+      buf<uint8_t>(b->rtab, (size_t)kReplayRows * kReplayRow);
+      hipLaunchKernelGGL(k_replay_table, dim3(1024), dim3(kBlock), 0, st, b->rtab.as<uint8_t>());
+      GX_HIP(hipGetLastError());
+    }
     ph_begin(b, PH_KREPLAY);
-    if (nlong) {
-      // a few hundred waves, each as long as its longest run: on the side
-      // stream, overlapping the short runs, the heads and the record sizes;
-      // joined before the records are written
-      side_init(b);
-      stream_after(b->st2, st, b->ev_fork);
-      side_open = true;
-      hipLaunchKernelGGL(k_replay_long<W>, dim3(grid_for(4 * nlong, kBlock, 1u << 16)), dim3(kBlock), 0, b->st2,
-                         nlong, rlist, rseg, rbytes, klo, khi, msk, k, nb, lists);
-      GX_HIP(hipGetLastError());
-    }
-    if (nrep > nlong) {
-      hipLaunchKernelGGL(k_replay<W>, dim3(grid_for(nrep - nlong, kBlock, 1u << 16)), dim3(kBlock), 0, st,
-                         nrep - nlong, rlist + nlong, rseg, rbytes, klo, khi, msk, k, nb, lists);
-      GX_HIP(hipGetLastError());
-    }
+    hipLaunchKernelGGL(k_replay<W>, dim3(grid_for(nent, 64, 1u << 16)), dim3(64), 0, st, nent, rk, rv, rseg, rbytes, klo,
+                       khi, b->rtab.as<uint8_t>(), k, nb, lists);
+    GX_HIP(hipGetLastError());
     ph_end(b, PH_KREPLAY);
   }
   ph_end(b, PH_REPLAY);
-  // replay inputs and order are dead (lists, needs and the node arrays
-  // stay); a free to make room drains the side stream first
-  b->reclaim.dead.insert(b->reclaim.dead.end(), {&b->nslot, &b->rcode, &b->selcnt, &b->seg, &b->rpos, &b->rkey,
+  // replay inputs and order are dead (lists, needs and the node arrays stay)
+  b->reclaim.dead.insert(b->reclaim.dead.end(), {&b->nslot, &b->rcode, &b->selcnt, &b->seg, &b->rkey,
                                                  &b->rval, &b->rkey2, &b->rval2});
 
   // 7. heads
@@ -4521,10 +4493,6 @@ static void run_build(gx_build* b) {
     b->part_rec[1] = nn;
     b->part_off[1] = total;
   }
-  if (side_open) {  // the records need every replayed list
-    stream_after(st, b->st2, b->ev_join);
-    side_open = false;
-  }
   uint8_t* out = buf<uint8_t>(b->out, total + 1);
   if (nn) {
     hipLaunchKernelGGL(k_ser_write<W>, dim3(grid_for(nn, kBlock, 0xffffffffu)), dim3(kBlock), 0, st, c, roff, out);
@@ -4578,7 +4546,7 @@ static void run_build(gx_build* b) {
   if (R > 1)  // the next range takes these buffers back as it needs them
     b->reclaim.dead.insert(b->reclaim.dead.end(),
                            {&b->klo, &b->khi, &b->cnt, &b->msk, &b->nslot, &b->nix_slots, &b->needs, &b->selcnt,
-                            &b->seg, &b->lists, &b->rpos, &b->rkey, &b->rval, &b->rkey2, &b->rval2, &b->rcode,
+                            &b->seg, &b->lists, &b->rkey, &b->rval, &b->rkey2, &b->rval2, &b->rcode,
                             &b->hcu, &b->hcf, &b->htot, &b->hstart, &b->uval, &b->rsize, &b->roff, &b->out, &b->ppid,
                             &b->pidx, &b->ppid2, &b->pidx2});
   }  // key ranges

@@ -5692,7 +5692,7 @@ struct VProps {
   uint64_t len;
   float cov;
   uint32_t nu, nf;
-  uint32_t self[4];
+  uint32_t self;  // self edges per type, a byte each (at most 16 edges)
 };
 
 template <int W, bool SELF>
@@ -5708,16 +5708,18 @@ __device__ inline VProps vertex_props(const VertexCtx& c, uint64_t i) {
     p.nf = c.hcf[i];
     if (SELF) {
       const KV v = node_key<W>(c.klo, c.khi, i);
-      for (uint32_t t = 0; t < 4; t++)
-        for (uint32_t x = 0; x < 4; x++)
-          if (((m >> (4 * t + x)) & 1) && keq<W>(neighbour<W>(v, c.k, t, x), v)) p.self[t]++;
+      const KV rv = revcomp<W>(v, c.k);
+      for (uint32_t b = m & 0xFFFFu; b; b &= b - 1) {
+        const uint32_t bit = (uint32_t)__builtin_ctz(b);
+        if (keq<W>(mask_neighbour<W>(v, rv, c.k, bit), v)) p.self += 1u << (8 * (bit >> 2));
+      }
     }
   } else {
     const uint32_t rep = c.urep_node[i];
     for (int e = 0; e < c.uecnt[i]; e++) {
       const uint32_t x = c.uedge[kUEdges * i + e], t = x >> kRepBits;
       p.deg[(t == ET_FF || t == ET_FR) ? 0 : 1]++;
-      if ((x & kRepMask) == rep) p.self[t]++;
+      if ((x & kRepMask) == rep) p.self += 1u << (8 * t);
     }
     p.len = c.ulen[i] + (uint64_t)c.k - 1;
     p.cov = (float)((double)c.ucov[i] / (double)c.ulen[i]);
@@ -5763,13 +5765,13 @@ __device__ inline bool stat_value(const VertexCtx& c, const VProps& p, int s, in
 // sum, least and largest value (and the totals), the second a histogram of
 // each whose range allows one.  A statistic at a time -- values to memory,
 // compacted, radix-sorted, binned -- moved about 100 bytes per vertex and
-// statistic: 27 ms for the 55 M nodes of the 5 Mbp workload, 1.5 ms now (0.73
-// and 0.67 ms a pass, 16 of its bytes per node and the self-edge tests).
-// Values are compared as value + 2^63, ordered like the signed ones.
+// statistic: 27 ms for the 55 M nodes of the 5 Mbp workload, 1.0 ms now (0.5
+// ms a pass over 24 and 16 bytes per node, bound by the 12 statistics'
+// arithmetic).  Values are compared as value + 2^63, ordered like the signed ones.
 constexpr uint64_t kStatBias = 0x8000000000000000ull;
 enum { SA_COUNT, SA_SUM, SA_HI, SA_LO, SA_N };  // acc[SA_N * s + .], then the totals
 constexpr int kStatAcc = SA_N * NSTAT + NTOT;
-constexpr unsigned kStatBlocks = 1024;  // one set of atomics per block
+constexpr unsigned kStatBlocks = 1024;
 
 // Wave sums, minima and maxima of 64-bit values (lane 0 holds the result).
 __device__ inline uint64_t wave_sum(uint64_t x) {
@@ -5785,21 +5787,47 @@ __device__ inline uint64_t wave_max(uint64_t x) {
   return x;
 }
 
-__global__ void k_stat_init(unsigned long long* __restrict__ acc) {
-  for (int q = threadIdx.x; q < kStatAcc; q += blockDim.x)
-    acc[q] = q < SA_N * NSTAT && q % SA_N == SA_LO ? ~0ull : 0ull;
+// Joins two values of accumulator q.
+__device__ inline unsigned long long stat_join(int q, unsigned long long x, unsigned long long y) {
+  if (q >= SA_N * NSTAT || q % SA_N < SA_HI) return x + y;
+  return q % SA_N == SA_HI ? max(x, y) : min(x, y);
+}
+__device__ inline unsigned long long stat_none(int q) {
+  return q < SA_N * NSTAT && q % SA_N == SA_LO ? ~0ull : 0ull;
+}
+
+// Each block's accumulators (part[block][.]) into one set (1024 blocks' atomics
+// on one set would follow each other at 13 ns a cache line).
+__global__ void __launch_bounds__(1024) k_stat_reduce(uint32_t blocks, const unsigned long long* __restrict__ part,
+                                                      unsigned long long* __restrict__ acc) {
+  constexpr int kWays = 16;
+  static_assert(kStatAcc <= 64, "one lane per accumulator");
+  __shared__ unsigned long long s[kWays][64];
+  const int q = threadIdx.x & 63, way = threadIdx.x >> 6;
+  unsigned long long x = stat_none(q);
+  if (q < kStatAcc)
+    for (uint32_t b = way; b < blocks; b += kWays) x = stat_join(q, x, part[(size_t)b * kStatAcc + q]);
+  s[way][q] = x;
+  __syncthreads();
+  if (way || q >= kStatAcc) return;
+  for (int w = 1; w < kWays; w++) x = stat_join(q, x, s[w][q]);
+  acc[q] = x;
 }
 
 template <int W>
-__global__ void __launch_bounds__(kBlock) k_stat_scan(VertexCtx c, unsigned long long* __restrict__ acc) {
+__global__ void __launch_bounds__(kBlock) k_stat_scan(VertexCtx c, unsigned long long* __restrict__ out) {
   __shared__ unsigned long long part[kStatAcc];
-  uint64_t sum[NSTAT], lo[NSTAT], hi[NSTAT];
+  // every value fits 32 bits: lengths below 2^30 + 63, Java ints, at most
+  // 2^30 heads on a side, coverages of at most 2^24
+  int64_t sum[NSTAT];
+  int32_t lo[NSTAT], hi[NSTAT];
   uint32_t cnt[NSTAT], tot[NTOT];
 #pragma unroll
   for (int s = 0; s < NSTAT; s++) {
     cnt[s] = 0;
-    sum[s] = hi[s] = 0;
-    lo[s] = ~0ull;
+    sum[s] = 0;
+    lo[s] = 0x7fffffff;
+    hi[s] = -0x7fffffff - 1;
   }
 #pragma unroll
   for (int q = 0; q < NTOT; q++) tot[q] = 0;
@@ -5812,25 +5840,24 @@ __global__ void __launch_bounds__(kBlock) k_stat_scan(VertexCtx c, unsigned long
     tot[TOT_TIPS_BOTH] += p.deg[0] == 0 && p.deg[1] == 0;
     tot[TOT_TIPS_ONE] += (p.deg[0] == 0) != (p.deg[1] == 0);
 #pragma unroll
-    for (int e = 0; e < 4; e++) tot[TOT_SELF_FF + e] += p.self[e];
+    for (int e = 0; e < 4; e++) tot[TOT_SELF_FF + e] += (p.self >> (8 * e)) & 0xff;
 #pragma unroll
     for (int s = 0; s < NSTAT; s++) {
       int64_t v;
       if (!stat_value<W>(c, p, s, &v)) continue;
-      const uint64_t key = (uint64_t)v + kStatBias;
       cnt[s]++;
-      sum[s] += (uint64_t)v;
-      lo[s] = min(lo[s], key);
-      hi[s] = max(hi[s], key);
+      sum[s] += (int32_t)v;
+      lo[s] = min(lo[s], (int32_t)v);
+      hi[s] = max(hi[s], (int32_t)v);
     }
   }
-  for (int q = threadIdx.x; q < kStatAcc; q += kBlock)
-    part[q] = q < SA_N * NSTAT && q % SA_N == SA_LO ? ~0ull : 0ull;
+  for (int q = threadIdx.x; q < kStatAcc; q += kBlock) part[q] = stat_none(q);
   __syncthreads();
   const bool lead = (threadIdx.x & 63) == 0;
 #pragma unroll
   for (int s = 0; s < NSTAT; s++) {
-    const uint64_t n = wave_sum(cnt[s]), x = wave_sum(sum[s]), l = wave_min(lo[s]), h = wave_max(hi[s]);
+    const uint64_t n = wave_sum(cnt[s]), x = wave_sum((uint64_t)sum[s]);
+    const uint64_t l = wave_min((uint64_t)(int64_t)lo[s] + kStatBias), h = wave_max((uint64_t)(int64_t)hi[s] + kStatBias);
     if (lead && n) {
       atomicAdd(&part[SA_N * s + SA_COUNT], (unsigned long long)n);
       atomicAdd(&part[SA_N * s + SA_SUM], (unsigned long long)x);
@@ -5844,26 +5871,18 @@ __global__ void __launch_bounds__(kBlock) k_stat_scan(VertexCtx c, unsigned long
     if (lead && x) atomicAdd(&part[SA_N * NSTAT + q], (unsigned long long)x);
   }
   __syncthreads();
-  for (int q = threadIdx.x; q < kStatAcc; q += kBlock) {
-    const unsigned long long x = part[q];
-    if (q >= SA_N * NSTAT || q % SA_N < SA_HI) {
-      if (x) atomicAdd(&acc[q], x);
-    } else if (q % SA_N == SA_HI) {
-      if (x) atomicMax(&acc[q], x);
-    } else if (x != ~0ull) {
-      atomicMin(&acc[q], x);
-    }
-  }
+  for (int q = threadIdx.x; q < kStatAcc; q += kBlock) out[(size_t)blockIdx.x * kStatAcc + q] = part[q];
 }
 
 // Histograms, one after the other in H: statistic s takes value - lo[s] at
 // off[s].  Each block counts the first kStatWin values of every statistic in
-// LDS and adds them up at its end; larger values, rare in read graphs, go to
-// H directly.  Most vertices share a value (a coverage of 1, a degree of 2),
+// LDS and adds them up at its end (one block per CU, so that few blocks meet
+// on H's first lines); larger values, rare in read graphs, go to H directly.  Most vertices share a value (a coverage of 1, a degree of 2),
 // so the lanes that hold the wave's first value count with one add.
 constexpr uint64_t kStatDense = 1ull << 22;  // widest histogram (16 MB); wider ranges are sorted
 constexpr uint32_t kStatWin = 1024;
-constexpr int kHistThreads = 512;
+constexpr int kHistThreads = 1024;
+constexpr unsigned kHistBlocks = 256;
 struct StatPlan {
   uint64_t lo[NSTAT], off[NSTAT];
   uint32_t mask;  // statistics that take a histogram
@@ -6030,13 +6049,13 @@ static void graph_stats(gx_build* b, int merged) {
   const unsigned G = b->grid;
   const VertexCtx c = vertex_ctx<W>(b, merged);
   const uint64_t n = c.n;
-  unsigned long long* acc = buf<unsigned long long>(b->s_acc, kStatAcc);
-  hipLaunchKernelGGL(k_stat_init, dim3(1), dim3(kBlock), 0, st, acc);
+  unsigned long long* acc = buf<unsigned long long>(b->s_acc, kStatAcc * (kStatBlocks + 1));
+  unsigned long long* part = acc + kStatAcc;
+  const unsigned sblocks = grid_for(n, kBlock, kStatBlocks);
+  hipLaunchKernelGGL(k_stat_scan<W>, dim3(sblocks), dim3(kBlock), 0, st, c, part);
   GX_HIP(hipGetLastError());
-  if (n) {
-    hipLaunchKernelGGL(k_stat_scan<W>, dim3(grid_for(n, kBlock, kStatBlocks)), dim3(kBlock), 0, st, c, acc);
-    GX_HIP(hipGetLastError());
-  }
+  hipLaunchKernelGGL(k_stat_reduce, dim3(1), dim3(1024), 0, st, sblocks, part, acc);
+  GX_HIP(hipGetLastError());
   unsigned long long a[kStatAcc];
   GX_HIP(hipMemcpyAsync(a, acc, sizeof(a), hipMemcpyDeviceToHost, st));
   GX_HIP(hipStreamSynchronize(st));
@@ -6070,7 +6089,7 @@ static void graph_stats(gx_build* b, int merged) {
     uint32_t* hflag = buf<uint32_t>(b->s_flag, nh + 1);
     uint64_t* hpos = buf<uint64_t>(b->s_pos, nh + 1);
     GX_HIP(hipMemsetAsync(H, 0, nh * 4, st));
-    hipLaunchKernelGGL(k_stat_hist<W>, dim3(grid_for(n, kHistThreads, kStatBlocks)), dim3(kHistThreads), 0, st, c, pl,
+    hipLaunchKernelGGL(k_stat_hist<W>, dim3(grid_for(n, kHistThreads, kHistBlocks)), dim3(kHistThreads), 0, st, c, pl,
                        H);
     GX_HIP(hipGetLastError());
     hipLaunchKernelGGL(k_hist_flag, dim3(grid_for(nh, kBlock, G)), dim3(kBlock), 0, st, nh, H, hflag);

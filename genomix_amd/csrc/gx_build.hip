@@ -2007,8 +2007,9 @@ __global__ void __launch_bounds__(64) k_replay(uint64_t n, const uint32_t* __res
 // ---------------------------------------------------------------------------
 // 7. 5' read heads (ReadHeadInfo.java:100-136; ReadsKeyValueParserFactory.java
 //    :129-135,142-144,165-170): one per valid mate on its first k-mer,
-//    unflipped at offset 0 or flipped at offset k-1.  Sort key =
-//    node<<31 | flipped<<30 | mate<<29 | readId: within a set the TreeSet
+//    unflipped at offset 0 or flipped at offset k-1.  Sort key = node,
+//    flipped, mate, readId from the top, the readId in the ridb bits its
+//    largest value needs (29 at most): within a set the TreeSet
 //    order (offset, lib = 0, mate, readId) of ReadHeadInfo.compareTo
 //    (:247-264); equal keys keep the first in emission order (TreeSet.add).
 // ---------------------------------------------------------------------------
@@ -2018,7 +2019,7 @@ __global__ void k_heads(uint64_t nmates, const uint8_t* __restrict__ valid, cons
                         const uint64_t* __restrict__ hidx, NodeIndex ix,
                         const int64_t* __restrict__ rid, const uint64_t* __restrict__ wbase,
                         const uint64_t* __restrict__ words, int k, uint64_t* __restrict__ hkey,
-                        uint32_t* __restrict__ hval, uint32_t tlo, uint32_t thi) {
+                        uint32_t* __restrict__ hval, uint32_t tlo, uint32_t thi, int ridb) {
   using SK = typename SortKeyOf<W>::T;
   for (uint64_t m = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; m < nmates; m += (uint64_t)gridDim.x * blockDim.x) {
     if (!valid[m] || nocc[m] == 0) continue;
@@ -2036,7 +2037,7 @@ __global__ void k_heads(uint64_t nmates, const uint8_t* __restrict__ valid, cons
     }
     uint64_t node = node_lookup<W>(ix, kk);
     uint64_t flipped = fwd ? 0 : 1;
-    uint64_t key = (node << 31) | (flipped << 30) | ((m & 1) << 29) | (uint64_t)rid[m >> 1];
+    uint64_t key = (((node << 1 | flipped) << 1 | (m & 1)) << ridb) | (uint64_t)rid[m >> 1];
     uint64_t j = hidx[m];
     hkey[j] = key;
     hval[j] = (uint32_t)m;
@@ -2069,13 +2070,14 @@ __global__ void k_head_unique(uint64_t nh, const uint64_t* __restrict__ hkey, ui
 
 __global__ void k_head_compact(uint64_t nh, const uint64_t* __restrict__ hkey, const uint32_t* __restrict__ hval,
                                const uint32_t* __restrict__ uflag, const uint64_t* __restrict__ upos,
-                               uint32_t* __restrict__ uval, uint32_t* __restrict__ hcu, uint32_t* __restrict__ hcf) {
+                               uint32_t* __restrict__ uval, uint32_t* __restrict__ hcu, uint32_t* __restrict__ hcf,
+                               int ridb) {
   for (uint64_t j = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; j < nh; j += (uint64_t)gridDim.x * blockDim.x) {
     if (!uflag[j]) continue;
-    uint64_t key = hkey[j];
-    uval[upos[j]] = hval[j] | ((uint32_t)((key >> 30) & 1) << 31);
-    uint64_t node = key >> 31;
-    atomicAdd(((key >> 30) & 1) ? &hcf[node] : &hcu[node], 1u);
+    const uint64_t key = hkey[j], node = key >> (ridb + 2);
+    const uint32_t flipped = (uint32_t)(key >> (ridb + 1)) & 1;
+    uval[upos[j]] = hval[j] | (flipped << 31);
+    atomicAdd(flipped ? &hcf[node] : &hcu[node], 1u);
   }
 }
 
@@ -2358,6 +2360,23 @@ __global__ void k_part_starts(uint64_t nn, const uint32_t* __restrict__ spid, ui
     uint32_t lo = j == 0 ? 0 : spid[j - 1] + 1;
     uint32_t hi = j == nn ? P : spid[j];
     for (uint32_t p = lo; p <= hi && p <= P; p++) start[p] = j;
+  }
+}
+
+// Largest readId (as an unsigned word), per block.
+constexpr unsigned kRidBlocks = 256;
+__global__ void __launch_bounds__(kBlock) k_rid_max(uint64_t nlines, const int64_t* __restrict__ rid,
+                                                    uint64_t* __restrict__ out) {
+  __shared__ uint64_t w[kBlock / 64];
+  uint64_t x = 0;
+  for (uint64_t i = (uint64_t)blockIdx.x * kBlock + threadIdx.x; i < nlines; i += (uint64_t)gridDim.x * kBlock)
+    x = max(x, (uint64_t)rid[i]);
+  for (int o = 32; o > 0; o >>= 1) x = max(x, (uint64_t)__shfl_xor(x, o));
+  if ((threadIdx.x & 63) == 0) w[threadIdx.x >> 6] = x;
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    for (int v = 1; v < kBlock / 64; v++) x = max(x, w[v]);
+    out[blockIdx.x] = x;
   }
 }
 
@@ -3029,7 +3048,9 @@ __global__ void k_unitig_heads(uint64_t nn, const uint64_t* __restrict__ hstart,
                                const uint32_t* __restrict__ upos,
                                const uint64_t* __restrict__ uid_of_rep, const int64_t* __restrict__ rid, int k,
                                Key128* __restrict__ key, uint32_t* __restrict__ val,
-                               unsigned long long* __restrict__ too_far) {
+                               unsigned long long* __restrict__ far) {
+  far += kTotLine * (blockIdx.x % kTotLines);
+  uint64_t most = 0;
   for (uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; i < nn; i += (uint64_t)gridDim.x * blockDim.x) {
     uint32_t nh = hcu[i] + hcf[i];
     if (!nh) continue;
@@ -3044,15 +3065,45 @@ __global__ void k_unitig_heads(uint64_t nn, const uint64_t* __restrict__ hstart,
       const uint32_t a = hoff ? hoff[h0 + j] : (f ? (uint32_t)(k - 1) : 0u);
       uint64_t off = upos[i] + (fwd ? a : (uint32_t)(k - 1) - a);
       if (off > kMaxHeadOffset) {  // ReadHeadInfo.makeUUID throws here (ReadHeadInfo.java:115-119)
-        atomicMin(too_far, (unsigned long long)off);
+        atomicMax(far + 1, ~(unsigned long long)off);
         off = 0;
       }
+      most = max(most, off);
       Key128 kk;
       kk.hi = u;
       kk.lo = ((uint64_t)nf << 53) | (off << 30) | ((uint64_t)(m & 1) << 29) | (uint64_t)rid[m >> 1];
       key[h0 + j] = kk;
       val[h0 + j] = m | ((uint32_t)nf << 31);
     }
+  }
+  for (int o = 32; o > 0; o >>= 1) most = max(most, (uint64_t)__shfl_xor(most, o));
+  if ((threadIdx.x & 63) == 0 && most) atomicMax(far, (unsigned long long)most);
+}
+
+// The same keys in the bits that the largest unitig, offset and readId need,
+// when those fit one word (they do up to 2^10 unitigs even with full readIds
+// and offsets): 7 sorted bytes instead of 12 for the 4 M unitigs of the 5
+// Mbp workload, 4 for those of a 5 kbp genome, and half the bytes a pass.
+struct HeadKeys {
+  const Key128* wide;      // hi = unitig, lo as above
+  const uint64_t* packed;  // or unitig, flipped, offset (offb bits), mate, readId (ridb bits)
+  int offb, ridb;
+  __device__ inline Key128 operator[](uint64_t j) const {
+    if (!packed) return wide[j];
+    const uint64_t x = packed[j], r = x & ((1ull << ridb) - 1), o = (x >> (ridb + 1)) & ((1ull << offb) - 1);
+    Key128 y;
+    y.hi = x >> (ridb + offb + 2);
+    y.lo = (((x >> (ridb + offb + 1)) & 1) << 53) | (o << 30) | (((x >> ridb) & 1) << 29) | r;
+    return y;
+  }
+};
+
+__global__ void k_uhead_pack(uint64_t nh, const Key128* __restrict__ key, int offb, int ridb,
+                             uint64_t* __restrict__ out) {
+  for (uint64_t j = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; j < nh; j += (uint64_t)gridDim.x * blockDim.x) {
+    const Key128 x = key[j];
+    const uint64_t off = (x.lo >> 30) & kMaxHeadOffset, r = x.lo & ((1ull << 29) - 1);
+    out[j] = ((((x.hi << 1 | (x.lo >> 53)) << offb | off) << 1 | ((x.lo >> 29) & 1)) << ridb) | r;
   }
 }
 
@@ -3069,7 +3120,7 @@ __device__ inline uint32_t uhead_bytes(const uint32_t* __restrict__ mlen, uint32
 // neighbours and add their count with one atomic: a cleaned graph's unitigs
 // carry 10^4 heads each, and an atomic per head waited on those few
 // addresses (2.4 ms for 1.7 M heads; 56 us now).
-__global__ void __launch_bounds__(kBlock) k_uhead_unique(uint64_t nh, const Key128* __restrict__ key,
+__global__ void __launch_bounds__(kBlock) k_uhead_unique(uint64_t nh, HeadKeys key,
                                                          const uint32_t* __restrict__ val,
                                                          const uint32_t* __restrict__ mlen,
                                                          uint32_t* __restrict__ uflag, uint32_t* __restrict__ usz,
@@ -3100,17 +3151,17 @@ __global__ void __launch_bounds__(kBlock) k_uhead_unique(uint64_t nh, const Key1
 // The unique heads in order, each with its unitig and the record bytes of
 // the unique heads before it (nhead + 1 entries).
 __global__ void k_uhead_compact(uint64_t nh, const uint32_t* __restrict__ uflag, const uint64_t* __restrict__ upos_,
-                                const uint64_t* __restrict__ ubytes, const Key128* __restrict__ key,
-                                const uint32_t* __restrict__ val, uint64_t* __restrict__ ukey_lo,
+                                const uint64_t* __restrict__ ubytes, HeadKeys key, const uint32_t* __restrict__ val, uint64_t* __restrict__ ukey_lo,
                                 uint32_t* __restrict__ uval_out, uint32_t* __restrict__ uunit,
                                 uint64_t* __restrict__ hbytes) {
   for (uint64_t j = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; j < nh; j += (uint64_t)gridDim.x * blockDim.x) {
     if (j == nh - 1) hbytes[upos_[nh]] = ubytes[nh];
     if (!uflag[j]) continue;
     const uint64_t q = upos_[j];
-    ukey_lo[q] = key[j].lo;
+    const Key128 x = key[j];
+    ukey_lo[q] = x.lo;
     uval_out[q] = val[j];
-    uunit[q] = (uint32_t)key[j].hi;
+    uunit[q] = (uint32_t)x.hi;
     hbytes[q] = ubytes[j];
   }
 }
@@ -3485,6 +3536,7 @@ struct gx_build {
   DevBuf u_lnk, u_tand, u_cut, u_ptr[2], u_flag, u_any, u_rep, u_pos, u_isrep, u_lenrep, u_walk, u_walk2;
   DevBuf u_uid, u_repnode, u_len, u_base, u_order, u_cov, u_edge, u_ecnt, u_hk, u_hk2, u_hv, u_hv2, u_uflag, u_uposh;
   DevBuf u_hu, u_hf, u_htot, u_hstart, u_hklo, u_hvc, u_rsize, u_roff, u_out;
+  int rid_bits = 29;  // of the largest readId of the build's input
   uint64_t nuheads = 0, u_bytes = 0, u_count = 0, u_rounds = 0, u_succ_reads = 0, u_walkers = 0;
   bool no_walk = false;  // rank by pointer jumping only (GX_UNITIG_RANK_POINTER_JUMPING)
   bool unitigs_done = false;
@@ -3497,6 +3549,7 @@ struct gx_build {
   DevBuf u_seqat;             // unitig pass: byte position of long sequences
   DevBuf u_hbytes;            // unitig pass: record bytes of the heads before each head
   DevBuf u_chunk;             // unitig pass: chunks of long sequences
+  DevBuf u_far;               // unitig pass: largest head offset, and the first beyond its field
   DevBuf u_headat;            // unitig pass: byte position of the heads of head-rich unitigs
   DevBuf u_ends;              // unitig pass: each node's outer letters, one byte per node
   DevBuf s_acc, s_k1, s_k2, s_v1, s_v2, s_flag, s_pos, s_bval, s_bst, s_out;  // statistics, FASTA
@@ -3765,7 +3818,7 @@ static void for_each_buf(gx_build* b, F&& f) {
         &b->u_base, &b->u_order, &b->u_cov, &b->u_edge, &b->u_ecnt, &b->u_hk, &b->u_hk2, &b->u_hv, &b->u_hv2,
         &b->u_uflag, &b->u_uposh, &b->u_hu, &b->u_hf, &b->u_htot, &b->u_hstart, &b->u_hklo, &b->u_hvc, &b->u_rsize,
         &b->u_roff, &b->u_out, &b->ppid, &b->pidx, &b->ppid2, &b->pidx2, &b->pbound, &b->sva, &b->svb,
-        &b->nix_dir, &b->nix_slots, &b->rcode, &b->u_seqat, &b->u_hbytes, &b->u_chunk, &b->tophist, &b->outacc, &b->blist, &b->hist2,
+        &b->nix_dir, &b->nix_slots, &b->rcode, &b->u_seqat, &b->u_hbytes, &b->u_chunk, &b->u_far, &b->tophist, &b->outacc, &b->blist, &b->hist2,
         &b->hregs, &b->sfeat, &b->spred, &b->c_keep, &b->c_pos, &b->c_klo, &b->c_khi, &b->c_cnt, &b->c_msk,
         &b->c_hcu, &b->c_hcf, &b->c_htot, &b->c_hstart, &b->c_uval, &b->hoff, &b->c_hoff, &b->bb_min, &b->bb_maj,
         &b->bb_typ, &b->bb_np, &b->bb_pbase, &b->bb_pairs, &b->bb_ed, &b->bb_into, &b->bb_hn, &b->bb_hb,
@@ -3835,13 +3888,21 @@ static void run_build(gx_build* b) {
   }
   // 3. pack
   uint64_t* wcnt = buf<uint64_t>(b->wcnt, nmates + 1);
-  uint64_t* wbase = buf<uint64_t>(b->wbase, nmates + 1);
+  uint64_t* wbase = buf<uint64_t>(b->wbase, nmates + 1 + kRidBlocks);  // and the blocks' largest readIds
   if (nmates) {
     hipLaunchKernelGGL(k_word_counts, dim3(grid_for(nmates, kBlock, G)), dim3(kBlock), 0, st, nmates, mlen, wcnt);
     GX_HIP(hipGetLastError());
   }
   exclusive_scan<uint64_t, uint64_t>(wcnt, wbase, nmates, scratch_for(b, scan_scratch_bytes<uint64_t>(nmates)), st);
-  uint64_t nwords = read1(st, wbase + nmates);
+  const unsigned rblocks = grid_for(nlines, kBlock, kRidBlocks);
+  hipLaunchKernelGGL(k_rid_max, dim3(rblocks), dim3(kBlock), 0, st, nlines, rid, wbase + nmates + 1);
+  GX_HIP(hipGetLastError());
+  uint64_t wr[1 + kRidBlocks];
+  GX_HIP(hipMemcpyAsync(wr, wbase + nmates, (1 + rblocks) * 8, hipMemcpyDeviceToHost, st));
+  GX_HIP(hipStreamSynchronize(st));
+  const uint64_t nwords = wr[0], rid_max = *std::max_element(wr + 1, wr + 1 + rblocks);
+  b->rid_bits = 1;  // valid readIds have at most 29 bits; those of lines that fail later may have more
+  while (b->rid_bits < 29 && (rid_max >> b->rid_bits)) b->rid_bits++;
   uint64_t* words = buf<uint64_t>(b->words, nwords + 4);
   uint8_t* valid = buf<uint8_t>(b->valid, nmates + 1);
   uint64_t* nocc = buf<uint64_t>(b->nocc, nmates + 1);
@@ -4386,7 +4447,7 @@ static void run_build(gx_build* b) {
   uint32_t* hv2 = buf<uint32_t>(b->hval2, nheads + 1);
   if (nmates) {
     hipLaunchKernelGGL(k_heads<W>, dim3(grid_for(nmates, kBlock, G)), dim3(kBlock), 0, st, nmates, valid, nocc, hidx,
-                       nix, rid, wbase, words, k, hk, hv, tlo, thi);
+                       nix, rid, wbase, words, k, hk, hv, tlo, thi, b->rid_bits);
     GX_HIP(hipGetLastError());
   }
   uint32_t* uflag = buf<uint32_t>(b->uflag, nheads + 1);
@@ -4404,7 +4465,7 @@ static void run_build(gx_build* b) {
     std::swap(hv, hv2);
   }
   int hbytes = 1;
-  while (hbytes < 8 && (((nn << 31) | ((1ull << 31) - 1)) >> (8 * hbytes)) > 0) hbytes++;
+  while (hbytes < 8 && ((((nn + 1) << (b->rid_bits + 2)) - 1) >> (8 * hbytes)) > 0) hbytes++;
   bool f3 = radix_sort<uint64_t>(hk, hv, hk2, hv2, nh, 0, hbytes, scratch_for(b, radix_scratch_bytes<uint64_t>(nh)),
                                  st);
   if (f3) { std::swap(hk, hk2); std::swap(hv, hv2); }
@@ -4424,7 +4485,7 @@ static void run_build(gx_build* b) {
   b->nuheads += nuh_r;
   if (nh) {
     hipLaunchKernelGGL(k_head_compact, dim3(grid_for(nh, kBlock, G)), dim3(kBlock), 0, st, nh, hk, hv, uflag, upos,
-                       uval, hcu, hcf);
+                       uval, hcu, hcf, b->rid_bits);
     GX_HIP(hipGetLastError());
   }
   if (nn) {
@@ -4844,19 +4905,49 @@ static void run_unitigs(gx_build* b) {
   Key128* hk2 = buf<Key128>(b->u_hk2, nh + 1);
   uint32_t* hv = buf<uint32_t>(b->u_hv, nh + 1);
   uint32_t* hv2 = buf<uint32_t>(b->u_hv2, nh + 1);
+  HeadKeys keys{hk, nullptr, 0, b->rid_bits};
   if (nn && nh) {
+    unsigned long long* far = buf<unsigned long long>(b->u_far, kTotLine * kTotLines);
+    GX_HIP(hipMemsetAsync(far, 0, kTotLine * kTotLines * 8, st));
     hipLaunchKernelGGL(k_unitig_heads, dim3(grid_for(nn, kBlock, G)), dim3(kBlock), 0, st, nn,
                        b->hstart.as<uint64_t>(), b->hcu.as<uint32_t>(), b->hcf.as<uint32_t>(), b->uval.as<uint32_t>(),
                        b->has_hoff ? b->hoff.as<uint8_t>() : nullptr, urep, upos, uid_of_rep, b->rid.as<int64_t>(), k,
-                       hk, hv, errw + 1);
+                       hk, hv, far);
     GX_HIP(hipGetLastError());
-    const unsigned long long far = read1(st, errw + 1);
-    if (far != ~0ull)
-      throw GxError(GX_ENOTSUP, "a read head lies at letter " + std::to_string(far) +
+    unsigned long long fr[kTotLine * kTotLines], most = 0, beyond = 0;
+    GX_HIP(hipMemcpyAsync(fr, far, sizeof(fr), hipMemcpyDeviceToHost, st));
+    GX_HIP(hipStreamSynchronize(st));
+    for (int l = 0; l < kTotLines; l++) {
+      most = std::max(most, fr[kTotLine * l]);
+      beyond = std::max(beyond, fr[kTotLine * l + 1]);
+    }
+    if (beyond)
+      throw GxError(GX_ENOTSUP, "a read head lies at letter " + std::to_string(~beyond) +
                                     " of its unitig; read-head offsets hold 23 bits");
+    auto bits_of = [](uint64_t x) {
+      int n = 0;
+      while (x >> n) n++;
+      return n;
+    };
+    const int offb = bits_of(most), all = bits_of(nu - 1) + offb + b->rid_bits + 2;
+    if (all <= 64) {
+      uint64_t* p1 = reinterpret_cast<uint64_t*>(hk2);  // both buffers of the packed keys
+      uint64_t* p2 = p1 + nh;
+      hipLaunchKernelGGL(k_uhead_pack, dim3(grid_for(nh, kBlock, G)), dim3(kBlock), 0, st, nh, hk, offb, b->rid_bits,
+                         p1);
+      GX_HIP(hipGetLastError());
+      const bool fl = radix_sort<uint64_t>(p1, hv, p2, hv2, nh, 0, (all + 7) / 8,
+                                           scratch_for(b, radix_scratch_bytes<uint64_t>(nh)), st);
+      if (fl) std::swap(hv, hv2);
+      keys.packed = fl ? p2 : p1;
+      keys.offb = offb;
+    } else {
+      const bool fl = radix_sort<Key128>(hk, hv, hk2, hv2, nh, 0, 12, scratch_for(b, radix_scratch_bytes<Key128>(nh)),
+                                         st);
+      if (fl) std::swap(hv, hv2);
+      keys.wide = fl ? hk2 : hk;
+    }
   }
-  bool fl = radix_sort<Key128>(hk, hv, hk2, hv2, nh, 0, 12, scratch_for(b, radix_scratch_bytes<Key128>(nh)), st);
-  if (fl) { std::swap(hk, hk2); std::swap(hv, hv2); }
   uint32_t* uflag = buf<uint32_t>(b->u_uflag, nh + 1);
   uint64_t* uposh = buf<uint64_t>(b->u_uposh, 2 * nh + 2);  // unique heads before each head, and their bytes
   uint64_t* ubytes = uposh + nh + 1;
@@ -4868,7 +4959,7 @@ static void run_unitigs(gx_build* b) {
   GX_HIP(hipMemsetAsync(hu, 0, (nu + 1) * 4, st));
   GX_HIP(hipMemsetAsync(hf, 0, (nu + 1) * 4, st));
   if (nh) {
-    hipLaunchKernelGGL(k_uhead_unique, dim3(grid_for(nh, kBlock, G)), dim3(kBlock), 0, st, nh, hk, hv,
+    hipLaunchKernelGGL(k_uhead_unique, dim3(grid_for(nh, kBlock, G)), dim3(kBlock), 0, st, nh, keys, hv,
                        b->mlen.as<uint32_t>(), uflag, usz, hu, hf);
     GX_HIP(hipGetLastError());
   }
@@ -4880,7 +4971,7 @@ static void run_unitigs(gx_build* b) {
   uint64_t* hbytes = buf<uint64_t>(b->u_hbytes, nh + 1);
   if (nh) {
     hipLaunchKernelGGL(k_uhead_compact, dim3(grid_for(nh, kBlock, G)), dim3(kBlock), 0, st, nh, uflag, uposh, ubytes,
-                       hk, hv, hkey_lo, hval_c, hunit, hbytes);
+                       keys, hv, hkey_lo, hval_c, hunit, hbytes);
     GX_HIP(hipGetLastError());
   }
   if (nu) {

@@ -283,6 +283,109 @@ __device__ __host__ inline uint32_t key_byte(const Key128& k, int b) {
 constexpr int kSortItems = 8;
 constexpr int kSortTile = kBlock * kSortItems;
 
+// Sorts of few elements: one block, every pass in LDS, one launch (three per
+// pass otherwise, 2.5 us each with nothing in between: 12 passes over the
+// 1600 heads of a 5 kbp genome took 100 us).  A wave holds a contiguous run
+// of the elements in registers, so its ranks need no barrier: a match over
+// the digit's bits plus the wave's own count of earlier equal digits; the
+// waves' counts are then summed per digit.
+constexpr int kSmallThreads = 1024, kSmallPer = 4;
+constexpr size_t kSmallSort = (size_t)kSmallThreads * kSmallPer;
+template <class KeyT, bool kVals, class ValT>
+__global__ void __launch_bounds__(kSmallThreads) k_radix_small(KeyT* __restrict__ keys, ValT* __restrict__ vals,
+                                                               uint32_t n, int byte_lo, int byte_hi) {
+  constexpr int kWaves = kSmallThreads / 64;
+  __shared__ KeyT sk[kSmallSort];
+  __shared__ ValT sv[kVals ? kSmallSort : 1];
+  __shared__ uint16_t wcnt[kWaves][256];
+  __shared__ uint32_t base[256], wsum[4];
+  const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
+  const uint64_t lt = (lane == 0) ? 0ull : (~0ull >> (64 - lane));
+  const uint32_t first = (uint32_t)wid * 64 * kSmallPer;
+  KeyT key[kSmallPer];
+  ValT val[kSmallPer];
+#pragma unroll
+  for (int r = 0; r < kSmallPer; r++) {
+    const uint32_t j = first + r * 64 + lane;
+    if (j < n) {
+      key[r] = keys[j];
+      if (kVals) val[r] = vals[j];
+    }
+  }
+  for (int byte = byte_lo; byte < byte_hi; byte++) {
+#pragma unroll
+    for (int q = 0; q < 4; q++) wcnt[wid][q * 64 + lane] = 0;
+    __builtin_amdgcn_wave_barrier();
+    uint32_t rank[kSmallPer], dig[kSmallPer];
+#pragma unroll
+    for (int r = 0; r < kSmallPer; r++) {
+      const bool valid = first + r * 64 + lane < n;
+      const uint32_t d = valid ? key_byte(key[r], byte) : 0;
+      uint64_t match = __ballot(valid);
+#pragma unroll
+      for (int b = 0; b < 8; b++) {
+        const uint64_t m = __ballot((d >> b) & 1);
+        match &= ((d >> b) & 1) ? m : ~m;
+      }
+      // the wave's LDS accesses run in order: read by every lane, then
+      // raised by the group's first
+      const uint32_t before = wcnt[wid][d];
+      rank[r] = before + __popcll(match & lt);
+      dig[r] = d;
+      __builtin_amdgcn_wave_barrier();
+      if (valid && (match & lt) == 0) wcnt[wid][d] = (uint16_t)(before + __popcll(match));
+      __builtin_amdgcn_wave_barrier();
+    }
+    __syncthreads();
+    uint32_t tot = 0, incl = 0;
+    if (threadIdx.x < 256) {
+      for (int w = 0; w < kWaves; w++) {
+        const uint32_t c = wcnt[w][threadIdx.x];
+        wcnt[w][threadIdx.x] = (uint16_t)tot;
+        tot += c;
+      }
+      incl = tot;
+#pragma unroll
+      for (int o = 1; o < 64; o <<= 1) {
+        const uint32_t y = __shfl_up(incl, o);
+        if (lane >= o) incl += y;
+      }
+      if (lane == 63) wsum[wid] = incl;
+    }
+    __syncthreads();
+    if (threadIdx.x < 256) {
+      uint32_t b = incl - tot;
+      for (int w = 0; w < wid; w++) b += wsum[w];
+      base[threadIdx.x] = b;
+    }
+    __syncthreads();
+#pragma unroll
+    for (int r = 0; r < kSmallPer; r++)
+      if (first + r * 64 + lane < n) {
+        const uint32_t pos = base[dig[r]] + wcnt[wid][dig[r]] + rank[r];
+        sk[pos] = key[r];
+        if (kVals) sv[pos] = val[r];
+      }
+    __syncthreads();
+#pragma unroll
+    for (int r = 0; r < kSmallPer; r++) {
+      const uint32_t j = first + r * 64 + lane;
+      if (j < n) {
+        key[r] = sk[j];
+        if (kVals) val[r] = sv[j];
+      }
+    }
+  }
+#pragma unroll
+  for (int r = 0; r < kSmallPer; r++) {
+    const uint32_t j = first + r * 64 + lane;
+    if (j < n) {
+      keys[j] = key[r];
+      if (kVals) vals[j] = val[r];
+    }
+  }
+}
+
 // Tile-local digit bases for a staged scatter: offs is the exclusive scan of
 // the digit-major per-tile counts (entry d * ntiles + tile, total last), so
 // this tile's count of digit d is the difference of two neighbours; lbase[d]
@@ -306,6 +409,47 @@ __device__ inline void tile_digit_bases(const uint64_t* __restrict__ offs, unsig
   for (int w = 0; w < wid; w++) before += wsum[w];
   lbase[threadIdx.x] = (IdxT)before;
   lrun[threadIdx.x] = (IdxT)before;
+}
+
+// The same from the counts themselves (hist, digit-major, not scanned), with
+// each digit's first output position in run: with few tiles every block adds
+// up the counts before its own, which saves the launches of a scan.
+constexpr unsigned kDirectTiles = 64;
+template <class IdxT>
+__device__ inline void tile_digit_bases_direct(const uint32_t* __restrict__ hist, unsigned ntiles, uint64_t* run,
+                                               IdxT* lbase, IdxT* lrun, uint32_t* wsum) {
+  const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
+  uint32_t before = 0, all = 0, mine = 0;
+#pragma unroll 8
+  for (unsigned t = 0; t < ntiles; t++) {
+    const uint32_t c = hist[(size_t)threadIdx.x * ntiles + t];
+    before += t < blockIdx.x ? c : 0;
+    mine = t == blockIdx.x ? c : mine;
+    all += c;
+  }
+  uint32_t ia = all, im = mine;
+#pragma unroll
+  for (int o = 1; o < 64; o <<= 1) {
+    const uint32_t ya = __shfl_up(ia, o), ym = __shfl_up(im, o);
+    if (lane >= o) {
+      ia += ya;
+      im += ym;
+    }
+  }
+  __shared__ uint32_t asum[kBlock / 64];
+  if (lane == 63) {
+    asum[wid] = ia;
+    wsum[wid] = im;
+  }
+  __syncthreads();
+  uint32_t ba = ia - all, bm = im - mine;
+  for (int w = 0; w < wid; w++) {
+    ba += asum[w];
+    bm += wsum[w];
+  }
+  run[threadIdx.x] = (uint64_t)ba + before;
+  lbase[threadIdx.x] = (IdxT)bm;
+  lrun[threadIdx.x] = (IdxT)bm;
 }
 
 template <class KeyT>
@@ -340,9 +484,11 @@ __device__ inline T load_stream(const T* p) {
 // written out as one contiguous run per digit (the tile's share of that
 // digit's output range): scattered element stores would leave lines partly
 // written across rounds, and the partial lines cost extra HBM writes.
-template <class KeyT, bool kVals, class ValT = uint32_t>
+// offs: the scanned counts, or (kDirect) the counts themselves.
+template <class KeyT, bool kVals, class ValT, bool kDirect>
 __global__ void __launch_bounds__(kBlock) k_radix_scatter(const KeyT* __restrict__ keys, const ValT* __restrict__ vals,
-                                                          size_t n, int byte, const uint64_t* __restrict__ offs,
+                                                          size_t n, int byte,
+                                                          const typename std::conditional<kDirect, uint32_t, uint64_t>::type* __restrict__ offs,
                                                           unsigned ntiles, KeyT* __restrict__ okeys,
                                                           ValT* __restrict__ ovals) {
   __shared__ uint64_t run[256];
@@ -351,8 +497,12 @@ __global__ void __launch_bounds__(kBlock) k_radix_scatter(const KeyT* __restrict
   __shared__ KeyT sk[kSortTile];
   __shared__ ValT sv[kVals ? kSortTile : 1];
   const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
-  run[threadIdx.x] = offs[(size_t)threadIdx.x * ntiles + blockIdx.x];
-  tile_digit_bases(offs, ntiles, lbase, lrun, wsum);
+  if constexpr (kDirect) {
+    tile_digit_bases_direct(offs, ntiles, run, lbase, lrun, wsum);
+  } else {
+    run[threadIdx.x] = offs[(size_t)threadIdx.x * ntiles + blockIdx.x];
+    tile_digit_bases(offs, ntiles, lbase, lrun, wsum);
+  }
   const uint64_t lt = (lane == 0) ? 0ull : (~0ull >> (64 - lane));
   size_t base = (size_t)blockIdx.x * kSortTile;
   for (int r = 0; r < kSortItems; r++) {
@@ -410,10 +560,16 @@ static size_t radix_scratch_bytes(size_t n) {
 
 // Sorts (keys, vals) by bytes [byte_lo, byte_hi).  Uses (k2, v2) as the
 // ping-pong buffers; returns true when the result ended in (k2, v2).
-template <class KeyT, class ValT = uint32_t>
-static bool radix_sort(KeyT* k1, ValT* v1, KeyT* k2, ValT* v2, size_t n, int byte_lo, int byte_hi,
-                       char* scratch, hipStream_t st) {
-  if (n <= 1) return false;
+template <class KeyT, bool kVals, class ValT>
+static bool radix_sort_impl(KeyT* k1, ValT* v1, KeyT* k2, ValT* v2, size_t n, int byte_lo, int byte_hi, char* scratch,
+                            hipStream_t st) {
+  if (n <= 1 || byte_lo >= byte_hi) return false;
+  if (n <= kSmallSort) {
+    hipLaunchKernelGGL((k_radix_small<KeyT, kVals, ValT>), dim3(1), dim3(kSmallThreads), 0, st, k1, v1, (uint32_t)n,
+                       byte_lo, byte_hi);
+    GX_HIP(hipGetLastError());
+    return false;
+  }
   unsigned ntiles = (unsigned)((n + kSortTile - 1) / kSortTile);
   size_t h = (size_t)256 * ntiles;
   uint32_t* hist = reinterpret_cast<uint32_t*>(scratch);
@@ -427,17 +583,25 @@ static bool radix_sort(KeyT* k1, ValT* v1, KeyT* k2, ValT* v2, size_t n, int byt
     ValT* ov = flip ? v1 : v2;
     hipLaunchKernelGGL((k_radix_hist<KeyT>), dim3(ntiles), dim3(kBlock), 0, st, ik, n, b, hist, ntiles);
     GX_HIP(hipGetLastError());
-    exclusive_scan<uint32_t, uint64_t>(hist, offs, h, sc, st);
-    if (v1)
-      hipLaunchKernelGGL((k_radix_scatter<KeyT, true, ValT>), dim3(ntiles), dim3(kBlock), 0, st, ik, iv, n, b, offs,
-                         ntiles, ok, ov);
-    else
-      hipLaunchKernelGGL((k_radix_scatter<KeyT, false, ValT>), dim3(ntiles), dim3(kBlock), 0, st, ik, iv, n, b,
+    if (ntiles <= kDirectTiles) {
+      hipLaunchKernelGGL((k_radix_scatter<KeyT, kVals, ValT, true>), dim3(ntiles), dim3(kBlock), 0, st, ik, iv, n, b,
+                         hist, ntiles, ok, ov);
+    } else {
+      exclusive_scan<uint32_t, uint64_t>(hist, offs, h, sc, st);
+      hipLaunchKernelGGL((k_radix_scatter<KeyT, kVals, ValT, false>), dim3(ntiles), dim3(kBlock), 0, st, ik, iv, n, b,
                          offs, ntiles, ok, ov);
+    }
     GX_HIP(hipGetLastError());
     flip = !flip;
   }
   return flip;
+}
+
+template <class KeyT, class ValT = uint32_t>
+static bool radix_sort(KeyT* k1, ValT* v1, KeyT* k2, ValT* v2, size_t n, int byte_lo, int byte_hi,
+                       char* scratch, hipStream_t st) {
+  return v1 ? radix_sort_impl<KeyT, true, ValT>(k1, v1, k2, v2, n, byte_lo, byte_hi, scratch, st)
+            : radix_sort_impl<KeyT, false, ValT>(k1, v1, k2, v2, n, byte_lo, byte_hi, scratch, st);
 }
 
 }  // namespace gx

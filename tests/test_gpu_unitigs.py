@@ -238,3 +238,34 @@ def test_node_index_of_uneven_buckets(gx, k, n):
     g = "".join(rng.choice("ACGT") for _ in range(3000))
     lines += [g[p:p + 100] for p in range(0, 2900, 20)]
     check(gx, "".join(f"{4 * i + 2}\t{s}\n" for i, s in enumerate(lines)).encode(), k)
+
+
+@pytest.mark.parametrize("n", [2, 4095, 4097, 131072, 131073])
+def test_head_sorts_of_every_size(gx, n):
+    """Read heads at the edges of the sorts: one block for all passes, few
+    tiles whose blocks add up the digit counts themselves, scanned counts;
+    many reads share a first k-mer and some repeat a readId."""
+    rng = random.Random(n)
+    k = 21
+    g = "".join(rng.choice("ACGT") for _ in range(400))
+    lines = []
+    for i in range(n):
+        p = rng.randrange(len(g) - 24)
+        s = g[p:p + 24]
+        rid = 4 * i + 2 if i % 50 else 2
+        lines.append(f"{rid}\t{s if rng.random() < 0.5 else rc(s)}\n")
+    check(gx, "".join(lines).encode(), k)
+
+
+def test_head_keys_wider_than_a_word(gx):
+    """Offsets of 20 bits, 29-bit readIds and more than 2^13 unitigs: the
+    unitig heads' sort keys need more than 64 bits."""
+    rng = random.Random(8)
+    k = 21
+    G = (1 << 19) + 3000
+    g = "".join(rng.choices("ACGT", k=G))
+    reads = [g[p:p + 100] for p in range(0, G - 99, 79)] + [g[-100:]]
+    reads += ["".join(rng.choices("ACGT", k=24)) for _ in range(9000)]
+    top = (1 << 29) - 1
+    text = "".join(f"{top - 3 * i}\t{s if rng.random() < 0.5 else rc(s)}\n" for i, s in enumerate(reads)).encode()
+    check(gx, text, k)

@@ -1512,11 +1512,14 @@ __global__ void k_big_move(const uint64_t* __restrict__ bstart, const uint32_t* 
   }
 }
 
-__global__ void k_big_sizes(uint32_t NB, const uint64_t* __restrict__ bstart, const uint32_t* __restrict__ big,
-                            uint64_t* __restrict__ sz) {
-  for (uint32_t b = blockIdx.x * blockDim.x + threadIdx.x; b < NB; b += gridDim.x * blockDim.x)
-    sz[b] = (big[b] == 1 && bstart[b + 1] >= bstart[b]) ? bstart[b + 1] - bstart[b] : 0;
-}
+// Records of an oversized bucket (0 for the others).
+struct BigSize {
+  const uint64_t* bstart;
+  const uint32_t* big;
+  __device__ inline uint64_t operator()(size_t b) const {
+    return (big[b] == 1 && bstart[b + 1] >= bstart[b]) ? bstart[b + 1] - bstart[b] : 0;
+  }
+};
 
 // Nodes are the runs of equal keys in the sorted records.  Run starts per
 // chunk of kEmitChunk records (a record starts a run when its key differs
@@ -2081,11 +2084,11 @@ __global__ void k_head_compact(uint64_t nh, const uint64_t* __restrict__ hkey, c
   }
 }
 
-__global__ void k_head_total(uint64_t nn, const uint32_t* __restrict__ hcu, const uint32_t* __restrict__ hcf,
-                             uint64_t* __restrict__ tot) {
-  for (uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; i < nn; i += (uint64_t)gridDim.x * blockDim.x)
-    tot[i] = (uint64_t)hcu[i] + hcf[i];
-}
+// Heads of a node or unitig.
+struct HeadTotal {
+  const uint32_t *u, *f;
+  __device__ inline uint64_t operator()(size_t i) const { return (uint64_t)u[i] + f[i]; }
+};
 
 // ---------------------------------------------------------------------------
 // 8. Node serialisation (Node.write, Node.java:408-487; VKmerList.write
@@ -2380,17 +2383,18 @@ __global__ void __launch_bounds__(kBlock) k_rid_max(uint64_t nlines, const int64
   }
 }
 
-// words per mate for the packed store
-__global__ void k_word_counts(uint64_t nmates, const uint32_t* __restrict__ mlen, uint64_t* __restrict__ wc) {
-  for (uint64_t m = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; m < nmates; m += (uint64_t)gridDim.x * blockDim.x)
-    wc[m] = (mlen[m] + 31) / 32 + 1;  // +1: k-mer loads may touch one word past the end
-}
+// words per mate for the packed store (+1: k-mer loads may touch one word past the end)
+struct MateWords {
+  const uint32_t* mlen;
+  __device__ inline uint64_t operator()(size_t m) const { return (mlen[m] + 31) / 32 + 1; }
+};
 
-__global__ void k_valid_u64(uint64_t nmates, const uint8_t* __restrict__ valid, const uint64_t* __restrict__ nocc,
-                            uint64_t* __restrict__ out) {
-  for (uint64_t m = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; m < nmates; m += (uint64_t)gridDim.x * blockDim.x)
-    out[m] = (valid[m] && nocc[m]) ? 1 : 0;
-}
+// 1 for a mate with k-mers
+struct MateHead {
+  const uint8_t* valid;
+  const uint64_t* nocc;
+  __device__ inline uint64_t operator()(size_t m) const { return (valid[m] && nocc[m]) ? 1 : 0; }
+};
 
 // ===========================================================================
 // Unitig compression (MERGE / P4 path merge) on the built graph.
@@ -3518,11 +3522,11 @@ struct gx_build {
   uint64_t src_len = 0;
   bool finished = false;
   // device buffers (grown on demand, reused across builds)
-  DevBuf text, scratch, blk, blk2, term, rid, mstart, mlen, wcnt, wbase, words, valid, nocc, occbase, hmask, hidx;
+  DevBuf text, scratch, blk, blk2, term, rid, mstart, mlen, wbase, words, valid, nocc, occbase, hidx;
   DevBuf table, occ_slot, occ_code, claimed;
   DevBuf ckey, cval, ckey2, cval2, nslot, klo, khi, cnt, msk, needs, selcnt, seg;
   DevBuf selflag, selpos, selk, selv, selk2, selv2, lists, rtot, rkey, rval, rkey2, rval2;
-  DevBuf hkey, hval, hkey2, hval2, uflag, upos, uval, hcu, hcf, htot, hstart, rsize, roff, out;
+  DevBuf hkey, hval, hkey2, hval2, uflag, upos, uval, hcu, hcf, hstart, rsize, roff, out;
   DevBuf errw;
   uint64_t stats[16] = {};
   // per-phase device timings (hipEvents on the handle's stream)
@@ -3535,7 +3539,7 @@ struct gx_build {
   // unitig pass
   DevBuf u_lnk, u_tand, u_cut, u_ptr[2], u_flag, u_any, u_rep, u_pos, u_isrep, u_lenrep, u_walk, u_walk2;
   DevBuf u_uid, u_repnode, u_len, u_base, u_order, u_cov, u_edge, u_ecnt, u_hk, u_hk2, u_hv, u_hv2, u_uflag, u_uposh;
-  DevBuf u_hu, u_hf, u_htot, u_hstart, u_hklo, u_hvc, u_rsize, u_roff, u_out;
+  DevBuf u_hu, u_hf, u_hstart, u_hklo, u_hvc, u_rsize, u_roff, u_out;
   int rid_bits = 29;  // of the largest readId of the build's input
   uint64_t nuheads = 0, u_bytes = 0, u_count = 0, u_rounds = 0, u_succ_reads = 0, u_walkers = 0;
   bool no_walk = false;  // rank by pointer jumping only (GX_UNITIG_RANK_POINTER_JUMPING)
@@ -3561,7 +3565,7 @@ struct gx_build {
   DevBuf blist;               // record sort: buckets listed for the larger LDS tiers
   DevBuf hist2;               // key ranges: the next range's per-tile digit counts
   // graph cleaning: the compacted graph; key ranges: the node graph of the ranges so far
-  DevBuf c_keep, c_pos, c_klo, c_khi, c_cnt, c_msk, c_hcu, c_hcf, c_htot, c_hstart, c_uval;
+  DevBuf c_keep, c_pos, c_klo, c_khi, c_cnt, c_msk, c_hcu, c_hcf, c_hstart, c_uval;
   DevBuf hoff, c_hoff;  // per node head: its letter in the node's k-mer (after a bubble merge)
   DevBuf bb_min, bb_maj, bb_typ, bb_np, bb_pbase, bb_pairs, bb_ed, bb_into, bb_hn, bb_hb, bb_addu, bb_addf, bb_cur,
       bb_tot, bb_astart, bb_hnode, bb_hmv, bb_hofs, bb_aval, bb_aoff;  // bubble merge
@@ -3808,19 +3812,19 @@ static void for_each_buf(gx_build* b, F&& f) {
   f(&b->u_ptr[1]);
   for (DevBuf* d :
        {&b->text2, &b->rtext, &b->fterm1, &b->fterm2, &b->fsz, &b->foff, &b->text, &b->scratch, &b->blk, &b->blk2,
-        &b->term, &b->rid, &b->mstart, &b->mlen, &b->wcnt, &b->wbase, &b->words, &b->valid, &b->nocc, &b->occbase,
-        &b->hmask, &b->hidx, &b->table, &b->occ_slot, &b->occ_code, &b->claimed, &b->ckey, &b->cval, &b->ckey2,
+        &b->term, &b->rid, &b->mstart, &b->mlen, &b->wbase, &b->words, &b->valid, &b->nocc, &b->occbase,
+        &b->hidx, &b->table, &b->occ_slot, &b->occ_code, &b->claimed, &b->ckey, &b->cval, &b->ckey2,
         &b->cval2, &b->nslot, &b->klo, &b->khi, &b->cnt, &b->msk, &b->needs, &b->selcnt, &b->seg, &b->selflag,
         &b->selpos, &b->selk, &b->selv, &b->selk2, &b->selv2, &b->lists, &b->rtot, &b->rkey, &b->rval, &b->rkey2,
         &b->rval2, &b->hkey, &b->hval, &b->hkey2, &b->hval2, &b->uflag, &b->upos, &b->uval, &b->hcu, &b->hcf,
-        &b->htot, &b->hstart, &b->rsize, &b->roff, &b->out, &b->errw, &b->u_lnk, &b->u_tand, &b->u_cut, &b->u_flag,
+        &b->hstart, &b->rsize, &b->roff, &b->out, &b->errw, &b->u_lnk, &b->u_tand, &b->u_cut, &b->u_flag,
         &b->u_any, &b->u_rep, &b->u_pos, &b->u_isrep, &b->u_lenrep, &b->u_uid, &b->u_repnode, &b->u_len,
         &b->u_base, &b->u_order, &b->u_cov, &b->u_edge, &b->u_ecnt, &b->u_hk, &b->u_hk2, &b->u_hv, &b->u_hv2,
-        &b->u_uflag, &b->u_uposh, &b->u_hu, &b->u_hf, &b->u_htot, &b->u_hstart, &b->u_hklo, &b->u_hvc, &b->u_rsize,
+        &b->u_uflag, &b->u_uposh, &b->u_hu, &b->u_hf, &b->u_hstart, &b->u_hklo, &b->u_hvc, &b->u_rsize,
         &b->u_roff, &b->u_out, &b->ppid, &b->pidx, &b->ppid2, &b->pidx2, &b->pbound, &b->sva, &b->svb,
         &b->nix_dir, &b->nix_slots, &b->rcode, &b->u_seqat, &b->u_hbytes, &b->u_chunk, &b->u_far, &b->tophist, &b->outacc, &b->blist, &b->hist2,
         &b->hregs, &b->sfeat, &b->spred, &b->c_keep, &b->c_pos, &b->c_klo, &b->c_khi, &b->c_cnt, &b->c_msk,
-        &b->c_hcu, &b->c_hcf, &b->c_htot, &b->c_hstart, &b->c_uval, &b->hoff, &b->c_hoff, &b->bb_min, &b->bb_maj,
+        &b->c_hcu, &b->c_hcf, &b->c_hstart, &b->c_uval, &b->hoff, &b->c_hoff, &b->bb_min, &b->bb_maj,
         &b->bb_typ, &b->bb_np, &b->bb_pbase, &b->bb_pairs, &b->bb_ed, &b->bb_into, &b->bb_hn, &b->bb_hb,
         &b->bb_addu, &b->bb_addf, &b->bb_cur, &b->bb_tot, &b->bb_astart, &b->bb_hnode, &b->bb_hmv, &b->bb_hofs,
         &b->bb_aval, &b->bb_aoff, &b->u_headat, &b->s_acc, &b->s_k1, &b->s_k2,
@@ -3887,13 +3891,8 @@ static void run_build(gx_build* b) {
     GX_HIP(hipGetLastError());
   }
   // 3. pack
-  uint64_t* wcnt = buf<uint64_t>(b->wcnt, nmates + 1);
   uint64_t* wbase = buf<uint64_t>(b->wbase, nmates + 1 + kRidBlocks);  // and the blocks' largest readIds
-  if (nmates) {
-    hipLaunchKernelGGL(k_word_counts, dim3(grid_for(nmates, kBlock, G)), dim3(kBlock), 0, st, nmates, mlen, wcnt);
-    GX_HIP(hipGetLastError());
-  }
-  exclusive_scan<uint64_t, uint64_t>(wcnt, wbase, nmates, scratch_for(b, scan_scratch_bytes<uint64_t>(nmates)), st);
+  exclusive_scan_of<uint64_t>(MateWords{mlen}, wbase, nmates, scratch_for(b, scan_scratch_bytes<uint64_t>(nmates)), st);
   const unsigned rblocks = grid_for(nlines, kBlock, kRidBlocks);
   hipLaunchKernelGGL(k_rid_max, dim3(rblocks), dim3(kBlock), 0, st, nlines, rid, wbase + nmates + 1);
   GX_HIP(hipGetLastError());
@@ -3917,13 +3916,9 @@ static void run_build(gx_build* b) {
   uint64_t* occbase = buf<uint64_t>(b->occbase, nmates + 1);
   exclusive_scan<uint64_t, uint64_t>(nocc, occbase, nmates, scratch_for(b, scan_scratch_bytes<uint64_t>(nmates)), st);
   uint64_t N = read1(st, occbase + nmates);
-  uint64_t* hm = buf<uint64_t>(b->hmask, nmates + 1);
   uint64_t* hidx = buf<uint64_t>(b->hidx, nmates + 1);
-  if (nmates) {
-    hipLaunchKernelGGL(k_valid_u64, dim3(grid_for(nmates, kBlock, G)), dim3(kBlock), 0, st, nmates, valid, nocc, hm);
-    GX_HIP(hipGetLastError());
-  }
-  exclusive_scan<uint64_t, uint64_t>(hm, hidx, nmates, scratch_for(b, scan_scratch_bytes<uint64_t>(nmates)), st);
+  exclusive_scan_of<uint64_t>(MateHead{valid, nocc}, hidx, nmates, scratch_for(b, scan_scratch_bytes<uint64_t>(nmates)),
+                              st);
   uint64_t nheads = read1(st, hidx + nmates);
 
   // 3b. sizing features: HLL sketch of the first 1% of the mates (at least
@@ -3992,8 +3987,8 @@ static void run_build(gx_build* b) {
     size_t fr = 0, tot = 0;
     GX_HIP(hipMemGetInfo(&fr, &tot));
     size_t live = 0;
-    for (DevBuf* d : {&b->text, &b->text2, &b->rtext, &b->term, &b->rid, &b->mstart, &b->mlen, &b->wcnt, &b->wbase,
-                      &b->words, &b->valid, &b->nocc, &b->occbase, &b->hmask, &b->hidx})
+    for (DevBuf* d : {&b->text, &b->text2, &b->rtext, &b->term, &b->rid, &b->mstart, &b->mlen, &b->wbase,
+                      &b->words, &b->valid, &b->nocc, &b->occbase, &b->hidx})
       live += d->cap;
     return (double)fr + (double)handle_bytes(b) - (double)live - kept - 0.1 * (double)tot - 48.0 * (double)nheads -
            16.0 * 256.0 * tiles;
@@ -4163,7 +4158,6 @@ static void run_build(gx_build* b) {
     const uint32_t bk0 = tlo << (8 * (bkb - 1)), bk1 = thi << (8 * (bkb - 1));
     uint64_t* bstart = buf<uint64_t>(b->hstart, NBK + 2);
     uint32_t* big = buf<uint32_t>(b->hcu, NBK + 1);
-    uint64_t* bsz = buf<uint64_t>(b->htot, NBK + 1);
     uint64_t* boff = buf<uint64_t>(b->upos, NBK + 2);
     GX_HIP(hipMemsetAsync(big, 0, (NBK + 1) * 4, st));
     hipLaunchKernelGGL(k_bucket_starts<SK>, dim3(grid_for(Nr + 1, kBlock, G)), dim3(kBlock), 0, st, Nr, kx, nb, bkb,
@@ -4203,9 +4197,7 @@ static void run_build(gx_build* b) {
       GX_HIP(hipGetLastError());
     }
     if (read1(st, errw + 2) != ~0ull) throw GxError(GX_EDEVICE, "internal error: unordered bucket bounds or lists");
-    hipLaunchKernelGGL(k_big_sizes, dim3(grid_for(NBK, kBlock, G)), dim3(kBlock), 0, st, NBK, bstart, big, bsz);
-    GX_HIP(hipGetLastError());
-    exclusive_scan<uint64_t, uint64_t>(bsz, boff, NBK, scratch_for(b, scan_scratch_bytes<uint64_t>(NBK)), st);
+    exclusive_scan_of<uint64_t>(BigSize{bstart, big}, boff, NBK, scratch_for(b, scan_scratch_bytes<uint64_t>(NBK)), st);
     const uint64_t nbig = read1(st, boff + NBK);
     if (nbig) {
       SK* tk = buf<SK>(b->hkey, nbig + 1);
@@ -4472,7 +4464,6 @@ static void run_build(gx_build* b) {
   uint32_t* uval = buf<uint32_t>(b->uval, nheads + 1);
   uint32_t* hcu = buf<uint32_t>(b->hcu, nn + 1);
   uint32_t* hcf = buf<uint32_t>(b->hcf, nn + 1);
-  uint64_t* htot = buf<uint64_t>(b->htot, nn + 1);
   uint64_t* hstart = buf<uint64_t>(b->hstart, nn + 1);
   GX_HIP(hipMemsetAsync(hcu, 0, (nn + 1) * 4, st));
   GX_HIP(hipMemsetAsync(hcf, 0, (nn + 1) * 4, st));
@@ -4488,11 +4479,7 @@ static void run_build(gx_build* b) {
                        uval, hcu, hcf, b->rid_bits);
     GX_HIP(hipGetLastError());
   }
-  if (nn) {
-    hipLaunchKernelGGL(k_head_total, dim3(grid_for(nn, kBlock, G)), dim3(kBlock), 0, st, nn, hcu, hcf, htot);
-    GX_HIP(hipGetLastError());
-  }
-  exclusive_scan<uint64_t, uint64_t>(htot, hstart, nn, scratch_for(b, scan_scratch_bytes<uint64_t>(nn)), st);
+  exclusive_scan_of<uint64_t>(HeadTotal{hcu, hcf}, hstart, nn, scratch_for(b, scan_scratch_bytes<uint64_t>(nn)), st);
   ph_end(b, PH_HEADS);
   // head sort arrays are dead; with several key ranges so is the range's
   // node index (rebuilt over the whole graph after the last range)
@@ -4608,7 +4595,7 @@ static void run_build(gx_build* b) {
     b->reclaim.dead.insert(b->reclaim.dead.end(),
                            {&b->klo, &b->khi, &b->cnt, &b->msk, &b->nslot, &b->nix_slots, &b->needs, &b->selcnt,
                             &b->seg, &b->lists, &b->rkey, &b->rval, &b->rkey2, &b->rval2, &b->rcode,
-                            &b->hcu, &b->hcf, &b->htot, &b->hstart, &b->uval, &b->rsize, &b->roff, &b->out, &b->ppid,
+                            &b->hcu, &b->hcf, &b->hstart, &b->uval, &b->rsize, &b->roff, &b->out, &b->ppid,
                             &b->pidx, &b->ppid2, &b->pidx2});
   }  // key ranges
 
@@ -4647,14 +4634,9 @@ static void run_build(gx_build* b) {
     }
     const uint64_t nn = tot_nn;
     if (nn < 0xffffffffull) {  // the node index and the graph steps number nodes in 32 bits
-      uint64_t* htot = buf<uint64_t>(b->htot, nn + 1);
       uint64_t* hstart = buf<uint64_t>(b->hstart, nn + 1);
-      if (nn) {
-        hipLaunchKernelGGL(k_head_total, dim3(grid_for(nn, kBlock, G)), dim3(kBlock), 0, st, nn,
-                           b->hcu.as<uint32_t>(), b->hcf.as<uint32_t>(), htot);
-        GX_HIP(hipGetLastError());
-      }
-      exclusive_scan<uint64_t, uint64_t>(htot, hstart, nn, scratch_for(b, scan_scratch_bytes<uint64_t>(nn)), st);
+      exclusive_scan_of<uint64_t>(HeadTotal{b->hcu.as<uint32_t>(), b->hcf.as<uint32_t>()}, hstart, nn,
+                                  scratch_for(b, scan_scratch_bytes<uint64_t>(nn)), st);
       ph_begin(b, PH_NIX);
       build_node_index<W>(b, b->st, nn, b->klo.as<uint64_t>(), W == 2 ? b->khi.as<uint64_t>() : nullptr,
                           b->msk.as<uint32_t>(), 0u, 256u);
@@ -4954,7 +4936,6 @@ static void run_unitigs(gx_build* b) {
   uint32_t* usz = hv2;  // the sort's spare buffer
   uint32_t* hu = buf<uint32_t>(b->u_hu, nu + 1);
   uint32_t* hf = buf<uint32_t>(b->u_hf, nu + 1);
-  uint64_t* htot = buf<uint64_t>(b->u_htot, nu + 1);
   uint64_t* hstart = buf<uint64_t>(b->u_hstart, nu + 1);
   GX_HIP(hipMemsetAsync(hu, 0, (nu + 1) * 4, st));
   GX_HIP(hipMemsetAsync(hf, 0, (nu + 1) * 4, st));
@@ -4974,11 +4955,7 @@ static void run_unitigs(gx_build* b) {
                        keys, hv, hkey_lo, hval_c, hunit, hbytes);
     GX_HIP(hipGetLastError());
   }
-  if (nu) {
-    hipLaunchKernelGGL(k_head_total, dim3(grid_for(nu, kBlock, G)), dim3(kBlock), 0, st, nu, hu, hf, htot);
-    GX_HIP(hipGetLastError());
-  }
-  exclusive_scan<uint64_t, uint64_t>(htot, hstart, nu, scratch_for(b, scan_scratch_bytes<uint64_t>(nu)), st);
+  exclusive_scan_of<uint64_t>(HeadTotal{hu, hf}, hstart, nu, scratch_for(b, scan_scratch_bytes<uint64_t>(nu)), st);
   // records (they list the outer edges)
   stream_after(st, b->st2, b->ev_join);
   USerCtx c;
@@ -5228,7 +5205,7 @@ __global__ void k_keep_nodes(uint64_t nn, const uint32_t* __restrict__ keep, con
                              const uint32_t* __restrict__ hcu, const uint32_t* __restrict__ hcf, AddedHeads ah,
                              uint64_t* __restrict__ klo2, uint64_t* __restrict__ khi2, uint32_t* __restrict__ cnt2,
                              uint32_t* __restrict__ msk2, uint32_t* __restrict__ hcu2, uint32_t* __restrict__ hcf2,
-                             uint64_t* __restrict__ htot2, unsigned long long* err) {
+                             unsigned long long* err) {
   for (uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; i < nn; i += (uint64_t)gridDim.x * blockDim.x) {
     if (!keep[i]) continue;
     const uint64_t j = pos[i];
@@ -5248,7 +5225,6 @@ __global__ void k_keep_nodes(uint64_t nn, const uint32_t* __restrict__ keep, con
     const uint32_t nu = hcu[i] + (ah.addu ? ah.addu[i] : 0u), nf = hcf[i] + (ah.addf ? ah.addf[i] : 0u);
     hcu2[j] = nu;
     hcf2[j] = nf;
-    htot2[j] = (uint64_t)nu + nf;
   }
 }
 
@@ -5302,16 +5278,15 @@ static void compact_graph(gx_build* b, uint32_t* keep, const AddedHeads& ah) {
   uint32_t* msk2 = buf<uint32_t>(b->c_msk, nn2 + 1);
   uint32_t* hcu2 = buf<uint32_t>(b->c_hcu, nn2 + 1);
   uint32_t* hcf2 = buf<uint32_t>(b->c_hcf, nn2 + 1);
-  uint64_t* htot2 = buf<uint64_t>(b->c_htot, nn2 + 1);
   uint64_t* hstart2 = buf<uint64_t>(b->c_hstart, nn2 + 1);
   if (nn) {
     hipLaunchKernelGGL(k_keep_nodes<W>, dim3(grid_for(nn, kBlock, G)), dim3(kBlock), 0, st, nn, keep, pos,
                        b->klo.as<uint64_t>(), W == 2 ? b->khi.as<uint64_t>() : nullptr, b->cnt.as<uint32_t>(),
                        b->msk.as<uint32_t>(), nix, b->cfg.k, b->hcu.as<uint32_t>(), b->hcf.as<uint32_t>(), ah, klo2,
-                       khi2, cnt2, msk2, hcu2, hcf2, htot2, errw);
+                       khi2, cnt2, msk2, hcu2, hcf2, errw);
     GX_HIP(hipGetLastError());
   }
-  exclusive_scan<uint64_t, uint64_t>(htot2, hstart2, nn2, scratch_for(b, scan_scratch_bytes<uint64_t>(nn2)), st);
+  exclusive_scan_of<uint64_t>(HeadTotal{hcu2, hcf2}, hstart2, nn2, scratch_for(b, scan_scratch_bytes<uint64_t>(nn2)), st);
   const uint64_t nh2 = read1(st, hstart2 + nn2);
   uint32_t* uval2 = buf<uint32_t>(b->c_uval, nh2 + 1);
   const bool offs = b->has_hoff || ah.aval;  // heads at letters other than the build's

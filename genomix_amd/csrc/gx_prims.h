@@ -146,15 +146,24 @@ static inline unsigned grid_for(size_t n, size_t per_block, unsigned cap = 1u <<
 }
 
 // ---------------------------------------------------------------------------
-// Exclusive scan: out[i] = sum(in[0..i)), out[n] = total.  out may not alias in.
+// Exclusive scan: out[i] = sum(in[0..i)), out[n] = total.  out may not alias
+// what in reads.  `in` is any device functor of the element number, so that
+// a value made of a few others needs no array and launch of its own; it is
+// called twice per element.
 // ---------------------------------------------------------------------------
 
 constexpr int kScanItems = 8;
 constexpr int kScanTile = kBlock * kScanItems;
 
-template <class T>
+template <class Tin>
+struct ScanArray {
+  const Tin* __restrict__ p;
+  __device__ inline Tin operator()(size_t i) const { return p[i]; }
+};
+
+template <class T, int kThreads = kBlock>
 __device__ inline T block_exclusive_scan(T v, T* total) {
-  __shared__ T wsum[kBlock / 64];
+  __shared__ T wsum[kThreads / 64];
   const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
   T x = v;
 #pragma unroll
@@ -166,7 +175,7 @@ __device__ inline T block_exclusive_scan(T v, T* total) {
   __syncthreads();
   T before = 0, all = 0;
 #pragma unroll
-  for (int w = 0; w < kBlock / 64; w++) {
+  for (int w = 0; w < kThreads / 64; w++) {
     if (w < wid) before += wsum[w];
     all += wsum[w];
   }
@@ -175,14 +184,14 @@ __device__ inline T block_exclusive_scan(T v, T* total) {
   return before + x - v;
 }
 
-template <class Tin, class T>
-__global__ void __launch_bounds__(kBlock) k_scan_reduce(const Tin* __restrict__ in, size_t n, T* __restrict__ part) {
+template <class In, class T>
+__global__ void __launch_bounds__(kBlock) k_scan_reduce(In in, size_t n, T* __restrict__ part) {
   size_t base = (size_t)blockIdx.x * kScanTile;
   T s = 0;
 #pragma unroll
   for (int i = 0; i < kScanItems; i++) {
     size_t j = base + (size_t)i * kBlock + threadIdx.x;
-    if (j < n) s += (T)in[j];
+    if (j < n) s += (T)in(j);
   }
   T tot;
   (void)block_exclusive_scan<T>(s, &tot);
@@ -194,8 +203,10 @@ __global__ void __launch_bounds__(kBlock) k_scan_reduce(const Tin* __restrict__ 
 // scanned with each thread on kScanItems consecutive elements.  Tile
 // position q sits at LDS slot q + q / kScanItems, so the threads' runs of
 // kScanItems fall on different banks.
-template <class Tin, class T>
-__global__ void __launch_bounds__(kBlock) k_scan_apply(const Tin* __restrict__ in, size_t n, const T* __restrict__ part,
+// part: the tiles' sums, scanned, or (kSumParts) as they are: each block
+// then adds up those before its own.
+template <class In, class T, bool kSumParts>
+__global__ void __launch_bounds__(kBlock) k_scan_apply(In in, size_t n, const T* __restrict__ part,
                                                        T* __restrict__ out) {
   __shared__ T tile[kScanTile + kBlock];
   const size_t base = (size_t)blockIdx.x * kScanTile;
@@ -203,7 +214,7 @@ __global__ void __launch_bounds__(kBlock) k_scan_apply(const Tin* __restrict__ i
   for (int i = 0; i < kScanItems; i++) {
     const uint32_t q = (uint32_t)(i * kBlock + threadIdx.x);
     const size_t j = base + q;
-    tile[q + q / kScanItems] = j < n ? (T)in[j] : (T)0;
+    tile[q + q / kScanItems] = j < n ? (T)in(j) : (T)0;
   }
   __syncthreads();
   const uint32_t run = threadIdx.x * (kScanItems + 1);  // slot of this thread's first element
@@ -214,8 +225,15 @@ __global__ void __launch_bounds__(kBlock) k_scan_apply(const Tin* __restrict__ i
     v[i] = tile[run + i];
     s += v[i];
   }
-  T tot;
-  T ex = block_exclusive_scan<T>(s, &tot) + (part ? part[blockIdx.x] : (T)0);
+  T tot, before = 0;
+  if constexpr (kSumParts) {
+    T mine = 0;
+    for (uint32_t q = threadIdx.x; q < blockIdx.x; q += kBlock) mine += part[q];
+    (void)block_exclusive_scan<T>(mine, &before);
+  } else {
+    before = part[blockIdx.x];
+  }
+  T ex = block_exclusive_scan<T>(s, &tot) + before;
 #pragma unroll
   for (int i = 0; i < kScanItems; i++) {  // the thread's own slots: no other thread reads them
     tile[run + i] = ex;
@@ -242,25 +260,64 @@ static size_t scan_scratch_bytes(size_t n) {
   return b + 256;
 }
 
-template <class Tin, class T>
-static void exclusive_scan(const Tin* in, T* out, size_t n, char* scratch, hipStream_t st) {
-  size_t tiles = (n + kScanTile - 1) / kScanTile;
-  if (tiles == 0) tiles = 1;
-  if (tiles == 1) {
-    hipLaunchKernelGGL((k_scan_apply<Tin, T>), dim3(1), dim3(kBlock), 0, st, in, n, (const T*)nullptr, out);
+// Short inputs: one block, tile after tile.
+constexpr int kScanOneThreads = 1024;
+constexpr size_t kScanOne = 2 * (size_t)kScanOneThreads * kScanItems;
+template <class In, class T>
+__global__ void __launch_bounds__(kScanOneThreads) k_scan_one(In in, size_t n, T* __restrict__ out) {
+  T carry = 0;
+  for (size_t base = 0; base < n; base += (size_t)kScanOneThreads * kScanItems) {
+    const size_t j0 = base + (size_t)threadIdx.x * kScanItems;
+    T v[kScanItems], s = 0, tot;
+#pragma unroll
+    for (int i = 0; i < kScanItems; i++) {
+      v[i] = j0 + i < n ? (T)in(j0 + i) : (T)0;
+      s += v[i];
+    }
+    T ex = block_exclusive_scan<T, kScanOneThreads>(s, &tot) + carry;
+#pragma unroll
+    for (int i = 0; i < kScanItems; i++) {
+      if (j0 + i < n) out[j0 + i] = ex;
+      ex += v[i];
+    }
+    carry += tot;
+  }
+  if (threadIdx.x == 0) out[n] = carry;
+}
+
+// One launch up to kScanOne elements, two (the tiles' sums, then the tiles)
+// while a block can add up the sums before its own, 2048 at most; beyond
+// that the sums are scanned in between.  (A launch costs 2.5 us: three of
+// them bounded every scan of a small graph.)
+constexpr size_t kSumTiles = 2048;
+template <class T, class In>
+static void exclusive_scan_of(In in, T* out, size_t n, char* scratch, hipStream_t st) {
+  if (n <= kScanOne) {
+    hipLaunchKernelGGL((k_scan_one<In, T>), dim3(1), dim3(kScanOneThreads), 0, st, in, n, out);
     GX_HIP(hipGetLastError());
     return;
   }
+  const size_t tiles = (n + kScanTile - 1) / kScanTile;
   T* part = reinterpret_cast<T*>(scratch);
   T* partscan = part + (tiles + 1);
   char* next = reinterpret_cast<char*>(partscan + tiles + 1);
   next = reinterpret_cast<char*>(((uintptr_t)next + 255) & ~(uintptr_t)255);
-  hipLaunchKernelGGL((k_scan_reduce<Tin, T>), dim3((unsigned)tiles), dim3(kBlock), 0, st, in, n, part);
+  hipLaunchKernelGGL((k_scan_reduce<In, T>), dim3((unsigned)tiles), dim3(kBlock), 0, st, in, n, part);
   GX_HIP(hipGetLastError());
-  exclusive_scan<T, T>(part, partscan, tiles, next, st);
-  hipLaunchKernelGGL((k_scan_apply<Tin, T>), dim3((unsigned)tiles), dim3(kBlock), 0, st, in, n,
-                     (const T*)partscan, out);
+  if (tiles <= kSumTiles) {
+    hipLaunchKernelGGL((k_scan_apply<In, T, true>), dim3((unsigned)tiles), dim3(kBlock), 0, st, in, n, (const T*)part,
+                       out);
+  } else {
+    exclusive_scan_of<T>(ScanArray<T>{part}, partscan, tiles, next, st);
+    hipLaunchKernelGGL((k_scan_apply<In, T, false>), dim3((unsigned)tiles), dim3(kBlock), 0, st, in, n,
+                       (const T*)partscan, out);
+  }
   GX_HIP(hipGetLastError());
+}
+
+template <class Tin, class T>
+static void exclusive_scan(const Tin* in, T* out, size_t n, char* scratch, hipStream_t st) {
+  exclusive_scan_of<T>(ScanArray<Tin>{in}, out, n, scratch, st);
 }
 
 // ---------------------------------------------------------------------------

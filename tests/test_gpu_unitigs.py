@@ -240,7 +240,7 @@ def test_node_index_of_uneven_buckets(gx, k, n):
     check(gx, "".join(f"{4 * i + 2}\t{s}\n" for i, s in enumerate(lines)).encode(), k)
 
 
-@pytest.mark.parametrize("n", [2, 4095, 4097, 131072, 131073])
+@pytest.mark.parametrize("n", [2, 4095, 4097, 8192, 8193, 131072, 131073])
 def test_head_sorts_of_every_size(gx, n):
     """Read heads at the edges of the sorts: one block for all passes, few
     tiles whose blocks add up the digit counts themselves, scanned counts;

@@ -3512,6 +3512,7 @@ struct gx_build {
   // outer edges beside their coverage and heads): ordered by events, created
   // on first use
   hipStream_t st2 = nullptr;
+  uint8_t* hostw = nullptr;  // pinned words for results the host waits for
   hipEvent_t ev_fork = nullptr, ev_join = nullptr;
   std::string err;
   uint64_t text_len = 0;
@@ -3673,12 +3674,33 @@ static void stream_after(hipStream_t waiter, hipStream_t producer, hipEvent_t ev
   GX_HIP(hipStreamWaitEvent(waiter, ev, 0));
 }
 
+// Small results read back by the host, several per wait: copies into the
+// handle's pinned words, then one wait.  (A copy to pageable memory and its
+// wait cost 12 us more than the wait alone, one to pinned memory 4 us; a
+// small build waits a dozen times.)
+constexpr size_t kHostBytes = 64 << 10;
+struct Fetch {
+  gx_build* b;
+  size_t at = 0;
+  explicit Fetch(gx_build* b_) : b(b_) {}
+  template <class T>
+  const T* get(const T* dptr, size_t n = 1) {
+    const size_t bytes = (n * sizeof(T) + 15) / 16 * 16;
+    if (at + bytes > kHostBytes) throw GxError(GX_EDEVICE, "internal error: read-back buffer too small");
+    T* h = reinterpret_cast<T*>(b->hostw + at);
+    at += bytes;
+    GX_HIP(hipMemcpyAsync(h, dptr, n * sizeof(T), hipMemcpyDeviceToHost, b->st));
+    return h;
+  }
+  void wait() { GX_HIP(hipStreamSynchronize(b->st)); }
+};
+
 template <class T>
-static T read1(hipStream_t st, const T* dptr) {
-  T v;
-  GX_HIP(hipMemcpyAsync(&v, dptr, sizeof(T), hipMemcpyDeviceToHost, st));
-  GX_HIP(hipStreamSynchronize(st));
-  return v;
+static T read1(gx_build* b, const T* dptr) {
+  Fetch f(b);
+  const T* p = f.get(dptr);
+  f.wait();
+  return *p;
 }
 
 static const char* errname(uint32_t code) {
@@ -3693,8 +3715,7 @@ static const char* errname(uint32_t code) {
   return "input error";
 }
 
-static void check_err(gx_build* b) {
-  unsigned long long e = read1(b->st, b->errw.as<unsigned long long>());
+static void check_err(unsigned long long e) {
   if (e != ~0ull) {
     uint32_t code = (uint32_t)(e & 0xff);
     uint64_t line = e >> 8;
@@ -3873,8 +3894,12 @@ static void run_build(gx_build* b) {
   hipLaunchKernelGGL(k_line_count, dim3(lblocks), dim3(kBlock), 0, st, t, n, blk, errw + 1);
   GX_HIP(hipGetLastError());
   exclusive_scan<uint64_t, uint64_t>(blk, blkb, lblocks, scratch_for(b, scan_scratch_bytes<uint64_t>(lblocks)), st);
-  uint64_t nlines = read1(st, blkb + lblocks);
-  unsigned long long na = read1(st, errw + 1);
+  Fetch fl(b);
+  const uint64_t* lines_p = fl.get(blkb + lblocks);
+  const unsigned long long* na_p = fl.get(errw + 1);
+  fl.wait();
+  const uint64_t nlines = *lines_p;
+  const unsigned long long na = *na_p;
   if (na != ~0ull) throw GxError(GX_EINPUT, "non-ASCII byte at offset " + std::to_string(na) + " (input must be ASCII)");
   uint64_t* term = buf<uint64_t>(b->term, nlines + 1);
   hipLaunchKernelGGL(k_line_write, dim3(lblocks), dim3(kBlock), 0, st, t, n, blkb, term, errw + 1);
@@ -3896,9 +3921,9 @@ static void run_build(gx_build* b) {
   const unsigned rblocks = grid_for(nlines, kBlock, kRidBlocks);
   hipLaunchKernelGGL(k_rid_max, dim3(rblocks), dim3(kBlock), 0, st, nlines, rid, wbase + nmates + 1);
   GX_HIP(hipGetLastError());
-  uint64_t wr[1 + kRidBlocks];
-  GX_HIP(hipMemcpyAsync(wr, wbase + nmates, (1 + rblocks) * 8, hipMemcpyDeviceToHost, st));
-  GX_HIP(hipStreamSynchronize(st));
+  Fetch fw(b);
+  const uint64_t* wr = fw.get(wbase + nmates, 1 + rblocks);
+  fw.wait();
   const uint64_t nwords = wr[0], rid_max = *std::max_element(wr + 1, wr + 1 + rblocks);
   b->rid_bits = 1;  // valid readIds have at most 29 bits; those of lines that fail later may have more
   while (b->rid_bits < 29 && (rid_max >> b->rid_bits)) b->rid_bits++;
@@ -3912,15 +3937,11 @@ static void run_build(gx_build* b) {
     GX_HIP(hipGetLastError());
   }
   ph_end(b, PH_PARSE);
-  check_err(b);
   uint64_t* occbase = buf<uint64_t>(b->occbase, nmates + 1);
   exclusive_scan<uint64_t, uint64_t>(nocc, occbase, nmates, scratch_for(b, scan_scratch_bytes<uint64_t>(nmates)), st);
-  uint64_t N = read1(st, occbase + nmates);
   uint64_t* hidx = buf<uint64_t>(b->hidx, nmates + 1);
   exclusive_scan_of<uint64_t>(MateHead{valid, nocc}, hidx, nmates, scratch_for(b, scan_scratch_bytes<uint64_t>(nmates)),
                               st);
-  uint64_t nheads = read1(st, hidx + nmates);
-
   // 3b. sizing features: HLL sketch of the first 1% of the mates (at least
   //     512), then, with a network attached, the predicted distinct count
   ph_begin(b, PH_SIZING);
@@ -3932,13 +3953,18 @@ static void run_build(gx_build* b) {
                        nocc, k, hr);
     GX_HIP(hipGetLastError());
   }
-  const uint64_t occ_s = read1(st, occbase + ns_m), valid_s = read1(st, hidx + ns_m);
-  {
-    std::vector<uint32_t> rh(kHllRegs);
-    GX_HIP(hipMemcpyAsync(rh.data(), hr, kHllRegs * 4, hipMemcpyDeviceToHost, st));
-    GX_HIP(hipStreamSynchronize(st));
-    for (int i = 0; i < kHllRegs; i++) b->regs_h[i] = (uint8_t)rh[i];
-  }
+  // the parse's error word and totals, and the sketch, in one wait
+  Fetch fs(b);
+  const unsigned long long* err_p = fs.get(errw);
+  const uint64_t* N_p = fs.get(occbase + nmates);
+  const uint64_t* nheads_p = fs.get(hidx + nmates);
+  const uint64_t* occ_p = fs.get(occbase + ns_m);
+  const uint64_t* valid_p = fs.get(hidx + ns_m);
+  const uint32_t* rh = fs.get(hr, kHllRegs);
+  fs.wait();
+  check_err(*err_p);
+  const uint64_t N = *N_p, nheads = *nheads_p, occ_s = *occ_p, valid_s = *valid_p;
+  for (int i = 0; i < kHllRegs; i++) b->regs_h[i] = (uint8_t)rh[i];
   sizing_features(b->regs_h, (double)occ_s, (double)valid_s, nmates ? (double)ns_m / (double)nmates : 0.0, k,
                   b->cfg.nparts, b->feat);
   b->pred[0] = b->pred[1] = 0;
@@ -4066,6 +4092,7 @@ static void run_build(gx_build* b) {
     if (P == 1) swap_buf(b->out, b->outacc);
   };
   if (acc_swap) swap_stores();
+  uint64_t most_cov = 0;  // largest count above 255 so far
   uint64_t cap = 0, rebuilds = 0, tot_nn = 0, tot_nrep = 0, tot_nsel = 0, tot_bytes = 0, acc_len = 0;
   std::vector<uint64_t> seg_src, seg_len;  // several ranges, no sink: range r's part p bytes in outacc
   uint64_t glen[7] = {};  // several ranges, no sink: bytes of the node graph so far (klo, khi, cnt, msk, heads)
@@ -4174,9 +4201,9 @@ static void run_build(gx_build* b) {
                        st, kx, vx, ky, rcodes, bstart, Nr, nb, bkb, bk0, bk1 - bk0, nullptr, big, blists, nlist,
                        NBK, errw + 2);
     GX_HIP(hipGetLastError());
-    uint32_t nl[3];
-    GX_HIP(hipMemcpyAsync(nl, nlist, 12, hipMemcpyDeviceToHost, st));
-    GX_HIP(hipStreamSynchronize(st));
+    Fetch fb(b);
+    const uint32_t* nl = fb.get(nlist, 3);
+    fb.wait();
     if (nl[0] > bk1 - bk0 || nl[1] > bk1 - bk0 || nl[2] > bk1 - bk0)
       throw GxError(GX_EDEVICE, "internal error: bucket list overflow");
     if (nl[0]) {
@@ -4196,9 +4223,13 @@ static void run_build(gx_build* b) {
                          nullptr, NBK, errw + 2);
       GX_HIP(hipGetLastError());
     }
-    if (read1(st, errw + 2) != ~0ull) throw GxError(GX_EDEVICE, "internal error: unordered bucket bounds or lists");
     exclusive_scan_of<uint64_t>(BigSize{bstart, big}, boff, NBK, scratch_for(b, scan_scratch_bytes<uint64_t>(NBK)), st);
-    const uint64_t nbig = read1(st, boff + NBK);
+    Fetch fe(b);
+    const unsigned long long* bad_p = fe.get(errw + 2);
+    const uint64_t* nbig_p = fe.get(boff + NBK);
+    fe.wait();
+    if (*bad_p != ~0ull) throw GxError(GX_EDEVICE, "internal error: unordered bucket bounds or lists");
+    const uint64_t nbig = *nbig_p;
     if (nbig) {
       SK* tk = buf<SK>(b->hkey, nbig + 1);
       SK* tk2 = buf<SK>(b->hkey2, nbig + 1);
@@ -4229,7 +4260,7 @@ static void run_build(gx_build* b) {
       GX_HIP(hipGetLastError());
     }
     exclusive_scan<uint32_t, uint64_t>(ccnt, coff, nch, scratch_for(b, scan_scratch_bytes<uint64_t>(nch)), st);
-    nn = read1(st, coff + nch);
+    nn = read1(b, coff + nch);
     if (nn >= 0xffffffffull) throw GxError(GX_ENOTSUP, "more than 2^32-1 distinct k-mers");
     klo = buf<uint64_t>(b->klo, nn + 1);
     khi = W == 2 ? buf<uint64_t>(b->khi, nn + 1) : nullptr;
@@ -4282,9 +4313,9 @@ static void run_build(gx_build* b) {
         GX_HIP(hipGetLastError());
         ph_end(b, PH_KINSERT);
       }
-      unsigned long long e = read1(st, errw);
+      unsigned long long e = read1(b, errw);
       if (e == ~0ull) break;
-      if ((e & 0xff) != ERR_TABLE || attempt > 8) check_err(b);
+      if ((e & 0xff) != ERR_TABLE || attempt > 8) check_err(e);
       // fallback: rebuild in a table twice as large, and at least as large as
       // the sizing from the occurrence count (the method without a prediction)
       uint64_t plain = 1024;
@@ -4302,7 +4333,7 @@ static void run_build(gx_build* b) {
     hipLaunchKernelGGL(k_compact_count<W>, dim3(cblocks), dim3(kBlock), 0, st, table, cap, cb);
     GX_HIP(hipGetLastError());
     exclusive_scan<uint64_t, uint64_t>(cb, cbb, cblocks, scratch_for(b, scan_scratch_bytes<uint64_t>(cblocks)), st);
-    nn = read1(st, cbb + cblocks);
+    nn = read1(b, cbb + cblocks);
     if (nn >= 0xffffffffull) throw GxError(GX_ENOTSUP, "more than 2^32-1 distinct k-mers");
     uint32_t* claimed = buf<uint32_t>(b->claimed, nn + 1);
     hipLaunchKernelGGL(k_compact_write<W>, dim3(cblocks), dim3(kBlock), 0, st, table, cap, cbb, claimed);
@@ -4330,7 +4361,7 @@ static void run_build(gx_build* b) {
       GX_HIP(hipMemsetAsync(errw + 2, 0xff, 8, st));
       hipLaunchKernelGGL(k_dup_check<W>, dim3(grid_for(nn, kBlock, G)), dim3(kBlock), 0, st, nn, klo, khi, errw + 2);
       GX_HIP(hipGetLastError());
-      unsigned long long dup = read1(st, errw + 2);
+      unsigned long long dup = read1(b, errw + 2);
       if (dup != ~0ull) throw GxError(GX_EDEVICE, "internal error: k-mer stored in two table slots (node " +
                                                       std::to_string(dup) + ")");
     }
@@ -4358,9 +4389,9 @@ static void run_build(gx_build* b) {
                        sorted ? nullptr : table, jdk7, needs, selcnt, rtot, errw + 3);
     GX_HIP(hipGetLastError());
   }
-  unsigned long long rt[kTotLine * kTotLines];
-  GX_HIP(hipMemcpyAsync(rt, rtot, sizeof(rt), hipMemcpyDeviceToHost, st));
-  GX_HIP(hipStreamSynchronize(st));
+  Fetch fr(b);
+  const unsigned long long* rt = fr.get(rtot, kTotLine * kTotLines);
+  fr.wait();
   uint64_t nsel = 0, nrep = 0, nent = 0;
   for (int l = 0; l < kTotLines; l++) {
     nsel += rt[kTotLine * l];
@@ -4449,7 +4480,7 @@ static void run_build(gx_build* b) {
     hipLaunchKernelGGL(k_head_in_range, dim3(grid_for(nheads, kBlock, G)), dim3(kBlock), 0, st, nheads, hk, uflag);
     GX_HIP(hipGetLastError());
     exclusive_scan<uint32_t, uint64_t>(uflag, upos, nheads, scratch_for(b, scan_scratch_bytes<uint64_t>(nheads)), st);
-    nh = read1(st, upos + nheads);
+    nh = read1(b, upos + nheads);
     hipLaunchKernelGGL(k_head_keep, dim3(grid_for(nheads, kBlock, G)), dim3(kBlock), 0, st, nheads, hk, hv, uflag,
                        upos, hk2, hv2);
     GX_HIP(hipGetLastError());
@@ -4472,7 +4503,7 @@ static void run_build(gx_build* b) {
     GX_HIP(hipGetLastError());
   }
   exclusive_scan<uint32_t, uint64_t>(uflag, upos, nh, scratch_for(b, scan_scratch_bytes<uint64_t>(nh)), st);
-  const uint64_t nuh_r = read1(st, upos + nh);  // unique heads of this range
+  const uint64_t nuh_r = read1(b, upos + nh);  // unique heads of this range
   b->nuheads += nuh_r;
   if (nh) {
     hipLaunchKernelGGL(k_head_compact, dim3(grid_for(nh, kBlock, G)), dim3(kBlock), 0, st, nh, hk, hv, uflag, upos,
@@ -4525,7 +4556,7 @@ static void run_build(gx_build* b) {
     GX_HIP(hipGetLastError());
   }
   exclusive_scan<uint64_t, uint64_t>(rsize, roff, nn, scratch_for(b, scan_scratch_bytes<uint64_t>(nn)), st);
-  uint64_t total = read1(st, roff + nn);
+  uint64_t total = read1(b, roff + nn);
   b->reclaim.dead.push_back(&b->rsize);
   b->part_rec.assign(P + 1, 0);
   b->part_off.assign(P + 1, 0);
@@ -4547,9 +4578,12 @@ static void run_build(gx_build* b) {
     GX_HIP(hipGetLastError());
   }
   ph_end(b, PH_SER);
-  GX_HIP(hipStreamSynchronize(st));
+  Fetch fd(b);
+  const unsigned long long* ew = fd.get(errw, 4);  // [1] first inconsistent node, [3] largest count
+  fd.wait();
   ph_collect(b, true);
-  unsigned long long badnode = read1(st, errw + 1);
+  const unsigned long long badnode = ew[1];
+  most_cov = ew[3];
   if (badnode != ~0ull)
     throw GxError(GX_EDEVICE, "internal error: replayed edge list inconsistent at node " + std::to_string(badnode));
   tot_nn += nn;
@@ -4658,7 +4692,7 @@ static void run_build(gx_build* b) {
   b->stats[3] = cap;
   b->stats[4] = tot_nrep;
   b->stats[5] = tot_nsel;
-  b->stats[6] = read1(st, errw + 3);
+  b->stats[6] = most_cov;
   b->stats[7] = (uint64_t)b->pred[0];
   b->stats[8] = rebuilds;
   b->stats[11] = R;
@@ -4721,14 +4755,17 @@ static void run_unitigs(gx_build* b) {
     uint32_t* ws = buf<uint32_t>(b->u_any, 4);  // [0] capped, [1] unranked nodes
     const unsigned gn = grid_for(nn, kBlock, G * 4);
     exclusive_scan<uint32_t, uint64_t>(endp, at, nn, scratch_for(b, scan_scratch_bytes<uint64_t>(nn)), st);
-    const uint64_t nw = read1(st, at + nn);
+    const uint64_t nw = read1(b, at + nn);
     // nodes from the walkers' records; true when every node has its rank
     auto finish_walks = [&](uint64_t nwalk, const uint64_t* sum, const uint32_t* before, uint32_t* wr) {
       hipLaunchKernelGGL(k_walk_final, dim3(gn), dim3(kBlock), 0, st, nn, E, nwalk, sum, before, urep, upos, isrep,
                          ulen_of_rep, ws + 1);
       GX_HIP(hipGetLastError());
-      GX_HIP(hipMemcpyAsync(wr, ws, 16, hipMemcpyDeviceToHost, st));
-      GX_HIP(hipStreamSynchronize(st));
+      Fetch f(b);
+      const uint32_t* w = f.get(ws, 2);
+      f.wait();
+      wr[0] = w[0];
+      wr[1] = w[1];
       b->u_walkers = nwalk;
       return wr[0] == 0 && wr[1] == 0;
     };
@@ -4738,7 +4775,7 @@ static void run_unitigs(gx_build* b) {
       GX_HIP(hipGetLastError());
       exclusive_scan<uint32_t, uint64_t>(flag, at, nn, scratch_for(b, scan_scratch_bytes<uint64_t>(nn)), st);
       GX_HIP(hipMemsetAsync(ws, 0, 16, st));
-      const uint64_t na = read1(st, at + nn), nel = 2 * na;
+      const uint64_t na = read1(b, at + nn), nel = 2 * na;
       uint32_t* list = buf<uint32_t>(b->u_walk2, na + 1);
       uint4* S[2];
       S[0] = buf<uint4>(b->u_ptr[1], 2 * nel + (3 * nel + 3) / 4 + 1);  // two ranking buffers, sums, nodes before
@@ -4819,7 +4856,7 @@ static void run_unitigs(gx_build* b) {
       GX_HIP(hipGetLastError());
       cur ^= 1;
       rounds++;
-      act = read1(st, anyflag);
+      act = read1(b, anyflag);
     }
     if (!act) break;
     if (attempt == 1) throw GxError(GX_EDEVICE, "internal error: unitig chains did not terminate after cutting cycles");
@@ -4836,15 +4873,15 @@ static void run_unitigs(gx_build* b) {
     hipLaunchKernelGGL(k_sum_reads, dim3(1), dim3(kBlock), 0, st, breads, jgrid, reinterpret_cast<uint64_t*>(errw + 2));
     GX_HIP(hipGetLastError());
   }
-  unsigned long long ew[3];  // [0] first node without its neighbour, [2] successor reads of the jumping rounds
-  GX_HIP(hipMemcpyAsync(ew, errw, sizeof(ew), hipMemcpyDeviceToHost, st));
-  GX_HIP(hipStreamSynchronize(st));
-  if (ew[0] != ~0ull) throw GxError(GX_EDEVICE, "internal error: neighbour k-mer missing from the table");
-  b->u_succ_reads = ew[2];
-
   uint64_t* uid_of_rep = buf<uint64_t>(b->u_uid, nn + 1);
   exclusive_scan<uint32_t, uint64_t>(isrep, uid_of_rep, nn, scratch_for(b, scan_scratch_bytes<uint64_t>(nn)), st);
-  uint64_t nu = read1(st, uid_of_rep + nn);
+  Fetch fu(b);
+  const unsigned long long* ew = fu.get(errw, 3);  // [0] first node without its neighbour, [2] reads of the jumps
+  const uint64_t* nu_p = fu.get(uid_of_rep + nn);
+  fu.wait();
+  if (ew[0] != ~0ull) throw GxError(GX_EDEVICE, "internal error: neighbour k-mer missing from the table");
+  b->u_succ_reads = ew[2];
+  const uint64_t nu = *nu_p;
   uint32_t* urep_node = buf<uint32_t>(b->u_repnode, nu + 1);
   uint64_t* ulen = buf<uint64_t>(b->u_len, nu + 1);
   uint64_t* ubase = buf<uint64_t>(b->u_base, nu + 1);
@@ -4896,9 +4933,10 @@ static void run_unitigs(gx_build* b) {
                        b->has_hoff ? b->hoff.as<uint8_t>() : nullptr, urep, upos, uid_of_rep, b->rid.as<int64_t>(), k,
                        hk, hv, far);
     GX_HIP(hipGetLastError());
-    unsigned long long fr[kTotLine * kTotLines], most = 0, beyond = 0;
-    GX_HIP(hipMemcpyAsync(fr, far, sizeof(fr), hipMemcpyDeviceToHost, st));
-    GX_HIP(hipStreamSynchronize(st));
+    unsigned long long most = 0, beyond = 0;
+    Fetch ff(b);
+    const unsigned long long* fr = ff.get(far, kTotLine * kTotLines);
+    ff.wait();
     for (int l = 0; l < kTotLines; l++) {
       most = std::max(most, fr[kTotLine * l]);
       beyond = std::max(beyond, fr[kTotLine * l + 1]);
@@ -4977,7 +5015,7 @@ static void run_unitigs(gx_build* b) {
     GX_HIP(hipGetLastError());
   }
   exclusive_scan<uint64_t, uint64_t>(rsize, roff, nu, scratch_for(b, scan_scratch_bytes<uint64_t>(nu)), st);
-  uint64_t total = read1(st, roff + nu);
+  uint64_t total = read1(b, roff + nu);
   uint8_t* out = buf<uint8_t>(b->u_out, total + 1);
   if (nu) {
     uint64_t* seq_at = buf<uint64_t>(b->u_seqat, nu + 1);
@@ -5096,7 +5134,7 @@ static uint64_t line_ends(gx_build* b, const uint8_t* t, uint64_t n, DevBuf& ter
   hipLaunchKernelGGL(k_line_count, dim3(lblocks), dim3(kBlock), 0, st, t, n, blk, nullptr);
   GX_HIP(hipGetLastError());
   exclusive_scan<uint64_t, uint64_t>(blk, blkb, lblocks, scratch_for(b, scan_scratch_bytes<uint64_t>(lblocks)), st);
-  uint64_t nl = read1(st, blkb + lblocks);
+  uint64_t nl = read1(b, blkb + lblocks);
   uint64_t* term = buf<uint64_t>(termbuf, nl + 1);
   hipLaunchKernelGGL(k_line_write, dim3(lblocks), dim3(kBlock), 0, st, t, n, blkb, term, nullptr);
   GX_HIP(hipGetLastError());
@@ -5129,7 +5167,7 @@ static void fastq_convert(gx_build* b) {
     GX_HIP(hipGetLastError());
   }
   exclusive_scan<uint64_t, uint64_t>(sz, off, nrec, scratch_for(b, scan_scratch_bytes<uint64_t>(nrec)), st);
-  uint64_t total = read1(st, off + nrec);
+  uint64_t total = read1(b, off + nrec);
   uint8_t* out = buf<uint8_t>(b->rtext, total + 64);
   if (nrec) {
     hipLaunchKernelGGL(k_fq_write, dim3(grid_for(nrec, kBlock / 64, 1u << 16)), dim3(kBlock), 0, st, nrec, t1, term1,
@@ -5271,7 +5309,7 @@ static void compact_graph(gx_build* b, uint32_t* keep, const AddedHeads& ah) {
   GX_HIP(hipMemsetAsync(errw, 0xff, 8, st));
   uint64_t* pos = buf<uint64_t>(b->c_pos, nn + 1);
   exclusive_scan<uint32_t, uint64_t>(keep, pos, nn, scratch_for(b, scan_scratch_bytes<uint64_t>(nn)), st);
-  const uint64_t nn2 = read1(st, pos + nn);
+  const uint64_t nn2 = read1(b, pos + nn);
   uint64_t* klo2 = buf<uint64_t>(b->c_klo, nn2 + 1);
   uint64_t* khi2 = W == 2 ? buf<uint64_t>(b->c_khi, nn2 + 1) : nullptr;
   uint32_t* cnt2 = buf<uint32_t>(b->c_cnt, nn2 + 1);
@@ -5287,7 +5325,12 @@ static void compact_graph(gx_build* b, uint32_t* keep, const AddedHeads& ah) {
     GX_HIP(hipGetLastError());
   }
   exclusive_scan_of<uint64_t>(HeadTotal{hcu2, hcf2}, hstart2, nn2, scratch_for(b, scan_scratch_bytes<uint64_t>(nn2)), st);
-  const uint64_t nh2 = read1(st, hstart2 + nn2);
+  Fetch fk(b);
+  const unsigned long long* bad_p = fk.get(errw);
+  const uint64_t* nh2_p = fk.get(hstart2 + nn2);
+  fk.wait();
+  if (*bad_p != ~0ull) throw GxError(GX_EDEVICE, "internal error: neighbour k-mer missing from the graph");
+  const uint64_t nh2 = *nh2_p;
   uint32_t* uval2 = buf<uint32_t>(b->c_uval, nh2 + 1);
   const bool offs = b->has_hoff || ah.aval;  // heads at letters other than the build's
   uint8_t* hoff2 = offs ? buf<uint8_t>(b->c_hoff, nh2 + 1) : nullptr;
@@ -5297,7 +5340,6 @@ static void compact_graph(gx_build* b, uint32_t* keep, const AddedHeads& ah) {
                        b->has_hoff ? b->hoff.as<uint8_t>() : nullptr, ah, b->cfg.k, hstart2, uval2, hoff2);
     GX_HIP(hipGetLastError());
   }
-  if (read1(st, errw) != ~0ull) throw GxError(GX_EDEVICE, "internal error: neighbour k-mer missing from the graph");
   swap_buf(b->klo, b->c_klo);
   if (W == 2) swap_buf(b->khi, b->c_khi);
   swap_buf(b->cnt, b->c_cnt);
@@ -5668,7 +5710,7 @@ static void bubble_graph(gx_build* b, float maxd, uint64_t maxlen) {
     GX_HIP(hipGetLastError());
   }
   exclusive_scan<uint32_t, uint64_t>(np, pbase, nu, scratch_for(b, scan_scratch_bytes<uint64_t>(nu)), st);
-  npairs = read1(st, pbase + nu);
+  npairs = read1(b, pbase + nu);
   b->bub_pairs = npairs;
   if (npairs) {
     uint4* pairs = buf<uint4>(b->bb_pairs, npairs);
@@ -5692,7 +5734,7 @@ static void bubble_graph(gx_build* b, float maxd, uint64_t maxlen) {
     GX_HIP(hipGetLastError());
   }
   exclusive_scan<uint32_t, uint64_t>(hn, hb, nu, scratch_for(b, scan_scratch_bytes<uint64_t>(nu)), st);
-  const uint64_t na = read1(st, hb + nu);
+  const uint64_t na = read1(b, hb + nu);
   AddedHeads ah;
   if (na) {
     uint32_t* addu = buf<uint32_t>(b->bb_addu, nn + 1);
@@ -6123,8 +6165,10 @@ static void graph_stats(gx_build* b, int merged) {
   hipLaunchKernelGGL(k_stat_reduce, dim3(1), dim3(1024), 0, st, sblocks, part, acc);
   GX_HIP(hipGetLastError());
   unsigned long long a[kStatAcc];
-  GX_HIP(hipMemcpyAsync(a, acc, sizeof(a), hipMemcpyDeviceToHost, st));
-  GX_HIP(hipStreamSynchronize(st));
+  Fetch fa(b);
+  const unsigned long long* ap = fa.get(acc, kStatAcc);
+  fa.wait();
+  std::copy(ap, ap + kStatAcc, a);  // later reads reuse the pinned words
   b->st_tot.assign(a + SA_N * NSTAT, a + kStatAcc);
   b->st_bins.assign(NSTAT, {});
   b->st_sum.assign(NSTAT, 0);
@@ -6161,7 +6205,7 @@ static void graph_stats(gx_build* b, int merged) {
     hipLaunchKernelGGL(k_hist_flag, dim3(grid_for(nh, kBlock, G)), dim3(kBlock), 0, st, nh, H, hflag);
     GX_HIP(hipGetLastError());
     exclusive_scan<uint32_t, uint64_t>(hflag, hpos, nh, scratch_for(b, scan_scratch_bytes<uint64_t>(nh)), st);
-    const uint64_t nbin = read1(st, hpos + nh);
+    const uint64_t nbin = read1(b, hpos + nh);
     uint2* bins = buf<uint2>(b->s_bval, nbin + 1);
     hipLaunchKernelGGL(k_hist_write, dim3(grid_for(nh, kBlock, G)), dim3(kBlock), 0, st, nh, H, hpos, bins);
     GX_HIP(hipGetLastError());
@@ -6199,7 +6243,7 @@ static void graph_stats(gx_build* b, int merged) {
     hipLaunchKernelGGL(k_bin_starts, dim3(grid_for(m, kBlock, G)), dim3(kBlock), 0, st, m, ks, flag);
     GX_HIP(hipGetLastError());
     exclusive_scan<uint32_t, uint64_t>(flag, pos, m, scratch_for(b, scan_scratch_bytes<uint64_t>(m)), st);
-    const uint64_t nbin = read1(st, pos + m);
+    const uint64_t nbin = read1(b, pos + m);
     int64_t* bval = buf<int64_t>(b->s_bval, nbin + 1);
     uint64_t* bst = buf<uint64_t>(b->s_bst, nbin + 1);
     hipLaunchKernelGGL(k_bin_write, dim3(grid_for(m, kBlock, G)), dim3(kBlock), 0, st, m, ks, lo, flag, pos, bval,
@@ -6232,7 +6276,7 @@ static uint64_t fasta_bytes(gx_build* b, int merged, uint8_t* dst, size_t cap) {
     GX_HIP(hipGetLastError());
   }
   exclusive_scan<uint64_t, uint64_t>(sz, off, n, scratch_for(b, scan_scratch_bytes<uint64_t>(n)), st);
-  const uint64_t total = read1(st, off + n);
+  const uint64_t total = read1(b, off + n);
   if (!dst) return total;
   if (cap < total) throw GxError(GX_EINVAL, "destination too small");
   uint8_t* out = buf<uint8_t>(b->s_out, total + 1);
@@ -6280,9 +6324,11 @@ int gx_build_create(const gx_build_cfg* cfg, gx_build** out) {
   int rc = guarded(b, [&] {
     GX_HIP(hipSetDevice(cfg->device));
     GX_HIP(hipStreamCreateWithFlags(&b->st, hipStreamNonBlocking));
+    GX_HIP(hipHostMalloc(reinterpret_cast<void**>(&b->hostw), kHostBytes, hipHostMallocDefault));
   });
   if (rc) {
     g_create_err = b->err;
+    if (b->st) (void)hipStreamDestroy(b->st);
     delete b;
     return rc;
   }
@@ -6818,6 +6864,7 @@ void gx_build_destroy(gx_build* b) {
     if (e) (void)hipEventDestroy(e);
   for (auto& e : b->evpj)
     if (e) (void)hipEventDestroy(e);
+  if (b->hostw) (void)hipHostFree(b->hostw);
   delete b;
 }
 

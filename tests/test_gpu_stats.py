@@ -61,6 +61,24 @@ def test_stats_of_wide_ranges(gx, copies):
         assert got["maximum"]["scaffoldSeedScore"] > 1 << 22
 
 
+@pytest.mark.parametrize("k,lengths", [(21, (1004, 1005, 1024, 2048, 2049)), (33, (992, 993, 5000))])
+def test_fasta_of_long_unitigs(gx, k, lengths):
+    """Sequences of one chunk, at its edge and of several chunks."""
+    import random
+    rng = random.Random(k)
+    lines = []
+    for G in lengths:
+        g = "".join(rng.choice("ACGT") for _ in range(G))
+        lines += [g[p:p + 100] for p in range(0, G - 99, 30)] + [g[-100:]]
+    text = "".join(f"{4 * i + 2}\t{s}\n" for i, s in enumerate(lines)).encode()
+    with gx.GraphBuilder(k) as b:
+        b.add_reads(text)
+        b.finish()
+        assert b.fasta("nodes") == oracle.dump_fasta(b.part_bytes(0), k)
+        u = b.unitigs()
+        assert b.fasta("unitigs") == oracle.dump_fasta(u, k)
+
+
 def test_stats_errors(gx):
     with gx.GraphBuilder(21) as b:
         b.add_reads(_text(3, G=5000, paired=False))

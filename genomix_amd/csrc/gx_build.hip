@@ -3217,7 +3217,7 @@ __device__ inline uint64_t useq_len(const USerCtx& c, uint64_t u) { return c.ule
 
 // Unitigs with more than kHeadsLong read heads have their heads written by
 // k_uheads_long (a thread per head); k_useq_write leaves the bytes to it.
-constexpr uint32_t kHeadsLong = 32;
+constexpr uint32_t kHeadsLong = 4;
 
 // One read head of unitig records: mate flag, uuid (offset in the unitig,
 // mate, readId), the read and its mate as VKmers.
@@ -3259,7 +3259,7 @@ __global__ void k_useq_size(USerCtx c, uint64_t* __restrict__ rsize) {
 // Sequences longer than kUseqLong bases are written by k_useq_long (a wave
 // per unitig, lanes over bytes); k_useq_write leaves their bytes to it and
 // records where they start.
-constexpr uint64_t kUseqLong = 256;
+constexpr uint64_t kUseqLong = 128;
 constexpr int kUSerStage = 30720;  // LDS stage of 256 unitig records (longer than node records)
 
 template <int W>
@@ -3450,9 +3450,10 @@ __global__ void __launch_bounds__(kBlock) k_uheads_long(USerCtx c, const uint64_
 
 // Long sequences in chunks of kSeqChunk bytes, so that one unitig's letters
 // are gathered by many waves: (unitig, chunk) entries, in any order.  A
-// unitig of m nodes longer than kUseqLong letters has at most m / 64 chunks.
-constexpr uint32_t kSeqChunk = 64;
-static_assert(kUseqLong >= 256 && kSeqChunk == 64, "the chunk table holds nn / 64 + 1 entries");
+// unitig of m nodes longer than kUseqLong letters (m > 66) has at most
+// (m + 62) / 256 + 2 < m / kChunkNodes chunks.
+constexpr uint32_t kSeqChunk = 64, kChunkNodes = 16;
+static_assert(kUseqLong >= 128 && kSeqChunk == 64 && kChunkNodes == 16, "the chunk table holds nn / 16 + 1 entries");
 __global__ void __launch_bounds__(kBlock) k_useq_chunks(USerCtx c, uint2* __restrict__ chunk,
                                                        unsigned long long* __restrict__ nchunk) {
   const int lane = threadIdx.x & 63;
@@ -5029,7 +5030,7 @@ static void run_unitigs(gx_build* b) {
                          head_at, out);
       GX_HIP(hipGetLastError());
     }
-    unsigned long long* nchunk = buf<unsigned long long>(b->u_chunk, nn / 64 + 2);  // the count, then the chunks
+    unsigned long long* nchunk = buf<unsigned long long>(b->u_chunk, nn / kChunkNodes + 2);  // the count, then the chunks
     uint2* chunk = reinterpret_cast<uint2*>(nchunk + 1);
     hipLaunchKernelGGL(k_set_u64, dim3(1), dim3(1), 0, st, reinterpret_cast<uint64_t*>(nchunk), 0ull);
     GX_HIP(hipGetLastError());

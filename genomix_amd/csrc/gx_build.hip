@@ -789,7 +789,7 @@ __global__ void k_compact_list(const void* table, const uint32_t* __restrict__ c
 //    << 8 | code); the records are sorted by (key, occurrence): two stable
 //    8-bit radix passes on the top 16 key bits -- the first fused with the
 //    k-mer extraction -- then a bitonic sort of each 16-bit bucket in LDS
-//    (buckets above kBucketCap records go through a global radix sort).
+//    (buckets above bucket_cap records go through a global radix sort).
 //    Nodes are the runs of equal keys, already in output order; a run's
 //    codes are its occurrences' records in emission order, as the JDK-7
 //    replay needs them.  All HBM traffic is streaming; there is no
@@ -825,7 +825,7 @@ __device__ inline bool sk_eq(uint64_t a, uint64_t b) { return a == b; }
 __device__ inline bool sk_eq(const Key128& a, const Key128& b) { return a.lo == b.lo && a.hi == b.hi; }
 
 // Record-sort bucket: the top `bkb` bytes of the sort key (2, or 3 for
-// passes of more than 2^28 records, so buckets stay LDS-sized; 1 when the
+// passes of more than about 3 * 10^8 records, so buckets stay LDS-sized; 1 when the
 // key has one byte).
 template <class SK>
 __device__ inline uint32_t sort_bucket(const SK& sk, int nb, int bkb) {
@@ -993,7 +993,6 @@ __global__ void __launch_bounds__(NT) k_nix_build(const uint64_t* __restrict__ k
 }
 
 constexpr int kNixSmall = 8192, kNixLarge = 16384;  // LDS slots of k_nix_build: 32 KB (512 threads), 64 KB (1024)
-constexpr int kBucketCap = 8192;  // records sorted per bucket in one block (72 KB / 144 KB of LDS)
 // HBM of a key-range pass, per occurrence (sizes the ranges): the records
 // (two key and two neighbour-code arrays, the sorted codes) and, per node (dfrac
 // nodes per occurrence), every node array of the pass -- key words, count,
@@ -1017,7 +1016,6 @@ __host__ inline double pass_bytes_per_occurrence(int W, int nb, double dfrac) {
 __host__ inline double kept_bytes_per_node(int W, int nb) {
   return 3.0 * (4 + nb) + 16 + 8.0 * W + 4 * 4 + 4 + 2.0 * (W == 1 ? 16 : 24) + 16;
 }
-constexpr int kIdxBits = 13;      // log2(kBucketCap)
 
 // The bucket bytes are sorted least significant first (LSD): the fused
 // extraction pass scatters by byte nb-bkb, radix passes after it by bytes
@@ -1283,25 +1281,41 @@ __global__ void k_bucket_starts(uint64_t N, const SK* __restrict__ keys, int nb,
   }
 }
 
-// In-bucket sort element: the key bits below the bucket, then the record's
-// index in the bucket (so ties keep the occurrence order).
-__device__ inline uint64_t bucket_elem(uint64_t sk, int nb, int bkb, uint32_t idx) {
-  int bits = 8 * (nb - bkb);  // <= 48
-  uint64_t low = bits >= 64 ? sk : (sk & ((1ull << bits) - 1));
-  return (low << kIdxBits) | idx;
+// In-bucket sort element: the low kb bits of the key, then ib bits of the
+// record's index (so ties keep the occurrence order).
+__device__ inline uint64_t bucket_elem(uint64_t sk, int kb, int ib, uint32_t idx) {
+  return ((kb >= 64 ? sk : (sk & ((1ull << kb) - 1))) << ib) | idx;
 }
-__device__ inline Key128 bucket_elem(const Key128& sk, int nb, int bkb, uint32_t idx) {
-  int bits = 8 * (nb - bkb);  // 40..112
+__device__ inline Key128 bucket_elem(const Key128& sk, int kb, int ib, uint32_t idx) {
   Key128 low = sk;
-  if (bits < 64) { low.lo &= (1ull << bits) - 1; low.hi = 0; }
-  else if (bits < 128) low.hi &= (bits == 64) ? 0ull : ((1ull << (bits - 64)) - 1);
+  if (kb < 64) { low.lo &= (1ull << kb) - 1; low.hi = 0; }
+  else if (kb < 128) low.hi &= (kb == 64) ? 0ull : ((1ull << (kb - 64)) - 1);
   Key128 r;
-  r.hi = (low.hi << kIdxBits) | (low.lo >> (64 - kIdxBits));
-  r.lo = (low.lo << kIdxBits) | idx;
+  r.hi = (low.hi << ib) | (low.lo >> (64 - ib));
+  r.lo = (low.lo << ib) | idx;
   return r;
 }
-__device__ inline uint32_t elem_idx(uint64_t e) { return (uint32_t)(e & (kBucketCap - 1)); }
-__device__ inline uint32_t elem_idx(const Key128& e) { return (uint32_t)(e.lo & (kBucketCap - 1)); }
+// The key of an element, given the key bits above its kb low ones.
+__device__ inline uint64_t elem_key(uint64_t e, int kb, int ib, uint64_t above) { return (above << kb) | (e >> ib); }
+__device__ inline Key128 elem_key(const Key128& e, int kb, int ib, uint64_t above) {
+  Key128 r;
+  r.lo = (e.lo >> ib) | (e.hi << (64 - ib));
+  r.hi = e.hi >> ib;
+  if (kb >= 64) {
+    r.hi |= above << (kb - 64);
+  } else {
+    r.lo |= above << kb;
+    r.hi |= kb ? above >> (64 - kb) : 0;
+  }
+  return r;
+}
+__device__ inline uint32_t elem_bits(uint64_t e, int from, uint32_t mask) { return (uint32_t)(e >> from) & mask; }
+__device__ inline uint32_t elem_bits(const Key128& e, int from, uint32_t mask) {
+  const uint64_t x = from >= 64 ? e.hi >> (from - 64) : from ? (e.lo >> from) | (e.hi << (64 - from)) : e.lo;
+  return (uint32_t)x & mask;
+}
+__device__ inline uint32_t elem_idx(uint64_t e, int ib) { return (uint32_t)e & ((1u << ib) - 1); }
+__device__ inline uint32_t elem_idx(const Key128& e, int ib) { return (uint32_t)e.lo & ((1u << ib) - 1); }
 __device__ inline bool elem_gt(uint64_t a, uint64_t b) { return a > b; }
 __device__ inline bool elem_gt(const Key128& a, const Key128& b) { return a.hi > b.hi || (a.hi == b.hi && a.lo > b.lo); }
 __device__ inline void elem_max(uint64_t& e) { e = ~0ull; }
@@ -1317,6 +1331,32 @@ __device__ inline Key128 lane_xor(const Key128& x, int m) {
   Key128 r;
   r.lo = lane_xor(x.lo, m);
   r.hi = lane_xor(x.hi, m);
+  return r;
+}
+// The same with M known at compile time and every lane active: M = 1, 2, 4
+// and 8 are lane moves of the vector unit (quad permutes, the half-row
+// mirror, a row rotation), 16 a swizzle; only 32 goes through the shuffle.
+template <int M>
+__device__ inline uint32_t lane_xor_c(uint32_t x) {
+  const int v = (int)x;
+  if constexpr (M == 1) return (uint32_t)__builtin_amdgcn_update_dpp(0, v, 0xB1, 0xf, 0xf, false);
+  else if constexpr (M == 2) return (uint32_t)__builtin_amdgcn_update_dpp(0, v, 0x4E, 0xf, 0xf, false);
+  else if constexpr (M == 4)  // ^7 (half-row mirror), then ^3
+    return (uint32_t)__builtin_amdgcn_update_dpp(0, __builtin_amdgcn_update_dpp(0, v, 0x141, 0xf, 0xf, false), 0x1B,
+                                                 0xf, 0xf, false);
+  else if constexpr (M == 8) return (uint32_t)__builtin_amdgcn_update_dpp(0, v, 0x128, 0xf, 0xf, false);
+  else if constexpr (M == 16) return (uint32_t)__builtin_amdgcn_ds_swizzle(v, 0x401F);
+  else return (uint32_t)__shfl_xor(v, M);
+}
+template <int M>
+__device__ inline uint64_t lane_xor_c(uint64_t x) {
+  return ((uint64_t)lane_xor_c<M>((uint32_t)(x >> 32)) << 32) | lane_xor_c<M>((uint32_t)x);
+}
+template <int M>
+__device__ inline Key128 lane_xor_c(const Key128& x) {
+  Key128 r;
+  r.lo = lane_xor_c<M>(x.lo);
+  r.hi = lane_xor_c<M>(x.hi);
   return r;
 }
 // Stages whose partner is in the same thread (stride S < elements per
@@ -1337,155 +1377,352 @@ __device__ inline void bitonic_in_thread(E* x, uint32_t size, bool up_t) {
   }
 }
 
-// One block per bucket: bitonic sort of (key below the bucket, index),
-// then the records are written in that order: the key and its neighbour
-// code (one byte per record: the replay's code array).  Each thread holds
-// EPT = CAP / NT consecutive elements in registers: stages of stride < EPT
-// run inside the thread, strides < 64 * EPT across the wave's lanes
-// (shuffles, no barrier), only the larger ones through LDS.  Element i
-// lives at LDS slot i + i / EPT, so the threads' blocks of EPT fall on
-// different banks.  Four tiers: one wave per bucket (CAP =
-// kSmallBucket) over every bucket of the key range; it lists the buckets
-// above that for the CAP = kBucketCap / 8 (256 threads), kBucketCap / 2
-// (512) and kBucketCap (1024) blocks, which run over their lists only
-// (buckets marked 4, 3, 2).  Oversized buckets (above kBucketCap) are
-// marked 1 and left to the global pass.
-constexpr int kSmallBucket = 256;
-template <int W, int CAP, int NT>
-__device__ inline void sort_one_bucket(uint32_t bk, typename SortKeyOf<W>::T* s,
-                                       const typename SortKeyOf<W>::T* __restrict__ ik,
-                                       const uint8_t* __restrict__ ic, typename SortKeyOf<W>::T* __restrict__ ok,
-                                       uint8_t* __restrict__ oc, const uint64_t* __restrict__ bstart, uint64_t N,
-                                       int nb, int bkb, uint32_t* __restrict__ big, uint32_t* __restrict__ lists,
-                                       uint32_t* __restrict__ nlist, uint32_t NBK, unsigned long long* err) {
-  using SK = typename SortKeyOf<W>::T;
-  using E = SK;  // uint64_t or Key128
-  const bool first = CAP == kSmallBucket;
-  const uint64_t a = bstart[bk], e = bstart[bk + 1];
-  if (a > e || e > N) {  // bucket bounds must be ordered: report, touch nothing
-    if (threadIdx.x == 0) atomicMin(err, (unsigned long long)bk);
-    return;
-  }
-  const uint32_t n = (uint32_t)(e - a);
-  if (n == 0) return;
-  if (first && n > CAP) {
-    if (n <= kBucketCap) {  // to the tier that fits it
-      if (threadIdx.x == 0) {
-        const int t = n <= kBucketCap / 8 ? 0 : n <= kBucketCap / 2 ? 1 : 2;
-        big[bk] = 4 - t;
-        lists[(size_t)t * NBK + atomicAdd(&nlist[t], 1u)] = bk;
-      }
-      return;
-    }
-    if (threadIdx.x == 0) big[bk] = 1;
-  }
-  if (n > (uint32_t)CAP) {  // the global pass sorts and writes it; in a listed tier, a bad list
-    if (!first && threadIdx.x == 0) atomicMin(err, (unsigned long long)bk);
-    return;
-  }
-  if (n == 1 || nb < 2) {
-    for (uint32_t i = threadIdx.x; i < n; i += NT) {
-      ok[a + i] = ik[a + i];
-      oc[a + i] = ic[a + i];
-    }
-    return;
-  }
-  constexpr uint32_t EPT = CAP / NT, WSPAN = 64 * EPT;  // elements per thread, per wave
-  static_assert(EPT == 4 || EPT == 8, "four or eight elements per thread");
-  uint32_t P = EPT;  // network width: a power of two >= n, at least one thread's share
-  while (P < n) P <<= 1;
-  for (uint32_t i = threadIdx.x; i < P; i += NT) {
-    E x;
-    if (i < n) x = bucket_elem(ik[a + i], nb, bkb, i);
-    else elem_max(x);
-    s[i + i / EPT] = x;
-  }
-  __syncthreads();
-  const uint32_t t = threadIdx.x, i0 = t * EPT, slot0 = i0 + t;  // slot of element i0 + e: slot0 + e
-  const bool act = i0 < P;  // threads past the network's width only take part in the barriers
-  E x[EPT];
-  if (act) {
+// Bitonic sort of 64 EPT elements by one wave, in registers, fully unrolled:
+// element i is x[i % EPT] of lane i / EPT.
+template <int EPT, int SIZE, int STRIDE, class E>
+__device__ inline void wave_stage(E* x, int lane) {
+  if constexpr (STRIDE > 0) {
+    const bool up = ((lane * EPT) & SIZE) == 0;
+    if constexpr (STRIDE < EPT) {
+      bitonic_in_thread<STRIDE, EPT>(x, SIZE, up);
+    } else {
+      const bool keep_min = ((lane & (STRIDE / EPT)) == 0) == up;
 #pragma unroll
-    for (uint32_t e = 0; e < EPT; e++) x[e] = s[slot0 + e];
-  }
-  for (uint32_t size = 2; size <= P; size <<= 1) {
-    for (uint32_t stride = size >> 1; stride > 0; stride >>= 1) {
-      // stride >= EPT: the stride and size bits of i0 + e are those of i0,
-      // so the direction is the thread's and the partner is element e of
-      // thread t ^ (stride / EPT)
-      const bool keep_min = ((i0 & stride) == 0) == ((i0 & size) == 0);
-      if (stride >= WSPAN) {  // partner in another wave
-        __syncthreads();
-        if (act) {
-#pragma unroll
-          for (uint32_t e = 0; e < EPT; e++) s[slot0 + e] = x[e];
-        }
-        __syncthreads();
-        if (act) {
-          const uint32_t pslot0 = (t ^ (stride / EPT)) * (EPT + 1);
-#pragma unroll
-          for (uint32_t e = 0; e < EPT; e++) {
-            const E y = s[pslot0 + e];
-            if (elem_gt(x[e], y) == keep_min) x[e] = y;
-          }
-        }
-      } else if (stride >= EPT) {  // partner in another lane (active: j < P)
-        if (act) {
-          const int m = (int)(stride / EPT);
-#pragma unroll
-          for (uint32_t e = 0; e < EPT; e++) {
-            const E y = lane_xor(x[e], m);
-            if (elem_gt(x[e], y) == keep_min) x[e] = y;
-          }
-        }
-      } else if (act) {
-        const bool up_t = (i0 & size) == 0;
-        if (stride == 1) bitonic_in_thread<1, EPT>(x, size, up_t);
-        else if (stride == 2) bitonic_in_thread<2, EPT>(x, size, up_t);
-        else if constexpr (EPT > 4) bitonic_in_thread<4, EPT>(x, size, up_t);
+      for (int e = 0; e < EPT; e++) {
+        const E y = lane_xor_c<STRIDE / EPT>(x[e]);
+        if (elem_gt(x[e], y) == keep_min) x[e] = y;
       }
     }
+    wave_stage<EPT, SIZE, STRIDE / 2>(x, lane);
   }
-  __syncthreads();
-  if (act) {
-#pragma unroll
-    for (uint32_t e = 0; e < EPT; e++) s[slot0 + e] = x[e];
-  }
-  __syncthreads();
-  if constexpr (W == 1) {
-    // the element holds the key bits below the bucket, and the bucket id
-    // is the bytes above them: the key needs no second read
-    const int bits = 8 * (nb - bkb);
-    for (uint32_t i = threadIdx.x; i < n; i += NT) {
-      const E el = s[i + i / EPT];
-      ok[a + i] = ((uint64_t)bk << bits) | (el >> kIdxBits);
-      oc[a + i] = ic[a + elem_idx(el)];
-    }
-  } else {
-    for (uint32_t i = threadIdx.x; i < n; i += NT) {
-      const uint32_t src = elem_idx(s[i + i / EPT]);
-      ok[a + i] = ik[a + src];
-      oc[a + i] = ic[a + src];
-    }
+}
+template <int EPT, int SIZE, class E>
+__device__ inline void wave_sort(E* x, int lane) {
+  if constexpr (SIZE <= 64 * EPT) {
+    wave_stage<EPT, SIZE, SIZE / 2>(x, lane);
+    wave_sort<EPT, SIZE * 2>(x, lane);
   }
 }
 
-// Blocks loop over the buckets (grid x block stays below 2^32 work-items):
-// the first tier over buckets [bucket0, bucket1), the others over a list.
-template <int W, int CAP, int NT>
-__global__ void __launch_bounds__(NT) k_bucket_sort(const typename SortKeyOf<W>::T* __restrict__ ik,
+// Record buckets are sorted by (key below the bucket, index) in three ways:
+//  * k_bucket_wave: up to kWaveMax records by one wave; several neighbouring
+//    buckets together when they are small;
+//  * k_bucket_part: larger buckets (up to bucket_cap) by a block that first
+//    spreads them in LDS over sub-buckets of about 100 records by the next
+//    key bits, then sorts those by a wave each;
+//  * k_bucket_block: a bucket with a sub-bucket above kWaveMax (a repeated
+//    k-mer) by one block-wide bitonic network;
+// and buckets above bucket_cap, or above kBlockCap with such a sub-bucket, by
+// the global radix sort.  The vector unit bounds them all: a network over n
+// elements costs each log2(n)^2 / 2 exchanges, 91 for a bucket of 8192 but 28
+// or 36 for a sub-bucket, whose exchanges are register moves besides.  The
+// 5 Mbp workload's 200 M records: 6.6 ms by block-wide networks over whole
+// buckets, 3.4 ms (1.1 TB/s of records read and written).  320 M records,
+// which needed a third bucket byte and a wave for each of 16 M buckets: 9.3
+// ms and a radix pass of 2.7, now 4.5 ms.
+constexpr uint32_t kWaveMax = 512;
+constexpr int kWaveIdxBits = 9, kIdxBits = 14;  // index bits of a wave's and a block's elements
+constexpr uint32_t kBlockCap = 8192;
+__host__ __device__ constexpr uint32_t bucket_cap(int W) { return W == 1 ? 16384 : 8192; }  // 128 KB of LDS
+constexpr int kBucketLists = 4;  // up to 2048 records, up to 8192, up to bucket_cap, for k_bucket_block
+constexpr uint32_t kPartSmall = 2048, kPartMid = 8192;
+
+// n (<= 64 EPT) elements of one wave, sorted and written as records from
+// position `at` on (codes at `codes` + their index).
+template <int EPT, class E, class Load>
+__device__ inline void wave_sort_write(uint32_t n, int lane, int kb, int ib, uint64_t above,
+                                       const uint8_t* __restrict__ codes, E* __restrict__ okeys,
+                                       uint8_t* __restrict__ ocodes, Load&& load) {
+  E x[EPT];
+#pragma unroll
+  for (int e = 0; e < EPT; e++) {
+    const uint32_t i = (uint32_t)(e * 64 + lane);
+    if (i < n) x[e] = load(i);
+    else elem_max(x[e]);
+  }
+  wave_sort<EPT, 2>(x, lane);
+#pragma unroll
+  for (int e = 0; e < EPT; e++) {
+    const uint32_t i = (uint32_t)(lane * EPT + e);
+    if (i < n) {
+      okeys[i] = elem_key(x[e], kb, ib, above);
+      ocodes[i] = codes[elem_idx(x[e], ib)];
+    }
+  }
+}
+template <class E, class Load>
+__device__ inline void wave_sort_any(uint32_t n, int lane, int kb, int ib, uint64_t above,
+                                     const uint8_t* __restrict__ codes, E* __restrict__ okeys,
+                                     uint8_t* __restrict__ ocodes, Load&& load) {
+  if (n <= 64) wave_sort_write<1, E>(n, lane, kb, ib, above, codes, okeys, ocodes, load);
+  else if (n <= 128) wave_sort_write<2, E>(n, lane, kb, ib, above, codes, okeys, ocodes, load);
+  else if (n <= 256) wave_sort_write<4, E>(n, lane, kb, ib, above, codes, okeys, ocodes, load);
+  else wave_sort_write<8, E>(n, lane, kb, ib, above, codes, okeys, ocodes, load);
+}
+
+// The buckets of [bucket0, bucket1) above kWaveMax records: into the list of
+// their size, or marked big.  A block reserves its entries with one atomic
+// per list (one per bucket followed each other at 13 ns: 0.6 ms for the 65536
+// buckets of the 5 Mbp workload).  Bucket bounds must be ordered: the first
+// that are not are reported.
+template <int W>
+__global__ void __launch_bounds__(kBlock) k_bucket_lists(const uint64_t* __restrict__ bstart, uint64_t N,
+                                                         uint32_t bucket0, uint32_t bucket1, uint32_t* __restrict__ big,
+                                                         uint32_t* __restrict__ lists, uint32_t list_len,
+                                                         uint32_t* __restrict__ nlist, unsigned long long* err) {
+  __shared__ uint32_t cnt[3], base[3];
+  for (uint64_t b0 = bucket0 + (uint64_t)blockIdx.x * kBlock; b0 < bucket1; b0 += (uint64_t)gridDim.x * kBlock) {
+    if (threadIdx.x < 3) cnt[threadIdx.x] = 0;
+    __syncthreads();
+    const uint64_t bk = b0 + threadIdx.x;
+    int l = -1;
+    uint32_t at = 0;
+    if (bk < bucket1) {
+      const uint64_t s = bstart[bk], t = bstart[bk + 1], n = t - s;
+      if (s > t || t > N) atomicMin(err, (unsigned long long)bk);
+      else if (n > bucket_cap(W)) l = 3;
+      else if (n > kWaveMax) l = n <= kPartSmall ? 0 : n <= kPartMid ? 1 : 2;
+      big[bk] = l == 3 ? 1 : 0;
+      if (l >= 0 && l < 3) at = atomicAdd(&cnt[l], 1u);
+    }
+    __syncthreads();
+    if (threadIdx.x < 3) base[threadIdx.x] = cnt[threadIdx.x] ? atomicAdd(&nlist[threadIdx.x], cnt[threadIdx.x]) : 0;
+    __syncthreads();
+    if (l >= 0 && l < 3) {
+      at += base[l];
+      if (at < list_len) lists[(size_t)l * list_len + at] = (uint32_t)bk;
+      else atomicMin(err, (unsigned long long)bk);
+    }
+    __syncthreads();
+  }
+}
+
+// A wave per group of 2^w neighbouring buckets (aligned; the element then
+// holds w bits of the bucket too), of buckets [bucket0, bucket1).  A group
+// above kWaveMax records is taken bucket by bucket; larger buckets are left
+// to the lists.
+template <int W>
+__global__ void __launch_bounds__(kBlock) k_bucket_wave(const typename SortKeyOf<W>::T* __restrict__ ik,
                                                         const uint8_t* __restrict__ ic,
                                                         typename SortKeyOf<W>::T* __restrict__ ok,
                                                         uint8_t* __restrict__ oc, const uint64_t* __restrict__ bstart,
                                                         uint64_t N, int nb, int bkb, uint32_t bucket0,
-                                                        uint32_t count, const uint32_t* __restrict__ list,
-                                                        uint32_t* __restrict__ big, uint32_t* __restrict__ lists,
-                                                        uint32_t* __restrict__ nlist, uint32_t NBK,
-                                                        unsigned long long* err) {
-  __shared__ typename SortKeyOf<W>::T s[CAP + NT];  // CAP elements, one padding slot per thread
+                                                        uint32_t bucket1, int w) {
+  using SK = typename SortKeyOf<W>::T;
+  const int lane = threadIdx.x & 63, bits = 8 * (nb - bkb);
+  const uint32_t nw = gridDim.x * (kBlock / 64);
+  auto sort_run = [&](uint64_t a, uint32_t n, int kb, uint64_t above) {
+    if (n == 1 || kb == 0) {  // equal keys are in order already
+      for (uint32_t i = lane; i < n; i += 64) {
+        ok[a + i] = ik[a + i];
+        oc[a + i] = ic[a + i];
+      }
+      return;
+    }
+    wave_sort_any<SK>(n, lane, kb, kWaveIdxBits, above, ic + a, ok + a, oc + a,
+                      [&](uint32_t i) { return bucket_elem(ik[a + i], kb, kWaveIdxBits, i); });
+  };
+  const uint32_t g0 = bucket0 >> w, g1 = (uint32_t)(((uint64_t)bucket1 + (1u << w) - 1) >> w);
+  for (uint32_t g = g0 + blockIdx.x * (kBlock / 64) + (threadIdx.x >> 6); g < g1; g += nw) {
+    const uint32_t ba = max(bucket0, g << w), bb = (uint32_t)min((uint64_t)bucket1, ((uint64_t)g + 1) << w);
+    const uint64_t a = bstart[ba], e = bstart[bb];
+    if (a >= e || e > N) continue;  // empty, or bounds that k_bucket_lists reports
+    if (e - a <= kWaveMax) {
+      sort_run(a, (uint32_t)(e - a), bits + w, g);
+      continue;
+    }
+    for (uint32_t bk = ba; bk < bb; bk++) {
+      const uint64_t s = bstart[bk], t = bstart[bk + 1];
+      if (s < t && t <= N && t - s <= kWaveMax) sort_run(s, (uint32_t)(t - s), bits, bk);
+    }
+  }
+}
+
+// A block per listed bucket of at most CAP records.
+template <int W, int CAP, int NT>
+__global__ void __launch_bounds__(NT) k_bucket_part(const typename SortKeyOf<W>::T* __restrict__ ik,
+                                                    const uint8_t* __restrict__ ic,
+                                                    typename SortKeyOf<W>::T* __restrict__ ok,
+                                                    uint8_t* __restrict__ oc, const uint64_t* __restrict__ bstart,
+                                                    int nb, int bkb, uint32_t count, const uint32_t* __restrict__ list,
+                                                    uint32_t* __restrict__ big, uint32_t* __restrict__ blist,
+                                                    uint32_t list_len, uint32_t* __restrict__ nblist,
+                                                    unsigned long long* err) {
+  using SK = typename SortKeyOf<W>::T;
+  constexpr int kPer = CAP / NT;
+  constexpr uint32_t kSubs = 256;
+  __shared__ SK s[CAP];
+  __shared__ uint32_t cnt[kSubs], start[kSubs + 1], wsum[4], most, next;
+  const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6, bits = 8 * (nb - bkb);
   for (uint32_t q = blockIdx.x; q < count; q += gridDim.x) {
-    const uint32_t bk = list ? list[q] : bucket0 + q;
-    sort_one_bucket<W, CAP, NT>(bk, s, ik, ic, ok, oc, bstart, N, nb, bkb, big, lists, nlist, NBK, err);
+    const uint32_t bk = list[q];
+    const uint64_t a = bstart[bk];
+    const uint64_t nfull = bstart[bk + 1] - a;
+    if (nfull > CAP) {  // a bad list
+      if (threadIdx.x == 0) atomicMin(err, (unsigned long long)bk);
+      continue;
+    }
+    const uint32_t n = (uint32_t)nfull;
+    int sb = 0;  // sub-buckets: the next sb key bits
+    while ((n >> sb) > 128 && (1u << sb) < kSubs && sb < bits) sb++;
+    const int from = kIdxBits + bits - sb;
+    const uint32_t mask = (1u << sb) - 1;
+    if (threadIdx.x < kSubs) cnt[threadIdx.x] = 0;
+    if (threadIdx.x == 0) most = next = 0;
+    __syncthreads();
+    SK x[kPer];
+#pragma unroll
+    for (int r = 0; r < kPer; r++) {
+      const uint32_t i = r * NT + threadIdx.x;
+      if (i < n) {
+        x[r] = bucket_elem(ik[a + i], bits, kIdxBits, i);
+        atomicAdd(&cnt[elem_bits(x[r], from, mask)], 1u);
+      }
+    }
+    __syncthreads();
+    uint32_t c = 0, incl = 0;
+    if (threadIdx.x < kSubs) {
+      c = incl = cnt[threadIdx.x];
+#pragma unroll
+      for (int o = 1; o < 64; o <<= 1) {
+        const uint32_t y = __shfl_up(incl, o);
+        if (lane >= o) incl += y;
+      }
+      if (lane == 63) wsum[wid] = incl;
+      if (c > kWaveMax) most = 1;
+    }
+    __syncthreads();
+    if (most) {  // uniform: a sub-bucket no wave can sort
+      if (threadIdx.x == 0) {
+        if (n > kBlockCap) {
+          big[bk] = 1;
+        } else {
+          const uint32_t at = atomicAdd(nblist, 1u);
+          if (at < list_len) blist[at] = bk;
+          else atomicMin(err, (unsigned long long)bk);
+        }
+      }
+      __syncthreads();
+      continue;
+    }
+    if (threadIdx.x < kSubs) {
+      uint32_t before = incl - c;
+      for (int v = 0; v < wid; v++) before += wsum[v];
+      start[threadIdx.x] = cnt[threadIdx.x] = before;
+      if (threadIdx.x == kSubs - 1) start[kSubs] = before + c;
+    }
+    __syncthreads();
+#pragma unroll
+    for (int r = 0; r < kPer; r++)
+      if ((uint32_t)(r * NT) + threadIdx.x < n) s[atomicAdd(&cnt[elem_bits(x[r], from, mask)], 1u)] = x[r];
+    __syncthreads();
+    for (;;) {  // the next sub-bucket goes to the next free wave
+      uint32_t d = 0;
+      if (lane == 0) d = atomicAdd(&next, 1u);
+      d = (uint32_t)__builtin_amdgcn_readfirstlane((int)d);
+      if (d > mask) break;
+      const uint32_t p = start[d], m = start[d + 1] - p;
+      if (m)
+        wave_sort_any<SK>(m, lane, bits, kIdxBits, bk, ic + a, ok + a + p, oc + a + p,
+                          [&](uint32_t i) { return s[p + i]; });
+    }
+    __syncthreads();  // s, cnt and start are reused by the next bucket
+  }
+}
+
+// One block-wide bitonic network per listed bucket of at most kBlockCap
+// records: each thread holds EPT = kBlockCap / NT consecutive elements in
+// registers; stages of stride < EPT run inside the thread, strides < 64 * EPT
+// across the wave's lanes (shuffles, no barrier), only the larger ones
+// through LDS.  Element i lives at LDS slot i + i / EPT, so the threads'
+// blocks of EPT fall on different banks.
+template <int W>
+__global__ void __launch_bounds__(1024) k_bucket_block(const typename SortKeyOf<W>::T* __restrict__ ik,
+                                                       const uint8_t* __restrict__ ic,
+                                                       typename SortKeyOf<W>::T* __restrict__ ok,
+                                                       uint8_t* __restrict__ oc, const uint64_t* __restrict__ bstart,
+                                                       int nb, int bkb, const uint32_t* __restrict__ count,
+                                                       const uint32_t* __restrict__ list, unsigned long long* err) {
+  using SK = typename SortKeyOf<W>::T;
+  using E = SK;  // uint64_t or Key128
+  constexpr uint32_t NT = 1024, EPT = kBlockCap / NT, WSPAN = 64 * EPT;  // elements per thread, per wave
+  static_assert(EPT == 8, "eight elements per thread");
+  __shared__ SK s[kBlockCap + NT];  // one padding slot per thread
+  const int bits = 8 * (nb - bkb);
+  const uint32_t nq = *count;
+  for (uint32_t q = blockIdx.x; q < nq; q += gridDim.x) {
+    const uint32_t bk = list[q];
+    const uint64_t a = bstart[bk], nfull = bstart[bk + 1] - a;
+    if (nfull > kBlockCap) {
+      if (threadIdx.x == 0) atomicMin(err, (unsigned long long)bk);
+      continue;
+    }
+    const uint32_t n = (uint32_t)nfull;
+    uint32_t P = EPT;  // network width: a power of two >= n, at least one thread's share
+    while (P < n) P <<= 1;
+    for (uint32_t i = threadIdx.x; i < P; i += NT) {
+      E x;
+      if (i < n) x = bucket_elem(ik[a + i], bits, kIdxBits, i);
+      else elem_max(x);
+      s[i + i / EPT] = x;
+    }
+    __syncthreads();
+    const uint32_t t = threadIdx.x, i0 = t * EPT, slot0 = i0 + t;  // slot of element i0 + e: slot0 + e
+    const bool act = i0 < P;  // threads past the network's width only take part in the barriers
+    E x[EPT];
+    if (act) {
+#pragma unroll
+      for (uint32_t e = 0; e < EPT; e++) x[e] = s[slot0 + e];
+    }
+    for (uint32_t size = 2; size <= P; size <<= 1) {
+      for (uint32_t stride = size >> 1; stride > 0; stride >>= 1) {
+        // stride >= EPT: the stride and size bits of i0 + e are those of i0,
+        // so the direction is the thread's and the partner is element e of
+        // thread t ^ (stride / EPT)
+        const bool keep_min = ((i0 & stride) == 0) == ((i0 & size) == 0);
+        if (stride >= WSPAN) {  // partner in another wave
+          __syncthreads();
+          if (act) {
+#pragma unroll
+            for (uint32_t e = 0; e < EPT; e++) s[slot0 + e] = x[e];
+          }
+          __syncthreads();
+          if (act) {
+            const uint32_t pslot0 = (t ^ (stride / EPT)) * (EPT + 1);
+#pragma unroll
+            for (uint32_t e = 0; e < EPT; e++) {
+              const E y = s[pslot0 + e];
+              if (elem_gt(x[e], y) == keep_min) x[e] = y;
+            }
+          }
+        } else if (stride >= EPT) {  // partner in another lane (active: j < P)
+          if (act) {
+            const int m = (int)(stride / EPT);
+#pragma unroll
+            for (uint32_t e = 0; e < EPT; e++) {
+              const E y = lane_xor(x[e], m);
+              if (elem_gt(x[e], y) == keep_min) x[e] = y;
+            }
+          }
+        } else if (act) {
+          const bool up_t = (i0 & size) == 0;
+          if (stride == 1) bitonic_in_thread<1, EPT>(x, size, up_t);
+          else if (stride == 2) bitonic_in_thread<2, EPT>(x, size, up_t);
+          else bitonic_in_thread<4, EPT>(x, size, up_t);
+        }
+      }
+    }
+    __syncthreads();
+    if (act) {
+#pragma unroll
+      for (uint32_t e = 0; e < EPT; e++) s[slot0 + e] = x[e];
+    }
+    __syncthreads();
+    for (uint32_t i = threadIdx.x; i < n; i += NT) {
+      const E el = s[i + i / EPT];
+      ok[a + i] = elem_key(el, bits, kIdxBits, bk);
+      oc[a + i] = ic[a + elem_idx(el, kIdxBits)];
+    }
     __syncthreads();  // s is reused by the next bucket
   }
 }
@@ -4101,8 +4338,12 @@ static void run_build(gx_build* b) {
   b->nuheads = 0;
   b->has_hoff = false;
   b->stats[9] = 0;
-  // record-sort bucket bytes of a pass of n records (LDS-sized buckets)
-  auto bkb_of = [&](uint64_t n) { return nb < 2 ? 1 : (nb >= 4 && n > (1ull << 28)) ? 3 : 2; };
+  // record-sort bucket bytes of a pass of n records: two while a mean bucket
+  // takes a third (one-word keys) or half of an LDS bucket, as the canonical
+  // choice skews the buckets to twice the mean; a third byte costs a radix
+  // pass (320 M records: 2.7 ms) and 16 M buckets of a few records
+  const uint64_t two_bytes = W == 1 ? 5ull << 26 : 1ull << 28;
+  auto bkb_of = [&](uint64_t n) { return nb < 2 ? 1 : (nb >= 4 && n > two_bytes) ? 3 : 2; };
   DevBuf *hcur = &b->selflag, *hnext = &b->hist2;  // per-tile digit counts: this range's, the next one's
   bool hist_ready = false;
   for (uint32_t ri = 0; ri < R; ri++) {
@@ -4187,41 +4428,61 @@ static void run_build(gx_build* b) {
     uint64_t* bstart = buf<uint64_t>(b->hstart, NBK + 2);
     uint32_t* big = buf<uint32_t>(b->hcu, NBK + 1);
     uint64_t* boff = buf<uint64_t>(b->upos, NBK + 2);
-    GX_HIP(hipMemsetAsync(big, 0, (NBK + 1) * 4, st));
+    if (bk1 - bk0 < NBK) GX_HIP(hipMemsetAsync(big, 0, (NBK + 1) * 4, st));  // buckets of other key ranges
     hipLaunchKernelGGL(k_bucket_starts<SK>, dim3(grid_for(Nr + 1, kBlock, G)), dim3(kBlock), 0, st, Nr, kx, nb, bkb,
                        bk0, bk1, bstart);
     GX_HIP(hipGetLastError());
     GX_HIP(hipMemsetAsync(errw + 2, 0xff, 8, st));
     // sorted records: keys in ky, neighbour codes (the replay's code array) in rcodes
     uint8_t* rcodes = buf<uint8_t>(b->rcode, Nr + 32);
-    uint32_t* blists = buf<uint32_t>(b->blist, 3 * (size_t)NBK + 3);
-    uint32_t* nlist = blists + 3 * (size_t)NBK;
-    GX_HIP(hipMemsetAsync(nlist, 0, 12, st));
-    const unsigned kMaxSortBlocks = 1u << 20;
-    hipLaunchKernelGGL((k_bucket_sort<W, kSmallBucket, 64>), dim3(std::min(bk1 - bk0, kMaxSortBlocks)), dim3(64), 0,
-                       st, kx, vx, ky, rcodes, bstart, Nr, nb, bkb, bk0, bk1 - bk0, nullptr, big, blists, nlist,
-                       NBK, errw + 2);
+    // listed buckets hold more than kWaveMax records each
+    const uint32_t list_len = (uint32_t)std::min<uint64_t>(NBK, Nr / kWaveMax + 1);
+    uint32_t* blists = buf<uint32_t>(b->blist, kBucketLists * (size_t)list_len + kBucketLists);
+    uint32_t* nlist = blists + kBucketLists * (size_t)list_len;
+    GX_HIP(hipMemsetAsync(nlist, 0, kBucketLists * 4, st));
+    // neighbouring buckets per wave: about 200 records, within the element's
+    // bits (key bits below the bucket, the bucket's low w bits, the index)
+    int w = 0;
+    const uint64_t nbk = bk1 - bk0;
+    while (w < 8 * bkb && 8 * (nb - bkb) + w + 1 + kWaveIdxBits <= (W == 1 ? 64 : 128) &&
+           (Nr << (w + 1)) / nbk <= 200)
+      w++;
+    hipLaunchKernelGGL((k_bucket_lists<W>), dim3(grid_for(nbk, kBlock, 256)), dim3(kBlock), 0, st, bstart, Nr, bk0, bk1,
+                       big, blists, list_len, nlist, errw + 2);
     GX_HIP(hipGetLastError());
     Fetch fb(b);
     const uint32_t* nl = fb.get(nlist, 3);
+    hipLaunchKernelGGL((k_bucket_wave<W>), dim3(grid_for((nbk >> w) + 2, kBlock / 64, 1u << 18)), dim3(kBlock), 0, st,
+                       kx, vx, ky, rcodes, bstart, Nr, nb, bkb, bk0, bk1, w);
+    GX_HIP(hipGetLastError());
     fb.wait();
-    if (nl[0] > bk1 - bk0 || nl[1] > bk1 - bk0 || nl[2] > bk1 - bk0)
+    if (nl[0] > list_len || nl[1] > list_len || nl[2] > list_len)
       throw GxError(GX_EDEVICE, "internal error: bucket list overflow");
+    uint32_t* nblock = nlist + 3;
+    uint32_t* lblock = blists + 3 * (size_t)list_len;
     if (nl[0]) {
-      hipLaunchKernelGGL((k_bucket_sort<W, kBucketCap / 8, 256>), dim3(std::min(nl[0], 65536u)), dim3(256), 0, st, kx,
-                         vx, ky, rcodes, bstart, Nr, nb, bkb, bk0, nl[0], blists, big, nullptr, nullptr, NBK, errw + 2);
+      hipLaunchKernelGGL((k_bucket_part<W, kPartSmall, 256>), dim3(std::min(nl[0], 65536u)), dim3(256), 0, st, kx, vx,
+                         ky, rcodes, bstart, nb, bkb, nl[0], blists, big, lblock, list_len, nblock, errw + 2);
       GX_HIP(hipGetLastError());
     }
     if (nl[1]) {
-      hipLaunchKernelGGL((k_bucket_sort<W, kBucketCap / 2, 512>), dim3(std::min(nl[1], 65536u)), dim3(512), 0, st, kx,
-                         vx, ky, rcodes, bstart, Nr, nb, bkb, bk0, nl[1], blists + NBK, big, nullptr, nullptr, NBK,
+      hipLaunchKernelGGL((k_bucket_part<W, kPartMid, 1024>), dim3(std::min(nl[1], 65536u)), dim3(1024), 0, st, kx, vx,
+                         ky, rcodes, bstart, nb, bkb, nl[1], blists + list_len, big, lblock, list_len, nblock,
                          errw + 2);
       GX_HIP(hipGetLastError());
     }
-    if (nl[2]) {
-      hipLaunchKernelGGL((k_bucket_sort<W, kBucketCap, 1024>), dim3(std::min(nl[2], 65536u)), dim3(1024), 0, st, kx,
-                         vx, ky, rcodes, bstart, Nr, nb, bkb, bk0, nl[2], blists + 2 * (size_t)NBK, big, nullptr,
-                         nullptr, NBK, errw + 2);
+    if constexpr (W == 1) {
+      if (nl[2]) {
+        hipLaunchKernelGGL((k_bucket_part<W, bucket_cap(1), 1024>), dim3(std::min(nl[2], 65536u)), dim3(1024), 0, st,
+                           kx, vx, ky, rcodes, bstart, nb, bkb, nl[2], blists + 2 * (size_t)list_len, big, lblock,
+                           list_len, nblock, errw + 2);
+        GX_HIP(hipGetLastError());
+      }
+    }
+    const uint32_t nlisted = nl[0] + nl[1] + nl[2];
+    if (nlisted) {
+      hipLaunchKernelGGL((k_bucket_block<W>), dim3(std::min(nlisted, 1024u)), dim3(1024), 0, st, kx, vx, ky, rcodes,
+                         bstart, nb, bkb, nblock, lblock, errw + 2);
       GX_HIP(hipGetLastError());
     }
     exclusive_scan_of<uint64_t>(BigSize{bstart, big}, boff, NBK, scratch_for(b, scan_scratch_bytes<uint64_t>(NBK)), st);

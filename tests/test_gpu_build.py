@@ -244,3 +244,30 @@ def test_plain_gpu_params_byte_parity(gx, case):
     assert hashlib.sha256(graph).hexdigest() == case["graph_sha256"]
     assert len(merged) == case["unitigs_bytes"]
     assert hashlib.sha256(merged).hexdigest() == case["unitigs_sha256"]
+
+
+@pytest.mark.parametrize("k", [9, 21, 31, 55])
+@pytest.mark.parametrize("n", [60, 65, 300, 513, 600, 2100, 8200, 16500])
+def test_record_bucket_sizes(gx, k, n):
+    """One key bucket of about n records (distinct k-mers that share their
+    first eight letters) beside small neighbours, and the same with a k-mer
+    repeated 600 times in it: groups of buckets and single buckets in a wave,
+    each size of block, sub-buckets above a wave's, oversized buckets."""
+    import random
+    rng = random.Random(1000 * k + n)
+
+    def rc(s):
+        return s[::-1].translate(str.maketrans("ACGT", "TGCA"))
+
+    for repeats in (0, 600):
+        reads = []
+        for i in range(n):
+            s = "AACAGATA" + "".join(rng.choice("ACGT") for _ in range(k - 8))
+            reads.append(s + "A")  # ends in A: read forward
+        one = "AACAGATA" + "C" * (k - 8) + "A"
+        reads += [one if rng.random() < 0.5 else rc(one) for _ in range(repeats)]
+        for _ in range(40):
+            reads.append("".join(rng.choice("ACGT") for _ in range(k + 30)))
+        rng.shuffle(reads)
+        text = "".join(f"{4 * i + 2}\t{s}\n" for i, s in enumerate(reads)).encode()
+        assert gx.build_graph(text, k)[0] == oracle.build_graph(text, k)[0], repeats

@@ -889,6 +889,21 @@ __global__ void k_nix_dir(uint64_t nn, const uint64_t* __restrict__ klo, const u
   }
 }
 
+// The same by a binary search per bucket (54.7 M nodes: 0.14 ms -> 15 us).
+template <int W>
+__global__ void k_nix_search(uint64_t nn, const uint64_t* __restrict__ klo, const uint64_t* __restrict__ khi, int nb,
+                             int bkb, uint32_t b0, uint32_t b1, uint32_t* __restrict__ dir) {
+  const uint64_t bk = b0 + (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (bk > b1) return;
+  uint64_t lo = 0, hi = nn;
+  while (lo < hi) {
+    const uint64_t mid = lo + (hi - lo) / 2;
+    if (node_bucket<W>(node_key<W>(klo, khi, mid), nb, bkb) < bk) lo = mid + 1;
+    else hi = mid;
+  }
+  dir[bk] = (uint32_t)lo;
+}
+
 __global__ void k_fill_u32(uint32_t* __restrict__ p, uint64_t from, uint64_t to, uint32_t v) {
   for (uint64_t i = from + (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; i < to; i += (uint64_t)gridDim.x * blockDim.x)
     p[i] = v;
@@ -1280,6 +1295,24 @@ __global__ void k_bucket_starts(uint64_t N, const SK* __restrict__ keys, int nb,
     for (uint32_t b = lo; b <= hi && b <= b1; b++) start[b] = j;
   }
 }
+
+// The same by a binary search per bucket, for buckets of many records: every
+// record's key is read otherwise (0.5 ms for 200 M records; 20 us for 65536
+// searches).
+template <class SK>
+__global__ void k_bucket_search(uint64_t N, const SK* __restrict__ keys, int nb, int bkb, uint32_t b0, uint32_t b1,
+                                uint64_t* __restrict__ start) {
+  const uint64_t bk = b0 + (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (bk > b1) return;
+  uint64_t lo = 0, hi = N;  // the first record of bucket bk or a later one
+  while (lo < hi) {
+    const uint64_t mid = lo + (hi - lo) / 2;
+    if (sort_bucket(keys[mid], nb, bkb) < bk) lo = mid + 1;
+    else hi = mid;
+  }
+  start[bk] = lo;
+}
+constexpr uint64_t kSearchRecords = 64;  // records per bucket from which the searches are the faster way
 
 // In-bucket sort element: the low kb bits of the key, then ib bits of the
 // record's index (so ties keep the occurrence order).
@@ -4043,8 +4076,12 @@ static NodeIndex build_node_index(gx_build* b, hipStream_t st, uint64_t nn, cons
                        (uint64_t)nbk + 1, (uint32_t)nn);
     GX_HIP(hipGetLastError());
   }
-  hipLaunchKernelGGL(k_nix_dir<W>, dim3(grid_for(nn + 1, kBlock, G)), dim3(kBlock), 0, st, nn, klo, khi, nb, xbkb, xb0,
-                     xb1, ndir);
+  if (nn >= kSearchRecords * (xb1 - xb0))
+    hipLaunchKernelGGL(k_nix_search<W>, dim3(grid_for(xb1 - xb0 + 1, kBlock)), dim3(kBlock), 0, st, nn, klo, khi, nb,
+                       xbkb, xb0, xb1, ndir);
+  else
+    hipLaunchKernelGGL(k_nix_dir<W>, dim3(grid_for(nn + 1, kBlock, G)), dim3(kBlock), 0, st, nn, klo, khi, nb, xbkb, xb0,
+                       xb1, ndir);
   GX_HIP(hipGetLastError());
   // buckets per block: as many as fill the small table, but at least 512
   // blocks; the large table (two blocks per CU) where one mean bucket would
@@ -4429,8 +4466,12 @@ static void run_build(gx_build* b) {
     uint32_t* big = buf<uint32_t>(b->hcu, NBK + 1);
     uint64_t* boff = buf<uint64_t>(b->upos, NBK + 2);
     if (bk1 - bk0 < NBK) GX_HIP(hipMemsetAsync(big, 0, (NBK + 1) * 4, st));  // buckets of other key ranges
-    hipLaunchKernelGGL(k_bucket_starts<SK>, dim3(grid_for(Nr + 1, kBlock, G)), dim3(kBlock), 0, st, Nr, kx, nb, bkb,
-                       bk0, bk1, bstart);
+    if (Nr >= kSearchRecords * (bk1 - bk0))
+      hipLaunchKernelGGL(k_bucket_search<SK>, dim3(grid_for(bk1 - bk0 + 1, kBlock)), dim3(kBlock), 0, st, Nr, kx, nb, bkb,
+                         bk0, bk1, bstart);
+    else
+      hipLaunchKernelGGL(k_bucket_starts<SK>, dim3(grid_for(Nr + 1, kBlock, G)), dim3(kBlock), 0, st, Nr, kx, nb, bkb,
+                         bk0, bk1, bstart);
     GX_HIP(hipGetLastError());
     GX_HIP(hipMemsetAsync(errw + 2, 0xff, 8, st));
     // sorted records: keys in ky, neighbour codes (the replay's code array) in rcodes

@@ -18,10 +18,11 @@ struct KV {
   uint64_t lo, hi;
 };
 
+// The 32 two-bit codes in reverse order: all bits reversed (one instruction
+// per 32), then each pair swapped back.
 __device__ __host__ inline uint64_t rev2_64(uint64_t x) {
-  x = ((x >> 2) & 0x3333333333333333ull) | ((x & 0x3333333333333333ull) << 2);
-  x = ((x >> 4) & 0x0F0F0F0F0F0F0F0Full) | ((x & 0x0F0F0F0F0F0F0F0Full) << 4);
-  return __builtin_bswap64(x);
+  x = __builtin_bitreverse64(x);
+  return ((x >> 1) & 0x5555555555555555ull) | ((x & 0x5555555555555555ull) << 1);
 }
 
 // Mask of the 2k valid bits.

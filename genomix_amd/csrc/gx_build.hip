@@ -2454,7 +2454,7 @@ __global__ void k_ser_size(SerCtx c, uint64_t* __restrict__ rsize) {
 // into single stores), never past the bytes asked for.
 
 // The n (<= 8) low bytes of x, least significant first.
-__device__ inline void put_le(uint8_t*& p, uint64_t x, int n) {
+__device__ __forceinline__ void put_le(uint8_t*& p, uint64_t x, int n) {
   if (n == 8) {
     memcpy(p, &x, 8);
     p += 8;
@@ -2475,13 +2475,13 @@ __device__ inline void put_le(uint8_t*& p, uint64_t x, int n) {
   if (n & 1) *p++ = (uint8_t)x;
 }
 
-__device__ inline void put32(uint8_t*& p, uint32_t v) {  // big endian
+__device__ __forceinline__ void put32(uint8_t*& p, uint32_t v) {  // big endian
   uint32_t b = __builtin_bswap32(v);
   memcpy(p, &b, 4);
   p += 4;
 }
 
-__device__ inline void put64(uint8_t*& p, uint64_t v) {  // big endian
+__device__ __forceinline__ void put64(uint8_t*& p, uint64_t v) {  // big endian
   uint64_t b = __builtin_bswap64(v);
   memcpy(p, &b, 8);
   p += 8;
@@ -2490,7 +2490,7 @@ __device__ inline void put64(uint8_t*& p, uint64_t v) {  // big endian
 // VKmer bytes: BE32(k), then the nb-byte big-endian form of V (whose
 // little-endian image is the sort key).
 template <int W>
-__device__ inline void put_key(uint8_t*& p, KV v, int k, int nb) {
+__device__ __forceinline__ void put_key(uint8_t*& p, KV v, int k, int nb) {
   put32(p, (uint32_t)k);
   if constexpr (W == 1) {
     put_le(p, sortkey64(v.lo, nb), nb);
@@ -2503,7 +2503,7 @@ __device__ inline void put_key(uint8_t*& p, KV v, int k, int nb) {
 
 // A read as VKmer bytes: BE32(L) then the packed stream's bytes reversed,
 // eight at a time as byte-swapped 64-bit windows of the stream.
-__device__ inline void put_read(uint8_t*& p, const uint64_t* w, uint32_t L) {
+__device__ __forceinline__ void put_read(uint8_t*& p, const uint64_t* w, uint32_t L) {
   put32(p, L);
   const int64_t nbl = nbytes_of(L);
   int64_t q = nbl - 8;  // lowest stream byte of the next window
@@ -2516,7 +2516,7 @@ __device__ inline void put_read(uint8_t*& p, const uint64_t* w, uint32_t L) {
 }
 
 template <int W>
-__device__ inline void write_record(const SerCtx& c, uint64_t i, uint8_t* p, uint64_t rec) {
+__device__ __forceinline__ void write_record(const SerCtx& c, uint64_t i, uint8_t* p, uint64_t rec) {
   // every per-node field is loaded here, before the first store: the
   // stores through p could alias them, which would order each later load
   // after them
@@ -2573,14 +2573,22 @@ __device__ inline void write_record(const SerCtx& c, uint64_t i, uint8_t* p, uin
 
 // Records of 256 consecutive nodes are contiguous in the output: each
 // thread writes its record into LDS, then the block stores the whole span
-// with coalesced 4-byte writes.  Spans larger than the staging buffer are
-// written directly.
-constexpr int kSerStage = 16384;  // 256 node records average ~60 bytes; a smaller stage keeps 8 waves per SIMD
+// with coalesced 4-byte writes.  Spans larger than the stage are written
+// directly.  The stage is sized at launch for 1.2 times the mean span: with
+// 16 KB for every k about half the spans at k = 31 (62 bytes a record) and
+// nearly all at k = 55 (77 bytes) missed it.  54.7 M records of k = 31 3.4 ->
+// 2.8 ms (2.1
+// TB/s of records and node fields), 4 x 20 M of k = 55 9.0 -> 5.2 ms.
+constexpr uint32_t kStageMax = 64 << 10;
+__host__ inline uint32_t stage_bytes(uint64_t total, uint64_t records) {
+  const double span = records ? (double)total / (double)records * kBlock : 0;
+  return (uint32_t)std::min<double>(kStageMax - 16, 1.2 * span + 512) / 16 * 16;
+}
 
 template <int W>
 __global__ void __launch_bounds__(kBlock) k_ser_write(SerCtx c, const uint64_t* __restrict__ roff,
-                                                      uint8_t* __restrict__ out) {
-  __shared__ __attribute__((aligned(16))) uint8_t stage[kSerStage + 8];
+                                                      uint8_t* __restrict__ out, uint32_t stage_len) {
+  extern __shared__ __attribute__((aligned(16))) uint8_t stage[];
   uint64_t first = (uint64_t)blockIdx.x * kBlock;
   if (first >= c.nn) return;
   uint64_t last = first + kBlock < c.nn ? first + kBlock : c.nn;
@@ -2588,10 +2596,12 @@ __global__ void __launch_bounds__(kBlock) k_ser_write(SerCtx c, const uint64_t* 
   uint64_t i = first + threadIdx.x;
   // the stage starts at the 4-byte boundary at or below s0
   uint64_t base = s0 & ~3ull;
-  bool staged = (s1 - base) <= kSerStage;
+  bool staged = (s1 - base) <= stage_len;
   if (i < last) {
     uint64_t rec = roff[i + 1] - roff[i];
-    write_record<W>(c, ser_node(c, i), staged ? stage + (roff[i] - base) : out + roff[i], rec);
+    // two calls: with the stage alone the stores are LDS ones
+    if (staged) write_record<W>(c, ser_node(c, i), stage + (roff[i] - base), rec);
+    else write_record<W>(c, ser_node(c, i), out + roff[i], rec);
   }
   if (!staged) return;
   __syncthreads();
@@ -3491,7 +3501,7 @@ constexpr uint32_t kHeadsLong = 4;
 
 // One read head of unitig records: mate flag, uuid (offset in the unitig,
 // mate, readId), the read and its mate as VKmers.
-__device__ inline void write_uhead(const USerCtx& c, uint64_t j, uint8_t*& p) {
+__device__ __forceinline__ void write_uhead(const USerCtx& c, uint64_t j, uint8_t*& p) {
   const uint32_t mi = c.hval[j] & 0x7fffffffu;
   const uint32_t L = c.mlen[mi], Lm = c.mlen[mi ^ 1];
   *p++ = Lm > 0 ? 1 : 0;
@@ -3530,7 +3540,6 @@ __global__ void k_useq_size(USerCtx c, uint64_t* __restrict__ rsize) {
 // per unitig, lanes over bytes); k_useq_write leaves their bytes to it and
 // records where they start.
 constexpr uint64_t kUseqLong = 128;
-constexpr int kUSerStage = 30720;  // LDS stage of 256 unitig records (longer than node records)
 
 template <int W>
 __device__ inline uint8_t useq_byte(const USerCtx& c, const uint32_t* ord, uint64_t len, uint64_t q) {
@@ -3555,7 +3564,7 @@ __device__ inline uint8_t useq_byte(const USerCtx& c, const uint32_t* ord, uint6
 // its record into an LDS stage and the block stores the span with
 // coalesced 4-byte writes (spans larger than the stage go direct).
 template <int W>
-__device__ inline void write_unitig_record(const USerCtx& c, uint64_t u, uint8_t* rs, uint64_t rec,
+__device__ __forceinline__ void write_unitig_record(const USerCtx& c, uint64_t u, uint8_t* rs, uint64_t rec,
                                            uint64_t rec_at, uint64_t* __restrict__ seq_at,
                                            uint64_t* __restrict__ head_at) {
   {
@@ -3674,18 +3683,21 @@ __device__ inline void write_unitig_record(const USerCtx& c, uint64_t u, uint8_t
 template <int W>
 __global__ void __launch_bounds__(kBlock) k_useq_write(USerCtx c, const uint64_t* __restrict__ roff,
                                                        uint8_t* __restrict__ out, uint64_t* __restrict__ seq_at,
-                                                       uint64_t* __restrict__ head_at) {
-  __shared__ __attribute__((aligned(16))) uint8_t stage[kUSerStage + 8];
+                                                       uint64_t* __restrict__ head_at, uint32_t stage_len) {
+  extern __shared__ __attribute__((aligned(16))) uint8_t stage[];
   const uint64_t first = (uint64_t)blockIdx.x * kBlock;
   if (first >= c.nu) return;
   const uint64_t last = first + kBlock < c.nu ? first + kBlock : c.nu;
   const uint64_t s0 = roff[first], s1 = roff[last];
   const uint64_t base = s0 & ~3ull;
-  const bool staged = (s1 - base) <= kUSerStage;
+  const bool staged = (s1 - base) <= stage_len;
   const uint64_t u = first + threadIdx.x;
-  if (u < last)
-    write_unitig_record<W>(c, u, staged ? stage + (roff[u] - base) : out + roff[u], roff[u + 1] - roff[u], roff[u],
-                           seq_at, head_at);
+  if (u < last) {  // two calls: with the stage alone the stores are LDS ones
+    if (staged)
+      write_unitig_record<W>(c, u, stage + (roff[u] - base), roff[u + 1] - roff[u], roff[u], seq_at, head_at);
+    else
+      write_unitig_record<W>(c, u, out + roff[u], roff[u + 1] - roff[u], roff[u], seq_at, head_at);
+  }
   if (!staged) return;
   __syncthreads();
   uint64_t a4 = (s0 + 3) & ~3ull, e4 = s1 & ~3ull;
@@ -4877,7 +4889,8 @@ static void run_build(gx_build* b) {
   }
   uint8_t* out = buf<uint8_t>(b->out, total + 1);
   if (nn) {
-    hipLaunchKernelGGL(k_ser_write<W>, dim3(grid_for(nn, kBlock, 0xffffffffu)), dim3(kBlock), 0, st, c, roff, out);
+    const uint32_t sb = stage_bytes(total, nn);
+    hipLaunchKernelGGL(k_ser_write<W>, dim3(grid_for(nn, kBlock, 0xffffffffu)), dim3(kBlock), sb + 16, st, c, roff, out, sb);
     GX_HIP(hipGetLastError());
   }
   ph_end(b, PH_SER);
@@ -5324,8 +5337,9 @@ static void run_unitigs(gx_build* b) {
     uint64_t* seq_at = buf<uint64_t>(b->u_seqat, nu + 1);
     uint64_t* head_at = buf<uint64_t>(b->u_headat, 2 * nu + 2);
     // one block per kBlock unitigs (no grid-stride loop: every block stages its own span)
-    hipLaunchKernelGGL(k_useq_write<W>, dim3(grid_for(nu, kBlock, 0xffffffffu)), dim3(kBlock), 0, st, c, roff, out,
-                       seq_at, head_at);
+    const uint32_t sb = stage_bytes(total, nu);
+    hipLaunchKernelGGL(k_useq_write<W>, dim3(grid_for(nu, kBlock, 0xffffffffu)), dim3(kBlock), sb + 16, st, c, roff,
+                       out, seq_at, head_at, sb);
     GX_HIP(hipGetLastError());
     if (nh) {
       hipLaunchKernelGGL(k_uheads_long, dim3(grid_for(nh, kBlock, 1u << 16)), dim3(kBlock), 0, st, c, uposh + nh, hunit,

@@ -2577,8 +2577,8 @@ __device__ __forceinline__ void write_record(const SerCtx& c, uint64_t i, uint8_
 // directly.  The stage is sized at launch for 1.2 times the mean span: with
 // 16 KB for every k about half the spans at k = 31 (62 bytes a record) and
 // nearly all at k = 55 (77 bytes) missed it.  54.7 M records of k = 31 3.4 ->
-// 2.8 ms (2.1
-// TB/s of records and node fields), 4 x 20 M of k = 55 9.0 -> 5.2 ms.
+// 2.8 ms (2.1 TB/s of records and node fields), 4 x 20 M of k = 55 9.0 ->
+// 5.2 ms.
 constexpr uint32_t kStageMax = 64 << 10;
 __host__ inline uint32_t stage_bytes(uint64_t total, uint64_t records) {
   const double span = records ? (double)total / (double)records * kBlock : 0;
@@ -2720,6 +2720,7 @@ __device__ inline int back_side(uint32_t t) { return (t == ET_FF || t == ET_RF) 
 // Initial walk records of a node end (ranking by walks, below): not yet
 // walked, or the end of a node that merges with nothing.
 constexpr uint64_t kEndUnvisited = ~0ull, kEndSingle = ~0ull - 1;
+constexpr uint32_t kCovMax = 1u << 24;  // coverage saturates like the reference's float sums
 constexpr uint32_t kWalkCap = 1024;  // claims of one walk; a longer path is ranked by walks between splitters
 
 // Neighbour y of k-mer v (reverse complement rv) for mask bit 4t + x:
@@ -2743,12 +2744,7 @@ __device__ inline bool self_listed(KV v, KV rv, int k, uint32_t mask) {
 
 // Per node: tandem flag, and for each side of degree 1 its partner
 // (node << 1 | partner side) or kEnd.  The two sides' lookups run
-// interleaved, so their loads overlap.  With E given (ranking by walks),
-// also each node end's walk entry: the next end on its merge path when
-// the link is mergeable (neither node a tandem repeat, the partner's side
-// of degree 1; the index slot holds the partner's neighbour mask) and the
-// record's initial value, and whether the node ends a path (one mergeable
-// side).
+// interleaved, so their loads overlap.
 // With half (odd k, where no k-mer is its own reverse complement, so each
 // node end has one partner end), a link is looked up only by the node of
 // the smaller key, which writes the partner entries of both its ends when
@@ -2758,8 +2754,7 @@ __device__ inline bool self_listed(KV v, KV rv, int k, uint32_t mask) {
 template <int W>
 __global__ void k_links(uint64_t nn, const uint64_t* __restrict__ klo, const uint64_t* __restrict__ khi,
                         const uint32_t* __restrict__ msk, NodeIndex ix, int k, bool half,
-                        uint32_t* __restrict__ lnk, uint8_t* __restrict__ tand, unsigned long long* err,
-                        uint4* __restrict__ E, uint32_t* __restrict__ endpoint) {
+                        uint32_t* __restrict__ lnk, uint8_t* __restrict__ tand, unsigned long long* err) {
   for (uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; i < nn; i += (uint64_t)gridDim.x * blockDim.x) {
     const KV v = node_key<W>(klo, khi, i);
     const KV rv = revcomp<W>(v, k);
@@ -2849,20 +2844,6 @@ __global__ void k_links(uint64_t nn, const uint64_t* __restrict__ klo, const uin
     }
     lnk[2 * i] = l[0];
     lnk[2 * i + 1] = l[1];
-    if (E) {
-      bool mg[2];
-      uint32_t nx[2];
-      for (int d = 0; d < 2; d++) {
-        mg[d] = l[d] != kEnd && !tnd && found[d] != (uint32_t)i &&
-                side_deg(pmask[d], (int)back[d]) == 1 &&
-                !self_listed<W>(z[d], revcomp<W>(z[d], k), k, pmask[d]);
-        nx[d] = mg[d] ? ((found[d] << 1) | (1u - back[d])) : kEnd;  // leave the partner by its other side
-      }
-      const uint64_t r = (mg[0] || mg[1]) ? kEndUnvisited : kEndSingle;
-      E[2 * i] = make_uint4(nx[0], 0u, (uint32_t)r, (uint32_t)(r >> 32));
-      E[2 * i + 1] = make_uint4(nx[1], 0u, (uint32_t)r, (uint32_t)(r >> 32));
-      endpoint[i] = mg[0] != mg[1] ? 1u : 0u;
-    }
   }
 }
 
@@ -2870,15 +2851,16 @@ __global__ void k_links(uint64_t nn, const uint64_t* __restrict__ klo, const uin
 // half): the next end leaves the partner by its other side; the record
 // starts unvisited on a node with a mergeable side, single otherwise; a
 // node with one mergeable side ends a path.
-__global__ void k_link_ends(uint64_t nn, const uint32_t* __restrict__ lnk, uint4* __restrict__ E,
-                            uint32_t* __restrict__ endpoint) {
+__global__ void k_link_ends(uint64_t nn, const uint32_t* __restrict__ lnk, const uint32_t* __restrict__ cnt,
+                            uint4* __restrict__ E, uint32_t* __restrict__ endpoint) {
   for (uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; i < nn; i += (uint64_t)gridDim.x * blockDim.x) {
     const uint2 l = reinterpret_cast<const uint2*>(lnk)[i];
     const bool m0 = l.x != kEnd, m1 = l.y != kEnd;
     const uint32_t n0 = m0 ? (l.x ^ 1u) : kEnd, n1 = m1 ? (l.y ^ 1u) : kEnd;
     const uint64_t r = (m0 || m1) ? kEndUnvisited : kEndSingle;
-    E[2 * i] = make_uint4(n0, 0u, (uint32_t)r, (uint32_t)(r >> 32));
-    E[2 * i + 1] = make_uint4(n1, 0u, (uint32_t)r, (uint32_t)(r >> 32));
+    const uint32_t c = min(cnt[i], kCovMax);
+    E[2 * i] = make_uint4(n0, c, (uint32_t)r, (uint32_t)(r >> 32));
+    E[2 * i + 1] = make_uint4(n1, c, (uint32_t)r, (uint32_t)(r >> 32));
     endpoint[i] = m0 != m1 ? 1u : 0u;
   }
 }
@@ -2914,10 +2896,11 @@ __device__ inline bool mergeable(uint64_t i, int d, const uint32_t* lnk, const u
 // its sides to one neighbour) take the pointer-jumping ranking instead.
 
 // One 16-byte entry per node end: .x = the next end on its path (kEnd at
-// the path's end), .z/.w = a 64-bit record; node i's record is the one of
-// its F end (entry 2i), in the same line as the entry of its R end, so a
-// walk step reads one line.  Record = walker << 32 | side << 31 | position,
-// or kEndUnvisited / kEndSingle.
+// the path's end), .y = the node's count, at most kCovMax (so a walk sums its
+// path's coverage from the lines it reads anyway), .z/.w = a 64-bit record;
+// node i's record is the one of its F end (entry 2i), in the same line as
+// the entry of its R end, so a walk step reads one line.  Record =
+// walker << 32 | side << 31 | position, or kEndUnvisited / kEndSingle.
 __device__ inline uint64_t end_record(const uint4& x) { return ((uint64_t)x.w << 32) | x.z; }
 
 // The walkers' start ends, in node order.
@@ -2931,16 +2914,21 @@ __global__ void k_walk_list(uint64_t nn, const uint32_t* __restrict__ endpoint, 
 // node the other walker of the path claimed.  claim[w] = nodes claimed <<
 // 32 | (the smallest of them is left by its R side) << 31 | that node
 // (0x7fffffff when none); met[w] = the record found on the first node
-// another walker claimed (~0 when the walk reached the path's end).
+// another walker claimed (~0 when the walk reached the path's end);
+// wcov[w] = the counts of the nodes it claimed (5 Mbp: 1.5 ms of gathers in
+// unitig order, a scan over 55 M nodes and flag arrays less than summing
+// them afterwards, for 0.03 ms here).
 __global__ void __launch_bounds__(kBlock) k_walk(uint32_t nwalk, const uint32_t* __restrict__ walkers,
                                                  uint4* __restrict__ E, uint64_t* __restrict__ claim,
-                                                 uint64_t* __restrict__ met, uint32_t* __restrict__ capped) {
+                                                 uint64_t* __restrict__ met, uint64_t* __restrict__ wcov,
+                                                 uint32_t* __restrict__ capped) {
   for (uint32_t w = blockIdx.x * blockDim.x + threadIdx.x; w < nwalk; w += gridDim.x * blockDim.x) {
     uint32_t e = walkers[w], idx = 0, mn = 0x7fffffffu, mn_rev = 0;
-    uint64_t other = ~0ull;
+    uint64_t other = ~0ull, cov = 0;
     for (;;) {
       const uint32_t i = e >> 1;
-      const uint32_t x = E[e].x;
+      const uint2 q = *reinterpret_cast<const uint2*>(E + e);
+      const uint32_t x = q.x;
       unsigned long long* rec = reinterpret_cast<unsigned long long*>(E + 2 * (uint64_t)i) + 1;
       const unsigned long long mine = ((unsigned long long)w << 32) | ((unsigned long long)(e & 1) << 31) | idx;
       const unsigned long long old = atomicCAS(rec, (unsigned long long)kEndUnvisited, mine);
@@ -2953,6 +2941,7 @@ __global__ void __launch_bounds__(kBlock) k_walk(uint32_t nwalk, const uint32_t*
         mn_rev = e & 1;
       }
       idx++;
+      cov += q.y;
       if (x == kEnd) break;
       if (idx >= kWalkCap) {
         *capped = 1u;
@@ -2962,15 +2951,18 @@ __global__ void __launch_bounds__(kBlock) k_walk(uint32_t nwalk, const uint32_t*
     }
     claim[w] = ((uint64_t)idx << 32) | ((uint64_t)mn_rev << 31) | mn;
     met[w] = other;
+    wcov[w] = cov;
   }
 }
 
 // Joins the two walks of each path: a walker that met the other writes
 // both walkers' summaries, sum = length << 32 | (the path's smallest node
 // is left by its R side, walking as this walker does) << 31 | that node.
-// When both met each other, both write the same values.
+// When both met each other, both write the same values.  pcov: the path's
+// coverage, likewise.
 __global__ void k_walk_join(uint32_t nwalk, const uint64_t* __restrict__ claim, const uint64_t* __restrict__ met,
-                            uint64_t* __restrict__ sum) {
+                            const uint64_t* __restrict__ wcov, uint64_t* __restrict__ sum,
+                            uint64_t* __restrict__ pcov) {
   for (uint32_t w = blockIdx.x * blockDim.x + threadIdx.x; w < nwalk; w += gridDim.x * blockDim.x) {
     const uint64_t m = met[w];
     if (m == ~0ull || (m >> 32) >= nwalk) continue;  // not another walker's record: no sum, so pointer jumping
@@ -2985,6 +2977,7 @@ __global__ void k_walk_join(uint32_t nwalk, const uint64_t* __restrict__ claim, 
     const uint32_t rev_w = own ? rw : 1u - rp, rev_p = own ? 1u - rw : rp;
     sum[w] = (len << 32) | ((uint64_t)rev_w << 31) | mn;
     sum[p] = (len << 32) | ((uint64_t)rev_p << 31) | mn;
+    pcov[w] = pcov[p] = wcov[w] + wcov[p];
   }
 }
 
@@ -3009,7 +3002,7 @@ constexpr uint32_t kSplitEvery = 16;
 // and rank 2 M of them).
 constexpr uint64_t kSplitMean = 64;
 
-// Nodes that end a path or split one (endpoint: from k_links / k_link_ends).
+// Nodes that end a path or split one (endpoint: from k_link_ends).
 __global__ void k_split_flags(uint64_t nn, const uint32_t* __restrict__ lnk, const uint32_t* __restrict__ endpoint,
                               uint32_t* __restrict__ flag) {
   for (uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; i < nn; i += (uint64_t)gridDim.x * blockDim.x) {
@@ -3020,16 +3013,15 @@ __global__ void k_split_flags(uint64_t nn, const uint32_t* __restrict__ lnk, con
 }
 
 // The splitters in node order; both entries of a splitter carry its number
-// + 1 in .y (0 for the other nodes), so a walk reads one entry per node.
+// + 1 in .y (0 for the other nodes, in place of their counts), so a walk reads
+// one entry per node.
 __global__ void k_split_list(uint64_t nn, const uint32_t* __restrict__ flag, const uint64_t* __restrict__ at,
                              uint32_t* __restrict__ list, uint4* __restrict__ E) {
-  for (uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; i < nn; i += (uint64_t)gridDim.x * blockDim.x)
-    if (flag[i]) {
-      const uint32_t a = (uint32_t)at[i];
-      list[a] = (uint32_t)i;
-      E[2 * i].y = a + 1;
-      E[2 * i + 1].y = a + 1;
-    }
+  for (uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; i < nn; i += (uint64_t)gridDim.x * blockDim.x) {
+    const uint32_t a = (uint32_t)at[i];
+    if (flag[i]) list[a] = (uint32_t)i;
+    E[2 * i].y = E[2 * i + 1].y = flag[i] ? a + 1 : 0;
+  }
 }
 
 // Element 2a + d leaves splitter a through side d and walks to the next
@@ -3081,15 +3073,13 @@ __global__ void k_split_join(uint32_t nel, const uint4* __restrict__ R, uint64_t
 // (bit 31 of its sum); the node reads backwards when that differs from the
 // side it leaves the node by.
 __global__ void k_walk_final(uint64_t nn, const uint4* __restrict__ E, uint64_t nwalk, const uint64_t* __restrict__ sum,
-                             const uint32_t* __restrict__ before, uint32_t* __restrict__ urep, uint32_t* __restrict__ upos, uint32_t* __restrict__ isrep,
-                             uint64_t* __restrict__ ulen_of_rep, uint32_t* __restrict__ unranked) {
+                             const uint32_t* __restrict__ before, uint32_t* __restrict__ urep,
+                             uint32_t* __restrict__ upos, uint32_t* __restrict__ unranked) {
   for (uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; i < nn; i += (uint64_t)gridDim.x * blockDim.x) {
     const uint64_t r = end_record(E[2 * i]);
     if (r == kEndSingle) {
       urep[i] = (uint32_t)i;
       upos[i] = 0;
-      isrep[i] = 1;
-      ulen_of_rep[i] = 1;
       continue;
     }
     if (r == kEndUnvisited || (r >> 32) >= nwalk) {
@@ -3109,8 +3099,6 @@ __global__ void k_walk_final(uint64_t nn, const uint4* __restrict__ E, uint64_t 
     const bool side = ((r >> 31) & 1) != 0;      // the walker leaves this node by its R side
     urep[i] = mn | (against != side ? 0x80000000u : 0u);
     upos[i] = against ? len - 1 - a : a;
-    isrep[i] = mn == (uint32_t)i ? 1u : 0u;
-    ulen_of_rep[i] = mn == (uint32_t)i ? len : 0u;
   }
 }
 
@@ -3195,8 +3183,7 @@ __global__ void k_pj_cut(uint64_t ne, const uint4* __restrict__ R, const uint32_
 }
 
 __global__ void k_pj_node_final(uint64_t nn, const uint4* __restrict__ R, uint32_t* __restrict__ urep,
-                                uint32_t* __restrict__ upos, uint32_t* __restrict__ isrep,
-                                uint64_t* __restrict__ ulen_of_rep) {
+                                uint32_t* __restrict__ upos, uint64_t* __restrict__ ulen_of_rep) {
   for (uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; i < nn; i += (uint64_t)gridDim.x * blockDim.x) {
     uint4 f = R[2 * i], b = R[2 * i + 1];
     uint32_t r = min(f.z, b.z);
@@ -3205,8 +3192,7 @@ __global__ void k_pj_node_final(uint64_t nn, const uint4* __restrict__ R, uint32
     uint32_t pos = m - 1 - (fwd ? f.y : b.y);
     urep[i] = r | (fwd ? 0u : 0x80000000u);
     upos[i] = pos;
-    isrep[i] = r == (uint32_t)i ? 1 : 0;
-    ulen_of_rep[i] = r == (uint32_t)i ? m : 0;
+    if (r == (uint32_t)i) ulen_of_rep[i] = m;
   }
 }
 
@@ -3215,8 +3201,7 @@ __global__ void k_pj_node_final(uint64_t nn, const uint4* __restrict__ R, uint32
 __global__ void k_order_cov(uint64_t nn, const uint32_t* __restrict__ order, const uint32_t* __restrict__ cnt,
                             uint32_t* __restrict__ c) {
   for (uint64_t j = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; j < nn; j += (uint64_t)gridDim.x * blockDim.x) {
-    const uint32_t x = cnt[order[j] & 0x7fffffffu];
-    c[j] = x > (1u << 24) ? (1u << 24) : x;
+    c[j] = min(cnt[order[j] & 0x7fffffffu], kCovMax);
   }
 }
 
@@ -3237,14 +3222,35 @@ __global__ void k_place(uint64_t nn, const uint32_t* __restrict__ urep, const ui
   }
 }
 
-__global__ void k_rep_list(uint64_t nn, const uint32_t* __restrict__ isrep, const uint64_t* __restrict__ uid_of_rep,
-                           const uint64_t* __restrict__ ulen_of_rep, uint32_t* __restrict__ urep_node,
-                           uint64_t* __restrict__ ulen) {
+// 1 for a unitig's representative.
+struct IsRep {
+  const uint32_t* urep;
+  __device__ inline uint32_t operator()(size_t i) const { return (urep[i] & 0x7fffffffu) == (uint32_t)i ? 1u : 0u; }
+};
+
+// The representatives in order, with their unitig's length and, after walks
+// from the endpoints (pcov), its coverage: from the representative's walk
+// record, or (pointer jumping) from ulen_of_rep.
+struct RankSource {
+  const uint4* E;
+  const uint64_t *sum, *pcov;
+  const uint64_t* ulen_of_rep;
+};
+__global__ void k_rep_list(uint64_t nn, const uint32_t* __restrict__ urep, const uint64_t* __restrict__ uid_of_rep,
+                           RankSource src, uint32_t* __restrict__ urep_node, uint64_t* __restrict__ ulen,
+                           unsigned long long* __restrict__ ucov) {
   for (uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; i < nn; i += (uint64_t)gridDim.x * blockDim.x) {
-    if (!isrep[i]) continue;
-    uint64_t u = uid_of_rep[i];
+    if ((urep[i] & 0x7fffffffu) != (uint32_t)i) continue;
+    const uint64_t u = uid_of_rep[i];
     urep_node[u] = (uint32_t)i;
-    ulen[u] = ulen_of_rep[i];
+    if (src.ulen_of_rep) {
+      ulen[u] = src.ulen_of_rep[i];
+      continue;
+    }
+    const uint4 e = src.E[2 * i];
+    const uint64_t r = end_record(e);
+    ulen[u] = r == kEndSingle ? 1 : src.sum[r >> 32] >> 32;
+    if (src.pcov) ucov[u] = r == kEndSingle ? e.y : src.pcov[r >> 32];
   }
 }
 
@@ -5123,7 +5129,7 @@ static void run_unitigs(gx_build* b) {
   uint8_t* tand = buf<uint8_t>(b->u_tand, nn + 1);
   uint8_t* cut = buf<uint8_t>(b->u_cut, ne + 1);
   GX_HIP(hipMemsetAsync(cut, 0, ne + 1, st));
-  // ranking by walks (odd k): k_links writes the walk entries too
+  // ranking by walks (odd k)
   const bool walk = nn && (k & 1) && !b->no_walk;
   uint4* E = walk ? buf<uint4>(b->u_ptr[0], ne + 1) : nullptr;  // the pointer-jumping buffers, free until a fallback
   uint32_t* endp = walk ? buf<uint32_t>(b->u_walk, nn + 1) : nullptr;
@@ -5132,17 +5138,16 @@ static void run_unitigs(gx_build* b) {
   if (half) GX_HIP(hipMemsetAsync(lnk, 0xff, (ne + 1) * 4, st));
   if (nn) {
     hipLaunchKernelGGL(k_links<W>, dim3(grid_for(nn, kBlock, G)), dim3(kBlock), 0, st, nn, klo, khi, msk, nix, k, half,
-                       lnk, tand, errw, half ? nullptr : E, endp);
+                       lnk, tand, errw);
     GX_HIP(hipGetLastError());
-    if (half && E) {
-      hipLaunchKernelGGL(k_link_ends, dim3(grid_for(nn, kBlock, G)), dim3(kBlock), 0, st, nn, lnk, E, endp);
+    if (E) {
+      hipLaunchKernelGGL(k_link_ends, dim3(grid_for(nn, kBlock, G)), dim3(kBlock), 0, st, nn, lnk, cnt, E, endp);
       GX_HIP(hipGetLastError());
     }
   }
   uint32_t* urep = buf<uint32_t>(b->u_rep, nn + 1);
   uint32_t* upos = buf<uint32_t>(b->u_pos, nn + 1);
-  uint32_t* isrep = buf<uint32_t>(b->u_isrep, nn + 1);
-  uint64_t* ulen_of_rep = buf<uint64_t>(b->u_lenrep, nn + 1);
+  RankSource src{};
   // ranking by walks (odd k), pointer jumping when a walk cannot rank every node
   const unsigned jgrid = 8192;
   uint64_t* breads = buf<uint64_t>(b->u_flag, jgrid + jgrid / 8);  // per-block counters of the jumping rounds, flags
@@ -5160,8 +5165,8 @@ static void run_unitigs(gx_build* b) {
     const uint64_t nw = read1(b, at + nn);
     // nodes from the walkers' records; true when every node has its rank
     auto finish_walks = [&](uint64_t nwalk, const uint64_t* sum, const uint32_t* before, uint32_t* wr) {
-      hipLaunchKernelGGL(k_walk_final, dim3(gn), dim3(kBlock), 0, st, nn, E, nwalk, sum, before, urep, upos, isrep,
-                         ulen_of_rep, ws + 1);
+      hipLaunchKernelGGL(k_walk_final, dim3(gn), dim3(kBlock), 0, st, nn, E, nwalk, sum, before, urep, upos,
+                         ws + 1);
       GX_HIP(hipGetLastError());
       Fetch f(b);
       const uint32_t* w = f.get(ws, 2);
@@ -5202,6 +5207,7 @@ static void run_unitigs(gx_build* b) {
       hipLaunchKernelGGL(k_split_join, dim3(grid_for(nel, kBlock, G)), dim3(kBlock), 0, st, (uint32_t)nel, S[cur], sum,
                          before);
       GX_HIP(hipGetLastError());
+      src = RankSource{E, sum, nullptr, nullptr};
       uint32_t wr[4];
       return finish_walks(nel, sum, before, wr);
     };
@@ -5209,9 +5215,13 @@ static void run_unitigs(gx_build* b) {
       walked = walk_splits();
     } else {
       uint32_t* walkers = buf<uint32_t>(b->u_walk2, nw + 1);
-      uint64_t* sum = buf<uint64_t>(b->u_ptr[1], 3 * (nw + 1));  // path sums, walker claims, meeting records
+      // path sums, walker claims, meeting records, walkers' and paths' coverages
+      uint64_t* sum = buf<uint64_t>(b->u_ptr[1], 5 * (nw + 1));
       uint64_t* claim = sum + (nw + 1);
       uint64_t* met = claim + (nw + 1);
+      uint64_t* wcov = met + (nw + 1);
+      uint64_t* pcov = wcov + (nw + 1);
+      src = RankSource{E, sum, pcov, nullptr};
       GX_HIP(hipMemsetAsync(ws, 0, 16, st));
       GX_HIP(hipMemsetAsync(sum, 0xff, (nw + 1) * 8, st));  // a sum no join writes leaves its nodes unranked
       if (nw) {
@@ -5220,10 +5230,10 @@ static void run_unitigs(gx_build* b) {
         // one resident wave set, each lane walking ~a dozen paths in turn: a
         // wave then waits for the longest of its lanes' sums, not of single paths
         hipLaunchKernelGGL(k_walk, dim3(grid_for(nw, kBlock, G)), dim3(kBlock), 0, st, (uint32_t)nw, walkers, E, claim,
-                           met, ws);
+                           met, wcov, ws);
         GX_HIP(hipGetLastError());
         hipLaunchKernelGGL(k_walk_join, dim3(grid_for(nw, kBlock, G)), dim3(kBlock), 0, st, (uint32_t)nw, claim, met,
-                           sum);
+                           wcov, sum, pcov);
         GX_HIP(hipGetLastError());
       }
       uint32_t wr[4];
@@ -5266,8 +5276,10 @@ static void run_unitigs(gx_build* b) {
     GX_HIP(hipGetLastError());
   }
   if (nn) {
+    uint64_t* ulen_of_rep = buf<uint64_t>(b->u_lenrep, nn + 1);
+    src = RankSource{nullptr, nullptr, nullptr, ulen_of_rep};
     hipLaunchKernelGGL(k_pj_node_final, dim3(grid_for(nn, kBlock, G)), dim3(kBlock), 0, st, nn, R[cur], urep, upos,
-                       isrep, ulen_of_rep);
+                       ulen_of_rep);
     GX_HIP(hipGetLastError());
   }
   }  // pointer jumping
@@ -5276,7 +5288,7 @@ static void run_unitigs(gx_build* b) {
     GX_HIP(hipGetLastError());
   }
   uint64_t* uid_of_rep = buf<uint64_t>(b->u_uid, nn + 1);
-  exclusive_scan<uint32_t, uint64_t>(isrep, uid_of_rep, nn, scratch_for(b, scan_scratch_bytes<uint64_t>(nn)), st);
+  exclusive_scan_of<uint64_t>(IsRep{urep}, uid_of_rep, nn, scratch_for(b, scan_scratch_bytes<uint64_t>(nn)), st);
   Fetch fu(b);
   const unsigned long long* ew = fu.get(errw, 3);  // [0] first node without its neighbour, [2] reads of the jumps
   const uint64_t* nu_p = fu.get(uid_of_rep + nn);
@@ -5287,14 +5299,14 @@ static void run_unitigs(gx_build* b) {
   uint32_t* urep_node = buf<uint32_t>(b->u_repnode, nu + 1);
   uint64_t* ulen = buf<uint64_t>(b->u_len, nu + 1);
   uint64_t* ubase = buf<uint64_t>(b->u_base, nu + 1);
+  unsigned long long* ucov = buf<unsigned long long>(b->u_cov, nu + 1);
   if (nn) {
-    hipLaunchKernelGGL(k_rep_list, dim3(grid_for(nn, kBlock, G)), dim3(kBlock), 0, st, nn, isrep, uid_of_rep,
-                       ulen_of_rep, urep_node, ulen);
+    hipLaunchKernelGGL(k_rep_list, dim3(grid_for(nn, kBlock, G)), dim3(kBlock), 0, st, nn, urep, uid_of_rep, src,
+                       urep_node, ulen, ucov);
     GX_HIP(hipGetLastError());
   }
   exclusive_scan<uint64_t, uint64_t>(ulen, ubase, nu, scratch_for(b, scan_scratch_bytes<uint64_t>(nu)), st);
   uint32_t* order = buf<uint32_t>(b->u_order, nn + 1);
-  unsigned long long* ucov = buf<unsigned long long>(b->u_cov, nu + 1);
   uint32_t* uedge = buf<uint32_t>(b->u_edge, kUEdges * (nu + 1));
   uint8_t* uecnt = buf<uint8_t>(b->u_ecnt, nu + 1);
   if (nn) {
@@ -5311,9 +5323,9 @@ static void run_unitigs(gx_build* b) {
                        order, klo, khi, msk, nix, urep, k, uedge, uecnt);
     GX_HIP(hipGetLastError());
   }
-  if (nn) {
-    uint32_t* ocov = buf<uint32_t>(b->u_isrep, nn + 1);  // isrep is read no more
-    uint64_t* cpre = buf<uint64_t>(b->u_lenrep, nn + 1);  // nor ulen_of_rep
+  if (nn && !src.pcov) {  // coverage sums where the ranking did not make them
+    uint32_t* ocov = buf<uint32_t>(b->u_isrep, nn + 1);
+    uint64_t* cpre = buf<uint64_t>(b->u_lenrep, nn + 1);  // ulen_of_rep is read no more
     hipLaunchKernelGGL(k_order_cov, dim3(grid_for(nn, kBlock, G)), dim3(kBlock), 0, st, nn, order, cnt, ocov);
     GX_HIP(hipGetLastError());
     exclusive_scan<uint32_t, uint64_t>(ocov, cpre, nn, scratch_for(b, scan_scratch_bytes<uint64_t>(nn)), st);

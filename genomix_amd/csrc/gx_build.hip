@@ -1035,7 +1035,11 @@ __host__ inline double kept_bytes_per_node(int W, int nb) {
 // The bucket bytes are sorted least significant first (LSD): the fused
 // extraction pass scatters by byte nb-bkb, radix passes after it by bytes
 // nb-bkb+1 .. nb-1; a one-byte key has a single pass on byte 0.
-constexpr int kTileMateCap = 512;
+// Occurrences are taken in tiles of kOccTile, a contiguous run of kOccPer *
+// 64 to each wave.
+constexpr int kOccThreads = 512, kOccWaves = kOccThreads / 64, kOccPer = 8;
+constexpr int kOccTile = kOccThreads * kOccPer;
+constexpr int kTileMateCap = 1024;
 
 // Mate holding occurrence j: the largest m in [lo, hi] with occbase[m] <= j.
 __device__ inline uint64_t mate_search(const uint64_t* __restrict__ ob, uint64_t lo, uint64_t hi, uint64_t j) {
@@ -1049,42 +1053,48 @@ __device__ inline uint64_t mate_search(const uint64_t* __restrict__ ob, uint64_t
 
 // The mates of a tile's occurrences [j0, j1), in LDS: the tile's first and
 // last mate (mr), and, when the mates fit (always, for mates of at least
-// kSortTile / kTileMateCap occurrences on average), their first occurrences
-// relative to the first mate's (lob) and a table giving each occurrence's
-// mate (mtab): every non-empty mate marks the slot of its first occurrence
-// and a running maximum over the tile fills the rest; otherwise each
-// occurrence searches occbase.
+// kOccTile / kTileMateCap occurrences on average), their first occurrences
+// and packed words relative to the first mate's (lob, lwb) and a table giving
+// each occurrence's mate (mtab): every non-empty mate marks the slot of its
+// first occurrence and a running maximum over the tile fills the rest;
+// otherwise each occurrence searches occbase.
 struct TileMates {
-  uint64_t* mr;    // [2] first and last mate; [2] = the first mate's first occurrence
+  uint64_t* mr;    // first and last mate; the first mate's first occurrence and first word; mates fit
   uint32_t* lob;   // [kTileMateCap] occbase[m0 + i] - occbase[m0]
-  uint16_t* mtab;  // [kSortTile] mate of occurrence j0 + q, relative to m0
+  uint32_t* lwb;   // [kTileMateCap] wbase[m0 + i] - wbase[m0]
+  uint16_t* mtab;  // [kOccTile] mate of occurrence j0 + q, relative to m0
 };
 
 __device__ inline void tile_mates_init(const TileMates& t, uint64_t j0, uint64_t j1, uint64_t nmates,
-                                       const uint64_t* __restrict__ occbase) {
-  __shared__ uint16_t wmax[kBlock / 64];
+                                       const uint64_t* __restrict__ occbase, const uint64_t* __restrict__ wbase) {
+  __shared__ uint16_t wmax[kOccWaves];
   if (threadIdx.x == 0) {
-    t.mr[0] = mate_search(occbase, 0, nmates - 1, j0);
-    t.mr[1] = mate_search(occbase, t.mr[0], nmates - 1, j1 - 1);
-    t.mr[2] = occbase[t.mr[0]];
+    const uint64_t m0 = mate_search(occbase, 0, nmates - 1, j0);
+    t.mr[0] = m0;
+    const uint64_t m1 = mate_search(occbase, m0, nmates - 1, j1 - 1);
+    t.mr[1] = m1;
+    t.mr[2] = occbase[m0];
+    t.mr[3] = wbase[m0];
+    t.mr[4] = m1 - m0 + 2 <= kTileMateCap && wbase[m1] - wbase[m0] < (1ull << 32);
   }
   __syncthreads();
-  const uint64_t m0 = t.mr[0], m1 = t.mr[1], b0 = t.mr[2];
-  if (m1 - m0 + 2 <= kTileMateCap) {
-    for (uint64_t i = threadIdx.x; i <= m1 - m0 + 1; i += kBlock)
-      t.lob[i] = i + m0 <= nmates ? (uint32_t)(occbase[m0 + i] - b0) : 0xffffffffu;
-    for (uint32_t q = threadIdx.x; q < kSortTile; q += kBlock) t.mtab[q] = 0;
+  const uint64_t m0 = t.mr[0], m1 = t.mr[1], b0 = t.mr[2], w0 = t.mr[3];
+  if (t.mr[4]) {
+    for (uint32_t i = threadIdx.x; i <= m1 - m0 + 1; i += kOccThreads) {
+      t.lob[i] = (uint32_t)(occbase[m0 + i] - b0);  // (occbase has nmates + 1 entries)
+      if (i <= m1 - m0) t.lwb[i] = (uint32_t)(wbase[m0 + i] - w0);
+    }
+    for (uint32_t q = threadIdx.x; q < kOccTile; q += kOccThreads) t.mtab[q] = 0;
     __syncthreads();
-    for (uint64_t i = threadIdx.x + 1; i <= m1 - m0; i += kBlock)
+    for (uint32_t i = threadIdx.x + 1; i <= m1 - m0; i += kOccThreads)
       if (t.lob[i + 1] > t.lob[i] && b0 + t.lob[i] < j1) t.mtab[b0 + t.lob[i] - j0] = (uint16_t)i;
     __syncthreads();
-    // running maximum: each thread over kSortTile / kBlock consecutive slots
-    constexpr int kPer = kSortTile / kBlock;
+    // running maximum: each thread over kOccPer consecutive slots
     const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
-    uint16_t* my = t.mtab + threadIdx.x * kPer;
+    uint16_t* my = t.mtab + threadIdx.x * kOccPer;
     uint32_t run = 0;
 #pragma unroll
-    for (int q = 0; q < kPer; q++) run = max(run, (uint32_t)my[q]);
+    for (int q = 0; q < kOccPer; q++) run = max(run, (uint32_t)my[q]);
     uint32_t incl = run;
 #pragma unroll
     for (int o = 1; o < 64; o <<= 1) {
@@ -1097,190 +1107,180 @@ __device__ inline void tile_mates_init(const TileMates& t, uint64_t j0, uint64_t
     if (lane == 0) before = 0;
     for (int v = 0; v < wid; v++) before = max(before, (uint32_t)wmax[v]);
 #pragma unroll
-    for (int q = 0; q < kPer; q++) {
+    for (int q = 0; q < kOccPer; q++) {
       before = max(before, (uint32_t)my[q]);
       my[q] = (uint16_t)before;
     }
-  } else {
-    __syncthreads();
   }
   __syncthreads();
 }
 
-// Canonical key (and, with CODES, neighbour code) of occurrence j of the tile.
+// Canonical key (and, with CODES, neighbour code) of occurrence j0 + q.  A
+// mate with occurrences has one per k-mer, so its length follows from them.
 template <int W, bool CODES>
-__device__ inline KV tile_occurrence(const TileMates& t, uint64_t j0, uint64_t j, const uint64_t* __restrict__ occbase,
-                                     const uint32_t* __restrict__ mlen, const uint64_t* __restrict__ wbase,
-                                     const uint64_t* __restrict__ words, int k, uint32_t* code) {
-  const uint64_t m0 = t.mr[0], m1 = t.mr[1];
-  const bool local = m1 - m0 + 2 <= kTileMateCap;
-  const uint64_t m = local ? m0 + t.mtab[j - j0] : mate_search(occbase, m0, m1, j);
-  const uint64_t mb = local ? t.mr[2] + t.lob[m - m0] : occbase[m];
-  uint32_t bits;
-  return occ_info<W, CODES>(words + wbase[m], mlen[m], (uint32_t)(j - mb), k, code, &bits);
-}
-
-// Occurrences [j0, j1) of a tile: calls f(round, valid, j, key, code) for
-// each, in rounds of kBlock consecutive occurrences.
-template <int W, bool CODES, class F>
-__device__ inline void for_tile_occurrences(const TileMates& t, uint64_t j0, uint64_t j1, uint64_t nmates,
-                                            const uint64_t* __restrict__ occbase, const uint32_t* __restrict__ mlen,
-                                            const uint64_t* __restrict__ wbase, const uint64_t* __restrict__ words,
-                                            int k, F&& f) {
-  tile_mates_init(t, j0, j1, nmates, occbase);
-  for (int r = 0; r < kSortItems; r++) {
-    uint64_t j = j0 + (uint64_t)r * kBlock + threadIdx.x;
-    bool valid = j < j1;
-    KV key{0, 0};
-    uint32_t code = 0;
-    if (valid) key = tile_occurrence<W, CODES>(t, j0, j, occbase, mlen, wbase, words, k, &code);
-    f(r, valid, j, key, code);
+__device__ inline KV tile_occurrence(const TileMates& t, uint64_t j0, uint32_t q, const uint64_t* __restrict__ occbase,
+                                     const uint64_t* __restrict__ wbase, const uint64_t* __restrict__ words, int k,
+                                     uint32_t* code) {
+  uint32_t p, nocc;
+  const uint64_t* w;
+  if (t.mr[4]) {
+    const uint32_t i = t.mtab[q], ob = t.lob[i];
+    p = (uint32_t)(j0 - t.mr[2]) + q - ob;
+    nocc = t.lob[i + 1] - ob;
+    w = words + t.mr[3] + t.lwb[i];
+  } else {
+    const uint64_t m = mate_search(occbase, t.mr[0], t.mr[1], j0 + q);
+    p = (uint32_t)(j0 + q - occbase[m]);
+    nocc = (uint32_t)(occbase[m + 1] - occbase[m]);
+    w = words + wbase[m];
   }
+  uint32_t bits;
+  return occ_info<W, CODES>(w, nocc + (uint32_t)k - 1, p, k, code, &bits);
 }
 
 template <int W>
-__global__ void __launch_bounds__(kBlock) k_occ_hist(uint64_t N, uint64_t nmates, const uint64_t* __restrict__ occbase,
-                                                     const uint32_t* __restrict__ mlen,
-                                                     const uint64_t* __restrict__ wbase,
-                                                     const uint64_t* __restrict__ words, int k, int nb,
-                                                     uint32_t* __restrict__ hist, unsigned ntiles, uint32_t tlo,
-                                                     uint32_t thi, int dbyte) {
+__global__ void __launch_bounds__(kOccThreads) k_occ_hist(uint64_t N, uint64_t nmates,
+                                                          const uint64_t* __restrict__ occbase,
+                                                          const uint64_t* __restrict__ wbase,
+                                                          const uint64_t* __restrict__ words, int k, int nb,
+                                                          uint32_t* __restrict__ hist, unsigned ntiles, uint32_t tlo,
+                                                          uint32_t thi, int dbyte) {
   using SK = typename SortKeyOf<W>::T;
   __shared__ uint32_t h[256];
-  __shared__ uint64_t mr[3];
-  __shared__ uint32_t lob[kTileMateCap];
-  __shared__ uint16_t mtab[kSortTile];
-  h[threadIdx.x] = 0;
-  uint64_t j0 = (uint64_t)blockIdx.x * kSortTile, j1 = j0 + kSortTile < N ? j0 + kSortTile : N;
-  for_tile_occurrences<W, false>(TileMates{mr, lob, mtab}, j0, j1, nmates, occbase, mlen, wbase, words, k,
-                                 [&](int, bool valid, uint64_t, KV key, uint32_t) {
-                                   if (valid) {
-                                     SK sk;
-                                     make_sort_key(key, nb, sk);
-                                     const uint32_t t = key_byte(sk, nb - 1);
-                                     if (t >= tlo && t < thi) atomicAdd(&h[key_byte(sk, dbyte)], 1u);
-                                   }
-                                 });
+  __shared__ uint64_t mr[5];
+  __shared__ uint32_t lob[kTileMateCap], lwb[kTileMateCap];
+  __shared__ uint16_t mtab[kOccTile];
+  if (threadIdx.x < 256) h[threadIdx.x] = 0;
+  const uint64_t j0 = (uint64_t)blockIdx.x * kOccTile, j1 = j0 + kOccTile < N ? j0 + kOccTile : N;
+  const TileMates tm{mr, lob, lwb, mtab};
+  tile_mates_init(tm, j0, j1, nmates, occbase, wbase);
+#pragma unroll 2
+  for (uint32_t q = threadIdx.x; q < (uint32_t)(j1 - j0); q += kOccThreads) {
+    uint32_t code;
+    SK sk;
+    make_sort_key(tile_occurrence<W, false>(tm, j0, q, occbase, wbase, words, k, &code), nb, sk);
+    const uint32_t t = key_byte(sk, nb - 1);
+    if (t >= tlo && t < thi) atomicAdd(&h[key_byte(sk, dbyte)], 1u);
+  }
   __syncthreads();
-  hist[(size_t)threadIdx.x * ntiles + blockIdx.x] = h[threadIdx.x];
+  if (threadIdx.x < 256) hist[(size_t)threadIdx.x * ntiles + blockIdx.x] = h[threadIdx.x];
 }
 
-// Stable scatter of the tile's records by the lower bucket byte (same
-// ranking as k_radix_scatter: wave match + lower waves' counts), staged in
-// LDS in digit order and written out as one contiguous run per digit.  The
-// stage holds 4 bytes per record (occurrence in the tile, neighbour code);
-// the write-out extracts each record's key again from the packed mates
-// (which the tile has just read, so they come from the caches), which
-// halves the block's LDS and doubles the blocks a CU holds.  A record is
-// its sort key and its neighbour code (one byte): the sorts after this are
-// stable or break ties by the record's index in its bucket, so occurrence
-// order among equal keys needs no stored occurrence number.
+// Stable scatter of the tile's records by the lower bucket byte (ranked as
+// in k_radix_scatter: each wave by itself), staged in LDS in digit order and
+// written out as one contiguous run per digit.  The stage holds 2 bytes per
+// record, its occurrence in the tile; the write-out extracts the record's key
+// again from the packed mates (which the tile has just read, so they come
+// from the caches) and with it the neighbour code, so records of other key
+// ranges cost their keys only.  A record is its sort key and its neighbour
+// code (one byte): the sorts after this are stable or break ties by the
+// record's index in its bucket, so occurrence order among equal keys needs no
+// stored occurrence number.  Bound by the integer work of the extraction.
+// 10 Mbp, k = 31: 3.9 -> 2.9 ms, 4 key ranges of k = 55 9.2 -> 7.3 ms, against
+// rounds of 256 occurrences with three barriers each, neighbour codes made
+// before the range test, and the mates' lengths and words read from memory
+// per occurrence.
 template <int W>
-__global__ void __launch_bounds__(kBlock) k_occ_scatter(uint64_t N, uint64_t nmates,
-                                                        const uint64_t* __restrict__ occbase,
-                                                        const uint32_t* __restrict__ mlen,
-                                                        const uint64_t* __restrict__ wbase,
-                                                        const uint64_t* __restrict__ words, int k, int nb,
-                                                        const uint64_t* __restrict__ offs, unsigned ntiles,
-                                                        typename SortKeyOf<W>::T* __restrict__ okeys,
-                                                        uint8_t* __restrict__ ocodes, uint32_t tlo, uint32_t thi,
-                                                        int dbyte, uint32_t nlo, uint32_t nhi, int ndbyte,
-                                                        uint32_t* __restrict__ nhist) {
+__global__ void __launch_bounds__(kOccThreads) k_occ_scatter(uint64_t N, uint64_t nmates,
+                                                             const uint64_t* __restrict__ occbase,
+                                                             const uint64_t* __restrict__ wbase,
+                                                             const uint64_t* __restrict__ words, int k, int nb,
+                                                             const uint64_t* __restrict__ offs, unsigned ntiles,
+                                                             typename SortKeyOf<W>::T* __restrict__ okeys,
+                                                             uint8_t* __restrict__ ocodes, uint32_t tlo, uint32_t thi,
+                                                             int dbyte, uint32_t nlo, uint32_t nhi, int ndbyte,
+                                                             uint32_t* __restrict__ nhist) {
   using SK = typename SortKeyOf<W>::T;
-  __shared__ uint64_t run[256];
-  __shared__ uint16_t lbase[256], lrun[256];  // (LDS kept under 20 KB: 8 blocks per CU)
-  __shared__ uint32_t wsum[kBlock / 64];
-  __shared__ uint16_t wcnt[kBlock / 64][256];
-  __shared__ uint64_t mr[3];
-  __shared__ uint32_t lob[kTileMateCap];
-  __shared__ uint16_t mtab[kSortTile];
+  __shared__ uint64_t run[256];  // output position of a digit's records less their place in the stage
+  __shared__ uint32_t wsum[4], last;
+  __shared__ uint16_t wcnt[kOccWaves][256];
+  __shared__ uint64_t mr[5];
+  __shared__ uint32_t lob[kTileMateCap], lwb[kTileMateCap];
+  __shared__ uint16_t mtab[kOccTile];
   __shared__ uint32_t h2[128];  // the next key range's digit counts (as k_occ_hist would give), two u16 per word
-  __shared__ uint32_t sv[kSortTile];  // (occurrence - j0) << 8 | code
+  __shared__ uint16_t sq[kOccTile];
   const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
-  run[threadIdx.x] = offs[(size_t)threadIdx.x * ntiles + blockIdx.x];
-  if (threadIdx.x < 128) h2[threadIdx.x] = 0;
-  tile_digit_bases(offs, ntiles, lbase, lrun, wsum);
   const uint64_t lt = (lane == 0) ? 0ull : (~0ull >> (64 - lane));
-  uint64_t j0 = (uint64_t)blockIdx.x * kSortTile, j1 = j0 + kSortTile < N ? j0 + kSortTile : N;
-  const TileMates tm{mr, lob, mtab};
-  for_tile_occurrences<W, true>(tm, j0, j1, nmates, occbase, mlen, wbase, words, k,
-                                [&](int, bool valid, uint64_t j, KV key, uint32_t code) {
-    for (int w = 0; w < kBlock / 64; w++) wcnt[w][threadIdx.x] = 0;
-    __syncthreads();
-    SK skey{};
+  const uint64_t out = threadIdx.x < 256 ? offs[(size_t)threadIdx.x * ntiles + blockIdx.x] : 0;
+  if (threadIdx.x < 128) h2[threadIdx.x] = 0;
+#pragma unroll
+  for (int r = 0; r < 4; r++) wcnt[wid][r * 64 + lane] = 0;
+  const uint64_t j0 = (uint64_t)blockIdx.x * kOccTile;
+  const uint32_t tn = (uint32_t)(N - j0 < (uint64_t)kOccTile ? N - j0 : (uint64_t)kOccTile);
+  const TileMates tm{mr, lob, lwb, mtab};
+  tile_mates_init(tm, j0, j0 + tn, nmates, occbase, wbase);
+  const uint32_t first = (uint32_t)wid * 64 * kOccPer + lane;
+  uint32_t rank[kOccPer];  // rank << 8 | digit, ~0 for no record of this range
+#pragma unroll
+  for (int r = 0; r < kOccPer; r++) {
+    const uint32_t q = first + r * 64;
+    bool valid = q < tn;
     uint32_t d = 0;
     if (valid) {
-      make_sort_key(key, nb, skey);
+      uint32_t code;
+      SK skey;
+      make_sort_key(tile_occurrence<W, false>(tm, j0, q, occbase, wbase, words, k, &code), nb, skey);
       d = key_byte(skey, dbyte);
       const uint32_t t = key_byte(skey, nb - 1);
       if (nhist && t >= nlo && t < nhi) {
         const uint32_t nd = key_byte(skey, ndbyte);
-        atomicAdd(&h2[nd >> 1], 1u << (16 * (nd & 1)));  // at most kSortTile per digit
+        atomicAdd(&h2[nd >> 1], 1u << (16 * (nd & 1)));  // at most kOccTile per digit
       }
       valid = t >= tlo && t < thi;  // key-range pass: other records wait for their range
     }
-    uint64_t act = __ballot(valid);
-    uint64_t match = act;
-#pragma unroll
-    for (int b = 0; b < 8; b++) {
-      uint64_t m = __ballot((d >> b) & 1);
-      match &= ((d >> b) & 1) ? m : ~m;
-    }
-    uint32_t rank = __popcll(match & lt);
-    if (valid && rank == 0) wcnt[wid][d] = (uint16_t)__popcll(match);
-    __syncthreads();
-    if (valid) {
-      uint32_t pos = lrun[d] + rank;
-      for (int w = 0; w < wid; w++) pos += wcnt[w][d];
-      sv[pos] = ((uint32_t)(j - j0) << 8) | code;
-    }
-    __syncthreads();
-    uint32_t tot = 0;
-    for (int w = 0; w < kBlock / 64; w++) tot += wcnt[w][threadIdx.x];
-    lrun[threadIdx.x] += tot;
-  });
-  __syncthreads();
-  const uint32_t tn = lrun[255];  // records of this range in the tile
-  for (uint32_t i = threadIdx.x; i < tn; i += kBlock) {
-    const uint32_t v = sv[i];
-    const uint64_t j = j0 + (v >> 8);
-    uint32_t code_unused;
-    SK skey;
-    make_sort_key(tile_occurrence<W, false>(tm, j0, j, occbase, mlen, wbase, words, k, &code_unused), nb, skey);
-    const uint32_t d = key_byte(skey, dbyte);
-    const uint64_t pos = run[d] + (i - lbase[d]);
-    okeys[pos] = skey;
-    ocodes[pos] = (uint8_t)v;
+    const uint32_t x = wave_rank(wcnt[wid], d, valid, lt);
+    rank[r] = valid ? (x << 8) | d : ~0u;
   }
-  if (nhist)
+  __syncthreads();
+  const uint32_t mine = threadIdx.x == 255 ? wcnt[kOccWaves - 1][255] : 0;
+  const uint32_t start = tile_digit_starts<kOccWaves>(wcnt, wsum);
+  if (threadIdx.x < 256) run[threadIdx.x] = out - start;
+  if (threadIdx.x == 255) last = wcnt[kOccWaves - 1][255] + mine;  // the records of this range in the tile
+  __syncthreads();
+#pragma unroll
+  for (int r = 0; r < kOccPer; r++)
+    if (rank[r] != ~0u) sq[wcnt[wid][rank[r] & 0xff] + (rank[r] >> 8)] = (uint16_t)(first + r * 64);
+  __syncthreads();
+  const uint32_t nrec = last;
+#pragma unroll 2
+  for (uint32_t i = threadIdx.x; i < nrec; i += kOccThreads) {
+    uint32_t code;
+    SK skey;
+    make_sort_key(tile_occurrence<W, true>(tm, j0, sq[i], occbase, wbase, words, k, &code), nb, skey);
+    const uint64_t pos = run[key_byte(skey, dbyte)] + i;
+    okeys[pos] = skey;
+    ocodes[pos] = (uint8_t)code;
+  }
+  if (nhist && threadIdx.x < 256)
     nhist[(size_t)threadIdx.x * ntiles + blockIdx.x] = (h2[threadIdx.x >> 1] >> (16 * (threadIdx.x & 1))) & 0xffffu;
 }
 
 // Occurrences per value of the sort key's top byte (the key ranges of a
 // multi-pass build are cut on it).
 template <int W>
-__global__ void __launch_bounds__(kBlock) k_top_hist(uint64_t N, uint64_t nmates, const uint64_t* __restrict__ occbase,
-                                                     const uint32_t* __restrict__ mlen,
-                                                     const uint64_t* __restrict__ wbase,
-                                                     const uint64_t* __restrict__ words, int k, int nb,
-                                                     unsigned long long* __restrict__ out) {
+__global__ void __launch_bounds__(kOccThreads) k_top_hist(uint64_t N, uint64_t nmates,
+                                                          const uint64_t* __restrict__ occbase,
+                                                          const uint64_t* __restrict__ wbase,
+                                                          const uint64_t* __restrict__ words, int k, int nb,
+                                                          unsigned long long* __restrict__ out) {
   using SK = typename SortKeyOf<W>::T;
   __shared__ uint32_t h[256];
-  __shared__ uint64_t mr[3];
-  __shared__ uint32_t lob[kTileMateCap];
-  __shared__ uint16_t mtab[kSortTile];
-  h[threadIdx.x] = 0;
-  uint64_t j0 = (uint64_t)blockIdx.x * kSortTile, j1 = j0 + kSortTile < N ? j0 + kSortTile : N;
-  for_tile_occurrences<W, false>(TileMates{mr, lob, mtab}, j0, j1, nmates, occbase, mlen, wbase, words, k,
-                                 [&](int, bool valid, uint64_t, KV key, uint32_t) {
-                                   if (valid) {
-                                     SK sk;
-                                     make_sort_key(key, nb, sk);
-                                     atomicAdd(&h[key_byte(sk, nb - 1)], 1u);
-                                   }
-                                 });
+  __shared__ uint64_t mr[5];
+  __shared__ uint32_t lob[kTileMateCap], lwb[kTileMateCap];
+  __shared__ uint16_t mtab[kOccTile];
+  if (threadIdx.x < 256) h[threadIdx.x] = 0;
+  const uint64_t j0 = (uint64_t)blockIdx.x * kOccTile, j1 = j0 + kOccTile < N ? j0 + kOccTile : N;
+  const TileMates tm{mr, lob, lwb, mtab};
+  tile_mates_init(tm, j0, j1, nmates, occbase, wbase);
+#pragma unroll 2
+  for (uint32_t q = threadIdx.x; q < (uint32_t)(j1 - j0); q += kOccThreads) {
+    uint32_t code;
+    SK sk;
+    make_sort_key(tile_occurrence<W, false>(tm, j0, q, occbase, wbase, words, k, &code), nb, sk);
+    atomicAdd(&h[key_byte(sk, nb - 1)], 1u);
+  }
   __syncthreads();
-  if (h[threadIdx.x]) atomicAdd(&out[threadIdx.x], (unsigned long long)h[threadIdx.x]);
+  if (threadIdx.x < 256 && h[threadIdx.x]) atomicAdd(&out[threadIdx.x], (unsigned long long)h[threadIdx.x]);
 }
 
 // First record of every bucket of [b0, b1) (start[b1] = N; empty buckets
@@ -4384,7 +4384,7 @@ static void run_build(gx_build* b) {
   const bool keep = !b->sink;          // several ranges keep their records and node graph
   DevBuf* const kept_bufs[8] = {&b->outacc, &b->c_klo, &b->c_khi, &b->c_cnt,
                                 &b->c_msk,  &b->c_hcu, &b->c_hcf, &b->c_uval};
-  const double tiles = (double)((N + kSortTile - 1) / kSortTile);
+  const double tiles = (double)((N + kOccTile - 1) / kOccTile);
   // HBM a pass may use: free now plus what this handle holds beyond the
   // parsed reads (its buffers from an earlier build are reused) and beyond
   // `kept` bytes this build holds for later, less a margin
@@ -4443,8 +4443,8 @@ static void run_build(gx_build* b) {
     if (target < N) {
       unsigned long long* th = buf<unsigned long long>(b->tophist, 256);
       GX_HIP(hipMemsetAsync(th, 0, 256 * 8, st));
-      const unsigned ntiles = (unsigned)((N + kSortTile - 1) / kSortTile);
-      hipLaunchKernelGGL(k_top_hist<W>, dim3(ntiles), dim3(kBlock), 0, st, N, nmates, occbase, mlen, wbase, words, k,
+      const unsigned ntiles = (unsigned)((N + kOccTile - 1) / kOccTile);
+      hipLaunchKernelGGL(k_top_hist<W>, dim3(ntiles), dim3(kOccThreads), 0, st, N, nmates, occbase, wbase, words, k,
                          nb, th);
       GX_HIP(hipGetLastError());
       GX_HIP(hipMemcpyAsync(toph.data(), th, 256 * 8, hipMemcpyDeviceToHost, st));
@@ -4524,7 +4524,7 @@ static void run_build(gx_build* b) {
     const size_t vbytes = std::max<size_t>(Nr + 2, 8 * (nch + 2));
     uint8_t* va = buf<uint8_t>(b->sva, vbytes);
     uint8_t* vb = buf<uint8_t>(b->svb, vbytes);
-    const unsigned ntiles = (unsigned)std::max<uint64_t>(1, (N + kSortTile - 1) / kSortTile);
+    const unsigned ntiles = (unsigned)std::max<uint64_t>(1, (N + kOccTile - 1) / kOccTile);
     // record-sort buckets: the top bkb key bytes (LDS-sized buckets)
     const int bkb = bkb_of(Nr);
     const int dbyte = nb - bkb;
@@ -4535,7 +4535,7 @@ static void run_build(gx_build* b) {
     if (Nr) {
       ph_begin(b, PH_KINSERT);
       if (!hist_ready) {
-        hipLaunchKernelGGL(k_occ_hist<W>, dim3(ntiles), dim3(kBlock), 0, st, N, nmates, occbase, mlen, wbase, words,
+        hipLaunchKernelGGL(k_occ_hist<W>, dim3(ntiles), dim3(kOccThreads), 0, st, N, nmates, occbase, wbase, words,
                            k, nb, hist, ntiles, tlo, thi, dbyte);
         GX_HIP(hipGetLastError());
       }
@@ -4546,7 +4546,7 @@ static void run_build(gx_build* b) {
       const uint32_t nlo = next_hist ? tb[ri + 1] : 0, nhi = next_hist ? tb[ri + 2] : 0;
       const int ndbyte = next_hist ? nb - bkb_of(rocc[ri + 1]) : 0;
       ph_begin(b, PH_KSCATTER);
-      hipLaunchKernelGGL(k_occ_scatter<W>, dim3(ntiles), dim3(kBlock), 0, st, N, nmates, occbase, mlen, wbase, words,
+      hipLaunchKernelGGL(k_occ_scatter<W>, dim3(ntiles), dim3(kOccThreads), 0, st, N, nmates, occbase, wbase, words,
                          k, nb, hoff, ntiles, ka, va, tlo, thi, dbyte, nlo, nhi, ndbyte, nh);
       GX_HIP(hipGetLastError());
       ph_end(b, PH_KSCATTER);

@@ -337,8 +337,65 @@ __device__ __host__ inline uint32_t key_byte(const Key128& k, int b) {
   return b < 8 ? (uint32_t)(k.lo >> (8 * b)) & 0xff : (uint32_t)(k.hi >> (8 * (b - 8))) & 0xff;
 }
 
-constexpr int kSortItems = 8;
-constexpr int kSortTile = kBlock * kSortItems;
+// A tile of the sort: kSortThreads threads with kPer elements each.  4096
+// elements over 256 digits leave runs of 16 on average, 128 bytes of 8-byte
+// keys (2048 left half a line each and twice the digit counts to scan).
+constexpr int kSortThreads = 512, kSortWaves = kSortThreads / 64;
+template <class KeyT>
+struct SortTile {
+  static constexpr int kPer = sizeof(KeyT) > 8 ? 4 : 8;
+  static constexpr int kTile = kSortThreads * kPer;
+};
+
+// Rank of each lane's digit among the wave's elements so far: count holds
+// the wave's elements of each digit (raised here), so successive calls rank
+// successive elements with no barrier between them.  All lanes call it.
+__device__ inline uint32_t wave_rank(uint16_t* count, uint32_t d, bool valid, uint64_t lt) {
+  uint64_t match = __ballot(valid);
+#pragma unroll
+  for (int b = 0; b < 8; b++) {
+    const uint64_t m = __ballot((d >> b) & 1);
+    match &= ((d >> b) & 1) ? m : ~m;
+  }
+  // the wave's LDS accesses run in order: read by every lane, then raised
+  // by the group's first
+  const uint32_t before = count[d];
+  __builtin_amdgcn_wave_barrier();
+  if (valid && (match & lt) == 0) count[d] = (uint16_t)(before + __popcll(match));
+  __builtin_amdgcn_wave_barrier();
+  return before + __popcll(match & lt);
+}
+
+// The waves' digit counts of a tile turned into each wave's first position
+// of each digit, in digit order and then wave order; returns (threads below
+// 256) the first position of digit threadIdx.x.  wsum: [4].  Barriers before
+// and after by the caller.
+template <int kWaves>
+__device__ inline uint32_t tile_digit_starts(uint16_t (*wcnt)[256], uint32_t* wsum) {
+  const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
+  uint32_t c[kWaves], tot = 0, incl = 0;
+  if (threadIdx.x < 256) {
+#pragma unroll
+    for (int w = 0; w < kWaves; w++) {
+      c[w] = tot;
+      tot += wcnt[w][threadIdx.x];
+    }
+    incl = tot;
+#pragma unroll
+    for (int o = 1; o < 64; o <<= 1) {
+      const uint32_t y = __shfl_up(incl, o);
+      if (lane >= o) incl += y;
+    }
+    if (lane == 63) wsum[wid] = incl;
+  }
+  __syncthreads();
+  if (threadIdx.x >= 256) return 0;
+  uint32_t b = incl - tot;
+  for (int w = 0; w < wid; w++) b += wsum[w];
+#pragma unroll
+  for (int w = 0; w < kWaves; w++) wcnt[w][threadIdx.x] = (uint16_t)(b + c[w]);
+  return b;
+}
 
 // Sorts of few elements: one block, every pass in LDS, one launch (three per
 // pass otherwise, 2.5 us each with nothing in between: 12 passes over the
@@ -355,7 +412,7 @@ __global__ void __launch_bounds__(kSmallThreads) k_radix_small(KeyT* __restrict_
   __shared__ KeyT sk[kSmallSort];
   __shared__ ValT sv[kVals ? kSmallSort : 1];
   __shared__ uint16_t wcnt[kWaves][256];
-  __shared__ uint32_t base[256], wsum[4];
+  __shared__ uint32_t wsum[4];
   const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
   const uint64_t lt = (lane == 0) ? 0ull : (~0ull >> (64 - lane));
   const uint32_t first = (uint32_t)wid * 64 * kSmallPer;
@@ -377,49 +434,16 @@ __global__ void __launch_bounds__(kSmallThreads) k_radix_small(KeyT* __restrict_
 #pragma unroll
     for (int r = 0; r < kSmallPer; r++) {
       const bool valid = first + r * 64 + lane < n;
-      const uint32_t d = valid ? key_byte(key[r], byte) : 0;
-      uint64_t match = __ballot(valid);
-#pragma unroll
-      for (int b = 0; b < 8; b++) {
-        const uint64_t m = __ballot((d >> b) & 1);
-        match &= ((d >> b) & 1) ? m : ~m;
-      }
-      // the wave's LDS accesses run in order: read by every lane, then
-      // raised by the group's first
-      const uint32_t before = wcnt[wid][d];
-      rank[r] = before + __popcll(match & lt);
-      dig[r] = d;
-      __builtin_amdgcn_wave_barrier();
-      if (valid && (match & lt) == 0) wcnt[wid][d] = (uint16_t)(before + __popcll(match));
-      __builtin_amdgcn_wave_barrier();
+      dig[r] = valid ? key_byte(key[r], byte) : 0;
+      rank[r] = wave_rank(wcnt[wid], dig[r], valid, lt);
     }
     __syncthreads();
-    uint32_t tot = 0, incl = 0;
-    if (threadIdx.x < 256) {
-      for (int w = 0; w < kWaves; w++) {
-        const uint32_t c = wcnt[w][threadIdx.x];
-        wcnt[w][threadIdx.x] = (uint16_t)tot;
-        tot += c;
-      }
-      incl = tot;
-#pragma unroll
-      for (int o = 1; o < 64; o <<= 1) {
-        const uint32_t y = __shfl_up(incl, o);
-        if (lane >= o) incl += y;
-      }
-      if (lane == 63) wsum[wid] = incl;
-    }
-    __syncthreads();
-    if (threadIdx.x < 256) {
-      uint32_t b = incl - tot;
-      for (int w = 0; w < wid; w++) b += wsum[w];
-      base[threadIdx.x] = b;
-    }
+    tile_digit_starts<kWaves>(wcnt, wsum);
     __syncthreads();
 #pragma unroll
     for (int r = 0; r < kSmallPer; r++)
       if (first + r * 64 + lane < n) {
-        const uint32_t pos = base[dig[r]] + wcnt[wid][dig[r]] + rank[r];
+        const uint32_t pos = wcnt[wid][dig[r]] + rank[r];
         sk[pos] = key[r];
         if (kVals) sv[pos] = val[r];
       }
@@ -443,92 +467,52 @@ __global__ void __launch_bounds__(kSmallThreads) k_radix_small(KeyT* __restrict_
   }
 }
 
-// Tile-local digit bases for a staged scatter: offs is the exclusive scan of
-// the digit-major per-tile counts (entry d * ntiles + tile, total last), so
-// this tile's count of digit d is the difference of two neighbours; lbase[d]
-// = elements of the tile with a smaller digit (IdxT: any type holding
-// kSortTile).  Block of kBlock = 256 threads, one digit each.
-template <class IdxT>
-__device__ inline void tile_digit_bases(const uint64_t* __restrict__ offs, unsigned ntiles, IdxT* lbase, IdxT* lrun,
-                                        uint32_t* wsum) {
-  const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
-  const size_t at = (size_t)threadIdx.x * ntiles + blockIdx.x;
-  const uint32_t c = (uint32_t)(offs[at + 1] - offs[at]);
-  uint32_t incl = c;
-#pragma unroll
-  for (int o = 1; o < 64; o <<= 1) {
-    const uint32_t y = __shfl_up(incl, o);
-    if (lane >= o) incl += y;
-  }
-  if (lane == 63) wsum[wid] = incl;
-  __syncthreads();
-  uint32_t before = incl - c;
-  for (int w = 0; w < wid; w++) before += wsum[w];
-  lbase[threadIdx.x] = (IdxT)before;
-  lrun[threadIdx.x] = (IdxT)before;
-}
-
-// The same from the counts themselves (hist, digit-major, not scanned), with
-// each digit's first output position in run: with few tiles every block adds
-// up the counts before its own, which saves the launches of a scan.
+// First output position of digit threadIdx.x (threads below 256) for a tile
+// from the tiles' counts themselves (hist, digit-major, not scanned): with
+// few tiles every block adds up the counts before its own, which saves the
+// launches of a scan.  wsum: [4].  All threads call it.
 constexpr unsigned kDirectTiles = 64;
-template <class IdxT>
-__device__ inline void tile_digit_bases_direct(const uint32_t* __restrict__ hist, unsigned ntiles, uint64_t* run,
-                                               IdxT* lbase, IdxT* lrun, uint32_t* wsum) {
+__device__ inline uint64_t direct_digit_start(const uint32_t* __restrict__ hist, unsigned ntiles, uint32_t* wsum) {
   const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
-  uint32_t before = 0, all = 0, mine = 0;
+  uint32_t before = 0, all = 0, incl = 0;
+  if (threadIdx.x < 256) {
 #pragma unroll 8
-  for (unsigned t = 0; t < ntiles; t++) {
-    const uint32_t c = hist[(size_t)threadIdx.x * ntiles + t];
-    before += t < blockIdx.x ? c : 0;
-    mine = t == blockIdx.x ? c : mine;
-    all += c;
-  }
-  uint32_t ia = all, im = mine;
-#pragma unroll
-  for (int o = 1; o < 64; o <<= 1) {
-    const uint32_t ya = __shfl_up(ia, o), ym = __shfl_up(im, o);
-    if (lane >= o) {
-      ia += ya;
-      im += ym;
+    for (unsigned t = 0; t < ntiles; t++) {
+      const uint32_t c = hist[(size_t)threadIdx.x * ntiles + t];
+      before += t < blockIdx.x ? c : 0;
+      all += c;
     }
-  }
-  __shared__ uint32_t asum[kBlock / 64];
-  if (lane == 63) {
-    asum[wid] = ia;
-    wsum[wid] = im;
+    incl = all;
+#pragma unroll
+    for (int o = 1; o < 64; o <<= 1) {
+      const uint32_t y = __shfl_up(incl, o);
+      if (lane >= o) incl += y;
+    }
+    if (lane == 63) wsum[wid] = incl;
   }
   __syncthreads();
-  uint32_t ba = ia - all, bm = im - mine;
-  for (int w = 0; w < wid; w++) {
-    ba += asum[w];
-    bm += wsum[w];
-  }
-  run[threadIdx.x] = (uint64_t)ba + before;
-  lbase[threadIdx.x] = (IdxT)bm;
-  lrun[threadIdx.x] = (IdxT)bm;
+  if (threadIdx.x >= 256) return 0;
+  uint32_t b = incl - all;
+  for (int w = 0; w < wid; w++) b += wsum[w];
+  return (uint64_t)b + before;
 }
 
 template <class KeyT>
-__global__ void __launch_bounds__(kBlock) k_radix_hist(const KeyT* __restrict__ keys, size_t n, int byte,
-                                                       uint32_t* __restrict__ hist, unsigned ntiles) {
+__global__ void __launch_bounds__(kSortThreads) k_radix_hist(const KeyT* __restrict__ keys, size_t n, int byte,
+                                                             uint32_t* __restrict__ hist, unsigned ntiles) {
   __shared__ uint32_t h[256];
-  h[threadIdx.x] = 0;
+  if (threadIdx.x < 256) h[threadIdx.x] = 0;
   __syncthreads();
-  size_t base = (size_t)blockIdx.x * kSortTile;
-#pragma unroll 4
-  for (int i = 0; i < kSortItems; i++) {
-    size_t j = base + (size_t)i * kBlock + threadIdx.x;
+  const size_t base = (size_t)blockIdx.x * SortTile<KeyT>::kTile;
+#pragma unroll
+  for (int i = 0; i < SortTile<KeyT>::kPer; i++) {
+    const size_t j = base + (size_t)i * kSortThreads + threadIdx.x;
     if (j < n) atomicAdd(&h[key_byte(keys[j], byte)], 1u);
   }
   __syncthreads();
-  hist[(size_t)threadIdx.x * ntiles + blockIdx.x] = h[threadIdx.x];
+  if (threadIdx.x < 256) hist[(size_t)threadIdx.x * ntiles + blockIdx.x] = h[threadIdx.x];
 }
 
-// Scatter with stable ranks: the tile is processed in kSortItems rounds of
-// 256 consecutive elements; inside a round the rank of an element among equal
-// digits comes from a wave-level match (8 ballots) plus the counts of the
-// lower waves, so ties keep their input order.
 // A load of data read once, in order: nontemporal for integer words, so
 // the stream does not evict lines other accesses reuse.
 template <class T>
@@ -537,79 +521,83 @@ __device__ inline T load_stream(const T* p) {
   else return *p;
 }
 
-// The tile's elements are ranked into an LDS stage in digit order, then
-// written out as one contiguous run per digit (the tile's share of that
-// digit's output range): scattered element stores would leave lines partly
-// written across rounds, and the partial lines cost extra HBM writes.
+// Scatter with stable ranks.  Each wave of the tile holds a contiguous run
+// of its elements in registers and ranks them by itself (wave_rank), so the
+// tile has five barriers in all; ranked in rounds of 256 elements with the
+// waves' counts exchanged in each, it had three per round and waited on them
+// (the records of 10 Mbp, k = 31: 3.9 -> 3.0 ms; of 4 x 20 M at k = 55 3.5 ->
+// 2.7 ms).  The elements then go through an LDS stage in digit order and leave as one
+// contiguous run per digit (the tile's share of that digit's output range):
+// scattered element stores would leave lines partly written, and the partial
+// lines cost extra HBM writes.
 // offs: the scanned counts, or (kDirect) the counts themselves.
 template <class KeyT, bool kVals, class ValT, bool kDirect>
-__global__ void __launch_bounds__(kBlock) k_radix_scatter(const KeyT* __restrict__ keys, const ValT* __restrict__ vals,
+__global__ void __launch_bounds__(kSortThreads) k_radix_scatter(const KeyT* __restrict__ keys, const ValT* __restrict__ vals,
                                                           size_t n, int byte,
                                                           const typename std::conditional<kDirect, uint32_t, uint64_t>::type* __restrict__ offs,
                                                           unsigned ntiles, KeyT* __restrict__ okeys,
                                                           ValT* __restrict__ ovals) {
-  __shared__ uint64_t run[256];
-  __shared__ uint32_t lbase[256], lrun[256], wsum[kBlock / 64];
-  __shared__ uint16_t wcnt[kBlock / 64][256];
-  __shared__ KeyT sk[kSortTile];
-  __shared__ ValT sv[kVals ? kSortTile : 1];
+  constexpr int kPer = SortTile<KeyT>::kPer, kTile = SortTile<KeyT>::kTile;
+  __shared__ uint64_t run[256];  // output position of a digit's elements less their place in the stage
+  __shared__ uint32_t wsum[4];
+  __shared__ uint16_t wcnt[kSortWaves][256];
+  __shared__ KeyT sk[kTile];
+  __shared__ ValT sv[kVals ? kTile : 1];
   const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
-  if constexpr (kDirect) {
-    tile_digit_bases_direct(offs, ntiles, run, lbase, lrun, wsum);
-  } else {
-    run[threadIdx.x] = offs[(size_t)threadIdx.x * ntiles + blockIdx.x];
-    tile_digit_bases(offs, ntiles, lbase, lrun, wsum);
-  }
   const uint64_t lt = (lane == 0) ? 0ull : (~0ull >> (64 - lane));
-  size_t base = (size_t)blockIdx.x * kSortTile;
-  for (int r = 0; r < kSortItems; r++) {
-    for (int w = 0; w < kBlock / 64; w++) wcnt[w][threadIdx.x] = 0;
-    __syncthreads();
-    size_t j = base + (size_t)r * kBlock + threadIdx.x;
-    bool valid = j < n;
-    KeyT key{};
-    ValT val = 0;
-    uint32_t d = 0;
-    if (valid) {
-      key = load_stream(keys + j);
-      if (kVals) val = load_stream(vals + j);
-      d = key_byte(key, byte);
-    }
-    uint64_t act = __ballot(valid);
-    uint64_t match = act;
+  const size_t base = (size_t)blockIdx.x * kTile;
+  const uint32_t tn = (uint32_t)(n - base < (size_t)kTile ? n - base : (size_t)kTile);
+  const uint32_t first = (uint32_t)wid * 64 * kPer + lane;
+  KeyT key[kPer];
+  ValT val[kPer];
+  uint32_t rank[kPer];
 #pragma unroll
-    for (int b = 0; b < 8; b++) {
-      uint64_t m = __ballot((d >> b) & 1);
-      match &= ((d >> b) & 1) ? m : ~m;
+  for (int r = 0; r < kPer; r++) {
+    const uint32_t i = first + r * 64;
+    key[r] = KeyT{};
+    if (i < tn) {
+      key[r] = load_stream(keys + base + i);
+      if (kVals) val[r] = load_stream(vals + base + i);
     }
-    uint32_t rank = __popcll(match & lt);
-    if (valid && rank == 0) wcnt[wid][d] = (uint16_t)__popcll(match);
-    __syncthreads();
-    if (valid) {
-      uint32_t pos = lrun[d] + rank;
-      for (int w = 0; w < wid; w++) pos += wcnt[w][d];
-      sk[pos] = key;
-      if (kVals) sv[pos] = val;
-    }
-    __syncthreads();
-    uint32_t tot = 0;
-    for (int w = 0; w < kBlock / 64; w++) tot += wcnt[w][threadIdx.x];
-    lrun[threadIdx.x] += tot;
   }
+  uint64_t out;
+  if constexpr (kDirect) {
+    out = direct_digit_start(offs, ntiles, wsum);
+  } else {
+    out = threadIdx.x < 256 ? offs[(size_t)threadIdx.x * ntiles + blockIdx.x] : 0;
+  }
+#pragma unroll
+  for (int q = 0; q < 4; q++) wcnt[wid][q * 64 + lane] = 0;
+  __builtin_amdgcn_wave_barrier();
+#pragma unroll
+  for (int r = 0; r < kPer; r++) rank[r] = wave_rank(wcnt[wid], key_byte(key[r], byte), first + r * 64 < tn, lt);
   __syncthreads();
-  const uint32_t tn = (uint32_t)(n - base < (size_t)kSortTile ? n - base : (size_t)kSortTile);
-  for (uint32_t i = threadIdx.x; i < tn; i += kBlock) {
-    const KeyT key = sk[i];
-    const uint32_t d = key_byte(key, byte);
-    const uint64_t pos = run[d] + (i - lbase[d]);
-    okeys[pos] = key;
-    if (kVals) ovals[pos] = sv[i];
+  const uint32_t start = tile_digit_starts<kSortWaves>(wcnt, wsum);
+  if (threadIdx.x < 256) run[threadIdx.x] = out - start;
+  __syncthreads();
+#pragma unroll
+  for (int r = 0; r < kPer; r++)
+    if (first + r * 64 < tn) {
+      const uint32_t pos = wcnt[wid][key_byte(key[r], byte)] + rank[r];
+      sk[pos] = key[r];
+      if (kVals) sv[pos] = val[r];
+    }
+  __syncthreads();
+#pragma unroll
+  for (int r = 0; r < kPer; r++) {
+    const uint32_t i = r * kSortThreads + threadIdx.x;
+    if (i < tn) {
+      const KeyT k = sk[i];
+      const uint64_t pos = run[key_byte(k, byte)] + i;
+      okeys[pos] = k;
+      if (kVals) ovals[pos] = sv[i];
+    }
   }
 }
 
 template <class KeyT>
 static size_t radix_scratch_bytes(size_t n) {
-  size_t ntiles = (n + kSortTile - 1) / kSortTile;
+  size_t ntiles = (n + SortTile<KeyT>::kTile - 1) / SortTile<KeyT>::kTile;
   if (ntiles == 0) ntiles = 1;
   size_t h = 256 * ntiles;
   return h * 4 + (h + 1) * 8 + scan_scratch_bytes<uint64_t>(h) + 1024;
@@ -627,7 +615,7 @@ static bool radix_sort_impl(KeyT* k1, ValT* v1, KeyT* k2, ValT* v2, size_t n, in
     GX_HIP(hipGetLastError());
     return false;
   }
-  unsigned ntiles = (unsigned)((n + kSortTile - 1) / kSortTile);
+  unsigned ntiles = (unsigned)((n + SortTile<KeyT>::kTile - 1) / SortTile<KeyT>::kTile);
   size_t h = (size_t)256 * ntiles;
   uint32_t* hist = reinterpret_cast<uint32_t*>(scratch);
   uint64_t* offs = reinterpret_cast<uint64_t*>(((uintptr_t)(hist + h) + 255) & ~(uintptr_t)255);
@@ -638,14 +626,14 @@ static bool radix_sort_impl(KeyT* k1, ValT* v1, KeyT* k2, ValT* v2, size_t n, in
     KeyT* ok = flip ? k1 : k2;
     ValT* iv = flip ? v2 : v1;
     ValT* ov = flip ? v1 : v2;
-    hipLaunchKernelGGL((k_radix_hist<KeyT>), dim3(ntiles), dim3(kBlock), 0, st, ik, n, b, hist, ntiles);
+    hipLaunchKernelGGL((k_radix_hist<KeyT>), dim3(ntiles), dim3(kSortThreads), 0, st, ik, n, b, hist, ntiles);
     GX_HIP(hipGetLastError());
     if (ntiles <= kDirectTiles) {
-      hipLaunchKernelGGL((k_radix_scatter<KeyT, kVals, ValT, true>), dim3(ntiles), dim3(kBlock), 0, st, ik, iv, n, b,
+      hipLaunchKernelGGL((k_radix_scatter<KeyT, kVals, ValT, true>), dim3(ntiles), dim3(kSortThreads), 0, st, ik, iv, n, b,
                          hist, ntiles, ok, ov);
     } else {
       exclusive_scan<uint32_t, uint64_t>(hist, offs, h, sc, st);
-      hipLaunchKernelGGL((k_radix_scatter<KeyT, kVals, ValT, false>), dim3(ntiles), dim3(kBlock), 0, st, ik, iv, n, b,
+      hipLaunchKernelGGL((k_radix_scatter<KeyT, kVals, ValT, false>), dim3(ntiles), dim3(kSortThreads), 0, st, ik, iv, n, b,
                          offs, ntiles, ok, ov);
     }
     GX_HIP(hipGetLastError());

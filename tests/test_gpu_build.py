@@ -271,3 +271,31 @@ def test_record_bucket_sizes(gx, k, n):
         rng.shuffle(reads)
         text = "".join(f"{4 * i + 2}\t{s}\n" for i, s in enumerate(reads)).encode()
         assert gx.build_graph(text, k)[0] == oracle.build_graph(text, k)[0], repeats
+
+
+@pytest.mark.parametrize("k", [21, 55])
+@pytest.mark.parametrize("occ", [2, 4, 5, 45])
+@pytest.mark.parametrize("n", [4095, 4096, 4097, 12289])
+def test_occurrence_tiles(gx, k, occ, n):
+    """About n occurrences in reads of occ k-mers each, every ninth read with
+    a letter outside ACGT (no occurrences): tiles of 4096 occurrences, full
+    and with a remainder, whose reads fit the tile's tables and do not, in
+    few letters so that keys repeat across the tile's waves."""
+    import random
+    rng = random.Random(n * occ + k)
+    genome = "".join(rng.choice("ACGT") for _ in range(900 + k))
+    left, reads = n, []
+    while left > 0:
+        i = len(reads)
+        length = k - 1 + max(2, min(occ, left))
+        at = rng.randrange(len(genome) - length + 1)
+        s = genome[at:at + length]
+        if rng.random() < 0.5:
+            s = s[::-1].translate(str.maketrans("ACGT", "TGCA"))
+        if i % 9 == 5:
+            s = s[:3] + "N" + s[4:]
+        else:
+            left -= length - k + 1
+        reads.append(s)
+    text = "".join(f"{i + 1}\t{s}\n" for i, s in enumerate(reads)).encode()
+    assert gx.build_graph(text, k)[0] == oracle.build_graph(text, k)[0]

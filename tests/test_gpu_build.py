@@ -299,3 +299,36 @@ def test_occurrence_tiles(gx, k, occ, n):
         reads.append(s)
     text = "".join(f"{i + 1}\t{s}\n" for i, s in enumerate(reads)).encode()
     assert gx.build_graph(text, k)[0] == oracle.build_graph(text, k)[0]
+
+
+@pytest.mark.parametrize("seed", range(6))
+def test_line_and_mate_lengths(gx, seed):
+    """Mates of every length up to 70, around the multiples of 32 and 128,
+    and on both sides of the lengths that a whole wave takes, one or two to a
+    line, in any alignment, upper and lower case, with other letters at any
+    place, readIds of up to 20 digits and a sign, empty second fields,
+    trailing tabs and every line end."""
+    import random
+    rng = random.Random(seed)
+    lengths = [n for n in range(14, 71)] + [95, 96, 97, 127, 128, 129, 255, 257, 1000, 1023, 1024, 1025, 2047, 2048,
+                                            2049, 2100, 4097, 9000]
+    rng.shuffle(lengths)
+
+    def mate(n):
+        s = "".join(rng.choice("ACGTacgt") for _ in range(n))
+        if rng.random() < 0.2:
+            i = rng.choice([0, n - 1, rng.randrange(n)])
+            s = s[:i] + rng.choice("NnBS@`-. ") + s[i + 1:]
+        return s
+
+    lines = []
+    for i, n in enumerate(lengths):
+        rid = str(3 * i + 1)
+        rid = rng.choice(["", "", "+"]) + "0" * rng.choice([0, 0, 1, 15 - len(rid), 16 - len(rid), 20 - len(rid)]) + rid
+        line = rid + "\t" + mate(n)
+        if rng.random() < 0.4:
+            line += "\t" + mate(rng.choice(lengths))
+        line += "\t" * rng.choice([0, 0, 0, 1, 9])
+        lines.append(line + rng.choice(["\n", "\n", "\r\n", "\r"]))
+    text = "".join(lines).encode()
+    assert gx.build_graph(text, 11)[0] == oracle.build_graph(text, 11)[0]

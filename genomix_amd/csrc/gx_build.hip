@@ -676,13 +676,13 @@ __device__ inline KV occ_info(const uint64_t* __restrict__ w, uint32_t L, uint32
   // letter is at bit end (read when p + k < L), the previous one at sh - 2
   const uint32_t wi = p >> 5, sh = 2 * (p & 31), end = sh + 2 * (uint32_t)k;
   const bool has_next = CODES && p + k < L, has_prev = CODES && p > 0;
-  const uint64_t wa = w[wi];
-  const uint64_t wb = (end > 64 || (has_next && end >= 64)) ? w[wi + 1] : 0;
-  const uint64_t wc = (W == 2 && (end > 128 || (has_next && end >= 128))) ? w[wi + 2] : 0;
+  // (the words after the k-mer's may be the next mate's: their bits are
+  // masked off, and a load costs less than the branch round it)
+  const uint64_t wa = w[wi], wb = w[wi + 1], wc = W == 2 ? w[wi + 2] : 0;
   const uint64_t wp = (has_prev && sh == 0) ? w[wi - 1] : 0;
   KV v;
-  v.lo = sh ? (wa >> sh) | (wb << (64 - sh)) : wa;
-  v.hi = W == 2 ? (sh ? (wb >> sh) | (wc << (64 - sh)) : wb) : 0;
+  v.lo = (wa >> sh) | ((wb << 1) << (63 - sh));
+  v.hi = W == 2 ? (wb >> sh) | ((wc << 1) << (63 - sh)) : 0;
   const KV km = kmask<W>(k);
   v.lo &= km.lo;
   v.hi &= km.hi;
@@ -1309,7 +1309,7 @@ __global__ void __launch_bounds__(kOccThreads) k_occ_hist(uint64_t N, uint64_t n
 // code (one byte): the sorts after this are stable or break ties by the
 // record's index in its bucket, so occurrence order among equal keys needs no
 // stored occurrence number.  Bound by the integer work of the extraction.
-// 10 Mbp, k = 31: 3.9 -> 2.9 ms, 4 key ranges of k = 55 9.2 -> 7.3 ms, against
+// 10 Mbp, k = 31: 3.9 -> 2.8 ms, 4 key ranges of k = 55 9.2 -> 6.9 ms, against
 // rounds of 256 occurrences with three barriers each, neighbour codes made
 // before the range test, and the mates' lengths and words read from memory
 // per occurrence.

@@ -2645,7 +2645,19 @@ __device__ __forceinline__ void put_read(uint8_t*& p, const uint64_t* w, uint32_
     uint64_t x = sh ? (w[a] >> sh) | (w[a + 1] << (64 - sh)) : w[a];
     put64(p, x);
   }
-  for (int64_t r = q + 7; r >= 0; r--) *p++ = (uint8_t)(w[r >> 3] >> (8 * (r & 7)));
+  const int left = (int)q + 8;  // the stream's first bytes, fewer than eight
+  if (left) put_le(p, __builtin_bswap64(w[0] << (64 - 8 * left)), left);
+}
+
+// What a read head's bytes are made from.
+struct HeadSrc {
+  uint32_t m, L, Lm;
+  int64_t rid;
+  const uint64_t *w, *wm;
+};
+__device__ __forceinline__ HeadSrc head_src(const SerCtx& c, uint64_t j) {
+  const uint32_t m = c.uval[j] & 0x7fffffffu;
+  return HeadSrc{m, c.mlen[m], c.mlen[m ^ 1], c.rid[m >> 1], c.words + c.wbase[m], c.words + c.wbase[m ^ 1]};
 }
 
 template <int W>
@@ -2658,6 +2670,8 @@ __device__ __forceinline__ void write_record(const SerCtx& c, uint64_t i, uint8_
   const uint32_t needs = c.jdk7 ? c.needs[i] : 0u;
   const uint64_t lists = needs ? c.lists[i] : 0ull;
   const uint64_t h0 = (nu | nf) ? c.hstart[i] : 0ull;
+  HeadSrc h{};  // the first head's, fetched behind the edges
+  if (nu | nf) h = head_src(c, h0);
   put32(p, (uint32_t)(rec - 8));
   put32(p, 4 + c.nb);
   put_key<W>(p, v, c.k, c.nb);
@@ -2686,14 +2700,13 @@ __device__ __forceinline__ void write_record(const SerCtx& c, uint64_t i, uint8_
     *p++ = 1;  // whole body in stream
     put32(p, cntf);
     for (uint64_t j = a; j < a + cntf; j++) {
-      uint32_t m = c.uval[j] & 0x7fffffffu;
-      uint32_t L = c.mlen[m], Lm = c.mlen[m ^ 1];
-      *p++ = Lm > 0 ? 1 : 0;
+      if (j > h0) h = head_src(c, j);
+      *p++ = h.Lm > 0 ? 1 : 0;
       uint64_t off = f ? (uint64_t)(c.k - 1) : 0;
-      uint64_t uuid = (off << 40) | ((uint64_t)(m & 1) << 35) | (uint64_t)c.rid[m >> 1];
+      uint64_t uuid = (off << 40) | ((uint64_t)(h.m & 1) << 35) | (uint64_t)h.rid;
       put64(p, uuid);
-      put_read(p, c.words + c.wbase[m], L);
-      if (Lm > 0) put_read(p, c.words + c.wbase[m ^ 1], Lm);
+      put_read(p, h.w, h.L);
+      if (h.Lm > 0) put_read(p, h.wm, h.Lm);
     }
   }
   // coverage: Java float accumulation of 1.0f saturates at 2^24
@@ -2706,12 +2719,15 @@ __device__ __forceinline__ void write_record(const SerCtx& c, uint64_t i, uint8_
 
 // Records of 256 consecutive nodes are contiguous in the output: each
 // thread writes its record into LDS, then the block stores the whole span
-// with coalesced 4-byte writes.  Spans larger than the stage are written
-// directly.  The stage is sized at launch for 1.2 times the mean span: with
+// with coalesced 16-byte writes.  Spans larger than the stage are written
+// directly.  Bound by latency: a wave has about two read heads at k = 31, five
+// dependent reads each, which the other lanes wait for; the first head's
+// fields are therefore fetched before the edges are written.  The stage is sized at launch for 1.2 times the mean span: with
 // 16 KB for every k about half the spans at k = 31 (62 bytes a record) and
-// nearly all at k = 55 (77 bytes) missed it.  54.7 M records of k = 31 3.4 ->
-// 2.8 ms (2.1 TB/s of records and node fields), 4 x 20 M of k = 55 9.0 ->
-// 5.2 ms.
+// nearly all at k = 55 (77 bytes) missed it (54.7 M records of k = 31 3.4 ->
+// 2.8 ms, 4 x 20 M of k = 55 9.0 -> 5.2).  16-byte words out, a read's last
+// bytes as one window and the early fetch: 94 M records of k = 31 4.75 -> 4.03
+// ms (2.1 TB/s of records and node fields), 4 x 20 M of k = 55 5.0 -> 4.7.
 constexpr uint32_t kStageMax = 64 << 10;
 __host__ inline uint32_t stage_bytes(uint64_t total, uint64_t records) {
   const double span = records ? (double)total / (double)records * kBlock : 0;
@@ -2727,26 +2743,28 @@ __global__ void __launch_bounds__(kBlock) k_ser_write(SerCtx c, const uint64_t* 
   uint64_t last = first + kBlock < c.nn ? first + kBlock : c.nn;
   uint64_t s0 = roff[first], s1 = roff[last];
   uint64_t i = first + threadIdx.x;
-  // the stage starts at the 4-byte boundary at or below s0
-  uint64_t base = s0 & ~3ull;
-  bool staged = (s1 - base) <= stage_len;
+  // the stage starts at the 16-byte boundary of the output at or below s0
+  uint8_t* const o = out + s0;
+  const uint32_t sh = (uint32_t)((uintptr_t)o & 15);
+  const bool staged = s1 - s0 + sh <= stage_len;
   if (i < last) {
     uint64_t rec = roff[i + 1] - roff[i];
     // two calls: with the stage alone the stores are LDS ones
-    if (staged) write_record<W>(c, ser_node(c, i), stage + (roff[i] - base), rec);
+    if (staged) write_record<W>(c, ser_node(c, i), stage + sh + (uint32_t)(roff[i] - s0), rec);
     else write_record<W>(c, ser_node(c, i), out + roff[i], rec);
   }
   if (!staged) return;
   __syncthreads();
-  // head and tail bytes that are not 4-byte aligned
-  uint64_t a4 = (s0 + 3) & ~3ull, e4 = s1 & ~3ull;
-  if (a4 > e4) { a4 = s1; e4 = s1; }
-  for (uint64_t x = s0 + threadIdx.x; x < a4; x += kBlock) out[x] = stage[x - base];
-  for (uint64_t x = e4 + threadIdx.x; x < s1; x += kBlock) out[x] = stage[x - base];
-  const uint32_t* src = reinterpret_cast<const uint32_t*>(stage + (a4 - base));
-  uint32_t* dst = reinterpret_cast<uint32_t*>(out + a4);
-  for (uint64_t x = threadIdx.x; x < (e4 - a4) / 4; x += kBlock)
-    __builtin_nontemporal_store(src[x], dst + x);  // written once, read by the caller later
+  // bytes [sh, end) of the stage; whole 16-byte words, then the two ends
+  using V4 = __attribute__((ext_vector_type(4))) uint32_t;
+  const uint32_t end = sh + (uint32_t)(s1 - s0), w0 = (sh + 15) / 16, w1 = max(end / 16, w0);
+  uint8_t* const ob = o - sh;
+  const V4* src = reinterpret_cast<const V4*>(stage);
+  for (uint32_t x = w0 + threadIdx.x; x < w1; x += kBlock)
+    __builtin_nontemporal_store(src[x], reinterpret_cast<V4*>(ob) + x);  // written once, read by the caller later
+  for (uint32_t x = sh + threadIdx.x; x < min(16 * w0, end); x += kBlock) ob[x] = stage[x];
+  for (uint32_t x = max(16 * w1, sh) + threadIdx.x; x < end; x += kBlock)
+    if (x >= 16 * w0) ob[x] = stage[x];
 }
 
 // Output partition of each node: nonneg(hashBytes(key)) % P, the reference's

@@ -4,13 +4,14 @@
 //   1. k_line_count / k_line_write   line terminators (Hadoop LineReader rules)
 //   2. k_parse_lines                 16 lanes per line: tab fields, readId
 //   3. k_pack_mates                  4 lanes per mate: validity + 2-bit pack
-//   4. k_insert<W>                   one wave per mate: canonical k-mers into an
-//                                    open-addressing table (count + neighbour
-//                                    mask with atomics), one record per
-//                                    occurrence in emission order
-//   5. k_compact / radix sort        dense node array in KmerPointable order
-//   6. replay (k_sel_*, radix sort, k_replay)
-//                                    JDK-7 HashSet edge order for nodes whose
+//   4. k_occ_hist, k_occ_scatter, radix passes, k_bucket_*
+//                                    a record (sort key, neighbour code) per
+//                                    occurrence, sorted by (key, occurrence)
+//      (or k_insert<W>               canonical k-mers into an open-addressing
+//                                    table, with atomics)
+//   5. k_run_count, k_node_emit      nodes = runs of equal keys, in
+//                                    KmerPointable order; k_nix_* their index
+//   6. k_replay_list, k_replay       JDK-7 HashSet edge order for nodes whose
 //                                    edge lists hold >= 2 k-mers
 //   7. heads (k_heads, radix sort)   TreeSet order of 5' read heads
 //   8. k_ser_size / k_ser_write      Node bytes, Java layout, big endian

@@ -1591,8 +1591,12 @@ constexpr uint32_t kWaveMax = 512;
 constexpr int kWaveIdxBits = 9, kIdxBits = 14;  // index bits of a wave's and a block's elements
 constexpr uint32_t kBlockCap = 8192;
 __host__ __device__ constexpr uint32_t bucket_cap(int W) { return W == 1 ? 16384 : 8192; }  // 128 KB of LDS
-constexpr int kBucketLists = 4;  // up to 2048 records, up to 8192, up to bucket_cap, for k_bucket_block
-constexpr uint32_t kPartSmall = 2048, kPartMid = 8192;
+constexpr int kBucketLists = 4;  // up to 2048 records, up to part_mid, up to bucket_cap, for k_bucket_block
+constexpr uint32_t kPartSmall = 2048;
+// half of bucket_cap: 64 KB of LDS, two blocks per CU (4 x 64 M two-word
+// records, whose buckets lie around 4096: 5.65 ms in blocks of 8192 alone, one
+// per CU; 4.70 with both)
+__host__ __device__ constexpr uint32_t part_mid(int W) { return bucket_cap(W) / 2; }
 
 // n (<= 64 EPT) elements of one wave, sorted and written as records from
 // position `at` on (codes at `codes` + their index).
@@ -1648,7 +1652,7 @@ __global__ void __launch_bounds__(kBlock) k_bucket_lists(const uint64_t* __restr
       const uint64_t s = bstart[bk], t = bstart[bk + 1], n = t - s;
       if (s > t || t > N) atomicMin(err, (unsigned long long)bk);
       else if (n > bucket_cap(W)) l = 3;
-      else if (n > kWaveMax) l = n <= kPartSmall ? 0 : n <= kPartMid ? 1 : 2;
+      else if (n > kWaveMax) l = n <= kPartSmall ? 0 : n <= part_mid(W) ? 1 : 2;
       big[bk] = l == 3 ? 1 : 0;
       if (l >= 0 && l < 3) at = atomicAdd(&cnt[l], 1u);
     }
@@ -2727,7 +2731,7 @@ __device__ __forceinline__ void write_record(const SerCtx& c, uint64_t i, uint8_
 // 16 KB for every k about half the spans at k = 31 (62 bytes a record) and
 // nearly all at k = 55 (77 bytes) missed it (54.7 M records of k = 31 3.4 ->
 // 2.8 ms, 4 x 20 M of k = 55 9.0 -> 5.2).  16-byte words out, a read's last
-// bytes as one window and the early fetch: 94 M records of k = 31 4.75 -> 4.03
+// bytes as one window and the early fetch: 90 M records of k = 31 4.75 -> 4.03
 // ms (2.1 TB/s of records and node fields), 4 x 20 M of k = 55 5.0 -> 4.7.
 constexpr uint32_t kStageMax = 64 << 10;
 __host__ inline uint32_t stage_bytes(uint64_t total, uint64_t records) {
@@ -4763,18 +4767,16 @@ static void run_build(gx_build* b) {
       GX_HIP(hipGetLastError());
     }
     if (nl[1]) {
-      hipLaunchKernelGGL((k_bucket_part<W, kPartMid, 1024>), dim3(std::min(nl[1], 65536u)), dim3(1024), 0, st, kx, vx,
+      hipLaunchKernelGGL((k_bucket_part<W, part_mid(W), 1024>), dim3(std::min(nl[1], 65536u)), dim3(1024), 0, st, kx, vx,
                          ky, rcodes, bstart, nb, bkb, nl[1], blists + list_len, big, lblock, list_len, nblock,
                          errw + 2);
       GX_HIP(hipGetLastError());
     }
-    if constexpr (W == 1) {
-      if (nl[2]) {
-        hipLaunchKernelGGL((k_bucket_part<W, bucket_cap(1), 1024>), dim3(std::min(nl[2], 65536u)), dim3(1024), 0, st,
-                           kx, vx, ky, rcodes, bstart, nb, bkb, nl[2], blists + 2 * (size_t)list_len, big, lblock,
-                           list_len, nblock, errw + 2);
-        GX_HIP(hipGetLastError());
-      }
+    if (nl[2]) {
+      hipLaunchKernelGGL((k_bucket_part<W, bucket_cap(W), 1024>), dim3(std::min(nl[2], 65536u)), dim3(1024), 0, st, kx,
+                         vx, ky, rcodes, bstart, nb, bkb, nl[2], blists + 2 * (size_t)list_len, big, lblock, list_len,
+                         nblock, errw + 2);
+      GX_HIP(hipGetLastError());
     }
     const uint32_t nlisted = nl[0] + nl[1] + nl[2];
     if (nlisted) {

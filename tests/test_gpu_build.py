@@ -332,3 +332,16 @@ def test_line_and_mate_lengths(gx, seed):
         lines.append(line + rng.choice(["\n", "\n", "\r\n", "\r"]))
     text = "".join(lines).encode()
     assert gx.build_graph(text, 11)[0] == oracle.build_graph(text, 11)[0]
+
+
+@pytest.mark.parametrize("n", [4060, 4100, 8150])
+def test_two_word_bucket_tiers(gx, n):
+    """A bucket of about n two-word records (distinct k-mers that share their
+    first eight letters), on both sides of the two block sizes' border."""
+    import random
+    rng = random.Random(n)
+    reads = ["AACAGATA" + "".join(rng.choice("ACGT") for _ in range(47)) + "A" for _ in range(n)]
+    reads += ["".join(rng.choice("ACGT") for _ in range(85)) for _ in range(40)]
+    rng.shuffle(reads)
+    text = "".join(f"{4 * i + 2}\t{s}\n" for i, s in enumerate(reads)).encode()
+    assert gx.build_graph(text, 55)[0] == oracle.build_graph(text, 55)[0]

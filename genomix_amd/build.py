@@ -7,7 +7,7 @@ HERE = os.path.dirname(os.path.abspath(__file__))
 ROOT = os.path.dirname(HERE)
 LIB = os.path.join(HERE, "libgenomix_gx.so")
 SOURCES = [os.path.join(HERE, "csrc", f) for f in ("gx_build.hip", "gx_sizer.hip", "gx_batch.hip")]
-HEADERS = [os.path.join(HERE, "csrc", f) for f in ("gx_prims.h", "gx_kmer.h", "gx_sizer.h")] + [
+HEADERS = [os.path.join(HERE, "csrc", f) for f in ("gx_host.h", "gx_prims.h", "gx_kmer.h", "gx_sizer.h")] + [
     os.path.join(ROOT, "include", f) for f in ("genomix_gx.h", "genomix_sizer.h", "genomix_batch.h")]
 
 HIPCC_FLAGS = [

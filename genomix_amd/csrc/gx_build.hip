@@ -27,6 +27,7 @@
 #include <vector>
 
 #include "../../include/genomix_gx.h"
+#include "gx_host.h"
 #include "gx_kmer.h"
 #include "gx_prims.h"
 #include "gx_sizer.h"
@@ -958,9 +959,9 @@ __device__ inline KV key_of_sort(const Key128& r, int nb) {
 __device__ inline bool sk_eq(uint64_t a, uint64_t b) { return a == b; }
 __device__ inline bool sk_eq(const Key128& a, const Key128& b) { return a.lo == b.lo && a.hi == b.hi; }
 
-// Record-sort bucket: the top `bkb` bytes of the sort key (2, or 3 for
-// passes of more than about 3 * 10^8 records, so buckets stay LDS-sized; 1 when the
-// key has one byte).
+// Record-sort bucket: the top `bkb` bytes of the sort key (2, or 3 where
+// those buckets would outgrow LDS, record_bucket_bytes; 1 when the key has
+// one byte).
 template <class SK>
 __device__ inline uint32_t sort_bucket(const SK& sk, int nb, int bkb) {
   uint32_t v = 0;
@@ -970,7 +971,7 @@ __device__ inline uint32_t sort_bucket(const SK& sk, int nb, int bkb) {
 
 // Key -> node index, built from the sorted nodes without global atomics:
 // the nodes of each key bucket (the top bkb bytes of the sort key: 2, or 3
-// above 2 * 10^8 nodes) are contiguous (dir[b] = first node), and each bucket
+// for large graphs, index_bucket_bytes) are contiguous (dir[b] = first node), and each bucket
 // owns a private open-addressing region of two slots per node, filled in
 // LDS by one block.  A lookup is the bucket's two dir entries plus one or
 // two slot probes.
@@ -1141,7 +1142,6 @@ __global__ void __launch_bounds__(NT) k_nix_build(const uint64_t* __restrict__ k
   }
 }
 
-constexpr int kNixSmall = 8192, kNixLarge = 16384;  // LDS slots of k_nix_build: 32 KB (512 threads), 64 KB (1024)
 // HBM of a key-range pass, per occurrence (sizes the ranges): the records
 // (two key and two neighbour-code arrays, the sorted codes) and, per node (dfrac
 // nodes per occurrence), every node array of the pass -- key words, count,
@@ -4309,19 +4309,18 @@ static void swap_buf(DevBuf& x, DevBuf& y) {
   std::swap(x.cap, y.cap);
 }
 
+// Occurrences by top key byte where none were counted.
+static const uint64_t kNoCounts[256] = {};
+
 // Key -> node index over nodes [0, nn) in key order whose keys' top byte
-// lies in [tlo, thi).
+// lies in [tlo, thi); top: occurrences by top key byte (gx_host.h).
 template <int W>
 static NodeIndex build_node_index(gx_build* b, hipStream_t st, uint64_t nn, const uint64_t* klo, const uint64_t* khi,
-                                  const uint32_t* msk, uint32_t tlo, uint32_t thi) {
+                                  const uint32_t* msk, const uint64_t* top, uint32_t tlo, uint32_t thi) {
   const int nb = b->nb;
   const unsigned G = b->grid;
   const size_t slotsz = W == 1 ? sizeof(Slot1) : sizeof(Slot2);
-  // two-byte buckets while the larger LDS table holds 2.5 times the mean
-  // bucket (the canonical choice skews the top byte between 0.1 and 2 times
-  // the mean); beyond that three-byte ones
-  const uint64_t slots2 = 5 * nn / 65536;  // slots of a two-byte bucket of 2.5 times the mean size
-  const int xbkb = nb < 2 ? 1 : (nb >= 4 && slots2 > kNixLarge) ? 3 : 2;
+  const int xbkb = index_bucket_bytes(nb, nn, top, tlo, thi);
   const uint32_t nbk = 1u << (8 * xbkb);
   const uint32_t xb0 = tlo << (8 * (xbkb - 1)), xb1 = thi << (8 * (xbkb - 1));
   b->nix_bkb = xbkb;
@@ -4344,9 +4343,9 @@ static NodeIndex build_node_index(gx_build* b, hipStream_t st, uint64_t nn, cons
                        xb1, ndir);
   GX_HIP(hipGetLastError());
   // buckets per block: as many as fill the small table, but at least 512
-  // blocks; the large table (two blocks per CU) where one mean bucket would
-  // not leave the small one room for the skew
-  const uint64_t per = std::max<uint64_t>(1, 5 * nn / nbk);
+  // blocks; the large table (two blocks per CU) where a bucket a quarter above
+  // the fullest would not fit the small one
+  const uint64_t per = std::max<uint64_t>(1, (uint64_t)(2.5 * fullest_bucket(nn, xbkb, top, tlo, thi)));
   uint32_t span = 1;
   while ((uint64_t)span * 2 * per <= kNixSmall && (xb1 - xb0) / (span * 2) >= 512) span *= 2;
   const unsigned blocks = std::min((xb1 - xb0 + span - 1) / span, 65536u);
@@ -4635,12 +4634,8 @@ static void run_build(gx_build* b) {
   b->nuheads = 0;
   b->has_hoff = false;
   b->stats[9] = 0;
-  // record-sort bucket bytes of a pass of n records: two while a mean bucket
-  // takes a third (one-word keys) or half of an LDS bucket, as the canonical
-  // choice skews the buckets to twice the mean; a third byte costs a radix
-  // pass (320 M records: 2.7 ms) and 16 M buckets of a few records
-  const uint64_t two_bytes = W == 1 ? 5ull << 26 : 1ull << 28;
-  auto bkb_of = [&](uint64_t n) { return nb < 2 ? 1 : (nb >= 4 && n > two_bytes) ? 3 : 2; };
+  // record-sort bucket bytes of range r
+  auto bkb_of = [&](uint32_t r) { return record_bucket_bytes(W, nb, rocc[r], toph.data(), tb[r], tb[r + 1]); };
   DevBuf *hcur = &b->selflag, *hnext = &b->hist2;  // per-tile digit counts: this range's, the next one's
   bool hist_ready = false;
   for (uint32_t ri = 0; ri < R; ri++) {
@@ -4682,7 +4677,7 @@ static void run_build(gx_build* b) {
     uint8_t* vb = buf<uint8_t>(b->svb, vbytes);
     const unsigned ntiles = (unsigned)std::max<uint64_t>(1, (N + kOccTile - 1) / kOccTile);
     // record-sort buckets: the top bkb key bytes (LDS-sized buckets)
-    const int bkb = bkb_of(Nr);
+    const int bkb = bkb_of(ri);
     const int dbyte = nb - bkb;
     const size_t hn = (size_t)256 * ntiles;
     uint32_t* hist = buf<uint32_t>(*hcur, hn + 1);
@@ -4700,7 +4695,7 @@ static void run_build(gx_build* b) {
       next_hist = ri + 1 < R && rocc[ri + 1] > 0;
       uint32_t* nh = next_hist ? buf<uint32_t>(*hnext, hn + 1) : nullptr;
       const uint32_t nlo = next_hist ? tb[ri + 1] : 0, nhi = next_hist ? tb[ri + 2] : 0;
-      const int ndbyte = next_hist ? nb - bkb_of(rocc[ri + 1]) : 0;
+      const int ndbyte = next_hist ? nb - bkb_of(ri + 1) : 0;
       ph_begin(b, PH_KSCATTER);
       hipLaunchKernelGGL(k_occ_scatter<W>, dim3(ntiles), dim3(kOccThreads), 0, st, N, nmates, occbase, wbase, words,
                          k, nb, hoff, ntiles, ka, va, tlo, thi, dbyte, nlo, nhi, ndbyte, nh);
@@ -4933,7 +4928,7 @@ static void run_build(gx_build* b) {
 
   // 5b. key -> node index (heads, unitig links)
   ph_begin(b, PH_NIX);
-  const NodeIndex nix = build_node_index<W>(b, st, nn, klo, khi, msk, tlo, thi);
+  const NodeIndex nix = build_node_index<W>(b, st, nn, klo, khi, msk, toph.data(), tlo, thi);
   if (sorted) cap = 2 * nn;
   ph_end(b, PH_NIX);
 
@@ -5235,7 +5230,7 @@ static void run_build(gx_build* b) {
                                   scratch_for(b, scan_scratch_bytes<uint64_t>(nn)), st);
       ph_begin(b, PH_NIX);
       build_node_index<W>(b, b->st, nn, b->klo.as<uint64_t>(), W == 2 ? b->khi.as<uint64_t>() : nullptr,
-                          b->msk.as<uint32_t>(), 0u, 256u);
+                          b->msk.as<uint32_t>(), toph.data(), 0u, 256u);
       ph_end(b, PH_NIX);
       GX_HIP(hipStreamSynchronize(st));
       ph_collect(b, true);
@@ -5943,7 +5938,7 @@ static void compact_graph(gx_build* b, uint32_t* keep, const AddedHeads& ah) {
   b->nnodes = nn2;
   b->nuheads = nh2;
   build_node_index<W>(b, b->st, nn2, b->klo.as<uint64_t>(), W == 2 ? b->khi.as<uint64_t>() : nullptr, b->msk.as<uint32_t>(),
-                      0, 256);
+                      kNoCounts, 0, 256);
   run_unitigs<W>(b);
 }
 

@@ -255,3 +255,33 @@ def test_large_pass_three_byte_buckets(gx, k):
         assert b.part_bytes(0) == one
         b.run_unitigs()
         assert b.unitig_count() == nu
+
+
+@pytest.mark.parametrize("k,n", [(21, 4_400_000), (33, 2_300_000)])
+def test_narrow_range_of_full_buckets(gx, k, n):
+    """A key range of one top byte that holds more records per two-byte bucket
+    than a block sorts, and more nodes than a block's index table: three-byte
+    buckets for the records and the range's node index (which the read heads
+    are found through), with the one-pass build's bytes and unitigs."""
+    import numpy as np
+    rng = np.random.default_rng(n + k)
+    codes = rng.integers(0, 4, (n, k + 1), dtype=np.uint8)
+    codes[:, :4] = [0, 0, 1, 0]
+    codes[:, -2:] = 0  # the reverse complement starts with TT: read forward
+    ids = np.arange(n)[:, None] // 10 ** np.arange(6, -1, -1) % 10 + 48
+    row = np.concatenate([ids.astype(np.uint8), np.full((n, 1), 9, np.uint8),
+                          np.frombuffer(b"ACGT", np.uint8)[codes], np.full((n, 1), 10, np.uint8)], axis=1)
+    text = row.tobytes()
+    with gx.GraphBuilder(k) as b:
+        b.add_reads(text)
+        b.finish()
+        assert b.stats()["key_ranges"] == 1
+        one, uone = b.part_bytes(0), b.unitigs()
+        b.reset()
+        b.set_stream(range_occurrences=n)
+        b.add_reads(text)
+        b.finish()
+        st = b.stats()
+        assert st["key_ranges"] > 1 and st["oversized_bucket_records"] == 0
+        assert b.part_bytes(0) == one
+        assert b.unitigs() == uone

@@ -4080,7 +4080,7 @@ struct gx_build {
   DevBuf ppid, pidx, ppid2, pidx2, pbound;
   DevBuf sva, svb;  // sorted aggregation: record neighbour codes
   DevBuf nix_dir, nix_slots;  // key -> node index
-  DevBuf rtab;                // replay transitions by hash bits (k_replay_table), the same for every build
+  FilledOnce<DevBuf> rtab;    // replay transitions by hash bits (k_replay_table), the same for every build
   DevBuf rcode;               // replay codes, one byte per record in node order
   DevBuf u_seqat;             // unitig pass: byte position of long sequences
   DevBuf u_hbytes;            // unitig pass: record bytes of the heads before each head
@@ -4359,7 +4359,6 @@ static NodeIndex build_node_index(gx_build* b, hipStream_t st, uint64_t nn, cons
   return NodeIndex{ndir, nslots, nb, nbk, xbkb};
 }
 
-// Device bytes the handle holds (all of its buffers).
 // Every device buffer of a handle.
 template <class F>
 static void for_each_buf(gx_build* b, F&& f) {
@@ -4384,25 +4383,26 @@ static void for_each_buf(gx_build* b, F&& f) {
         &b->bb_addu, &b->bb_addf, &b->bb_cur, &b->bb_tot, &b->bb_astart, &b->bb_hnode, &b->bb_hmv, &b->bb_hofs,
         &b->bb_aval, &b->bb_aoff, &b->u_headat, &b->s_acc, &b->s_k1, &b->s_k2,
         &b->s_v1, &b->s_v2, &b->s_flag, &b->s_pos, &b->s_bval, &b->s_bst, &b->s_out, &b->u_walk, &b->u_walk2,
-        &b->u_ends})
+        &b->u_ends, &b->rtab.buf})
     f(d);
 }
 
+// Device bytes the handle holds (all of its buffers).
 static size_t handle_bytes(gx_build* b) {
   size_t s = 0;
   for_each_buf(b, [&](DevBuf* d) { s += d->cap; });
   return s;
 }
 
-// At the start of a build every buffer but the input is the last build's
-// and may be freed when an allocation would otherwise fail; a buffer the
+// At the start of a build every buffer but the input and the replay table is
+// the last build's and may be freed when an allocation would otherwise fail; a buffer the
 // build uses leaves the list on its first use (DevBuf::ensure).
 static void results_dead(gx_build* b) {
   auto& dead = b->reclaim.dead;
   dead.clear();
   for_each_buf(b, [&](DevBuf* d) {
     if (d != &b->text && d != &b->text2 && d != &b->rtext && d != &b->fterm1 && d != &b->fterm2 && d != &b->fsz &&
-        d != &b->foff && d->p)
+        d != &b->foff && d != &b->rtab.buf && d->p)
       dead.push_back(d);
   });
 }
@@ -4541,14 +4541,14 @@ static void run_build(gx_build* b) {
                                 &b->c_msk,  &b->c_hcu, &b->c_hcf, &b->c_uval};
   const double tiles = (double)((N + kOccTile - 1) / kOccTile);
   // HBM a pass may use: free now plus what this handle holds beyond the
-  // parsed reads (its buffers from an earlier build are reused) and beyond
-  // `kept` bytes this build holds for later, less a margin
+  // parsed reads and the replay table (its buffers from an earlier build are
+  // reused) and beyond `kept` bytes this build holds for later, less a margin
   auto pass_budget = [&](double kept) {
     size_t fr = 0, tot = 0;
     GX_HIP(hipMemGetInfo(&fr, &tot));
     size_t live = 0;
     for (DevBuf* d : {&b->text, &b->text2, &b->rtext, &b->term, &b->rid, &b->mstart, &b->mlen, &b->wbase,
-                      &b->words, &b->valid, &b->nocc, &b->occbase, &b->hidx})
+                      &b->words, &b->valid, &b->nocc, &b->occbase, &b->hidx, &b->rtab.buf})
       live += d->cap;
     return (double)fr + (double)handle_bytes(b) - (double)live - kept - 0.1 * (double)tot - 48.0 * (double)nheads -
            16.0 * 256.0 * tiles;
@@ -5002,14 +5002,13 @@ static void run_build(gx_build* b) {
         rv = rv2;
       }
     }
-    if (!b->rtab.p) {
-      buf<uint8_t>(b->rtab, (size_t)kReplayRows * kReplayRow);
-      hipLaunchKernelGGL(k_replay_table, dim3(1024), dim3(kBlock), 0, st, b->rtab.as<uint8_t>());
+    const uint8_t* rtab = static_cast<const uint8_t*>(b->rtab.get((size_t)kReplayRows * kReplayRow, [&](void* p) {
+      hipLaunchKernelGGL(k_replay_table, dim3(1024), dim3(kBlock), 0, st, static_cast<uint8_t*>(p));
       GX_HIP(hipGetLastError());
-    }
+    }));
     ph_begin(b, PH_KREPLAY);
     hipLaunchKernelGGL(k_replay<W>, dim3(grid_for(nent, 64, 1u << 16)), dim3(64), 0, st, nent, rk, rv, rseg, rbytes, klo,
-                       khi, b->rtab.as<uint8_t>(), k, nb, lists);
+                       khi, rtab, k, nb, lists);
     GX_HIP(hipGetLastError());
     ph_end(b, PH_KREPLAY);
   }

@@ -2,9 +2,28 @@
 // can be checked without a GPU.
 #pragma once
 
+#include <cstddef>
 #include <cstdint>
 
 namespace gx {
+
+// A buffer that is filled once and kept.  It counts as filled only after its
+// fill returned: one that threw (a failed launch) is run again.
+template <class Buf>
+struct FilledOnce {
+  Buf buf;
+  bool filled = false;
+  template <class Fill>
+  void* get(size_t bytes, Fill&& fill) {
+    if (!buf.p) filled = false;
+    void* p = buf.ensure(bytes);
+    if (!filled) {
+      fill(p);
+      filled = true;
+    }
+    return p;
+  }
+};
 
 // Items (records, nodes) of the fullest key bucket among n whose keys' top
 // byte lies in [tlo, thi); a bucket is the keys that share their top `bytes`

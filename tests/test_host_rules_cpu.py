@@ -9,8 +9,33 @@ import pytest
 from .conftest import ROOT
 
 SHIM = r"""
+#include <cstdlib>
+#include <stdexcept>
 #include "gx_host.h"
+struct Heap {
+  void* p = nullptr;
+  ~Heap() { free(p); }
+  void* ensure(size_t n) { return p ? p : p = malloc(n); }
+};
 extern "C" {
+// A fill that throws at its first `fails` calls: its calls after `gets`
+// requests of the buffer, whose last must have succeeded.
+int fill_calls(int fails, int gets) {
+  gx::FilledOnce<Heap> t;
+  int calls = 0, ok = 0;
+  for (int i = 0; i < gets; i++) {
+    ok = 0;
+    try {
+      char* p = (char*)t.get(16, [&](void* q) {
+        if (calls++ < fails) throw std::runtime_error("launch");
+        *(char*)q = 7;
+      });
+      ok = *p == 7;
+    } catch (const std::runtime_error&) {
+    }
+  }
+  return ok ? calls : -1;
+}
 int record_bytes(int words, int key_bytes, uint64_t n, const uint64_t* top, unsigned lo, unsigned hi) {
   return gx::record_bucket_bytes(words, key_bytes, n, top, lo, hi);
 }
@@ -106,3 +131,11 @@ def test_bucket_bytes_of_an_empty_range(rules):
     top = _top([0] * 128 + [10] * 128)
     assert rules.record_bytes(1, 8, 0, top, 0, 64) == 2
     assert rules.fullest(0, 2, top, 0, 64) == 0
+
+
+@pytest.mark.parametrize("fails", [0, 1, 3])
+def test_buffer_filled_once(rules, fails):
+    """A fill that failed is run again by the next request, one that returned
+    is not."""
+    assert rules.fill_calls(fails, fails + 1) == fails + 1
+    assert rules.fill_calls(fails, fails + 4) == fails + 1

@@ -2877,7 +2877,6 @@ __device__ inline int back_side(uint32_t t) { return (t == ET_FF || t == ET_RF) 
 // walked, or the end of a node that merges with nothing.
 constexpr uint64_t kEndUnvisited = ~0ull, kEndSingle = ~0ull - 1;
 constexpr uint32_t kCovMax = 1u << 24;  // coverage saturates like the reference's float sums
-constexpr uint32_t kWalkCap = 1024;  // claims of one walk; a longer path is ranked by walks between splitters
 
 // Neighbour y of k-mer v (reverse complement rv) for mask bit 4t + x:
 // FF w[1:]+x, FR rc(w[1:]+x) = comp(x)+rc(w)[:-1], RF rc(x+w[:-1]) =
@@ -3077,7 +3076,7 @@ __global__ void k_walk_list(uint64_t nn, const uint32_t* __restrict__ endpoint, 
 __global__ void __launch_bounds__(kBlock) k_walk(uint32_t nwalk, const uint32_t* __restrict__ walkers,
                                                  uint4* __restrict__ E, uint64_t* __restrict__ claim,
                                                  uint64_t* __restrict__ met, uint64_t* __restrict__ wcov,
-                                                 uint32_t* __restrict__ capped) {
+                                                 uint32_t cap, uint32_t* __restrict__ capped) {
   for (uint32_t w = blockIdx.x * blockDim.x + threadIdx.x; w < nwalk; w += gridDim.x * blockDim.x) {
     uint32_t e = walkers[w], idx = 0, mn = 0x7fffffffu, mn_rev = 0;
     uint64_t other = ~0ull, cov = 0;
@@ -3099,7 +3098,7 @@ __global__ void __launch_bounds__(kBlock) k_walk(uint32_t nwalk, const uint32_t*
       idx++;
       cov += q.y;
       if (x == kEnd) break;
-      if (idx >= kWalkCap) {
+      if (idx >= cap) {
         *capped = 1u;
         break;
       }
@@ -5378,7 +5377,7 @@ static void run_unitigs(gx_build* b) {
         // one resident wave set, each lane walking ~a dozen paths in turn: a
         // wave then waits for the longest of its lanes' sums, not of single paths
         hipLaunchKernelGGL(k_walk, dim3(grid_for(nw, kBlock, G)), dim3(kBlock), 0, st, (uint32_t)nw, walkers, E, claim,
-                           met, wcov, ws);
+                           met, wcov, walk_cap(nn), ws);
         GX_HIP(hipGetLastError());
         hipLaunchKernelGGL(k_walk_join, dim3(grid_for(nw, kBlock, G)), dim3(kBlock), 0, st, (uint32_t)nw, claim, met,
                            wcov, sum, pcov);

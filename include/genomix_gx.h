@@ -130,11 +130,11 @@ int gx_unitig_emit(gx_build* b, uint8_t* dst, size_t cap, size_t* written);
 /* How the unitig pass ranks the nodes of its merge paths:
  * GX_RANK_AUTO (default) walks each path from both its endpoints toward
  * each other when k is odd; graphs of long paths (more than 64 nodes on
- * average, or a walk of more than 1024) are walked between splitter nodes,
- * whose chains are ranked by pointer jumping.  It falls back to pointer
- * jumping over every node for even k (palindromic k-mers) and cycles;
- * GX_RANK_POINTER_JUMPING always uses that.  The records are the same
- * either way. */
+ * average, or a walk of more than 1024 to 4096, by the graph's size) are
+ * walked between splitter nodes, whose chains are ranked by pointer jumping.
+ * It falls back to pointer jumping over every node for even k (palindromic
+ * k-mers) and cycles; GX_RANK_POINTER_JUMPING always uses that.  The records
+ * are the same either way. */
 #define GX_RANK_AUTO 0
 #define GX_RANK_POINTER_JUMPING 1
 int gx_unitig_set_ranking(gx_build* b, int mode);

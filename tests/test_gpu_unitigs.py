@@ -269,3 +269,54 @@ def test_head_keys_wider_than_a_word(gx):
     top = (1 << 29) - 1
     text = "".join(f"{top - 3 * i}\t{s if rng.random() < 0.5 else rc(s)}\n" for i, s in enumerate(reads)).encode()
     check(gx, text, k)
+
+
+def _short_and_long_paths(rng, k, short, long):
+    """Reads of a graph of linear paths: genomes of `short` letters in one read
+    each, and one of `long` letters."""
+    lines = ["".join(rng.choices("ACGT", k=n)) for n in short]
+    g = "".join(rng.choices("ACGT", k=long))
+    lines += [g[p:p + 100] for p in range(0, long - 99, 40)] + [g[-100:]]
+    return "".join(f"{4 * i + 2}\t{s if rng.random() < 0.5 else rc(s)}\n" for i, s in enumerate(lines)).encode()
+
+
+@pytest.mark.parametrize("k", [21, 33])
+def test_walks_that_meet_their_cap(gx, k):
+    """A low mean length with one long path: the walks from the paths' ends
+    start, one meets its cap, and the graph is ranked again between
+    splitters."""
+    rng = random.Random(k)
+    paths = 301
+    text = _short_and_long_paths(rng, k, [k + 39] * (paths - 1), 5200)
+    outs = []
+    for mode in ("auto", "pointer_jumping"):
+        with gx.GraphBuilder(k) as b:
+            b.set_ranking(mode)
+            b.add_reads(text)
+            b.finish()
+            outs.append(b.unitigs())
+            st = b.stats()
+            if mode == "auto":
+                assert b.unitig_count() == paths and st["distinct"] <= 64 * paths  # the walks are tried first
+                assert st["pj_rounds"] > 0  # over the splitters
+                assert 4 * paths < st["walkers"] < st["distinct"]  # two per splitter, every path's ends among them
+    assert outs[0] == outs[1]
+    assert outs[0] == oracle.unitigs(oracle.build_graph(text, k)[0], k)
+
+
+def test_long_path_of_a_large_graph_is_walked(gx):
+    """Ranking the whole of a large graph anew costs more than walking one path
+    of a few thousand nodes: no splitters."""
+    rng = random.Random(11)
+    k = 21
+    text = _short_and_long_paths(rng, k, [70] * 170_000, 2300)
+    outs = []
+    for mode in ("auto", "pointer_jumping"):
+        with gx.GraphBuilder(k) as b:
+            b.set_ranking(mode)
+            b.add_reads(text)
+            b.finish()
+            outs.append(b.unitigs())
+            if mode == "auto":
+                assert b.stats()["distinct"] > 8_400_000 and b.stats()["pj_rounds"] == 0
+    assert outs[0] == outs[1]

@@ -42,6 +42,7 @@ int record_bytes(int words, int key_bytes, uint64_t n, const uint64_t* top, unsi
 int index_bytes(int key_bytes, uint64_t n, const uint64_t* top, unsigned lo, unsigned hi) {
   return gx::index_bucket_bytes(key_bytes, n, top, lo, hi);
 }
+unsigned walk_cap(uint64_t nodes) { return gx::walk_cap(nodes); }
 double fullest(uint64_t n, int bytes, const uint64_t* top, unsigned lo, unsigned hi) {
   return gx::fullest_bucket(n, bytes, top, lo, hi);
 }
@@ -61,6 +62,7 @@ def rules(tmp_path_factory):
     u64, u64p, u32, i32 = ctypes.c_uint64, ctypes.POINTER(ctypes.c_uint64), ctypes.c_uint, ctypes.c_int
     L.record_bytes.argtypes = [i32, i32, u64, u64p, u32, u32]
     L.index_bytes.argtypes = [i32, u64, u64p, u32, u32]
+    L.walk_cap.argtypes = [u64]
     L.fullest.argtypes = [u64, i32, u64p, u32, u32]
     L.fullest.restype = ctypes.c_double
     return L
@@ -139,3 +141,10 @@ def test_buffer_filled_once(rules, fails):
     is not."""
     assert rules.fill_calls(fails, fails + 1) == fails + 1
     assert rules.fill_calls(fails, fails + 4) == fails + 1
+
+
+def test_walk_cap(rules):
+    """Large graphs walk paths of 8192 nodes from both ends; small ones turn to
+    the splitters after 1024 nodes a walk."""
+    assert [rules.walk_cap(n) for n in (0, 1, 4096 * 1024, 4096 * 1025, 4096 * 4096, 1 << 30)] == [
+        1024, 1024, 1024, 1025, 4096, 4096]

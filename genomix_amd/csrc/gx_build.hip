@@ -5320,8 +5320,9 @@ static void run_unitigs(gx_build* b) {
       f.wait();
       wr[0] = w[0];
       wr[1] = w[1];
-      b->u_walkers = nwalk;
-      return wr[0] == 0 && wr[1] == 0;
+      const bool all = wr[0] == 0 && wr[1] == 0;
+      if (all) b->u_walkers = nwalk;
+      return all;
     };
     auto walk_splits = [&] {
       uint32_t* flag = upos;  // until k_walk_final

@@ -320,3 +320,22 @@ def test_long_path_of_a_large_graph_is_walked(gx):
             if mode == "auto":
                 assert b.stats()["distinct"] > 8_400_000 and b.stats()["pj_rounds"] == 0
     assert outs[0] == outs[1]
+
+
+def test_walkers_of_the_ranking_that_was_used(gx):
+    """The count of walks is that of the walks that ranked the graph: none
+    where a circular genome beside linear ones is left to pointer jumping."""
+    rng = random.Random(78)
+    k = 21
+    genome = "".join(rng.choices("ACGT", k=3000))
+    line = "".join(rng.choices("ACGT", k=1500))
+    for g, walked in ((genome, True), (genome + genome[:200], False)):
+        reads = [s[p:p + 120] for s in (g, line) for p in range(0, len(s) - 119, 40)]
+        text = "".join(f"{4 * i + 2}\t{s}\n" for i, s in enumerate(reads)).encode()
+        with gx.GraphBuilder(k) as b:
+            b.add_reads(text)
+            b.finish()
+            got = b.unitigs()
+            st = b.stats()
+            assert (st["walkers"] > 0) == walked and st["pj_rounds"] > 0
+        assert got == oracle.unitigs(oracle.build_graph(text, k)[0], k)

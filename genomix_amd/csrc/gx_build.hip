@@ -590,32 +590,6 @@ __device__ inline uint64_t table_insert(void* table, uint64_t cap, KV key, uint6
 
 constexpr uint32_t kEnd = 0xffffffffu;
 
-// Read-only lookup of a key that is known to be in the table.
-template <int W>
-__device__ inline uint64_t table_find(const void* table, uint64_t cap, KV key) {
-  uint64_t s = slot_home(khash<W>(key), cap);
-  for (uint64_t probe = 0; probe < cap; probe++) {
-    if (W == 1) {
-      uint64_t cur = ((const Slot1*)table)[s].key;
-      if (cur == key.lo) return s;
-      if (cur == kEmpty) return ~0ull;
-    } else {
-      uint64_t cur = ((const Slot2*)table)[s].hi;
-      if (cur == key.hi && ((const Slot2*)table)[s].lo == key.lo) return s;
-      if (cur == kEmpty) return ~0ull;
-    }
-    s = slot_next(s, cap);
-  }
-  return ~0ull;
-}
-
-template <int W>
-__device__ inline uint32_t node_of_key(const void* table, uint64_t cap, KV key) {
-  uint64_t s = table_find<W>(table, cap, key);
-  if (s == ~0ull) return kEnd;
-  return W == 1 ? ((const Slot1*)table)[s].count : ((const Slot2*)table)[s].count;
-}
-
 template <int W>
 __device__ inline KV node_key(const uint64_t* klo, const uint64_t* khi, uint64_t i) {
   KV v;
@@ -2048,38 +2022,6 @@ __global__ void k_set_u64(uint64_t* p, uint64_t v) {
 __global__ void k_node_cnt(uint64_t nn, const uint64_t* __restrict__ nstart, uint32_t* __restrict__ cnt) {
   for (uint64_t n = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; n < nn; n += (uint64_t)gridDim.x * blockDim.x)
     cnt[n] = (uint32_t)(nstart[n + 1] - nstart[n]);
-}
-
-// Key -> node lookup table (the unitig pass and the read heads find nodes
-// by key): distinct keys, so a failed claim always means another key.
-template <int W>
-__global__ void k_node_table(uint64_t nn, const uint64_t* __restrict__ klo, const uint64_t* __restrict__ khi,
-                             void* table, uint64_t cap, unsigned long long* err) {
-  for (uint64_t n = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; n < nn; n += (uint64_t)gridDim.x * blockDim.x) {
-    KV key = node_key<W>(klo, khi, n);
-    uint64_t s = slot_home(khash<W>(key), cap);
-    bool done = false;
-    for (uint64_t probe = 0; probe < cap && !done; probe++) {
-      if (W == 1) {
-        Slot1* T = (Slot1*)table;
-        if (atomicCAS((unsigned long long*)&T[s].key, (unsigned long long)kEmpty, (unsigned long long)key.lo) ==
-            kEmpty) {
-          T[s].count = (uint32_t)n;
-          done = true;
-        }
-      } else {
-        Slot2* T = (Slot2*)table;
-        if (atomicCAS((unsigned long long*)&T[s].hi, (unsigned long long)kEmpty, (unsigned long long)key.hi) ==
-            kEmpty) {
-          T[s].lo = key.lo;
-          T[s].count = (uint32_t)n;
-          done = true;
-        }
-      }
-      s = slot_next(s, cap);
-    }
-    if (!done) report(err, ~0ull >> 8, ERR_TABLE);
-  }
 }
 
 // Sorted node keys must be strictly increasing: one key in two table

@@ -4283,12 +4283,15 @@ static NodeIndex build_node_index(gx_build* b, hipStream_t st, uint64_t nn, cons
     hipLaunchKernelGGL(k_nix_dir<W>, dim3(grid_for(nn + 1, kBlock, G)), dim3(kBlock), 0, st, nn, klo, khi, nb, xbkb, xb0,
                        xb1, ndir);
   GX_HIP(hipGetLastError());
-  // buckets per block: as many as fill the small table, but at least 512
-  // blocks; the large table (two blocks per CU) where a bucket a quarter above
+  // buckets per block: as many as fill half of the small table, but at least
+  // 512 blocks (the whole table gains nothing for buckets of up to 60 nodes,
+  // a block's threads have enough to do, and fuller ones are better off alone:
+  // two-word buckets of about 300 nodes, 4.5 G in all, 113-118 ms against
+  // 107); the large table (two blocks per CU) where a bucket a quarter above
   // the fullest would not fit the small one
   const uint64_t per = std::max<uint64_t>(1, (uint64_t)(2.5 * fullest_bucket(nn, xbkb, top, tlo, thi)));
   uint32_t span = 1;
-  while ((uint64_t)span * 2 * per <= kNixSmall && (xb1 - xb0) / (span * 2) >= 512) span *= 2;
+  while ((uint64_t)span * 4 * per <= kNixSmall && (xb1 - xb0) / (span * 2) >= 512) span *= 2;
   const unsigned blocks = std::min((xb1 - xb0 + span - 1) / span, 65536u);
   if (per <= kNixSmall)
     hipLaunchKernelGGL((k_nix_build<W, kNixSmall, 512>), dim3(blocks), dim3(512), 0, st, klo, khi, msk, ndir, nslots,

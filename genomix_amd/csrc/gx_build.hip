@@ -894,11 +894,12 @@ __global__ void k_compact_list(const void* table, const uint32_t* __restrict__ c
 // node's output rank once its count has been copied out.
 // ---------------------------------------------------------------------------
 // 4'-5'. Sort-partitioned aggregation (the default method).  Every k-mer
-//    occurrence becomes a record (KmerPointable sort key, occurrence index
-//    << 8 | code); the records are sorted by (key, occurrence): two stable
-//    8-bit radix passes on the top 16 key bits -- the first fused with the
-//    k-mer extraction -- then a bitonic sort of each 16-bit bucket in LDS
-//    (buckets above bucket_cap records go through a global radix sort).
+//    occurrence becomes a record (KmerPointable sort key, neighbour code);
+//    the records are sorted by (key, occurrence): stable 8-bit radix passes
+//    on the top 16 key bits (24 where those buckets would outgrow LDS) -- the
+//    first fused with the k-mer extraction -- then each bucket by itself, in
+//    registers and LDS (buckets above bucket_cap records go through a global
+//    radix sort).
 //    Nodes are the runs of equal keys, already in output order; a run's
 //    codes are its occurrences' records in emission order, as the JDK-7
 //    replay needs them.  All HBM traffic is streaming; there is no
@@ -2099,7 +2100,7 @@ __global__ void __launch_bounds__(kBlock) k_node_info(uint64_t nn, const uint32_
   uint64_t all;
   (void)block_exclusive_scan<uint64_t>(rec, &all);
   if (threadIdx.x == 0 && all) atomicAdd(&tot[0], (unsigned long long)all);
-  (void)block_exclusive_scan<uint64_t>((nodes << 32) | entries, &all);  // at most 4 * 2^30 / blocks entries each
+  (void)block_exclusive_scan<uint64_t>((nodes << 32) | entries, &all);  // fits: 2^32 nodes over at least 64 blocks
   if (threadIdx.x == 0 && all) {
     atomicAdd(&tot[1], (unsigned long long)(all >> 32));
     atomicAdd(&tot[2], (unsigned long long)(all & 0xffffffffull));
@@ -3726,8 +3727,8 @@ __global__ void k_useq_size(USerCtx c, uint64_t* __restrict__ rsize) {
 }
 
 // Sequences longer than kUseqLong bases are written by k_useq_long (a wave
-// per unitig, lanes over bytes); k_useq_write leaves their bytes to it and
-// records where they start.
+// per chunk of 64 bytes); k_useq_write leaves their bytes to it and records
+// where they start.
 constexpr uint64_t kUseqLong = 128;
 
 template <int W>

@@ -339,7 +339,8 @@ __device__ __host__ inline uint32_t key_byte(const Key128& k, int b) {
 
 // A tile of the sort: kSortThreads threads with kPer elements each.  4096
 // elements over 256 digits leave runs of 16 on average, 128 bytes of 8-byte
-// keys (2048 left half a line each and twice the digit counts to scan).
+// keys (2048 left half a line each and twice the digit counts to scan); of
+// 16-byte keys 2048 do.
 constexpr int kSortThreads = 512, kSortWaves = kSortThreads / 64;
 template <class KeyT>
 struct SortTile {
